@@ -100,9 +100,6 @@ struct Ctx {
   bool prof_count = false;  // kernels with a byte model count their bytes (extra device work)
   void* pinned = nullptr;  // small pinned host buffer for scalar read-backs (allocated on first use)
   Tuning tune;
-  // device bytes the refinement's inbound-set event stage may take at once (0: half of what
-  // the device has free, cached blocks included)
-  uint64_t event_budget = 0;
   // side streams for independent kernels of one stage (created on first use, default priority)
   static constexpr int SIDES = 3;
   hipStream_t side[SIDES] = {};

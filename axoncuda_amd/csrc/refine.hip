@@ -54,14 +54,13 @@ __device__ __forceinline__ uint64_t ordered_i64(int64_t g) { return (uint64_t)g 
 
 // ---- 1. per-hedge partition lists ------------------------------------------------------
 // Per-hedge partition lists for hedges of at most PP_SMALL pins (one thread per hedge).
-// With INB, also the destination counts and the per-partition inbound sizes; those are
-// aggregated in an LDS histogram when the partition count fits it (k_lds > 0), so a few
+// With INB, also the per-partition inbound sizes; those are aggregated in an LDS histogram when the partition count fits it (k_lds > 0), so a few
 // hot partitions do not serialize millions of global atomics.
 template <bool INB>
 __global__ void __launch_bounds__(256) k_pp_small(const uint32_t* __restrict__ hedges, const uint64_t* __restrict__ hoff,
                                                   const uint32_t* __restrict__ srcc, const uint32_t* __restrict__ part,
                                                   const float* __restrict__ w, uint32_t E, uint2* __restrict__ pp,
-                                                  uint32_t* __restrict__ pp_dcnt, uint32_t* __restrict__ lambda,
+                                                  uint32_t* __restrict__ lambda,
                                                   uint4* __restrict__ hinfo, uint32_t* __restrict__ large_flag,
                                                   uint32_t* inbsz, uint32_t k_lds) {
   extern __shared__ uint32_t hist[];
@@ -136,12 +135,9 @@ __global__ void __launch_bounds__(256) k_pp_small(const uint32_t* __restrict__ h
       for (uint32_t k = 0; k < PP_SMALL; ++k) {
         if (k < m) {
           pp[s + k] = make_uint2(qs[k], cs[k]);
-          if (INB) {
-            pp_dcnt[s + k] = ds[k];
-            if (ds[k]) {
-              if (k_lds) atomicAdd(&hist[qs[k]], 1u);
-              else atomicAdd(&inbsz[qs[k]], 1u);
-            }
+          if (INB && ds[k]) {
+            if (k_lds) atomicAdd(&hist[qs[k]], 1u);
+            else atomicAdd(&inbsz[qs[k]], 1u);
           }
         }
       }
@@ -178,8 +174,8 @@ __global__ void __launch_bounds__(64) k_pp_large(const uint32_t* __restrict__ he
                                                  const float* __restrict__ w,
                                                  const uint32_t* __restrict__ list, uint32_t cap, uint32_t k,
                                                  const uint64_t* __restrict__ goff, uint32_t* __restrict__ gtab,
-                                                 uint2* __restrict__ pp, uint32_t* __restrict__ pp_dcnt,
-                                                 uint32_t* __restrict__ lambda, uint4* __restrict__ hinfo,
+                                                 uint2* __restrict__ pp, uint32_t* __restrict__ lambda,
+                                                 uint4* __restrict__ hinfo,
                                                  uint32_t* inbsz) {
   extern __shared__ uint32_t lds[];
   const uint32_t e = list[blockIdx.x];
@@ -264,7 +260,6 @@ __global__ void __launch_bounds__(64) k_pp_large(const uint32_t* __restrict__ he
   const uint64_t s0 = s;
   for (uint32_t o = l; o < base; o += 64) {
     pp[s0 + o] = make_uint2(ld(&keys[o]), ld(&cnt[o]));
-    if (INB) pp_dcnt[s0 + o] = ld(&dcnt[o]);
   }
   if (l == 0) {
     lambda[e] = base;
@@ -1453,7 +1448,7 @@ __global__ void k_compact_u64(const uint32_t* __restrict__ flag, const uint64_t*
 // then pins and weights at the scanned offsets
 // The small-hedge CSR: hedge i (hedge keys[i], or i without keys) keeps its pins from a
 // multiple of 4, padded to a multiple of 4 with its last pin, so a thread loads them as 16-byte
-// vectors; its record is start << 5 | length (lengths 2..16).
+// vectors; its record is start << 10 | sources << 5 | length (lengths 1..16).
 __device__ __forceinline__ uint32_t small_hedge_id(const uint64_t* keys, uint32_t i) {
   return keys ? (uint32_t)keys[i] : i;
 }
@@ -1466,7 +1461,7 @@ __global__ void k_small_lens(const uint64_t* __restrict__ keys, uint32_t m, cons
 }
 __global__ void k_small_fill(const uint64_t* __restrict__ keys, uint32_t m, const uint64_t* __restrict__ hoff,
                              const uint32_t* __restrict__ hedges, const float* __restrict__ w,
-                             uint64_t* __restrict__ rec, uint32_t* __restrict__ pins, float* __restrict__ sw) {
+                             const uint32_t* __restrict__ srcc, uint64_t* __restrict__ rec, uint32_t* __restrict__ pins, float* __restrict__ sw) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= m) return;
   const uint32_t e = small_hedge_id(keys, i);
@@ -1474,7 +1469,7 @@ __global__ void k_small_fill(const uint64_t* __restrict__ keys, uint32_t m, cons
   for (uint64_t j = 0; j < len; ++j) pins[o + j] = hedges[s + j];
   for (uint64_t j = len; j < ((len + 3) & ~3ull); ++j) pins[o + j] = hedges[s + len - 1];
   sw[i] = w[e];
-  rec[i] = (o << 5) | len;
+  rec[i] = (o << 10) | ((uint64_t)(srcc ? srcc[e] : 0u) << 5) | len;
 }
 __global__ void k_compact(const uint32_t* __restrict__ flag, const uint64_t* __restrict__ pos, uint32_t n,
                           uint32_t* __restrict__ out) {
@@ -1808,6 +1803,10 @@ struct CascadeArgs {
   const uint2* pm2;
   int incc;
   unsigned long long* seq;
+  // inbound-constrained mode only: source counts, and per rank the hedges whose destinations
+  // leave (low word) and enter (high word) a partition with that move (see k_inbound_deltas)
+  const uint32_t* srcc;
+  unsigned long long* dio;
 };
 constexpr uint32_t PM2_MAX_K = 0xFFFFu;  // partition ids < 0xFFFF leave 0xFFFF for "no move"
 
@@ -1846,17 +1845,18 @@ __device__ __forceinline__ int64_t cascade_term(int incc, int64_t W, int64_t cp,
   return t;
 }
 
-// Cascade classes of a level's hedges: 2..CAS_SMALL pins (the thread-per-hedge kernel; the
+// Cascade classes of a level's hedges: min_len..CAS_SMALL pins (the thread-per-hedge kernel; the
 // key orders them by their first pin), the sorted kernels (up to CAS_SORT_S or sort_max
-// pins) and the direct LDS/HBM kernel.  A hedge of one pin adds nothing: its pin finds itself
-// alone in p and nobody in q, so the two terms of cascade_term cancel.
+// pins) and the direct LDS/HBM kernel.  A hedge of one pin adds nothing to the cascade: its pin
+// finds itself alone in p and nobody in q, so the two terms of cascade_term cancel.  It does
+// count for the inbound sets, so min_len is 2 in k-way mode and 1 in inbound-constrained mode.
 __global__ void k_cascade_classes(const uint32_t* __restrict__ hedges, const uint64_t* __restrict__ hoff, uint32_t E,
-                                  uint32_t sort_max, uint32_t* __restrict__ f_small, uint64_t* __restrict__ k_small,
+                                  uint32_t min_len, uint32_t sort_max, uint32_t* __restrict__ f_small, uint64_t* __restrict__ k_small,
                                   uint32_t* __restrict__ f_s, uint32_t* __restrict__ f_m, uint32_t* __restrict__ f_big) {
   const uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= E) return;
   const uint64_t s = hoff[e], hl = hoff[e + 1] - s;
-  const bool small = hl >= 2 && hl <= CAS_SMALL;
+  const bool small = hl >= min_len && hl <= CAS_SMALL;
   const bool sorted = hl > CAS_SMALL && hl <= sort_max;
   f_small[e] = small ? 1u : 0u;
   k_small[e] = small ? ((uint64_t)hedges[s] << 32) | e : 0ull;
@@ -1869,7 +1869,7 @@ __global__ void k_cascade_classes(const uint32_t* __restrict__ hedges, const uin
 // once per level): offsets, pins and weights are read coalesced, and nearby threads gather the
 // records of nearby nodes.
 struct SmallHedges {
-  const uint64_t* rec;  // start << 5 | length; starts are multiples of 4
+  const uint64_t* rec;  // start << 10 | sources << 5 | length; starts are multiples of 4
   const uint32_t* pins;
   const float* w;
   uint32_t m;
@@ -1880,13 +1880,18 @@ struct SmallHedges {
 // P16 (packed records, k < PM2_MAX_K): a pin's partition and target stay packed in one
 // register (partition | target << 16, 0xFFFF = none), so the pins take 32 registers instead
 // of 48 and more waves fit on a SIMD.
-template <bool P16>
+// INCC: a moving destination pin also counts the hedge's destinations in its source partition
+// and its target just before the move.  The hedge leaves the source's inbound set when they are
+// all this node (a hedge that lists a node twice counts it once, at the first of its pins), and
+// enters the target's when there are none: one 64-bit atomic per pin that changes either.
+template <bool P16, bool INCC>
 __global__ void k_cascade_small(CascadeArgs a, SmallHedges h) {
   const uint32_t i = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
   if (i >= h.m) return;
   const uint64_t rec = h.rec[i];
-  const uint64_t s = rec >> 5;
+  const uint64_t s = rec >> 10;
   const uint32_t len = (uint32_t)(rec & 31u);
+  const uint32_t sc = (uint32_t)(rec >> 5) & 31u;  // pins from here on are destinations
   const uint4* p4 = reinterpret_cast<const uint4*>(h.pins + s);  // 16-byte aligned: s % 4 == 0
   // per pin: partition (with P16 also the target), target, rank
   uint32_t pt[CAS_SMALL], mv[P16 ? 1 : CAS_SMALL], rk[CAS_SMALL];
@@ -1955,6 +1960,8 @@ __global__ void k_cascade_small(CascadeArgs a, SmallHedges h) {
     if (i < jmax && moves(i)) {
       const uint32_t p = part_of(i), q = move_of(i), r = rk[i];
       int32_t cp = 0, cq = 0;
+      uint32_t dp = 0, dq = 0, own = 0;  // destinations in p and q, and those that are this node
+      bool again = false;                // an earlier destination pin is this node
 #pragma unroll
       for (uint32_t j = 0; j < CAS_SMALL; ++j) {
         if (j < jmax) {
@@ -1962,10 +1969,24 @@ __global__ void k_cascade_small(CascadeArgs a, SmallHedges h) {
           const uint32_t now = before ? move_of(j) : part_of(j);  // its partition when pin i moves
           cp += now == p;
           cq += now == q;
+          if constexpr (INCC) {
+            const bool dst = j >= sc;
+            const bool same = dst && moves(j) && rk[j] == r;
+            dp += dst && now == p;
+            dq += dst && now == q;
+            own += same;
+            if (j < i) again |= same;
+          }
         }
       }
       const int64_t term = cascade_term(a.incc, W, cp, cq);
       if (term) atomicAdd(&a.seq[r], (unsigned long long)term);
+      if constexpr (INCC) {
+        if (i >= sc && !again) {
+          const unsigned long long io = (dp == own ? 1ull : 0ull) | (dq == 0 ? 1ull << 32 : 0ull);
+          if (io) atomicAdd(&a.dio[r], io);
+        }
+      }
     }
   }
 }
@@ -1979,7 +2000,7 @@ __global__ __launch_bounds__(256) void k_cascade_small_bytes(CascadeArgs a, Smal
   const uint32_t i0 = blockIdx.x * blockDim.x + threadIdx.x;
   uint64_t b = 0;
   if (i0 < h.m) {
-    const uint64_t s = h.rec[i0] >> 5, len = h.rec[i0] & 31u, rec = a.pm2 ? 8 : 16;
+    const uint64_t s = h.rec[i0] >> 10, len = h.rec[i0] & 31u, rec = a.pm2 ? 8 : 16;
     uint32_t moving = 0;
     for (uint64_t i = s; i < s + len; ++i) moving += pm_at(a, h.pins[i]).y != NONE;
     b = 8 + (4 + rec) * len + (moving ? 4 + 8 * (uint64_t)moving : 0);
@@ -1992,12 +2013,15 @@ __global__ __launch_bounds__(256) void k_cascade_small_bytes(CascadeArgs a, Smal
     atomicAdd(&prof[blockIdx.x % PROF_SLOTS], (unsigned long long)(part[0] + part[1] + part[2] + part[3]));
 }
 
+// INCC: as in k_cascade_small.
+template <bool INCC>
 __global__ void __launch_bounds__(64) k_cascade_large(CascadeArgs a, const uint32_t* __restrict__ list) {
   __shared__ uint32_t s_pt[CAS_LDS], s_mv[CAS_LDS], s_rk[CAS_LDS];
   const uint32_t e = list[blockIdx.x];
   const uint32_t l = lane_id();
   const uint64_t s = a.hoff[e];
   const uint32_t len = (uint32_t)(a.hoff[e + 1] - s);
+  const uint32_t sc = INCC ? a.srcc[e] : 0u;
   const bool in_lds = len <= CAS_LDS;
   bool any = false;
   if (in_lds) {
@@ -2023,8 +2047,19 @@ __global__ void __launch_bounds__(64) k_cascade_large(CascadeArgs a, const uint3
     if (q == NONE) continue;
     const uint32_t p = PT(i), r = RK(i);
     int64_t cp = 0, cq = 0;
+    uint32_t dp = 0, dq = 0, own = 0;
+    bool again = false;
     for (uint32_t j = 0; j < len; ++j) {
       const uint32_t pj = PT(j), mj = MV(j);
+      if (INCC && j >= sc) {
+        const uint32_t rj = mj != NONE ? RK(j) : NONE;
+        const uint32_t now = mj != NONE && rj < r ? mj : pj;
+        const bool same = mj != NONE && rj == r;
+        dp += now == p;
+        dq += now == q;
+        own += same;
+        if (j < i) again |= same;
+      }
       cp += pj == p;
       cq += pj == q;
       if (mj != NONE && RK(j) < r) {
@@ -2035,6 +2070,10 @@ __global__ void __launch_bounds__(64) k_cascade_large(CascadeArgs a, const uint3
       }
     }
     atomicAdd(&a.seq[r], (unsigned long long)cascade_term(a.incc, W, cp, cq));
+    if (INCC && i >= sc && !again) {
+      const unsigned long long io = (dp == own ? 1ull : 0ull) | (dq == 0 ? 1ull << 32 : 0ull);
+      if (io) atomicAdd(&a.dio[r], io);
+    }
   }
 }
 
@@ -2047,6 +2086,9 @@ __global__ void __launch_bounds__(64) k_cascade_large(CascadeArgs a, const uint3
 // c_p and c_q of the cascade term, in O(m log^2 m) for m moving pins instead of
 // O(len * m).
 // key = partition << (rb + 11) | (rank + 1) << 11 | dir << 10 | local index (dir 1 = in).
+// INCC: the same scan carries the destination pins' deltas in its high half (and the table their
+// counts), which gives the destinations in the source just before an out event and in the target
+// just before an in event; a node listed twice passes its events one after the other.
 __device__ __forceinline__ int32_t wave_seg_scan(int32_t v, bool& flag) {
   const uint32_t l = lane_id();
 #pragma unroll
@@ -2061,7 +2103,7 @@ __device__ __forceinline__ int32_t wave_seg_scan(int32_t v, bool& flag) {
   return v;
 }
 
-template <uint32_t PINS, uint32_t EVS, uint32_t NT>
+template <uint32_t PINS, uint32_t EVS, uint32_t NT, bool INCC>
 __global__ void __launch_bounds__(NT) k_cascade_sorted(CascadeArgs a, const uint32_t* __restrict__ list, int rb) {
   static_assert(EVS >= 2 * PINS && (EVS & (EVS - 1)) == 0, "two event slots per pin, a power of two");
   constexpr uint32_t HS = EVS;  // partition table: at least twice the pins, so it never fills
@@ -2069,11 +2111,13 @@ __global__ void __launch_bounds__(NT) k_cascade_sorted(CascadeArgs a, const uint
   __shared__ uint32_t s_hk[HS], s_hc[HS];
   __shared__ uint32_t s_rk[PINS];
   __shared__ int32_t s_cp[PINS], s_cq[PINS];
+  __shared__ uint8_t s_out[INCC ? PINS : 1], s_in[INCC ? PINS : 1];  // the hedge leaves / enters an inbound set
   __shared__ uint32_t s_moving;
   const uint32_t e = list[blockIdx.x];
   const uint32_t l = lane_id(), tid = threadIdx.x;
   const uint64_t s = a.hoff[e];
   const uint32_t len = (uint32_t)(a.hoff[e + 1] - s);
+  const uint32_t sc = INCC ? a.srcc[e] : 0u;
   if (tid == 0) s_moving = 0;
   for (uint32_t h = tid; h < HS; h += NT) {
     s_hk[h] = NONE;
@@ -2091,7 +2135,7 @@ __global__ void __launch_bounds__(NT) k_cascade_sorted(CascadeArgs a, const uint
       if (old == NONE || old == p) break;
       h = (h + 1) & (HS - 1);
     }
-    atomicAdd(&s_hc[h], 1u);
+    atomicAdd(&s_hc[h], INCC && i >= sc ? 0x10001u : 1u);  // INCC: destinations in the high half
     s_rk[i] = q == NONE ? NONE : q4.z;
     // event slots: one LDS atomic per wave (the lowest moving lane's), not one per moving pin
     const uint64_t mv = __ballot(q != NONE);
@@ -2140,7 +2184,10 @@ __global__ void __launch_bounds__(NT) k_cascade_sorted(CascadeArgs a, const uint
       const bool act = i < nev;
       const uint64_t key = act ? s_ev[i] : ~0ull;
       const bool dir_in = (key >> 10) & 1u;
-      const int32_t d = !act ? 0 : (dir_in ? 1 : -1);
+      const uint32_t idx = (uint32_t)(key & 1023u);
+      const bool dst = INCC && idx >= sc;
+      const int32_t d1 = !act ? 0 : (dir_in ? 1 : -1);
+      const int32_t d = dst ? d1 * 0x10001 : d1;
       bool flag = act && (i == 0 || (s_ev[i - 1] >> shift) != (key >> shift));
       int32_t v = wave_seg_scan(d, flag);
       if (!flag) v += carry;  // segment continues from the previous chunk
@@ -2156,9 +2203,16 @@ __global__ void __launch_bounds__(NT) k_cascade_sorted(CascadeArgs a, const uint
           if (kx == NONE) break;
           h = (h + 1) & (HS - 1);
         }
-        const uint32_t idx = (uint32_t)(key & 1023u);
-        if (dir_in) s_cq[idx] = (int32_t)cnt + v - d;
-        else s_cp[idx] = (int32_t)cnt + v - d;
+        // counts just before the event; INCC: two signed 16-bit halves, each below 2^11
+        const int32_t before = (int32_t)cnt + v - d;
+        const int32_t all = INCC ? (int32_t)(int16_t)before : before;
+        if (dir_in) s_cq[idx] = all;
+        else s_cp[idx] = all;
+        if (INCC) {
+          const int32_t dsts = (before - all) >> 16;
+          if (dir_in) s_in[idx] = dst && dsts == 0;
+          else s_out[idx] = dst && dsts == 1;
+        }
       }
       carry = __shfl(v, 63, 64);
     }
@@ -2169,10 +2223,16 @@ __global__ void __launch_bounds__(NT) k_cascade_sorted(CascadeArgs a, const uint
     const uint32_t r = s_rk[i];
     if (r == NONE) continue;
     atomicAdd(&a.seq[r], (unsigned long long)cascade_term(a.incc, W, s_cp[i], s_cq[i]));
+    if (INCC) {
+      const unsigned long long io = (unsigned long long)s_out[i] | ((unsigned long long)s_in[i] << 32);
+      if (io) atomicAdd(&a.dio[r], io);
+    }
   }
 }
 
 // ---- 5. events ----------------------------------------------------------------------------
+// The two events of every move, at 2 * rank (out of its partition) and 2 * rank + 1 (into its
+// target): key = partition << (rb + 1) | rank << 1 | dir, value = the node's signed size.
 __global__ void k_size_events(const uint32_t* __restrict__ part, const uint32_t* __restrict__ moves,
                               const uint32_t* __restrict__ ranks, const uint32_t* __restrict__ sizes, uint32_t n, int rb,
                               uint64_t* __restrict__ keys, uint32_t* __restrict__ vals) {
@@ -2180,23 +2240,26 @@ __global__ void k_size_events(const uint32_t* __restrict__ part, const uint32_t*
   if (v >= n) return;
   const uint32_t q = moves[v];
   if (q == NONE) return;
-  const uint32_t r = ranks[v];
-  keys[2 * (uint64_t)r] = ((uint64_t)part[v] << rb) | r;
-  vals[2 * (uint64_t)r] = (uint32_t)(-(int32_t)sizes[v]);
-  keys[2 * (uint64_t)r + 1] = ((uint64_t)q << rb) | r;
-  vals[2 * (uint64_t)r + 1] = sizes[v];
+  const uint64_t r = ranks[v];
+  keys[2 * r] = ((uint64_t)part[v] << (rb + 1)) | (r << 1);
+  vals[2 * r] = (uint32_t)(-(int32_t)sizes[v]);
+  keys[2 * r + 1] = ((uint64_t)q << (rb + 1)) | (r << 1) | 1u;
+  vals[2 * r + 1] = sizes[v];
 }
 __global__ void k_to_i64(const uint32_t* __restrict__ vals, uint64_t m, int64_t* __restrict__ out) {
   uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < m) out[i] = (int64_t)(int32_t)vals[i];
+}
+__device__ __forceinline__ uint32_t event_rank(uint64_t key, int rb) {
+  return (uint32_t)((key >> 1) & (((uint64_t)1 << rb) - 1));
 }
 __global__ void k_size_flags(const uint64_t* __restrict__ keys, const uint32_t* __restrict__ vals,
                              const int64_t* __restrict__ cum, const uint64_t* __restrict__ poff, uint64_t m, int rb,
                              const uint32_t* __restrict__ psizes, uint32_t omega, int32_t* sv) {
   uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= m) return;
-  const uint32_t q = (uint32_t)(keys[i] >> rb);
-  const uint32_t r = (uint32_t)(keys[i] & (((uint64_t)1 << rb) - 1));
+  const uint32_t q = (uint32_t)(keys[i] >> (rb + 1));
+  const uint32_t r = event_rank(keys[i], rb);
   const uint64_t st = poff[q];
   const int64_t before_seg = st == 0 ? 0 : cum[st - 1];
   const int64_t c = cum[i] - before_seg;
@@ -2206,131 +2269,41 @@ __global__ void k_size_flags(const uint64_t* __restrict__ keys, const uint32_t* 
   atomicAdd(&sv[r], (int32_t)ex);
 }
 
-// inbound events: (partition, hedge, rank) +-1 for every inbound hedge of every move
-// events of partitions in [plo, phi) only (the stage runs in chunks of partitions when all
-// events at once would not fit the device)
-__global__ void k_inbound_event_counts(const uint32_t* __restrict__ part, const uint32_t* __restrict__ moves,
-                                       const uint32_t* __restrict__ inb, uint32_t n, uint32_t plo, uint32_t phi,
-                                       uint32_t* __restrict__ cnt) {
-  uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= n) return;
-  const uint32_t q = moves[v], p = part[v];
-  const uint32_t in = q == NONE ? 0u : (uint32_t)(p >= plo && p < phi) + (uint32_t)(q >= plo && q < phi);
-  cnt[v] = in * inb[v];
+// Inbound-set events on the order of the size events.  All hedges whose destinations leave a
+// partition (or enter one) with one move change its inbound-set size in the same direction, so
+// the cascade kernels count them per move (dio) and the move is one event of that many hedges
+// for its source and one for its target.  One move's hedges cross the cap at most once, so the
+// violations per rank are those of hedge-by-hedge events, at 2 events per move instead of two
+// per moving inbound incidence (on an 8 x 8191-neuron network of fan-out 64 the events, their
+// 43-bit sort and the searches of their runs took 250 of a 530 ms partitioning).
+// Scanned together: the signed change in the low `db` bits, and above them the number of events
+// that change anything (the first of a partition assumes it started valid).
+__global__ void k_inbound_deltas(const uint64_t* __restrict__ keys, const unsigned long long* __restrict__ dio,
+                                 uint64_t m, int rb, int db, int64_t* __restrict__ out) {
+  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= m) return;
+  const unsigned long long x = dio[event_rank(keys[i], rb)];
+  const int64_t d = (keys[i] & 1u) ? (int64_t)(x >> 32) : -(int64_t)(x & 0xFFFFFFFFull);
+  out[i] = d + (d != 0 ? (int64_t)1 << db : 0);
 }
-__global__ void k_inbound_events(const uint32_t* __restrict__ part, const uint32_t* __restrict__ moves,
-                                 const uint32_t* __restrict__ ranks, const uint32_t* __restrict__ tch,
-                                 const uint64_t* __restrict__ toff, const uint32_t* __restrict__ inb,
-                                 const uint64_t* __restrict__ eoff, uint32_t n, int eb, int rb, uint32_t plo,
-                                 uint32_t phi, uint64_t* __restrict__ keys, uint32_t* __restrict__ vals) {
-  uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= n) return;
-  const uint32_t q = moves[v];
-  if (q == NONE) return;
-  const uint32_t p = part[v], r = ranks[v];
-  const bool pin = p >= plo && p < phi, qin = q >= plo && q < phi;
-  uint64_t o = eoff[v];
-  for (uint64_t j = toff[v]; j < toff[v] + inb[v]; ++j) {
-    const uint64_t e = tch[j];
-    if (pin) {
-      keys[o] = ((uint64_t)p << (eb + rb)) | (e << rb) | r;
-      vals[o++] = 0xFFFFFFFFu;  // -1
-    }
-    if (qin) {
-      keys[o] = ((uint64_t)q << (eb + rb)) | (e << rb) | r;
-      vals[o++] = 1u;
-    }
-  }
-}
-// count of destination pins of hedge e in partition q (0 when absent).  The lists start at
-// the hedge's pin offset; a list of one entry is read from the record.  Lists of more than
-// PP_SMALL entries (only hedges of more than PP_SMALL pins have them) are sorted by
-// partition id: binary search; shorter ones are scanned.
-__device__ __forceinline__ int64_t dst_count(const uint4* hinfo, const uint64_t* hoff, const uint2* pp,
-                                             const uint32_t* pp_dcnt, uint32_t e, uint32_t q) {
-  const uint4 hi = hinfo[e];
-  const uint64_t s = hoff[e];
-  if (hi.z == 1) return hi.x == q ? pp_dcnt[s] : 0;
-  if (hi.z <= PP_SMALL) {
-    for (uint32_t i = 0; i < hi.z; ++i)
-      if (pp[s + i].x == q) return pp_dcnt[s + i];
-    return 0;
-  }
-  uint32_t lo = 0, n = hi.z;  // first entry with partition >= q
-  while (n > 0) {
-    const uint32_t h = n / 2;
-    if (pp[s + lo + h].x < q) {
-      lo += h + 1;
-      n -= h + 1;
-    } else {
-      n = h;
-    }
-  }
-  return lo < hi.z && pp[s + lo].x == q ? pp_dcnt[s + lo] : 0;
-}
-// The first event of every (partition, hedge) run looks up the run's starting destination
-// count once (a scan of the hedge's partition list); the run's other events read it there.
-__global__ void k_inbound_group_init(const uint64_t* __restrict__ keys, uint64_t m, int eb, int rb,
-                                     const uint4* __restrict__ hinfo, const uint64_t* __restrict__ hoff,
-                                     const uint2* __restrict__ pp,
-                                     const uint32_t* __restrict__ pp_dcnt, int64_t* __restrict__ ginit) {
+__global__ void k_inbound_flags(const uint64_t* __restrict__ keys, const unsigned long long* __restrict__ dio,
+                                const int64_t* __restrict__ cum, const uint64_t* __restrict__ poff, uint64_t m, int rb,
+                                int db, const uint32_t* __restrict__ isz, uint32_t delta, int32_t* iv) {
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= m) return;
   const uint64_t key = keys[i];
-  if (i > 0 && (keys[i - 1] >> rb) == (key >> rb)) return;
-  const uint32_t q = (uint32_t)(key >> (eb + rb));
-  const uint32_t e = (uint32_t)((key >> rb) & (((uint64_t)1 << eb) - 1));
-  ginit[i] = dst_count(hinfo, hoff, pp, pp_dcnt, e, q);
-}
-__global__ void k_inbound_transitions(const uint64_t* __restrict__ keys, const uint32_t* __restrict__ vals,
-                                      const int64_t* __restrict__ cum, uint64_t m, int rb,
-                                      const int64_t* __restrict__ ginit, uint32_t* __restrict__ tflag,
-                                      int32_t* __restrict__ tdelta) {
-  uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= m) return;
-  const uint64_t key = keys[i];
-  const uint64_t grp = key >> rb;  // (partition, hedge)
-  // start of this (partition, hedge) run: binary search backwards
-  uint64_t lo = 0, hi = i;
-  while (lo < hi) {
-    const uint64_t mid = (lo + hi) / 2;
-    if ((keys[mid] >> rb) < grp) lo = mid + 1;
-    else hi = mid;
-  }
-  const int64_t before = lo == 0 ? 0 : cum[lo - 1];
-  const int64_t init = ginit[lo];
-  const int64_t cur = init + (cum[i] - before);
-  const int64_t prev = cur - (int64_t)(int32_t)vals[i];
-  int32_t d = 0;
-  if (prev == 0 && cur > 0) d = 1;
-  else if (prev > 0 && cur == 0) d = -1;
-  tflag[i] = d != 0;
-  tdelta[i] = d;
-}
-__global__ void k_inbound_size_events(const uint64_t* __restrict__ keys, const uint32_t* __restrict__ tflag,
-                                      const int32_t* __restrict__ tdelta, const uint64_t* __restrict__ tpos, uint64_t m,
-                                      int eb, int rb, uint64_t* __restrict__ okeys, uint32_t* __restrict__ ovals) {
-  uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= m || !tflag[i]) return;
-  const uint64_t key = keys[i];
-  const uint64_t q = key >> (eb + rb);
-  const uint64_t r = key & (((uint64_t)1 << rb) - 1);
-  okeys[tpos[i]] = (q << rb) | r;
-  ovals[tpos[i]] = (uint32_t)tdelta[i];
-}
-__global__ void k_inbound_flags(const uint64_t* __restrict__ keys, const uint32_t* __restrict__ vals,
-                                const int64_t* __restrict__ cum, const uint64_t* __restrict__ poff, uint64_t m, int rb,
-                                const uint32_t* __restrict__ isz, uint32_t delta, int32_t* iv) {
-  uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= m) return;
-  const uint32_t q = (uint32_t)(keys[i] >> rb);
-  const uint32_t r = (uint32_t)(keys[i] & (((uint64_t)1 << rb) - 1));
+  const uint32_t r = event_rank(key, rb);
+  const unsigned long long x = dio[r];
+  const int64_t d = (key & 1u) ? (int64_t)(x >> 32) : -(int64_t)(x & 0xFFFFFFFFull);
+  if (d == 0) return;
+  const uint32_t q = (uint32_t)(key >> (rb + 1));
   const uint64_t st = poff[q];
-  const int64_t before_seg = st == 0 ? 0 : cum[st - 1];
-  const int64_t cur = (int64_t)isz[q] + (cum[i] - before_seg);
-  const int64_t prev = cur - (int64_t)(int32_t)vals[i];
+  const int64_t c = cum[i] - (st == 0 ? 0 : cum[st - 1]);
+  const int64_t change = (int64_t)((uint64_t)c << (64 - db)) >> (64 - db);
+  const bool first = ((c - change) >> db) == 1;
+  const int64_t cur = (int64_t)isz[q] + change, prev = cur - d;
   // the first event of a partition assumes it started valid (kernels/refinement.cu:643-644)
-  const bool was_valid = i == st || prev <= (int64_t)delta, is_valid = cur <= (int64_t)delta;
+  const bool was_valid = first || prev <= (int64_t)delta, is_valid = cur <= (int64_t)delta;
   if (was_valid && !is_valid) atomicAdd(&iv[r], 1);
   if (!was_valid && is_valid) atomicSub(&iv[r], 1);
 }
@@ -2462,13 +2435,13 @@ namespace {
 struct PartitionLists {
   DBuf<uint2> pp;      // (partition, pin count) per list entry, at the hedge's own offsets
   DBuf<uint4> hinfo;   // per hedge: list start (lo, hi) or its one entry, length, fixed-point weight
-  DBuf<uint32_t> dcnt, lambda, inbsz;
+  DBuf<uint32_t> lambda, inbsz;
   DBuf<uint4> hm;      // instead of the lists (k-way, k <= MASK_K): per hedge, its partition masks
   uint64_t P = 0;      // pins of the level
 };
 
-// Partition lists of every hedge.  want_inbound adds the destination counts and the
-// per-partition inbound sizes (the inbound-set constraint needs them; k-way does not).
+// Partition lists of every hedge.  want_inbound adds the per-partition inbound sizes (the
+// inbound-set constraint needs them; k-way does not).
 // The hedge classes of a level depend only on hedge lengths and k, so refine() computes them
 // in its first round and reuses them: for the partition-list kernels the pin count, the
 // hedges of more than PP_SMALL pins with LDS tables, those with HBM tables and their table
@@ -2519,7 +2492,6 @@ void build_partition_lists(Ctx& c, const RefineLevel& L, const uint32_t* part, P
   pl.hinfo = DBuf<uint4>(c, L.e);
   pl.lambda = DBuf<uint32_t>(c, L.e);
   if (want_inbound) {
-    pl.dcnt = DBuf<uint32_t>(c, P);
     pl.inbsz = DBuf<uint32_t>(c, std::max<uint32_t>(L.k, 1));
     memset_async(c, pl.inbsz.get(), 0, (uint64_t)L.k * sizeof(uint32_t));
   }
@@ -2528,11 +2500,10 @@ void build_partition_lists(Ctx& c, const RefineLevel& L, const uint32_t* part, P
   if (want_inbound) {
     const uint32_t k_lds = L.k <= PP_HIST_CAP ? L.k : 0u;
     HGP_LAUNCH((k_pp_small<true>), ceil_div(L.e, 256), 256, k_lds * sizeof(uint32_t), c, L.hedges, L.hoff, L.srcc, part,
-               L.w, L.e, pl.pp.get(), pl.dcnt.get(), pl.lambda.get(), pl.hinfo.get(), lflag.get(), pl.inbsz.get(),
-               k_lds);
+               L.w, L.e, pl.pp.get(), pl.lambda.get(), pl.hinfo.get(), lflag.get(), pl.inbsz.get(), k_lds);
   } else {
     HGP_LAUNCH((k_pp_small<false>), ceil_div(L.e, 256), 256, 0, c, L.hedges, L.hoff, L.srcc, part, L.w, L.e,
-               pl.pp.get(), (uint32_t*)nullptr, pl.lambda.get(), pl.hinfo.get(), lflag.get(), (uint32_t*)nullptr, 0u);
+               pl.pp.get(), pl.lambda.get(), pl.hinfo.get(), lflag.get(), (uint32_t*)nullptr, 0u);
   }
   // Distinct partitions per hedge <= min(k, len).  Tables of up to PP_LDS_CAP slots sit in
   // LDS; hedges needing more (len and k both above ~2K) get HBM tables.
@@ -2574,8 +2545,7 @@ void build_partition_lists(Ctx& c, const RefineLevel& L, const uint32_t* part, P
     constexpr bool INB = decltype(inb)::value, GMEM = decltype(gmem)::value;
     if (m == 0) return;
     HGP_LAUNCH((k_pp_large<INB, GMEM>), m, 64, GMEM ? 0 : 3 * cap * sizeof(uint32_t), c, L.hedges, L.hoff, L.srcc, part,
-               L.w, lst, cap, L.k, goff, gtab, pl.pp.get(), INB ? pl.dcnt.get() : (uint32_t*)nullptr, pl.lambda.get(),
-               pl.hinfo.get(), INB ? pl.inbsz.get() : (uint32_t*)nullptr);
+               L.w, lst, cap, L.k, goff, gtab, pl.pp.get(), pl.lambda.get(), pl.hinfo.get(), INB ? pl.inbsz.get() : (uint32_t*)nullptr);
   };
   using T = std::true_type;
   using F = std::false_type;
@@ -2589,21 +2559,6 @@ void build_partition_lists(Ctx& c, const RefineLevel& L, const uint32_t* part, P
 }
 
 uint32_t discount_of(uint32_t rep, uint32_t R) { return rep < R / 3 ? 1u : (rep < 2 * R / 3 ? 2u : NONE); }
-
-// peak device bytes per inbound-set event: keys and values with their sort buffers and tile
-// counts, running sums, transition flags, deltas, group starts and positions
-constexpr uint64_t INBOUND_EVENT_BYTES = 64;
-
-uint64_t event_budget(Ctx& c) {
-  if (c.event_budget) return c.event_budget;
-  size_t free_b = 0, total_b = 0;
-  if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) {
-    (void)hipGetLastError();
-    return 16ull << 30;
-  }
-  return std::max<uint64_t>(1ull << 26, ((uint64_t)free_b + c.cached) / 2);
-}
-
 
 // Algorithmic bytes of the gain kernels over `list` (evaluated only while the kernel is
 // profiled): per node 36 (partition, size, two offsets, move and gain out) + 20 per touching
@@ -2827,10 +2782,15 @@ void analyze_round(Ctx& c, const RefineLevel& L, int mode, uint32_t omega, uint3
   if (V == 0) return;
   HGP_LAUNCH(k_zero3, ceil_div(V, 256), 256, 0, c, st.seq.get(), (uint32_t*)st.sv.get(), (uint32_t*)st.iv.get(),
              (uint64_t)V);
+  DBuf<unsigned long long> dio;
+  if (incc) {
+    dio = DBuf<unsigned long long>(c, V);
+    fill_u32(c, (uint32_t*)dio.get(), 0u, 2ull * V);
+  }
   // cascade.  The hedges of 2..CAS_SMALL pins first, alone on the stream; then, with bit 1 of
-  // the side_streams tuning, the sorted and direct classes on side streams beside the size and
-  // inbound events (all classes add their terms to seq with atomics; the node records stay
-  // alive until the join before seq's prefix sum).
+  // the side_streams tuning, the sorted and direct classes on side streams beside the size
+  // events (all classes add their terms to seq and dio with atomics; the node records stay
+  // alive until the join before they are read).
   DBuf<uint4> pm;
   DBuf<uint2> pm2;
   std::optional<Fork> cas_fork;
@@ -2843,7 +2803,7 @@ void analyze_round(Ctx& c, const RefineLevel& L, int mode, uint32_t omega, uint3
       pm = DBuf<uint4>(c, n);
       HGP_LAUNCH(k_pack_nodes, g, 256, 0, c, part, st.moves.get(), st.ranks.get(), n, pm.get());
     }
-    CascadeArgs a{L.hedges, L.hoff, L.w, pm.get(), pm2.get(), incc ? 1 : 0, st.seq.get()};
+    CascadeArgs a{L.hedges, L.hoff, L.w, pm.get(), pm2.get(), incc ? 1 : 0, st.seq.get(), L.srcc, dio.get()};
     const int crb = std::max(1, bit_width(V));  // rank + 1 <= V
     const int cpb = std::max(1, bit_width(L.k));
     const uint32_t sort_max = cpb + crb + 11 < 64 ? CAS_SORT : 0u;
@@ -2854,7 +2814,7 @@ void analyze_round(Ctx& c, const RefineLevel& L, int mode, uint32_t omega, uint3
       DBuf<uint32_t> fl[4];
       for (int cls = 0; cls < 4; ++cls) fl[cls] = DBuf<uint32_t>(c, L.e);
       DBuf<uint64_t> ks(c, std::max<uint32_t>(L.e, 1));
-      HGP_LAUNCH(k_cascade_classes, ceil_div(L.e, 256), 256, 0, c, L.hedges, L.hoff, L.e, sort_max, fl[3].get(),
+      HGP_LAUNCH(k_cascade_classes, ceil_div(L.e, 256), 256, 0, c, L.hedges, L.hoff, L.e, incc ? 1u : 2u, sort_max, fl[3].get(),
                  ks.get(), fl[0].get(), fl[1].get(), fl[2].get());
       DBuf<uint64_t> pos(c, (uint64_t)L.e + 1);
       for (int cls = 0; cls < 3; ++cls) {
@@ -2872,7 +2832,7 @@ void analyze_round(Ctx& c, const RefineLevel& L, int mode, uint32_t omega, uint3
         DBuf<uint64_t> kc(c, m);
         HGP_LAUNCH(k_compact_u64, ceil_div(L.e, 256), 256, 0, c, fl[3].get(), pos.get(), L.e, ks.get(), kc.get());
         radix_sort(c, kc.get(), nullptr, m, 32 + std::max(1, bit_width(L.n)));
-        Y.cs = small_csr(c, kc.get(), m, L.hoff, L.hedges, L.w);
+        Y.cs = small_csr(c, kc.get(), m, L.hoff, L.hedges, L.w, incc ? L.srcc : nullptr);
       }
     }
     auto small_cascade = [&] {
@@ -2880,8 +2840,10 @@ void analyze_round(Ctx& c, const RefineLevel& L, int mode, uint32_t omega, uint3
       if (!m) return;
       const SmallHedges sh{Y.cs.rec.get(), Y.cs.pins.get(), Y.cs.w.get(), m};
       const uint32_t cb = c.tune.cascade_block;  // 256 unless the autotuner chose otherwise
-      if (a.pm2) HGP_LAUNCH(k_cascade_small<true>, ceil_div(m, cb), cb, 0, c, a, sh);
-      else HGP_LAUNCH(k_cascade_small<false>, ceil_div(m, cb), cb, 0, c, a, sh);
+      if (a.pm2 && incc) HGP_LAUNCH((k_cascade_small<true, true>), ceil_div(m, cb), cb, 0, c, a, sh);
+      else if (incc) HGP_LAUNCH((k_cascade_small<false, true>), ceil_div(m, cb), cb, 0, c, a, sh);
+      else if (a.pm2) HGP_LAUNCH((k_cascade_small<true, false>), ceil_div(m, cb), cb, 0, c, a, sh);
+      else HGP_LAUNCH((k_cascade_small<false, false>), ceil_div(m, cb), cb, 0, c, a, sh);
       if (prof_match(c, "k_cascade_small") && c.prof_count && c.prof_dev)
         HGP_LAUNCH(k_cascade_small_bytes, ceil_div(m, 256), 256, 0, c, a, sh, c.prof_dev);
     };
@@ -2895,96 +2857,56 @@ void analyze_round(Ctx& c, const RefineLevel& L, int mode, uint32_t omega, uint3
       if (m == 0) continue;
       const uint32_t* lst = Y.cas_list[cls].get();
       cas_fork->on(cls, [&] {
-        if (cls == 0) HGP_LAUNCH((k_cascade_sorted<CAS_SORT_S, 2 * CAS_SORT_S, 64>), m, 64, 0, c, a, lst, crb);
-        else if (cls == 1)
-          HGP_LAUNCH((k_cascade_sorted<CAS_SORT, CAS_EV, CAS_SORT_NT>), m, CAS_SORT_NT, 0, c, a, lst, crb);
-        else HGP_LAUNCH(k_cascade_large, m, 64, 0, c, a, lst);
+        auto launch = [&](auto mode_incc) {
+          constexpr bool INCC = decltype(mode_incc)::value;
+          if (cls == 0)
+            HGP_LAUNCH((k_cascade_sorted<CAS_SORT_S, 2 * CAS_SORT_S, 64, INCC>), m, 64, 0, c, a, lst, crb);
+          else if (cls == 1)
+            HGP_LAUNCH((k_cascade_sorted<CAS_SORT, CAS_EV, CAS_SORT_NT, INCC>), m, CAS_SORT_NT, 0, c, a, lst, crb);
+          else HGP_LAUNCH((k_cascade_large<INCC>), m, 64, 0, c, a, lst);
+        };
+        if (incc) launch(std::true_type{});
+        else launch(std::false_type{});
       });
     }
     if (early) small_cascade();
   }
   const int rb = std::max(1, bit_width(V - 1));
   const int kb = std::max(1, bit_width(L.k));
-  // size events
+  // size events; in inbound-constrained mode the inbound-set events on the same order (with
+  // k-way's Delta = INT32_MAX every prefix is valid)
   {
     const uint64_t m = 2ull * V;
     DBuf<uint64_t> keys(c, m), poff(c, (uint64_t)L.k + 1);
     DBuf<uint32_t> vals(c, m);
     DBuf<int64_t> cum(c, m);
+    // inbound events: m of them counted above a change of at most P destination pins either way
+    const int db = 63 - bit_width(m);
+    if (incc) {
+      // partition, hedge and rank in one 64-bit word: larger levels are refused
+      const int eb = std::max(1, bit_width(L.e));
+      HGP_REQUIRE(kb + eb + rb <= 64, HGP_E_CAPACITY, "inbound events: key exceeds 64 bits");
+      HGP_REQUIRE(pl.P < (1ull << (db - 1)), HGP_E_CAPACITY, "inbound events: too many moves and pins");
+    }
     HGP_LAUNCH(k_size_events, g, 256, 0, c, part, st.moves.get(), st.ranks.get(), L.sizes, n, rb, keys.get(), vals.get());
     // the events sit at 2 * rank (+1), so they are already in rank order: sorting by the
     // partition bits alone orders them by (partition, rank)
-    radix_sort_buf(c, keys, vals, m, rb, rb + kb);
+    radix_sort_buf(c, keys, vals, m, rb + 1, rb + 1 + kb);
     HGP_LAUNCH(k_to_i64, ceil_div(m, 256), 256, 0, c, vals.get(), m, cum.get());
     inclusive_scan(c, cum.get(), cum.get(), m);
-    segment_offsets(c, keys.get(), rb, m, L.k, poff.get());
+    segment_offsets(c, keys.get(), rb + 1, m, L.k, poff.get());
     HGP_LAUNCH(k_size_flags, ceil_div(m, 256), 256, 0, c, keys.get(), vals.get(), cum.get(), poff.get(), m, rb, psizes,
                omega, st.sv.get());
     inclusive_scan(c, st.sv.get(), st.sv.get(), V);
-  }
-  // inbound-set events (INCC only: with k-way's Delta = INT32_MAX every prefix is valid)
-  if (incc) {
-    const int eb = std::max(1, bit_width(L.e));
-    HGP_REQUIRE(kb + eb + rb <= 64, HGP_E_CAPACITY, "inbound events: key exceeds 64 bits");
-    DBuf<uint32_t> ecnt(c, n);
-    DBuf<uint64_t> eoff(c, (uint64_t)n + 1);
-    // All events at once need about INBOUND_EVENT_BYTES each (keys and values with their
-    // sort buffers, running sums, transition flags, deltas, group starts, positions); when that
-    // exceeds the event budget the partitions are split into ranges whose events are processed
-    // one range after the other.  Every event stays with its partition, so the violations
-    // summed over the ranges are exact.
-    HGP_LAUNCH(k_inbound_event_counts, g, 256, 0, c, part, st.moves.get(), L.inb, n, 0u, L.k, ecnt.get());
-    exclusive_scan(c, ecnt.get(), eoff.get(), n);
-    const uint64_t m_all = read_scalar(c, eoff.get() + n);
-    const uint64_t budget = event_budget(c);
-    const uint32_t chunks = (uint32_t)std::min<uint64_t>(
-        std::max<uint32_t>(L.k, 1), std::max<uint64_t>(1, (m_all * INBOUND_EVENT_BYTES + budget - 1) / budget));
-    if (c.verbose >= 2 && chunks > 1)
-      fprintf(stderr, "  inbound events: %llu in %u partition ranges\n", (unsigned long long)m_all, chunks);
-    for (uint32_t ch = 0; ch < chunks && m_all; ++ch) {
-      const uint32_t plo = (uint32_t)((uint64_t)L.k * ch / chunks), phi = (uint32_t)((uint64_t)L.k * (ch + 1) / chunks);
-      if (chunks > 1) {
-        HGP_LAUNCH(k_inbound_event_counts, g, 256, 0, c, part, st.moves.get(), L.inb, n, plo, phi, ecnt.get());
-        exclusive_scan(c, ecnt.get(), eoff.get(), n);
-      }
-      const uint64_t m = chunks > 1 ? read_scalar(c, eoff.get() + n) : m_all;
-      if (!m) continue;
-      DBuf<uint64_t> keys(c, m);
-      DBuf<uint32_t> vals(c, m);
-      HGP_LAUNCH(k_inbound_events, g, 256, 0, c, part, st.moves.get(), st.ranks.get(), L.tch, L.toff, L.inb, eoff.get(), n,
-                 eb, rb, plo, phi, keys.get(), vals.get());
-      radix_sort(c, keys.get(), vals.get(), m, kb + eb + rb);
-      DBuf<int64_t> cum(c, m);
-      HGP_LAUNCH(k_to_i64, ceil_div(m, 256), 256, 0, c, vals.get(), m, cum.get());
+    cas_fork.reset();  // the main stream waits for the cascade's side streams
+    if (incc) {
+      HGP_LAUNCH(k_inbound_deltas, ceil_div(m, 256), 256, 0, c, keys.get(), dio.get(), m, rb, db, cum.get());
       inclusive_scan(c, cum.get(), cum.get(), m);
-      DBuf<uint32_t> tflag(c, m);
-      DBuf<int32_t> tdelta(c, m);
-      DBuf<int64_t> ginit(c, m);
-      HGP_LAUNCH(k_inbound_group_init, ceil_div(m, 256), 256, 0, c, keys.get(), m, eb, rb, pl.hinfo.get(), L.hoff,
-                 pl.pp.get(), pl.dcnt.get(), ginit.get());
-      HGP_LAUNCH(k_inbound_transitions, ceil_div(m, 256), 256, 0, c, keys.get(), vals.get(), cum.get(), m, rb,
-                 ginit.get(), tflag.get(), tdelta.get());
-      DBuf<uint64_t> tpos(c, m + 1);
-      exclusive_scan(c, tflag.get(), tpos.get(), m);
-      const uint64_t T = read_scalar(c, tpos.get() + m);
-      if (T) {
-        DBuf<uint64_t> ok(c, T), poff(c, (uint64_t)L.k + 1);
-        DBuf<uint32_t> ov(c, T);
-        HGP_LAUNCH(k_inbound_size_events, ceil_div(m, 256), 256, 0, c, keys.get(), tflag.get(), tdelta.get(), tpos.get(),
-                   m, eb, rb, ok.get(), ov.get());
-        keys.reset();
-        radix_sort(c, ok.get(), ov.get(), T, rb + kb);
-        DBuf<int64_t> cum2(c, T);
-        HGP_LAUNCH(k_to_i64, ceil_div(T, 256), 256, 0, c, ov.get(), T, cum2.get());
-        inclusive_scan(c, cum2.get(), cum2.get(), T);
-        segment_offsets(c, ok.get(), rb, T, L.k, poff.get());
-        HGP_LAUNCH(k_inbound_flags, ceil_div(T, 256), 256, 0, c, ok.get(), ov.get(), cum2.get(), poff.get(), T, rb,
-                   pl.inbsz.get(), delta, st.iv.get());
-      }
+      HGP_LAUNCH(k_inbound_flags, ceil_div(m, 256), 256, 0, c, keys.get(), dio.get(), cum.get(), poff.get(), m, rb, db,
+                 pl.inbsz.get(), delta, st.iv.get());
+      inclusive_scan(c, st.iv.get(), st.iv.get(), V);
     }
-    inclusive_scan(c, st.iv.get(), st.iv.get(), V);
   }
-  cas_fork.reset();  // the main stream waits for the cascade's side streams
   inclusive_scan(c, (const int64_t*)st.seq.get(), (int64_t*)st.seq.get(), V);
   // best prefix
   {
@@ -3089,7 +3011,7 @@ uint32_t jacobi_round(Ctx& c, const RefineLevel& L, uint32_t omega, uint32_t rou
 }
 
 SmallCsr small_csr(Ctx& c, const uint64_t* keys, uint32_t m, const uint64_t* hoff, const uint32_t* hedges,
-                   const float* w) {
+                   const float* w, const uint32_t* srcc) {
   SmallCsr r;
   r.m = m;
   if (!m) return r;
@@ -3099,20 +3021,20 @@ SmallCsr small_csr(Ctx& c, const uint64_t* keys, uint32_t m, const uint64_t* hof
   const uint64_t sp = read_scalar(c, r.rec.get() + m);
   r.pins = DBuf<uint32_t>(c, sp);
   r.w = DBuf<float>(c, m);
-  HGP_LAUNCH(k_small_fill, ceil_div(m, 256), 256, 0, c, keys, m, hoff, hedges, w, r.rec.get(), r.pins.get(),
-             r.w.get());
+  HGP_LAUNCH(k_small_fill, ceil_div(m, 256), 256, 0, c, keys, m, hoff, hedges, w, srcc, r.rec.get(),
+             r.pins.get(), r.w.get());
   return r;
 }
 
 float time_cascade_small(Ctx& c, const SmallCsr& cs, const uint2* pm2, uint32_t block, unsigned long long* seq) {
   const uint32_t m = cs.m;
-  CascadeArgs a{nullptr, nullptr, nullptr, nullptr, pm2, 0, seq};
+  CascadeArgs a{nullptr, nullptr, nullptr, nullptr, pm2, 0, seq, nullptr, nullptr};
   const SmallHedges sh{cs.rec.get(), cs.pins.get(), cs.w.get(), m};
   hipEvent_t t0, t1;
   HGP_HIP(hipEventCreate(&t0));
   HGP_HIP(hipEventCreate(&t1));
   HGP_HIP(hipEventRecord(t0, c.stream));
-  HGP_LAUNCH(k_cascade_small<true>, ceil_div(m, block), block, 0, c, a, sh);
+  HGP_LAUNCH((k_cascade_small<true, false>), ceil_div(m, block), block, 0, c, a, sh);
   HGP_HIP(hipEventRecord(t1, c.stream));
   HGP_HIP(hipEventSynchronize(t1));
   float ms = 0;

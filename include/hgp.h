@@ -89,10 +89,10 @@ typedef struct hgp_params {
   uint32_t ip_rounds;
   uint32_t ip_nodes_per_part;
   uint32_t ip_refine_repeats;
-  /* INCC refinement: device bytes its inbound-set event stage may take at once; the events of
-   * a round that need more are processed in ranges of partitions, one after the other, with
-   * the same result (0, the default: half of the device memory free at that moment).  The
-   * reference sizes this stage without a bound (sources/refinement.cu:307-491). */
+  /* INCC refinement: device bytes for its inbound-set events.  Accepted and without effect: the
+   * stage takes two events per move whatever the number of inbound hedges (under 64 bytes per
+   * node), so nothing is split.  The reference sizes this stage by the moving inbound
+   * incidences, without a bound (sources/refinement.cu:307-491). */
   uint64_t refine_event_budget;
 } hgp_params;
 

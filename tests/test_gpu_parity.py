@@ -306,6 +306,42 @@ def test_refine_analyze_huge_lists(dev, mode, k, fm_repeat, chainup, n, e, max_s
     assert got["best"] == exp["best"]
 
 
+@pytest.mark.parametrize("k", [5, 300, 66000])
+@pytest.mark.parametrize("dup", [False, True])
+def test_refine_analyze_inbound_by_hedge_size(dev, k, dup, rng):
+    """The cascade kernels count which hedges leave and enter inbound sets: hedges of one pin, at
+    the edges of every hedge class, with and without sources, and (not deduplicated) hedges that
+    list a destination twice; k = 66000 takes the unpacked node records."""
+    lens = [1, 2, 4, 5, 15, 16, 17, 63, 64, 65, 127, 128, 129, 1023, 1024, 1025, 2049] * 4 + [1, 2, 3] * 200
+    n, off, pins, srcc = 3000, [0], [], []
+    for i, ln in enumerate(lens):
+        nodes = list(rng.choice(n, size=ln, replace=False))
+        ns = min(int(rng.integers(0, 3)), ln - 1) if i % 3 else 0
+        if dup and i % 2:
+            nodes.append(nodes[int(rng.integers(ns, ln))])
+        pins.extend(int(x) for x in nodes)
+        off.append(len(pins))
+        srcc.append(ns)
+    hg = O.HG(n, np.array(off, np.uint64), np.array(pins, np.uint32), np.array(srcc, np.uint32),
+              np.ones(len(lens), np.float32))
+    sizes = rng.integers(1, 3, size=n).astype(np.uint32)
+    part = rng.integers(0, min(k, 300), size=n).astype(np.uint32)
+    part[:5] = k - 1 - np.arange(5)
+    psizes = np.bincount(part, weights=sizes, minlength=k).astype(np.uint32)
+    omega, delta = int(psizes.max()) + 3, int(O.inbound_sizes(hg, part, k).max()) - 1
+    L = G.Level(dev, hg)
+    L.build_touching()
+    ro, rt, ri = O.touching(hg)
+    got = G.refine_analyze(dev, L, sizes, k, 0, omega, delta, 16, 0, True, part, psizes)
+    exp = O.refine_analyze(0, omega, delta, 16, hg, ro, rt, ri, sizes, k, 0, True, part, psizes)
+    assert exp["iv"].any(), "the case must have inbound violations"
+    # the cascade of a node listed twice is counted pin by pin on the device (the oracle applies
+    # both pins at once), so seq and the best prefix are compared on deduplicated hedges only
+    for key in ("moves", "gains", "ranks", "sv", "iv") + (() if dup else ("seq",)):
+        assert np.array_equal(got[key], exp[key]), f"{key} differs"
+    assert dup or got["best"] == exp["best"]
+
+
 @pytest.mark.parametrize("rc", REFINE_CASES, ids=[r[0] for r in REFINE_CASES])
 def test_refine_loop(dev, rc, rng):
     name, mode, k, case_name = rc
