@@ -300,6 +300,19 @@ __device__ __forceinline__ T swap16_move(T v) {  // lane i <- lane i ^ 16
     return (T)sw((uint32_t)v);
   }
 }
+// lane i <- lane i ^ mask, for mask one of 1, 2, 4, 8, 16, 32 (constant after unrolling): DPP moves
+// inside a row of 16 (xor 4 as the half-row mirror, xor 7, and the quad reversal, xor 3), a
+// ds_swizzle for 16 and a cross-lane read for 32.
+__device__ __forceinline__ uint32_t lane_xor(uint32_t v, uint32_t mask) {
+  switch (mask) {
+    case 1: return dpp_u32<0xB1>(v);
+    case 2: return dpp_u32<0x4E>(v);
+    case 4: return dpp_u32<0x1B>(dpp_u32<0x141>(v));
+    case 8: return dpp_u32<0x128>(v);
+    case 16: return swap16_move(v);
+    default: return (uint32_t)__shfl_xor((int)v, 32, 64);
+  }
+}
 template <typename T>
 __device__ __forceinline__ T lane_value(T v, int lane) {
   if constexpr (sizeof(T) == 8) {
@@ -319,6 +332,39 @@ __device__ __forceinline__ T wave_reduce(T v, Op op) {
   v = op(v, dpp_move<0x140>(v));  // row_mirror: the two halves of each 16
   v = op(v, swap16_move(v));      // the two rows of each 32
   return op(lane_value(v, 0), lane_value(v, 32));
+}
+
+// Ascending bitonic sort of 64 * R keys held by the wave, key[r] of lane l at position
+// 64 * r + l: strides below 64 exchange lanes, larger ones registers; no LDS, no barrier.
+template <uint32_t R>
+__device__ __forceinline__ void wave_sort(uint32_t (&key)[R]) {
+  static_assert((R & (R - 1)) == 0, "a power of two of registers");
+  const uint32_t l = lane_id();
+#pragma unroll
+  for (uint32_t k = 2; k <= 64 * R; k <<= 1) {
+#pragma unroll
+    for (uint32_t j = k >> 1; j > 0; j >>= 1) {
+      if (j >= 64) {
+#pragma unroll
+        for (uint32_t r = 0; r < R; ++r) {
+          const uint32_t o = r ^ (j / 64);
+          if (r < o) {
+            const uint32_t a = key[r], b = key[o];
+            const bool up = ((64 * r) & k) == 0;
+            key[r] = up ? min(a, b) : max(a, b);
+            key[o] = up ? max(a, b) : min(a, b);
+          }
+        }
+      } else {
+#pragma unroll
+        for (uint32_t r = 0; r < R; ++r) {
+          const uint32_t other = lane_xor(key[r], j);
+          const bool up = ((64 * r + l) & k) == 0, low = (l & j) == 0;
+          key[r] = up == low ? min(key[r], other) : max(key[r], other);
+        }
+      }
+    }
+  }
 }
 
 template <typename T>

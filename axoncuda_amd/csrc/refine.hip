@@ -28,6 +28,9 @@ namespace hgp {
 namespace {
 
 constexpr uint32_t PP_SMALL = 16;
+constexpr uint32_t PP_WAVE = 256;       // pins of a hedge whose list a wave sorts in registers
+constexpr uint32_t PP_REPLICAS = 64;    // copies of the inbound sizes that the list kernels add to (at most)
+constexpr uint32_t PP_REPLICA_CAP = 16384;  // ... and their counters together
 constexpr uint32_t PP_HIST_CAP = 8192;  // partitions whose inbound counts aggregate in LDS
 constexpr uint32_t PP_LDS_CAP = 4096;  // 3 x 16 KiB of dynamic LDS per wave
 constexpr uint32_t GAIN_CAP = 1024;
@@ -62,8 +65,9 @@ __global__ void __launch_bounds__(256) k_pp_small(const uint32_t* __restrict__ h
                                                   const float* __restrict__ w, uint32_t E, uint2* __restrict__ pp,
                                                   uint32_t* __restrict__ lambda,
                                                   uint4* __restrict__ hinfo, uint32_t* __restrict__ large_flag,
-                                                  uint32_t* inbsz, uint32_t k_lds) {
+                                                  uint32_t* inbsz, uint32_t k_lds, uint32_t k, uint32_t replicas) {
   extern __shared__ uint32_t hist[];
+  if (INB) inbsz += (uint64_t)(blockIdx.x & (replicas - 1)) * k;
   if (INB && k_lds) {
     for (uint32_t i = threadIdx.x; i < k_lds; i += blockDim.x) hist[i] = 0;
     __syncthreads();
@@ -163,7 +167,99 @@ __host__ __device__ __forceinline__ uint32_t pp_table_cap(uint64_t len, uint32_t
   return cap;
 }
 
-// One wave per hedge with more than 16 pins.  GMEM = false: the (partition, count, dst
+// Lists of hedges of PP_SMALL < len <= PP_WAVE pins: one wave sorts the pins' partitions in
+// registers; a run's head writes its entry (the list comes sorted by partition id, as below) and
+// its last pin, a destination when the run has one (the low key bit), adds to the inbound size.
+// An LDS table per wave, sized for the longest hedge, left room for few waves on a CU and was
+// cleared and compacted slot by slot, and every hedge added to one counter per partition, hence
+// the replicas: 8,092 hedges of up to 65 pins took 112 us a launch that way and take 7 us here,
+// 57,337 of them 691 and 18 us; 425,000 nets at k = 256 (those above 16 pins) 46 and 9 us, 25 us
+// more for the few above 256 pins.
+template <uint32_t R, bool INB>
+__device__ __forceinline__ void pp_wave_list(const uint32_t* __restrict__ hedges, const uint32_t* __restrict__ part,
+                                             uint64_t s, uint32_t len, uint32_t sc, uint2* __restrict__ pp,
+                                             uint32_t* inbsz, uint32_t& lambda, uint2& first) {
+  constexpr uint32_t SH = INB ? 1 : 0;  // INB: the low key bit marks a destination
+  const uint32_t l = lane_id();
+  uint32_t key[R];
+#pragma unroll
+  for (uint32_t r = 0; r < R; ++r) key[r] = hedges[s + min(64 * r + l, len - 1)];
+#pragma unroll
+  for (uint32_t r = 0; r < R; ++r) {
+    const uint32_t i = 64 * r + l;
+    const uint32_t q = part[key[r]];
+    key[r] = i < len ? (q << SH) | (INB && i >= sc ? 1u : 0u) : NONE;
+  }
+  wave_sort(key);
+  uint64_t head[R];  // positions where a run starts; the padding's start ends the last run
+#pragma unroll
+  for (uint32_t r = 0; r < R; ++r) {
+    const uint32_t up = __shfl_up(key[r], 1, 64);
+    const uint32_t prev = l ? up : (r ? lane_value(key[r ? r - 1 : 0], 63) : 0u);
+    head[r] = __ballot((r == 0 && l == 0) || (prev >> SH) != (key[r] >> SH));
+  }
+  uint32_t base = 0;
+#pragma unroll
+  for (uint32_t r = 0; r < R; ++r) {
+    const uint32_t i = 64 * r + l;
+    const bool real = i < len;
+    const bool mine = real && ((head[r] >> l) & 1ull);
+    // where this position's run ends: the next head, or the end of all positions
+    const uint64_t above = l == 63 ? 0ull : head[r] & (~0ull << (l + 1));
+    uint32_t end = 64 * R;
+#pragma unroll
+    for (uint32_t x = R; x-- > r + 1;)
+      if (head[x]) end = 64 * x + (uint32_t)__ffsll((unsigned long long)head[x]) - 1u;
+    if (above) end = 64 * r + (uint32_t)__ffsll((unsigned long long)above) - 1u;
+    if (mine) {
+      const uint32_t o = base + lanes_below(head[r]);
+      pp[s + o] = make_uint2(key[r] >> SH, end - i);
+    }
+    if (INB && real && end == i + 1 && (key[r] & 1u)) atomicAdd(&inbsz[key[r] >> 1], 1u);
+    base += (uint32_t)__popcll(__ballot(mine));
+  }
+  lambda = base;
+  first = make_uint2(lane_value(key[0], 0) >> SH, len);  // the one entry of a list of one
+}
+
+template <bool INB>
+__global__ void __launch_bounds__(256) k_pp_wave(const uint32_t* __restrict__ hedges, const uint64_t* __restrict__ hoff,
+                                                 const uint32_t* __restrict__ srcc, const uint32_t* __restrict__ part,
+                                                 const float* __restrict__ w, const uint32_t* __restrict__ list,
+                                                 uint32_t m, uint2* __restrict__ pp, uint32_t* __restrict__ lambda,
+                                                 uint4* __restrict__ hinfo, uint32_t* inbsz, uint32_t k,
+                                                 uint32_t replicas) {
+  const uint32_t x = blockIdx.x * 4 + threadIdx.x / 64;
+  if (x >= m) return;
+  const uint32_t e = (uint32_t)__builtin_amdgcn_readfirstlane((int)list[x]);
+  const uint64_t s = hoff[e];
+  const uint32_t len = (uint32_t)(hoff[e + 1] - s), sc = INB ? srcc[e] : 0u;
+  uint32_t* isz = INB ? inbsz + (uint64_t)(x & (replicas - 1)) * k : nullptr;
+  uint32_t lam;
+  uint2 first;
+  if (len <= 64) pp_wave_list<1, INB>(hedges, part, s, len, sc, pp, isz, lam, first);
+  else if (len <= 128) pp_wave_list<2, INB>(hedges, part, s, len, sc, pp, isz, lam, first);
+  else pp_wave_list<4, INB>(hedges, part, s, len, sc, pp, isz, lam, first);
+  if (lane_id() == 0) {
+    lambda[e] = lam;
+    // a single entry rides in the record in place of the list start
+    const uint64_t o = lam == 1 ? (((uint64_t)first.y << 32) | first.x) : s;
+    hinfo[e] = make_uint4((uint32_t)o, (uint32_t)(o >> 32), lam, w ? fixed_weight(w[e]) : 0u);
+  }
+}
+
+// out[q] = the sum of the replicas' counters of partition q
+__global__ void k_sum_replicas(const uint32_t* __restrict__ in, uint32_t k, uint32_t replicas,
+                               uint32_t* __restrict__ out) {
+  const uint32_t q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= k) return;
+  uint32_t t = 0;
+#pragma unroll 16
+  for (uint32_t r = 0; r < replicas; ++r) t += in[(uint64_t)r * k + q];
+  out[q] = t;
+}
+
+// One wave per hedge with more than PP_WAVE pins.  GMEM = false: the (partition, count, dst
 // count) table lives in LDS with `cap` slots; GMEM = true (hedges whose table would not fit
 // in LDS): in HBM at gtab + 3 * goff[i], sized by pp_table_cap.  The list is written sorted
 // by partition id (the table, compacted into its own first slots and padded to a power of
@@ -175,15 +271,14 @@ __global__ void __launch_bounds__(64) k_pp_large(const uint32_t* __restrict__ he
                                                  const uint32_t* __restrict__ list, uint32_t cap, uint32_t k,
                                                  const uint64_t* __restrict__ goff, uint32_t* __restrict__ gtab,
                                                  uint2* __restrict__ pp, uint32_t* __restrict__ lambda,
-                                                 uint4* __restrict__ hinfo,
-                                                 uint32_t* inbsz) {
+                                                 uint4* __restrict__ hinfo, uint32_t* inbsz, uint32_t replicas) {
   extern __shared__ uint32_t lds[];
   const uint32_t e = list[blockIdx.x];
-  uint32_t* keys = lds;
-  if (GMEM) {
-    cap = pp_table_cap(hoff[e + 1] - hoff[e], k);
-    keys = gtab + 3 * goff[blockIdx.x];
-  }
+  uint32_t* keys = GMEM ? gtab + 3 * goff[blockIdx.x] : lds;
+  // only the slots this hedge needs are cleared and compacted
+  const uint32_t need = pp_table_cap(hoff[e + 1] - hoff[e], k);
+  cap = GMEM ? need : min(need, cap);
+  if (INB) inbsz += (uint64_t)(blockIdx.x & (replicas - 1)) * k;
   uint32_t* cnt = keys + cap;
   uint32_t* dcnt = keys + 2 * cap;
   const uint32_t l = lane_id();
@@ -2444,14 +2539,14 @@ struct PartitionLists {
 // inbound-set constraint needs them; k-way does not).
 // The hedge classes of a level depend only on hedge lengths and k, so refine() computes them
 // in its first round and reuses them: for the partition-list kernels the pin count, the
-// hedges of more than PP_SMALL pins with LDS tables, those with HBM tables and their table
-// offsets; for the cascade the three classes of hedges above CAS_SMALL pins (for the
-// sort_max they were built with).
+// hedges of PP_SMALL < len <= PP_WAVE pins, the longer ones with LDS tables, those with HBM
+// tables and their table offsets; for the cascade the three classes of hedges above CAS_SMALL
+// pins (for the sort_max they were built with).
 struct LevelLayout {
   bool ready = false;
   uint64_t P = 0;
-  uint32_t nl = 0, ng = 0;
-  DBuf<uint32_t> large, glist;
+  uint32_t nl = 0, nlds = 0, ng = 0;
+  DBuf<uint32_t> large, llist, glist;  // large: all above PP_SMALL pins (masks), or up to PP_WAVE (lists)
   DBuf<uint64_t> goff;
   uint64_t gslots = 0;
   uint32_t cas_sort_max = 0xFFFFFFFFu;
@@ -2491,19 +2586,24 @@ void build_partition_lists(Ctx& c, const RefineLevel& L, const uint32_t* part, P
   pl.pp = DBuf<uint2>(c, P);
   pl.hinfo = DBuf<uint4>(c, L.e);
   pl.lambda = DBuf<uint32_t>(c, L.e);
+  DBuf<uint32_t> isz;  // replicas of the inbound sizes
+  uint32_t replicas = 1;
   if (want_inbound) {
-    pl.inbsz = DBuf<uint32_t>(c, std::max<uint32_t>(L.k, 1));
-    memset_async(c, pl.inbsz.get(), 0, (uint64_t)L.k * sizeof(uint32_t));
+    const uint32_t k1 = std::max<uint32_t>(L.k, 1);
+    while (replicas < PP_REPLICAS && 2ull * replicas * k1 <= PP_REPLICA_CAP) replicas <<= 1;
+    pl.inbsz = DBuf<uint32_t>(c, k1);
+    isz = DBuf<uint32_t>(c, (uint64_t)replicas * k1);
+    fill_u32(c, isz.get(), 0u, (uint64_t)replicas * k1);
   }
   DBuf<uint32_t> lflag;
   if (!Y.ready) lflag = DBuf<uint32_t>(c, L.e);
   if (want_inbound) {
     const uint32_t k_lds = L.k <= PP_HIST_CAP ? L.k : 0u;
     HGP_LAUNCH((k_pp_small<true>), ceil_div(L.e, 256), 256, k_lds * sizeof(uint32_t), c, L.hedges, L.hoff, L.srcc, part,
-               L.w, L.e, pl.pp.get(), pl.lambda.get(), pl.hinfo.get(), lflag.get(), pl.inbsz.get(), k_lds);
+               L.w, L.e, pl.pp.get(), pl.lambda.get(), pl.hinfo.get(), lflag.get(), isz.get(), k_lds, L.k, replicas);
   } else {
     HGP_LAUNCH((k_pp_small<false>), ceil_div(L.e, 256), 256, 0, c, L.hedges, L.hoff, L.srcc, part, L.w, L.e,
-               pl.pp.get(), pl.lambda.get(), pl.hinfo.get(), lflag.get(), (uint32_t*)nullptr, 0u);
+               pl.pp.get(), pl.lambda.get(), pl.hinfo.get(), lflag.get(), (uint32_t*)nullptr, 0u, 0u, 1u);
   }
   // Distinct partitions per hedge <= min(k, len).  Tables of up to PP_LDS_CAP slots sit in
   // LDS; hedges needing more (len and k both above ~2K) get HBM tables.
@@ -2514,25 +2614,32 @@ void build_partition_lists(Ctx& c, const RefineLevel& L, const uint32_t* part, P
     DBuf<uint64_t> pos(c, (uint64_t)L.e + 1);
     exclusive_scan(c, lflag.get(), pos.get(), L.e);
     Y.nl = (uint32_t)read_scalar(c, pos.get() + L.e);
-    if (Y.nl == 0) return;
-    Y.large = DBuf<uint32_t>(c, Y.nl);
-    DBuf<uint32_t> small(c, L.e - Y.nl);
-    // k_split puts flagged (large) entries first list
-    HGP_LAUNCH(k_split, ceil_div(L.e, 256), 256, 0, c, lflag.get(), pos.get(), L.e, Y.large.get(), small.get());
-    if (L.k > lds_max_len) {
-      DBuf<uint32_t> gflag(c, Y.nl);
-      DBuf<uint64_t> gpos(c, (uint64_t)Y.nl + 1);
-      HGP_LAUNCH(k_flag_longer, ceil_div(Y.nl, 256), 256, 0, c, Y.large.get(), Y.nl, L.hoff, (uint64_t)lds_max_len,
-                 gflag.get());
-      exclusive_scan(c, gflag.get(), gpos.get(), Y.nl);
-      Y.ng = (uint32_t)read_scalar(c, gpos.get() + Y.nl);
+    if (Y.nl) {
+      Y.large = DBuf<uint32_t>(c, Y.nl);
+      DBuf<uint32_t> small(c, L.e - Y.nl);
+      // k_split puts flagged (large) entries first list
+      HGP_LAUNCH(k_split, ceil_div(L.e, 256), 256, 0, c, lflag.get(), pos.get(), L.e, Y.large.get(), small.get());
+      // moves the listed hedges of more than max_len pins to a list of their own
+      auto split_longer = [&](DBuf<uint32_t>& list, uint32_t& m, uint64_t max_len, DBuf<uint32_t>& longer, uint32_t& ml) {
+        if (m == 0) return;
+        DBuf<uint32_t> flag(c, m);
+        DBuf<uint64_t> lpos(c, (uint64_t)m + 1);
+        HGP_LAUNCH(k_flag_longer, ceil_div(m, 256), 256, 0, c, list.get(), m, L.hoff, max_len, flag.get());
+        exclusive_scan(c, flag.get(), lpos.get(), m);
+        ml = (uint32_t)read_scalar(c, lpos.get() + m);
+        if (ml == 0) return;
+        DBuf<uint32_t> rest(c, m - ml);
+        longer = DBuf<uint32_t>(c, ml);
+        HGP_LAUNCH(k_split_list, ceil_div(m, 256), 256, 0, c, flag.get(), lpos.get(), list.get(), m, longer.get(),
+                   rest.get());
+        list = std::move(rest);
+        m -= ml;
+      };
+      // (the wave's keys hold a partition id and a bit when the inbound sizes are wanted)
+      const bool wide_ids = want_inbound && L.k > 0x7FFFFFFFu;
+      split_longer(Y.large, Y.nl, wide_ids ? PP_SMALL : PP_WAVE, Y.llist, Y.nlds);
+      if (L.k > lds_max_len) split_longer(Y.llist, Y.nlds, lds_max_len, Y.glist, Y.ng);
       if (Y.ng) {
-        DBuf<uint32_t> lds_list(c, Y.nl - Y.ng);
-        Y.glist = DBuf<uint32_t>(c, Y.ng);
-        HGP_LAUNCH(k_split_list, ceil_div(Y.nl, 256), 256, 0, c, gflag.get(), gpos.get(), Y.large.get(), Y.nl,
-                   Y.glist.get(), lds_list.get());
-        Y.large = std::move(lds_list);
-        Y.nl -= Y.ng;
         DBuf<uint64_t> gcap(c, Y.ng);
         Y.goff = DBuf<uint64_t>(c, (uint64_t)Y.ng + 1);
         HGP_LAUNCH(k_pp_gcap, ceil_div(Y.ng, 256), 256, 0, c, Y.glist.get(), Y.ng, L.hoff, L.k, gcap.get());
@@ -2541,20 +2648,25 @@ void build_partition_lists(Ctx& c, const RefineLevel& L, const uint32_t* part, P
       }
     }
   }
-  auto launch = [&](auto inb, auto gmem, const uint32_t* lst, uint32_t m, const uint64_t* goff, uint32_t* gtab) {
-    constexpr bool INB = decltype(inb)::value, GMEM = decltype(gmem)::value;
-    if (m == 0) return;
-    HGP_LAUNCH((k_pp_large<INB, GMEM>), m, 64, GMEM ? 0 : 3 * cap * sizeof(uint32_t), c, L.hedges, L.hoff, L.srcc, part,
-               L.w, lst, cap, L.k, goff, gtab, pl.pp.get(), pl.lambda.get(), pl.hinfo.get(), INB ? pl.inbsz.get() : (uint32_t*)nullptr);
+  DBuf<uint32_t> gtab(c, 3 * Y.gslots);
+  auto launch = [&](auto inb) {
+    constexpr bool INB = decltype(inb)::value;
+    if (Y.nl)
+      HGP_LAUNCH((k_pp_wave<INB>), ceil_div(Y.nl, 4), 256, 0, c, L.hedges, L.hoff, L.srcc, part, L.w, Y.large.get(),
+                 Y.nl, pl.pp.get(), pl.lambda.get(), pl.hinfo.get(), isz.get(), L.k, replicas);
+    if (Y.nlds)
+      HGP_LAUNCH((k_pp_large<INB, false>), Y.nlds, 64, 3 * cap * sizeof(uint32_t), c, L.hedges, L.hoff, L.srcc, part,
+                 L.w, Y.llist.get(), cap, L.k, (const uint64_t*)nullptr, (uint32_t*)nullptr, pl.pp.get(),
+                 pl.lambda.get(), pl.hinfo.get(), isz.get(), replicas);
+    if (Y.ng)
+      HGP_LAUNCH((k_pp_large<INB, true>), Y.ng, 64, 0, c, L.hedges, L.hoff, L.srcc, part, L.w, Y.glist.get(), cap, L.k,
+                 Y.goff.get(), gtab.get(), pl.pp.get(), pl.lambda.get(), pl.hinfo.get(), isz.get(), replicas);
   };
-  using T = std::true_type;
-  using F = std::false_type;
-  if (want_inbound) launch(T{}, F{}, Y.large.get(), Y.nl, nullptr, nullptr);
-  else launch(F{}, F{}, Y.large.get(), Y.nl, nullptr, nullptr);
-  if (Y.ng) {
-    DBuf<uint32_t> gtab(c, 3 * Y.gslots);
-    if (want_inbound) launch(T{}, T{}, Y.glist.get(), Y.ng, Y.goff.get(), gtab.get());
-    else launch(F{}, T{}, Y.glist.get(), Y.ng, Y.goff.get(), gtab.get());
+  if (want_inbound) {
+    launch(std::true_type{});
+    HGP_LAUNCH(k_sum_replicas, ceil_div(L.k, 256), 256, 0, c, isz.get(), L.k, replicas, pl.inbsz.get());
+  } else {
+    launch(std::false_type{});
   }
 }
 

@@ -306,6 +306,34 @@ def test_refine_analyze_huge_lists(dev, mode, k, fm_repeat, chainup, n, e, max_s
     assert got["best"] == exp["best"]
 
 
+@pytest.mark.parametrize("k,spread", [(1, 1), (70, 70), (70, 2), (40000, 40000)])
+def test_partition_lists_by_hedge_length(dev, k, spread, rng):
+    """Partition lists at the edges of their kernels (16 pins by thread, up to 64, 128 and 256 in a
+    wave's registers, longer ones in LDS and HBM tables): the inbound sizes and lambda-1 that
+    follow from them, with few and with many distinct partitions per hedge."""
+    lens = [1, 2, 16, 17, 63, 64, 65, 127, 128, 129, 255, 256, 257, 511, 2016, 2017, 2500] * 3
+    n, off, pins, srcc = 4000, [0], [], []
+    for i, ln in enumerate(lens):
+        pins.extend(int(x) for x in rng.choice(n, size=ln, replace=False))
+        off.append(len(pins))
+        srcc.append(min(i % 3, ln))
+    hg = O.HG(n, np.array(off, np.uint64), np.array(pins, np.uint32), np.array(srcc, np.uint32),
+              rng.integers(1, 5, size=len(lens)).astype(np.float32))
+    part = (rng.integers(0, spread, size=n) + k - spread).astype(np.uint32)
+    L = G.Level(dev, hg)
+    d_part = dev.upload(part)
+    d_out = dev.alloc(4 * k)
+    dev.check(dev.lib.hgp_inbound_sizes(dev.ctx, G.V(L.pins), G.V(L.off), G.V(L.srcc), G.V(d_part), hg.e, k,
+                                        G.V(d_out)), "inbound sizes")
+    assert np.array_equal(dev.download(d_out, k, np.uint32), O.inbound_sizes(hg, part, k))
+    for p2 in (part, part + np.uint32(0xFFFE0000)):  # ids that fill 32 bits
+        d_p2 = dev.upload(p2)
+        km1 = C.c_int64()
+        dev.check(dev.lib.hgp_connectivity(dev.ctx, G.V(L.pins), G.V(L.off), G.V(L.w), G.V(d_p2), hg.e, C.byref(km1)),
+                  "connectivity")
+        assert km1.value == O.connectivity_fixed(hg, part)
+
+
 @pytest.mark.parametrize("k", [5, 300, 66000])
 @pytest.mark.parametrize("dup", [False, True])
 def test_refine_analyze_inbound_by_hedge_size(dev, k, dup, rng):
