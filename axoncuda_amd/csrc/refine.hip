@@ -1527,6 +1527,24 @@ __global__ void __launch_bounds__(256) k_jacobi_apply(const uint32_t* __restrict
 }
 
 // partitions in descending mix32(q + repeat) order (mix32 is a bijection: no ties)
+// up to ORDER_DIRECT partitions: every thread counts the hashes above its own (they are distinct)
+// in LDS, one launch of a few microseconds instead of the four passes of a 32-bit sort (23 us)
+constexpr uint32_t ORDER_DIRECT = 4096;
+__global__ void __launch_bounds__(256) k_order_direct(uint32_t k, uint32_t repeat, uint32_t* __restrict__ order) {
+  __shared__ __align__(16) uint32_t h[ORDER_DIRECT];
+  const uint32_t k4 = (k + 3) & ~3u;  // padded with zeros: below or equal to every hash, never above
+  for (uint32_t q = threadIdx.x; q < k4; q += 256) h[q] = q < k ? mix32(q + repeat) : 0u;
+  __syncthreads();
+  const uint32_t q = blockIdx.x * 256 + threadIdx.x;
+  if (q >= k) return;
+  const uint32_t mine = h[q];
+  uint32_t above = 0;
+  for (uint32_t i = 0; i < k4; i += 4) {
+    const uint4 x = *reinterpret_cast<const uint4*>(&h[i]);
+    above += (x.x > mine) + (x.y > mine) + (x.z > mine) + (x.w > mine);
+  }
+  order[above] = q;
+}
 __global__ void k_order_keys(uint32_t k, uint32_t repeat, uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
   const uint32_t q = blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= k) return;
@@ -1594,35 +1612,123 @@ __global__ void k_heavy_tabcap(const uint32_t* __restrict__ list, const uint64_t
 }
 
 // ---- 3. ranking -------------------------------------------------------------------------
-__global__ void k_rank_keys_gain(const uint32_t* __restrict__ moves, const int64_t* __restrict__ gains, uint32_t n,
-                                 uint64_t* __restrict__ keys, uint32_t* __restrict__ vals) {
-  uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
+// Sort keys are built over the bits that vary.  Gains are 2^18 fixed point, so with whole-number
+// weights their low 18 bits are zero, and a round's gains span a few hundred whole numbers: one
+// pass over the moves finds their range, the trailing zeros they share and how many there are,
+// and the sorts' keys are (more significant class) << gb | (max - gain) >> tz.
+struct KeyStats {
+  unsigned long long mn, mx;  // smallest and largest value (ordered_i64)
+  unsigned long long bits;    // OR of the values: trailing zeros are shared by all
+  unsigned long long count;   // valid entries
+  unsigned long long odd;     // chaining: a component without its head exists
+};
+struct KeyCode {
+  uint64_t mx = 0;
+  int tz = 0, bits = 0;  // code = (mx - ordered value) >> tz, below 2^bits
+};
+KeyCode key_code(const KeyStats& st) {
+  KeyCode k;
+  if (st.count == 0 || st.mx == st.mn) {
+    k.mx = st.mx;
+    k.tz = st.count ? 63 : 0;  // all equal: every code is 0
+    return k;
+  }
+  k.mx = st.mx;
+  k.tz = st.bits ? __builtin_ctzll(st.bits) : 0;
+  k.bits = bit_width((st.mx - st.mn) >> k.tz);
+  return k;
+}
+__device__ __forceinline__ uint64_t gain_code(int64_t g, uint64_t mx, int tz) { return (mx - ordered_i64(g)) >> tz; }
+
+__global__ void k_init_stats(KeyStats* st) { *st = KeyStats{~0ull, 0ull, 0ull, 0ull, 0ull}; }
+// this thread's (min, max, or, count) into *st, one set of atomics per workgroup of 256
+__device__ __forceinline__ void add_stats(uint64_t mn, uint64_t mx, uint64_t bits, uint32_t count, KeyStats* st) {
+  __shared__ uint64_t s_mn[4], s_mx[4], s_or[4];
+  __shared__ uint32_t s_n[4];
+  mn = wave_min(mn);
+  mx = wave_max(mx);
+  bits = wave_reduce(bits, [](uint64_t a, uint64_t b) { return a | b; });
+  count = wave_sum(count);
+  if (lane_id() == 0) {
+    const uint32_t w = threadIdx.x / 64;
+    s_mn[w] = mn;
+    s_mx[w] = mx;
+    s_or[w] = bits;
+    s_n[w] = count;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int i = 1; i < 4; ++i) {
+      mn = s_mn[i] < mn ? s_mn[i] : mn;
+      mx = s_mx[i] > mx ? s_mx[i] : mx;
+      bits |= s_or[i];
+      count += s_n[i];
+    }
+    if (count) {
+      atomicMin(&st->mn, (unsigned long long)mn);
+      atomicMax(&st->mx, (unsigned long long)mx);
+      atomicOr(&st->bits, (unsigned long long)bits);
+      atomicAdd(&st->count, (unsigned long long)count);
+    }
+  }
+}
+__global__ void __launch_bounds__(256) k_gain_stats(const uint32_t* __restrict__ moves, const int64_t* __restrict__ gains,
+                                                    uint32_t n, KeyStats* st) {
+  uint64_t mn = ~0ull, mx = 0, bits = 0;
+  uint32_t count = 0;
+  for (uint32_t v = blockIdx.x * 256 + threadIdx.x; v < n; v += gridDim.x * 256) {
+    if (moves[v] == NONE) continue;
+    const int64_t g = gains[v];
+    const uint64_t o = ordered_i64(g);
+    mn = o < mn ? o : mn;
+    mx = o > mx ? o : mx;
+    bits |= (uint64_t)g;
+    ++count;
+  }
+  add_stats(mn, mx, bits, count, st);
+}
+// the summed gains of the components of valid moves, and the component count (the scan's total)
+__global__ void __launch_bounds__(256) k_comp_stats(const uint32_t* __restrict__ cflag, const long long* __restrict__ cw,
+                                                    const uint32_t* __restrict__ cinv, uint32_t n, KeyStats* st) {
+  uint64_t mn = ~0ull, mx = 0, bits = 0;
+  uint32_t count = 0;
+  for (uint32_t j = blockIdx.x * 256 + threadIdx.x; j < n; j += gridDim.x * 256) {
+    if (!cflag[j]) continue;
+    if (!cinv[j]) {
+      const int64_t g = (int64_t)cw[j];
+      const uint64_t o = ordered_i64(g);
+      mn = o < mn ? o : mn;
+      mx = o > mx ? o : mx;
+      bits |= (uint64_t)g;
+    }
+    ++count;
+  }
+  add_stats(mn, mx, bits, count, st);
+}
+// key = (source partition << 1 | invalid) << gb | gain code (part == nullptr: no partition); with
+// gb < 0 the gain code alone
+template <typename K>
+__global__ void k_move_keys(const uint32_t* __restrict__ part, const uint32_t* __restrict__ moves,
+                            const int64_t* __restrict__ gains, uint32_t n, uint64_t mx, int tz, int gb,
+                            K* __restrict__ keys, uint32_t* __restrict__ vals) {
+  const uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
   if (v >= n) return;
-  keys[v] = moves[v] == NONE ? 0ull : ~ordered_i64(gains[v]);
+  const bool invalid = moves[v] == NONE;
+  const K hi = (part ? (K)part[v] << 1 : (K)0) | (invalid ? 1u : 0u);
+  keys[v] = (gb < 0 ? (K)0 : (K)(hi << gb)) | (invalid ? (K)0 : (K)gain_code(gains[v], mx, tz));
   vals[v] = v;
 }
-__global__ void k_invalid_keys(const uint32_t* __restrict__ moves, const uint32_t* __restrict__ vals, uint32_t n,
-                               uint32_t* __restrict__ keys) {
-  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) keys[i] = moves[vals[i]] == NONE ? 1u : 0u;
+// (source partition << 1) | invalid (part == nullptr: invalid), in the order of vals
+__global__ void k_part_keys(const uint32_t* __restrict__ part, const uint32_t* __restrict__ moves,
+                            const uint32_t* __restrict__ vals, uint32_t n, uint32_t* __restrict__ k2) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const uint32_t v = vals[i];
+  k2[i] = (part ? part[v] << 1 : 0u) | (moves[v] == NONE ? 1u : 0u);
 }
 __global__ void k_scatter_ranks(const uint32_t* __restrict__ vals, uint32_t n, uint32_t* __restrict__ ranks) {
   uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
   if (r < n) ranks[vals[r]] = r;
-}
-// grid-stride count, reduced per workgroup: one atomic per workgroup
-__global__ void __launch_bounds__(256) k_count_valid(const uint32_t* __restrict__ moves, uint32_t n, uint32_t* cnt) {
-  __shared__ uint32_t s_part[4];
-  uint32_t c = 0;
-  for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += gridDim.x * blockDim.x)
-    c += moves[v] != NONE ? 1u : 0u;
-  c = wave_sum(c);
-  if (lane_id() == 0) s_part[threadIdx.x / 64] = c;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const uint32_t t = s_part[0] + s_part[1] + s_part[2] + s_part[3];
-    if (t) atomicAdd(cnt, t);
-  }
 }
 
 // zeroes three arrays of n entries in one launch (instead of three fills)
@@ -1638,69 +1744,46 @@ __global__ void k_zero3(unsigned long long* __restrict__ a, uint32_t* __restrict
 // chaining: edges in sorted space j (by source partition asc, valid first, gain desc)
 struct ChainArrays {
   const uint32_t* orig;  // j -> node
-  uint32_t* src;
-  uint32_t* dst;
-  uint32_t* sz;
-  int64_t* w;
-  uint32_t* ok;
-  uint32_t* ob;
-  uint32_t* oe;
+  uint4* pk;             // per entry: gain (lo, hi), size, valid
+  uint2* range;          // per entry: its target partition's entries (empty when invalid)
+  uint32_t* from;        // per entry: where its next proposal scan starts
   uint32_t* next;
   uint32_t* prev;
   unsigned long long* claim;
-  uint32_t* progress;  // progress[it] != 0: iteration it committed a link
-  uint4* pk;           // per entry: gain (lo, hi), size, valid -- what a proposal scan reads
-  uint32_t* from;      // per entry: where its next proposal scan starts
+  uint32_t* progress;    // progress[it] != 0: iteration it committed a link
+  // components, by head entry: summed gain, moves, holds an invalid move, exists
+  long long* cw;
+  uint32_t* csize;
+  uint32_t* cinv;
+  uint32_t* cflag;
 };
 // An iteration after one that committed nothing would repeat it exactly: skip it.
 __device__ __forceinline__ bool chain_stalled(const ChainArrays& c, int it) {
   return it > 0 && c.progress[it - 1] == 0;
 }
 
-__global__ void k_chain_sortkeys(const uint32_t* __restrict__ part, const uint32_t* __restrict__ moves,
-                                 const int64_t* __restrict__ gains, uint32_t n, uint64_t* __restrict__ k1,
-                                 uint32_t* __restrict__ vals) {
-  uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= n) return;
-  k1[v] = moves[v] == NONE ? 0ull : ~ordered_i64(gains[v]);
-  vals[v] = v;
-}
-// second (more significant) pass key: (source partition << 1) | invalid
-__global__ void k_chain_sortkeys2(const uint32_t* __restrict__ part, const uint32_t* __restrict__ moves,
-                                  const uint32_t* __restrict__ vals, uint32_t n, uint32_t* __restrict__ k2) {
-  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const uint32_t v = vals[i];
-  k2[i] = (part[v] << 1) | (moves[v] == NONE ? 1u : 0u);
-}
-__global__ void k_chain_gather(ChainArrays c, const uint32_t* __restrict__ part, const uint32_t* __restrict__ moves,
-                               const int64_t* __restrict__ gains, const uint32_t* __restrict__ sizes, uint32_t n) {
-  uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
+// Everything an entry starts with, in one launch.  poff: the entries of each source partition.
+__global__ void k_chain_gather(ChainArrays c, const uint32_t* __restrict__ moves, const int64_t* __restrict__ gains,
+                               const uint32_t* __restrict__ sizes, const uint64_t* __restrict__ poff, uint32_t n,
+                               KeyStats* comp_stats) {
+  const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (j < 4) c.progress[j] = 0u;
+  if (j == 0) *comp_stats = KeyStats{~0ull, 0ull, 0ull, 0ull, 0ull};
   if (j >= n) return;
   const uint32_t v = c.orig[j];
-  c.src[j] = part[v];
-  c.dst[j] = moves[v];
-  c.sz[j] = sizes[v];
-  c.w[j] = gains[v];
-  c.ok[j] = moves[v] != NONE;
-  c.pk[j] = make_uint4((uint32_t)(uint64_t)gains[v], (uint32_t)((uint64_t)gains[v] >> 32), sizes[v],
-                       moves[v] != NONE ? 1u : 0u);
+  const uint32_t q = moves[v];
+  const int64_t g = gains[v];
+  c.pk[j] = make_uint4((uint32_t)(uint64_t)g, (uint32_t)((uint64_t)g >> 32), sizes[v], q != NONE ? 1u : 0u);
+  const uint2 r = q != NONE ? make_uint2((uint32_t)poff[q], (uint32_t)poff[q + 1]) : make_uint2(0u, 0u);
+  c.range[j] = r;
+  c.from[j] = r.x;
   c.next[j] = NONE;
   c.prev[j] = NONE;
   c.claim[j] = 0ull;
-}
-__global__ void k_chain_ranges(ChainArrays c, const uint64_t* __restrict__ poff, uint32_t n) {
-  uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= n) return;
-  if (!c.ok[j]) {
-    c.ob[j] = 0;
-    c.oe[j] = 0;
-    return;
-  }
-  const uint32_t q = c.dst[j];
-  c.ob[j] = (uint32_t)poff[q];
-  c.oe[j] = (uint32_t)poff[q + 1];
-  c.from[j] = c.ob[j];
+  c.cw[j] = 0;
+  c.csize[j] = 0u;
+  c.cinv[j] = 0u;
+  c.cflag[j] = 0u;
 }
 __device__ __forceinline__ int size_bucket(uint32_t s) { return s == 0 ? 0 : 31 - __clz(s); }
 
@@ -1728,11 +1811,13 @@ __global__ void __launch_bounds__(RESOLVE_BLOCK) k_chain_propose(ChainArrays c, 
   }
   const uint32_t i = blockIdx.x * RESOLVE_BLOCK + threadIdx.x;
   uint32_t choice = NONE;
-  if (i < n && c.next[i] == NONE && c.ob[i] < c.oe[i]) {
-    const uint32_t si = c.sz[i];
+  const uint2 range = i < n ? c.range[i] : make_uint2(0u, 0u);
+  uint32_t si = 0, choice_size = 0;
+  if (range.x < range.y && c.next[i] == NONE) {
+    si = c.pk[i].z;
     const int bi = size_bucket(si);
-    const uint32_t lim = min(c.oe[i], c.ob[i] + 256u);
-    const uint32_t j0 = max(c.from[i], c.ob[i]);
+    const uint32_t lim = min(range.y, range.x + 256u);
+    const uint32_t j0 = c.from[i];
     uint32_t first = lim;  // first entry that could be chosen (scan end when none)
     int64_t bw = 0;
     uint32_t bd = 0;
@@ -1769,6 +1854,7 @@ __global__ void __launch_bounds__(RESOLVE_BLOCK) k_chain_propose(ChainArrays c, 
         if (choice == NONE) first = j;
         if (choice == NONE || wj > bw || (wj == bw && d < bd)) {
           choice = j;
+          choice_size = sj;
           bw = wj;
           bd = d;
           if (d == 0) {  // later entries gain no more and cannot have a smaller difference
@@ -1782,7 +1868,7 @@ __global__ void __launch_bounds__(RESOLVE_BLOCK) k_chain_propose(ChainArrays c, 
   }
   __syncthreads();  // the table is cleared
   if (choice != NONE && c.prev[choice] == NONE) {
-    const uint32_t d = c.sz[i] > c.sz[choice] ? c.sz[i] - c.sz[choice] : c.sz[choice] - c.sz[i];
+    const uint32_t d = si > choice_size ? si - choice_size : choice_size - si;
     const unsigned long long key = ((unsigned long long)(0xFFFFFFFFu - d) << 32) | (0xFFFFFFFFu - i);
     uint32_t h = slot_hash(choice) & (RESOLVE_SLOTS - 1);
     for (;;) {
@@ -1810,12 +1896,23 @@ __global__ void k_chain_commit(ChainArrays c, uint32_t n, int it) {
 }
 // comp / pos: each move's component (its chain's head) and its distance from the head; a
 // chain whose head is not found within 256 steps (a cycle, or a longer chain) is keyed by
-// its lowest index at position 0 and raises *odd.  csize counts each component's moves.
+// its lowest index at position 0 and raises odd.  csize counts each component's moves.  A move
+// without links is its component's only member: plain stores.
 __global__ void k_chain_comp(ChainArrays c, uint32_t n, uint32_t* __restrict__ comp, uint32_t* __restrict__ pos,
-                             uint32_t* __restrict__ cflag, long long* __restrict__ cw,
-                             uint32_t* __restrict__ cinv, uint32_t* __restrict__ csize, uint32_t* __restrict__ odd) {
+                             KeyStats* st) {
   uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
+  const uint4 e = c.pk[i];
+  const long long w = (long long)(((uint64_t)e.y << 32) | e.x);
+  if (c.prev[i] == NONE && c.next[i] == NONE) {
+    comp[i] = i;
+    pos[i] = 0;
+    c.cflag[i] = 1u;
+    c.csize[i] = 1u;
+    if (e.w) c.cw[i] = w;
+    else c.cinv[i] = 1u;
+    return;
+  }
   uint32_t cur = i, mn = i, cc = NONE, ps = 0;
   for (uint32_t d = 0; d < 256; ++d) {
     const uint32_t p = c.prev[cur];
@@ -1830,34 +1927,35 @@ __global__ void k_chain_comp(ChainArrays c, uint32_t n, uint32_t* __restrict__ c
   if (cc == NONE) {
     cc = mn;
     ps = 0;
-    *odd = 1u;
+    st->odd = 1ull;
   }
   comp[i] = cc;
   pos[i] = ps;
-  cflag[cc] = 1u;
-  atomicAdd(&csize[cc], 1u);
-  if (c.ok[i]) atomicAdd((unsigned long long*)&cw[cc], (unsigned long long)c.w[i]);  // two's complement sum
-  else atomicOr(&cinv[cc], 1u);
+  c.cflag[cc] = 1u;
+  atomicAdd(&c.csize[cc], 1u);
+  if (e.w) atomicAdd((unsigned long long*)&c.cw[cc], (unsigned long long)w);  // two's complement sum
+  else atomicOr(&c.cinv[cc], 1u);
 }
-__global__ void k_comp_list(const uint32_t* __restrict__ cflag, const uint64_t* __restrict__ cpos, uint32_t n,
-                            const long long* __restrict__ cw, const uint32_t* __restrict__ cinv,
-                            uint32_t* __restrict__ clist, uint64_t* __restrict__ ckey, uint32_t* __restrict__ cinvk) {
+// the components in ascending head order with their sort keys: invalid << gb | code of the summed
+// gain (a component made of an invalid move sums to 0 and goes behind every valid one); with
+// gb < 0 the code alone
+template <typename K>
+__global__ void k_comp_list(ChainArrays c, const uint64_t* __restrict__ cpos, uint32_t n, uint64_t mx, int tz, int gb,
+                            uint32_t* __restrict__ clist, K* __restrict__ ckey) {
   uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= n || !cflag[j]) return;
+  if (j >= n || !c.cflag[j]) return;
   const uint64_t o = cpos[j];
   clist[o] = j;
-  ckey[o] = ~ordered_i64((int64_t)cw[j]);
-  cinvk[o] = cinv[j];
+  ckey[o] = c.cinv[j] ? (gb < 0 ? (K)0 : (K)1 << gb) : (K)gain_code((int64_t)c.cw[j], mx, tz);
 }
-__global__ void k_comp_rank(const uint32_t* __restrict__ clist, uint32_t m, uint32_t* __restrict__ crank) {
-  uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r < m) crank[clist[r]] = r;
-}
-// sizes of the components in rank order
-__global__ void k_comp_sizes(const uint32_t* __restrict__ clist, const uint32_t* __restrict__ csize, uint32_t m,
-                             uint32_t* __restrict__ out) {
+// rank of each component, and the sizes in rank order
+__global__ void k_comp_rank(const uint32_t* __restrict__ clist, const uint32_t* __restrict__ csize, uint32_t m,
+                            uint32_t* __restrict__ crank, uint32_t* __restrict__ rsz) {
   const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r < m) out[r] = csize[clist[r]];
+  if (r >= m) return;
+  const uint32_t j = clist[r];
+  crank[j] = r;
+  rsz[r] = csize[j];
 }
 // Every chain has its head: a move's rank is its component's start (the sizes of the
 // components ranked before it) plus its distance from the head -- the position the stable
@@ -1868,16 +1966,13 @@ __global__ void k_chain_direct_ranks(const uint32_t* __restrict__ comp, const ui
   const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
   if (j < n) ranks[orig[j]] = (uint32_t)(start[crank[comp[j]]] + pos[j]);
 }
-__global__ void k_pack2(const uint64_t* __restrict__ a, const uint32_t* __restrict__ b, uint64_t* __restrict__ out) {
-  out[0] = a[0];
-  out[1] = b[0];
-}
+template <typename K>
 __global__ void k_edge_keys(const uint32_t* __restrict__ comp, const uint32_t* __restrict__ pos,
-                            const uint32_t* __restrict__ crank, uint32_t n, uint64_t* __restrict__ keys,
+                            const uint32_t* __restrict__ crank, uint32_t n, K* __restrict__ keys,
                             uint32_t* __restrict__ vals) {
   uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= n) return;
-  keys[j] = ((uint64_t)crank[comp[j]] << 8) | pos[j];
+  keys[j] = ((K)crank[comp[j]] << 8) | pos[j];
   vals[j] = j;
 }
 __global__ void k_edge_ranks(const uint32_t* __restrict__ sorted_j, const uint32_t* __restrict__ orig, uint32_t n,
@@ -2680,9 +2775,14 @@ void compute_gains(Ctx& c, const RefineLevel& L, const PartitionLists& pl, int m
                    uint32_t discount, const uint32_t* part, const uint32_t* psizes, uint32_t* moves, int64_t* gains) {
   // hash order of partitions for the non-adjacent fallback, sorted on the device
   const uint32_t kk = std::max<uint32_t>(L.k, 1);
-  DBuf<uint32_t> okeys(c, kk), dorder(c, kk);
-  HGP_LAUNCH(k_order_keys, ceil_div(L.k, 256), 256, 0, c, L.k, repeat, okeys.get(), dorder.get());
-  radix_sort(c, okeys.get(), dorder.get(), L.k, 32);
+  DBuf<uint32_t> dorder(c, kk);
+  if (L.k <= ORDER_DIRECT) {
+    HGP_LAUNCH(k_order_direct, ceil_div(L.k, 256), 256, 0, c, L.k, repeat, dorder.get());
+  } else {
+    DBuf<uint32_t> okeys(c, kk);
+    HGP_LAUNCH(k_order_keys, ceil_div(L.k, 256), 256, 0, c, L.k, repeat, okeys.get(), dorder.get());
+    radix_sort(c, okeys.get(), dorder.get(), L.k, 32);
+  }
   GainArgs a{};
   a.tch = L.tch;
   a.toff = L.toff;
@@ -2774,75 +2874,105 @@ void compute_gains(Ctx& c, const RefineLevel& L, const PartitionLists& pl, int m
   }
 }
 
-void rank_by_gain(Ctx& c, uint32_t n, const uint32_t* moves, const int64_t* gains, uint32_t* ranks) {
+KeyStats gain_stats(Ctx& c, uint32_t n, const uint32_t* moves, const int64_t* gains) {
+  DBuf<KeyStats> st(c, 1);
+  HGP_LAUNCH(k_init_stats, 1, 1, 0, c, st.get());
+  HGP_LAUNCH(k_gain_stats, std::min<uint32_t>(ceil_div(n, 256), 256), 256, 0, c, moves, gains, n, st.get());
+  return read_scalar(c, st.get());
+}
+
+// Runs f with a 32-bit key type when the keys fit, else with a 64-bit one.
+template <typename F>
+void with_key_type(int bits, F&& f) {
+  if (bits <= 32) f(uint32_t{});
+  else f(uint64_t{});
+}
+
+// vals = the nodes by (source partition asc, when part is given; valid first; gain desc; id).
+// poff (with part): the entries of each partition.
+void sort_moves(Ctx& c, uint32_t n, uint32_t k, const uint32_t* part, const uint32_t* moves, const int64_t* gains,
+                const KeyStats& gst, DBuf<uint32_t>& vals, uint64_t* poff) {
+  const uint32_t g = ceil_div(n, 256);
+  const KeyCode kc = key_code(gst);
+  const int pb = part ? std::max(2, bit_width(2ull * k - 1)) : 1;
+  if (kc.bits + pb <= 64) {
+    with_key_type(kc.bits + pb, [&](auto key) {
+      DBuf<decltype(key)> keys(c, n);
+      HGP_LAUNCH((k_move_keys<decltype(key)>), g, 256, 0, c, part, moves, gains, n, kc.mx, kc.tz, kc.bits, keys.get(),
+                 vals.get());
+      radix_sort_buf(c, keys, vals, n, 0, kc.bits + pb);
+      if (part) segment_offsets(c, keys.get(), kc.bits + 1, n, k, poff);
+    });
+    return;
+  }
+  // a wider range of gains: by gain, then stably by (partition, invalid)
   DBuf<uint64_t> keys(c, n);
-  DBuf<uint32_t> vals(c, n), k2(c, n);
-  HGP_LAUNCH(k_rank_keys_gain, ceil_div(n, 256), 256, 0, c, moves, gains, n, keys.get(), vals.get());
-  radix_sort_range_buf(c, keys, vals, n);
-  HGP_LAUNCH(k_invalid_keys, ceil_div(n, 256), 256, 0, c, moves, vals.get(), n, k2.get());
-  radix_sort_buf(c, k2, vals, n, 0, 1);
+  DBuf<uint32_t> k2(c, n);
+  HGP_LAUNCH((k_move_keys<uint64_t>), g, 256, 0, c, part, moves, gains, n, kc.mx, kc.tz, -1, keys.get(), vals.get());
+  radix_sort_buf(c, keys, vals, n, 0, kc.bits);
+  HGP_LAUNCH(k_part_keys, g, 256, 0, c, part, moves, vals.get(), n, k2.get());
+  radix_sort_buf(c, k2, vals, n, 0, pb);
+  if (part) segment_offsets(c, k2.get(), 1, n, k, poff);
+}
+
+// by (valid first, gain desc, node id)
+void rank_by_gain(Ctx& c, uint32_t n, const uint32_t* moves, const int64_t* gains, const KeyStats& gst,
+                  uint32_t* ranks) {
+  if (n == 0) return;
+  DBuf<uint32_t> vals(c, n);
+  sort_moves(c, n, 1, nullptr, moves, gains, gst, vals, nullptr);
   HGP_LAUNCH(k_scatter_ranks, ceil_div(n, 256), 256, 0, c, vals.get(), n, ranks);
 }
 
 void rank_by_chaining(Ctx& c, uint32_t n, uint32_t k, const uint32_t* part, const uint32_t* moves, const int64_t* gains,
-                      const uint32_t* sizes, uint32_t* ranks) {
+                      const KeyStats& gst, const uint32_t* sizes, uint32_t* ranks) {
+  if (n == 0) return;
   const uint32_t g = ceil_div(n, 256);
   // sorted space: stable by (src partition asc, valid first, gain desc), ties by node id
-  DBuf<uint64_t> k1(c, n);
-  DBuf<uint32_t> orig(c, n), k2(c, n);
-  HGP_LAUNCH(k_chain_sortkeys, g, 256, 0, c, part, moves, gains, n, k1.get(), orig.get());
-  radix_sort_range_buf(c, k1, orig, n);
-  HGP_LAUNCH(k_chain_sortkeys2, g, 256, 0, c, part, moves, orig.get(), n, k2.get());
-  radix_sort_buf(c, k2, orig, n, 0, bit_width(2ull * k + 1));
-  k1.reset();
-  DBuf<uint32_t> src(c, n), dst(c, n), sz(c, n), ok(c, n), ob(c, n), oe(c, n), next(c, n), prev(c, n);
-  DBuf<int64_t> w(c, n);
-  DBuf<unsigned long long> claim(c, n);
-  DBuf<uint32_t> progress(c, 4);
-  DBuf<uint4> pk(c, n);
-  DBuf<uint32_t> from(c, n);
-  fill_u32(c, progress.get(), 0u, 4);
-  ChainArrays ca{orig.get(), src.get(), dst.get(), sz.get(), w.get(), ok.get(), ob.get(), oe.get(),
-                 next.get(), prev.get(), claim.get(), progress.get(), pk.get(), from.get()};
-  HGP_LAUNCH(k_chain_gather, g, 256, 0, c, ca, part, moves, gains, sizes, n);
+  DBuf<uint32_t> orig(c, n);
   DBuf<uint64_t> poff(c, (uint64_t)k + 1);
-  // src partitions of sorted space are the k2 keys >> 1
-  segment_offsets(c, k2.get(), 1, n, k, poff.get());
-  HGP_LAUNCH(k_chain_ranges, g, 256, 0, c, ca, poff.get(), n);
+  sort_moves(c, n, k, part, moves, gains, gst, orig, poff.get());
+  DBuf<uint32_t> next(c, n), prev(c, n), from(c, n), progress(c, 4);
+  DBuf<unsigned long long> claim(c, n);
+  DBuf<uint4> pk(c, n);
+  DBuf<uint2> range(c, n);
+  DBuf<uint32_t> cflag(c, n), cinv(c, n), csize(c, n);
+  DBuf<long long> cw(c, n);
+  DBuf<KeyStats> cst(c, 1);
+  ChainArrays ca{orig.get(), pk.get(), range.get(), from.get(), next.get(), prev.get(), claim.get(), progress.get(),
+                 cw.get(), csize.get(), cinv.get(), cflag.get()};
+  HGP_LAUNCH(k_chain_gather, g, 256, 0, c, ca, moves, gains, sizes, poff.get(), n, cst.get());
   for (int it = 0; it < 4; ++it) {
     HGP_LAUNCH(k_chain_propose, ceil_div(n, RESOLVE_BLOCK), RESOLVE_BLOCK, 0, c, ca, n, it);
     HGP_LAUNCH(k_chain_commit, g, 256, 0, c, ca, n, it);
   }
-  DBuf<uint32_t> comp(c, n), pos(c, n), cflag(c, n), cinv(c, n), csize(c, n), odd(c, 1);
-  DBuf<long long> cw(c, n);
-  HGP_LAUNCH(k_zero3, g, 256, 0, c, (unsigned long long*)cw.get(), cflag.get(), cinv.get(), (uint64_t)n);
-  fill_u32(c, csize.get(), 0u, n);
-  fill_u32(c, odd.get(), 0u, 1);
-  HGP_LAUNCH(k_chain_comp, g, 256, 0, c, ca, n, comp.get(), pos.get(), cflag.get(), cw.get(), cinv.get(), csize.get(),
-             odd.get());
-  DBuf<uint64_t> cpos(c, (uint64_t)n + 1), mo(c, 2);
+  DBuf<uint32_t> comp(c, n), pos(c, n);
+  HGP_LAUNCH(k_chain_comp, g, 256, 0, c, ca, n, comp.get(), pos.get(), cst.get());
+  HGP_LAUNCH(k_comp_stats, std::min<uint32_t>(g, 256), 256, 0, c, cflag.get(), cw.get(), cinv.get(), n, cst.get());
+  DBuf<uint64_t> cpos(c, (uint64_t)n + 1);
   exclusive_scan(c, cflag.get(), cpos.get(), n);
-  HGP_LAUNCH(k_pack2, 1, 1, 0, c, cpos.get() + n, odd.get(), mo.get());  // one read-back for both
-  uint64_t mo_h[2];
-  copy_d2h(c, mo_h, mo.get(), sizeof mo_h);
-  const uint32_t m = (uint32_t)mo_h[0];
-  const bool direct = mo_h[1] == 0;
-  DBuf<uint32_t> clist(c, m), cinvk(c, m), crank(c, n);
-  DBuf<uint64_t> ckey(c, m);
-  HGP_LAUNCH(k_comp_list, g, 256, 0, c, cflag.get(), cpos.get(), n, cw.get(), cinv.get(), clist.get(), ckey.get(),
-             cinvk.get());
+  const KeyStats cs = read_scalar(c, cst.get());
+  const uint32_t m = (uint32_t)cs.count;
   // components by (valid first, summed gain desc, head id asc): the list starts in ascending
-  // head id; a stable sort on the summed gain, then a stable 1-bit pass that moves the
-  // components made of an invalid move (summed gain 0) behind every valid one
-  radix_sort_range_buf(c, ckey, clist, m);
-  DBuf<uint32_t> inv2(c, m);
-  HGP_LAUNCH(k_gather_u32, ceil_div(m, 256), 256, 0, c, cinv.get(), clist.get(), m, inv2.get());
-  radix_sort_buf(c, inv2, clist, m, 0, 1);
-  HGP_LAUNCH(k_comp_rank, ceil_div(m, 256), 256, 0, c, clist.get(), m, crank.get());
-  if (direct) {  // every chain has its head: ranks from component starts and distances
-    DBuf<uint32_t> rsz(c, m);
+  // head id and the sort is stable
+  DBuf<uint32_t> clist(c, m), crank(c, n), rsz(c, m);
+  KeyCode cc;
+  if (cs.mn <= cs.mx) cc = key_code(cs);  // else no component of valid moves
+  const bool one = cc.bits < 64;  // the class bit fits above the code (else a pass of its own)
+  with_key_type(cc.bits + 1, [&](auto key) {
+    DBuf<decltype(key)> ckey(c, m);
+    HGP_LAUNCH((k_comp_list<decltype(key)>), g, 256, 0, c, ca, cpos.get(), n, cc.mx, cc.tz, one ? cc.bits : -1,
+               clist.get(), ckey.get());
+    radix_sort_buf(c, ckey, clist, m, 0, one ? cc.bits + 1 : 64);
+  });
+  if (!one) {
+    DBuf<uint32_t> inv2(c, m);
+    HGP_LAUNCH(k_gather_u32, ceil_div(m, 256), 256, 0, c, cinv.get(), clist.get(), m, inv2.get());
+    radix_sort_buf(c, inv2, clist, m, 0, 1);
+  }
+  HGP_LAUNCH(k_comp_rank, ceil_div(m, 256), 256, 0, c, clist.get(), csize.get(), m, crank.get(), rsz.get());
+  if (cs.odd == 0) {  // every chain has its head: ranks from component starts and distances
     DBuf<uint64_t> start(c, (uint64_t)m + 1);
-    HGP_LAUNCH(k_comp_sizes, ceil_div(m, 256), 256, 0, c, clist.get(), csize.get(), m, rsz.get());
     exclusive_scan(c, rsz.get(), start.get(), m);
     HGP_LAUNCH(k_chain_direct_ranks, g, 256, 0, c, comp.get(), pos.get(), crank.get(), start.get(), orig.get(), n,
                ranks);
@@ -2850,10 +2980,13 @@ void rank_by_chaining(Ctx& c, uint32_t n, uint32_t k, const uint32_t* part, cons
   }
   // final order: (component rank, position), ties in sorted-space index order: the keys are
   // laid out in index order and the sort is stable
-  DBuf<uint64_t> ek(c, n);
+  const int eb = bit_width(m - 1) + 8;
   DBuf<uint32_t> ev(c, n);
-  HGP_LAUNCH(k_edge_keys, g, 256, 0, c, comp.get(), pos.get(), crank.get(), n, ek.get(), ev.get());
-  radix_sort_buf(c, ek, ev, n, 0, bit_width(m) + 8);
+  with_key_type(eb, [&](auto key) {
+    DBuf<decltype(key)> ek(c, n);
+    HGP_LAUNCH((k_edge_keys<decltype(key)>), g, 256, 0, c, comp.get(), pos.get(), crank.get(), n, ek.get(), ev.get());
+    radix_sort_buf(c, ek, ev, n, 0, eb);
+  });
   HGP_LAUNCH(k_edge_ranks, g, 256, 0, c, ev.get(), orig.get(), n, ranks);
 }
 
@@ -2878,14 +3011,10 @@ void analyze_round(Ctx& c, const RefineLevel& L, int mode, uint32_t omega, uint3
   st.gains = DBuf<int64_t>(c, n);
   st.ranks = DBuf<uint32_t>(c, n);
   compute_gains(c, L, pl, mode, omega, rep, discount_of(rep, R), part, psizes, st.moves.get(), st.gains.get());
-  if (chainup) rank_by_gain(c, n, st.moves.get(), st.gains.get(), st.ranks.get());
-  else rank_by_chaining(c, n, L.k, part, st.moves.get(), st.gains.get(), L.sizes, st.ranks.get());
-  {
-    DBuf<uint32_t> cnt(c, 1);
-    memset_async(c, cnt.get(), 0, 4);
-    HGP_LAUNCH(k_count_valid, std::min<uint32_t>(g, 1024), 256, 0, c, st.moves.get(), n, cnt.get());
-    st.V = read_scalar(c, cnt.get());
-  }
+  const KeyStats gst = gain_stats(c, n, st.moves.get(), st.gains.get());
+  st.V = (uint32_t)gst.count;
+  if (chainup) rank_by_gain(c, n, st.moves.get(), st.gains.get(), gst, st.ranks.get());
+  else rank_by_chaining(c, n, L.k, part, st.moves.get(), st.gains.get(), gst, L.sizes, st.ranks.get());
   const uint32_t V = st.V;
   st.seq = DBuf<unsigned long long>(c, std::max<uint32_t>(V, 1));
   st.sv = DBuf<int32_t>(c, std::max<uint32_t>(V, 1));

@@ -306,6 +306,42 @@ def test_refine_analyze_huge_lists(dev, mode, k, fm_repeat, chainup, n, e, max_s
     assert got["best"] == exp["best"]
 
 
+@pytest.mark.parametrize("mode,k,scale,chainup", [
+    (1, 2, 1.0, False),            # whole-number gains: few varying bits, cycles of moves
+    (0, 300, 1.0, True),
+    (0, 4096, 0.37, False),        # the largest partition order ranked by counting
+    (0, 4097, 0.37, False),        # ... and the smallest sorted one
+    (0, 1 << 19, 16000.0, False),  # gain and partition bits together above 64: two sorts
+    (0, 1 << 19, 16000.0, True),
+])
+def test_refine_analyze_move_keys(dev, mode, k, scale, chainup, rng):
+    """The order of the moves over the bits of the gains that vary: unit and fractional weights,
+    weights near the top of the fixed-point range on nodes of thousands of hedges."""
+    heavy = scale > 1000
+    n, e = 3000, 20000 if heavy else 3000
+    n, off, pins, srcc, w = gen.random_hypergraph(n, e, rng, max_size=5, src_prob=0.3, max_src=1)
+    rows = [list(pins[off[i]:off[i + 1]]) + ([0, 1] if heavy else []) for i in range(e)]  # two nodes of every hedge
+    w = (np.ones(e) if scale == 1.0 else scale * (0.5 + 0.5 * rng.random(e))).astype(np.float32)
+    hg = O.dedup(O.HG(n, np.cumsum([0] + [len(r) for r in rows]).astype(np.uint64),
+                      np.array([x for r in rows for x in r], np.uint32), srcc, w))
+    sizes = rng.integers(1, 3, size=n).astype(np.uint32)
+    part = (rng.integers(0, min(k, 2000), size=n) + max(0, k - 2000)).astype(np.uint32)
+    part[1] = part[0]
+    psizes = np.bincount(part, weights=sizes, minlength=k).astype(np.uint32)
+    omega, delta = int(psizes.max()) + 2, 2**31 - 1
+    L = G.Level(dev, hg)
+    L.build_touching()
+    ro, rt, ri = O.touching(hg)
+    got = G.refine_analyze(dev, L, sizes, k, mode, omega, delta, 16, 0, chainup, part, psizes)
+    exp = O.refine_analyze(mode, omega, delta, 16, hg, ro, rt, ri, sizes, k, 0, chainup, part, psizes)
+    if heavy:
+        g = exp["gains"][exp["moves"] != 2**32 - 1]
+        assert (int(g.max()) - int(g.min())).bit_length() + 20 > 64, "the case must need two sorts"
+    for key in ("moves", "gains", "ranks", "seq", "sv", "iv"):
+        assert np.array_equal(got[key], exp[key]), f"{key} differs"
+    assert got["best"] == exp["best"]
+
+
 @pytest.mark.parametrize("k,spread", [(1, 1), (70, 70), (70, 2), (40000, 40000)])
 def test_partition_lists_by_hedge_length(dev, k, spread, rng):
     """Partition lists at the edges of their kernels (16 pins by thread, up to 64, 128 and 256 in a
