@@ -54,7 +54,7 @@ struct ProfRec {
 // Launch parameters chosen by the autotuner (hgp_tuning in the C ABI).  They change speed
 // only: every stage returns the same result under any valid setting.
 struct Tuning {
-  uint32_t sort_rounds[40] = {};     // radix-sort keys per thread and tile, by floor(log2 n); 0 = rule
+  uint32_t sort_rounds[40] = {};     // radix-sort keys per thread of a tile, by floor(log2 n); 0 = rule
   uint32_t heavy_slots = 65536;      // first-attempt HBM hash table of a heavy candidate node
   uint32_t heavy_fill16 = 12;        // its fill limit in sixteenths
   uint32_t cascade_block = 256;      // threads per workgroup of the thread-per-hedge cascade
@@ -63,8 +63,8 @@ struct Tuning {
   uint32_t mask_wide16_degree = 512;  // 4 (16) waves per node
   uint32_t side_streams = 2;          // bit 0: candidate tiers, bit 1: cascade classes beside events,
                                       // bit 2: ... and beside the small-hedge cascade
-  uint32_t coop_max_n = 65536;        // sorts of RS1 .. this many keys run every pass in one launch
-  uint32_t coop_tile = 1024;          // keys per workgroup of those launches (at least)
+  uint32_t coop_max_n = 65536;        // kept for saved tunings (no sort reads them)
+  uint32_t coop_tile = 1024;
   bool tuned = false;
 };
 
@@ -87,8 +87,6 @@ struct Ctx {
   void* scan_agg = nullptr;
   void* scan_incl = nullptr;
   unsigned long long* scan_ticket = nullptr;
-  unsigned int* coop_bar = nullptr;  // grid-barrier counter of the cooperative sorts (prim.hip)
-  uint64_t coop_issued = 0;
   uint32_t scan_cap_tiles = 0;
   uint32_t scan_gen = 0;
   uint64_t scan_tickets_issued = 0;

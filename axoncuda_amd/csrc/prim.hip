@@ -1,9 +1,11 @@
 // prim.hip - scans, stable radix sort and small helpers for gfx950 (wave64).
 //
 // Scans: one pass with decoupled look-back over 4096-element tiles.
-// Radix sort: reduce-then-scan LSD with 8-bit digits; the scatter ranks keys within a tile
-// in 256-key rounds, using eight ballots per key to find same-digit lanes of a wave (a
-// stable in-wave rank) and LDS prefix sums across the four waves of the workgroup.
+// Radix sort: LSD with digits of up to 8 bits; up to 8,192 keys in one workgroup's registers and
+// LDS, larger ones in tiles (counts, offsets, scatter) per pass.
+#include <algorithm>
+#include <type_traits>
+
 #include "prim.hpp"
 
 namespace hgp {
@@ -246,22 +248,6 @@ void scan_status(Ctx& c, uint32_t tiles) {
   c.scan_cap_tiles = cap;
 }
 
-// Grid-barrier counter of the context's cooperative sorts: returns the count that a launch
-// making `arrivals` arrivals starts from, resetting the counter (on the stream) before it
-// could wrap.  The caller adds the arrivals to c.coop_issued once the launch is queued, so a
-// launch that fails to queue leaves the count as the device has it.
-unsigned int coop_barrier_base(Ctx& c, uint32_t arrivals) {
-  if (!c.coop_bar) {
-    c.coop_bar = (unsigned int*)dmalloc(c, 4);
-    c.coop_issued = 1u << 31;  // forces the reset below
-  }
-  if (c.coop_issued + (uint64_t)arrivals >= (1ull << 31)) {
-    fill_u32(c, c.coop_bar, 0u, 1);
-    c.coop_issued = 0;
-  }
-  return (unsigned int)c.coop_issued;
-}
-
 // in == out is safe: each workgroup reads only its own tile before writing it.
 template <typename TI, typename TO>
 void scan_impl(Ctx& c, const TI* in, TO* out, uint64_t n, bool exclusive) {
@@ -296,366 +282,393 @@ void scan_impl(Ctx& c, const TI* in, TO* out, uint64_t n, bool exclusive) {
 }
 
 // ---------------------------------------------------------------------------------------
-// radix sort
+// radix sort (stable, least significant digit first; digits of at most 8 bits, the passes of a
+// sort sharing its bits evenly)
 constexpr int RS_BLOCK = 256;
-constexpr uint32_t RS_MAX_ROUNDS = 16;  // keys per thread and tile of a large sort
-constexpr uint32_t RS_TARGET_TILES = 512;  // small sorts shrink their tiles to spread over the CUs
 
-// Rounds of RS_BLOCK keys per tile: one tile per workgroup, so a small sort runs many short
-// workgroups side by side instead of a few that walk 16 rounds one after another.  The
-// autotuner may set the rounds per size class (floor(log2 n)); the result is the same.
-inline uint32_t rs_rounds(const Ctx& c, uint64_t n) {
-  const int cls = bit_width(n) - 1;
-  if (cls >= 0 && cls < 40 && c.tune.sort_rounds[cls]) return std::min(c.tune.sort_rounds[cls], RS_MAX_ROUNDS);
-  return (uint32_t)std::min<uint64_t>(RS_MAX_ROUNDS, std::max<uint64_t>(1, ceil_div(n, (uint64_t)RS_BLOCK * RS_TARGET_TILES)));
-}
-
-template <typename K>
-__global__ void k_rs_hist(const K* __restrict__ keys, uint64_t n, int shift, uint32_t nblocks, uint32_t rounds,
-                          K kmin, uint32_t* __restrict__ counts) {
-  __shared__ uint32_t h[256];
-  h[threadIdx.x] = 0;
-  __syncthreads();
-  uint64_t base = (uint64_t)blockIdx.x * RS_BLOCK * rounds;
-  for (uint32_t r = 0; r < rounds; ++r) {
-    uint64_t i = base + (uint64_t)r * RS_BLOCK + threadIdx.x;
-    if (i < n) atomicAdd(&h[(uint32_t)((keys[i] - kmin) >> shift) & 0xFFu], 1u);
-  }
-  __syncthreads();
-  counts[(uint64_t)threadIdx.x * nblocks + blockIdx.x] = h[threadIdx.x];
-}
-
-template <typename K, bool HAS_VALS>
-__global__ void __launch_bounds__(RS_BLOCK) k_rs_scatter(const K* __restrict__ keys, const uint32_t* __restrict__ vals,
-                                                         K* __restrict__ okeys, uint32_t* __restrict__ ovals,
-                                                         uint64_t n, int shift, uint32_t nblocks, uint32_t rounds,
-                                                         K kmin, const uint64_t* __restrict__ offsets) {
-  __shared__ uint64_t run[256];
-  __shared__ uint32_t wcnt[RS_BLOCK / 64][256];
-  const uint32_t t = threadIdx.x, w = t / 64;
-  run[t] = offsets[(uint64_t)t * nblocks + blockIdx.x];
-  uint64_t base = (uint64_t)blockIdx.x * RS_BLOCK * rounds;
-  for (uint32_t r = 0; r < rounds; ++r) {
-    uint64_t i = base + (uint64_t)r * RS_BLOCK + t;
-    if (base + (uint64_t)r * RS_BLOCK >= n) break;  // uniform across the block
+// Ranking.  A wave owns consecutive keys, 64 per round; lanes with equal digits find each other
+// with one ballot per digit bit, the lowest of them adds the group to the wave's own counter of
+// that digit, and a key's rank is the counter before its group plus its place in it.  The
+// counters belong to the wave (LDS operations of a wave are in order), so rounds need no barrier.
+// Returns the rank among the wave's keys of the same digit so far.
+__device__ __forceinline__ uint32_t wave_digit_rank(bool valid, uint32_t d, int nb, uint32_t* cnt) {
+  uint64_t peers = __ballot(valid);
 #pragma unroll
-    for (int q = 0; q < RS_BLOCK / 64; ++q) wcnt[q][t] = 0;
-    __syncthreads();
-    const bool valid = i < n;
-    K key = valid ? keys[i] : (K)0;
-    uint32_t val = 0;
-    if (HAS_VALS && valid) val = vals[i];
-    const uint32_t d = (uint32_t)((key - kmin) >> shift) & 0xFFu;
-    uint64_t peers = __ballot(valid);
-#pragma unroll
-    for (int b = 0; b < 8; ++b) {
+  for (int b = 0; b < 8; ++b) {
+    if (b < nb) {  // uniform
       const bool bit = (d >> b) & 1u;
       const uint64_t bb = __ballot(bit);
       peers &= bit ? bb : ~bb;
     }
-    const uint32_t rank = lanes_below(peers);
-    if (valid && rank == 0) wcnt[w][d] = (uint32_t)__popcll(peers);
-    __syncthreads();
-    // per digit: exclusive prefix over waves (thread t handles digit t)
-    uint32_t acc = 0;
-#pragma unroll
-    for (int q = 0; q < RS_BLOCK / 64; ++q) {
-      uint32_t c = wcnt[q][t];
-      wcnt[q][t] = acc;
-      acc += c;
-    }
-    __syncthreads();
-    if (valid) {
-      uint64_t pos = run[d] + wcnt[w][d] + rank;
-      okeys[pos] = key;
-      if (HAS_VALS) ovals[pos] = val;
-    }
-    __syncthreads();
-    run[t] += acc;
   }
+  const uint32_t below = lanes_below(peers);
+  uint32_t before = 0;
+  if (valid) before = cnt[d];
+  __builtin_amdgcn_wave_barrier();
+  if (valid && below == 0) cnt[d] = before + (uint32_t)__popcll(peers);
+  __builtin_amdgcn_wave_barrier();
+  return before + below;
 }
 
-// Whole LSD sort of a small array by one workgroup: each pass (digit histogram, digit
-// offsets, stable scatter in rounds of RS1_BLOCK keys) runs between barriers, so a small sort
-// costs one launch instead of three or four per pass.  Keys of the pass stay in registers
-// between the histogram and the scatter.  Ends in kb/vb after an odd pass count.
-constexpr int RS1_BLOCK = 1024;
-constexpr uint32_t RS1_MAX_ROUNDS = 16;
-constexpr uint64_t RS1_MAX_N = (uint64_t)RS1_BLOCK * RS1_MAX_ROUNDS;
+// Whole sort of at most 1024 * IT keys by one workgroup: keys and values stay in registers, every
+// pass ranks them and exchanges them through LDS, and memory is read and written once.  The
+// exchange through global memory this replaces cost 64 cycles per scattered 64-lane store: two
+// passes over 8,191 64-bit keys with values took 37 us and take 20 us this way, 4,096 keys 25 and
+// 13 us, 64 keys 14 and 7.5 us.  Past 8,192 keys one CU's ranking is the bound (16,384 keys: 38 us)
+// and the tiles below are faster (16,385 keys: 18 us).
+constexpr uint32_t RS1_BLOCK = 1024;
+constexpr uint32_t RS1_MAX_IT = 8;
+constexpr uint64_t RS1_MAX_N = (uint64_t)RS1_BLOCK * RS1_MAX_IT;
 
-template <typename K, bool HAS_VALS>
-__global__ void __launch_bounds__(RS1_BLOCK) k_rs_small(K* ka, uint32_t* va, K* kb, uint32_t* vb, uint32_t n,
-                                                        int lo, int bits, K kmin) {
-  __shared__ uint32_t h[256];
-  __shared__ uint32_t run[256];
-  __shared__ uint32_t s_w[4];
-  __shared__ uint32_t wcnt[RS1_BLOCK / 64][256];
+template <typename K, bool HAS_VALS, uint32_t IT>
+__global__ void __launch_bounds__(RS1_BLOCK) k_rs_block(K* keys, uint32_t* vals, uint32_t n, int lo, int bits, int nb,
+                                                        K kmin) {
+  constexpr uint32_t W = RS1_BLOCK / 64;
+  __shared__ K s_key[RS1_BLOCK * IT];
+  __shared__ uint32_t s_cnt[W][256];
+  __shared__ uint32_t s_w[W];
   const uint32_t t = threadIdx.x, w = t / 64, l = lane_id();
-  const uint32_t rounds = (n + RS1_BLOCK - 1) / RS1_BLOCK;
-  for (int shift = lo; shift < bits; shift += 8) {
-    K key[RS1_MAX_ROUNDS];
-    uint32_t val[RS1_MAX_ROUNDS];
-    if (t < 256) h[t] = 0;
-    __syncthreads();
+  const uint32_t first = w * 64 * IT + l;  // this lane's keys: first + 64 * r
+  K key[IT];
+  uint32_t val[IT];
 #pragma unroll
-    for (uint32_t r = 0; r < RS1_MAX_ROUNDS; ++r) {
-      const uint32_t i = r * RS1_BLOCK + t;
-      key[r] = 0;
-      val[r] = 0;
-      if (i < n) {
-        key[r] = ka[i];
-        if (HAS_VALS) val[r] = va[i];
-        atomicAdd(&h[(uint32_t)((key[r] - kmin) >> shift) & 0xFFu], 1u);
-      }
-    }
-    __syncthreads();
-    // run[d]: keys of digits below d (exclusive scan of the histogram by the first four waves)
-    uint32_t x = 0, inc = 0;
-    if (t < 256) {
-      x = h[t];
-      inc = wave_scan_incl(x);
-      if (l == 63) s_w[w] = inc;
-    }
-    __syncthreads();
-    if (t < 256) {
-      uint32_t b = 0;
-      for (uint32_t q = 0; q < w; ++q) b += s_w[q];
-      run[t] = b + inc - x;
-    }
-#pragma unroll
-    for (uint32_t r = 0; r < RS1_MAX_ROUNDS; ++r) {
-      if (r < rounds) {  // uniform across the block
-#pragma unroll
-        for (int q = 0; q < 4; ++q) (&wcnt[0][0])[q * RS1_BLOCK + t] = 0;
-        __syncthreads();
-        const uint32_t i = r * RS1_BLOCK + t;
-        const bool valid = i < n;
-        const uint32_t d = (uint32_t)((key[r] - kmin) >> shift) & 0xFFu;
-        uint64_t peers = __ballot(valid);
-#pragma unroll
-        for (int b = 0; b < 8; ++b) {
-          const bool bit = (d >> b) & 1u;
-          const uint64_t bb = __ballot(bit);
-          peers &= bit ? bb : ~bb;
-        }
-        const uint32_t rank = lanes_below(peers);
-        if (valid && rank == 0) wcnt[w][d] = (uint32_t)__popcll(peers);
-        __syncthreads();
-        // per digit (thread t < 256 handles digit t): exclusive prefix over the waves
-        uint32_t acc = 0;
-        if (t < 256) {
-#pragma unroll
-          for (int q = 0; q < RS1_BLOCK / 64; ++q) {
-            const uint32_t cq = wcnt[q][t];
-            wcnt[q][t] = acc;
-            acc += cq;
-          }
-        }
-        __syncthreads();
-        if (valid) {
-          const uint32_t pos = run[d] + wcnt[w][d] + rank;
-          kb[pos] = key[r];
-          if (HAS_VALS) vb[pos] = val[r];
-        }
-        __syncthreads();
-        if (t < 256) run[t] += acc;
-      }
-    }
-    K* tk = ka;
-    ka = kb;
-    kb = tk;
-    uint32_t* tv = va;
-    va = vb;
-    vb = tv;
-    __threadfence();  // the next pass reads what this one wrote
-    __syncthreads();
+  for (uint32_t r = 0; r < IT; ++r) {
+    const uint32_t i = first + 64 * r;
+    key[r] = i < n ? keys[i] : (K)0;
+    val[r] = HAS_VALS && i < n ? vals[i] : 0u;
   }
-}
-
-// Whole LSD sort of a mid-size array in one launch: B workgroups each own a contiguous tile and
-// meet at grid barriers.  B <= COOP_MAX_BLOCKS = 64 is far below what the device holds at once
-// (at least 4 such workgroups per CU, 256 CUs), and every other kernel that may run beside one
-// finishes on its own (look-back scans wait only on tiles already running; serving workers do
-// not use these sorts), so all B workgroups become resident and every barrier is reached.  A pass counts its tile's digits, publishes the counts, and after a
-// barrier every workgroup derives its tile's digit offsets from all counts (digit totals
-// scanned over digits, plus the counts of the tiles before its own), scatters its keys stably
-// in rounds of 256, and waits at a second barrier before the next pass reads the output.
-// The barrier counter only grows; arrival k of a launch waits for base + B * k.
-constexpr uint32_t COOP_MAX_BLOCKS = 64;
-
-__device__ __forceinline__ void grid_barrier(unsigned int* ctr, unsigned int target) {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");  // this thread's writes before the arrival
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    atomicAdd(ctr, 1u);
-    while (__hip_atomic_load(ctr, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) < target) __builtin_amdgcn_s_sleep(1);
-  }
-  __syncthreads();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");  // the other workgroups' writes after it
-}
-
-template <typename K, bool HAS_VALS>
-__global__ void __launch_bounds__(RS_BLOCK) k_rs_coop(K* ka, uint32_t* va, K* kb, uint32_t* vb, uint32_t n,
-                                                      uint32_t tile, int lo, int bits, K kmin,
-                                                      uint32_t* __restrict__ counts, unsigned int* bar,
-                                                      unsigned int bar_base) {
-  __shared__ uint32_t h[256];
-  __shared__ uint32_t run[256];
-  __shared__ uint32_t s_w[RS_BLOCK / 64];
-  __shared__ uint32_t wcnt[RS_BLOCK / 64][256];
-  const uint32_t B = gridDim.x, b = blockIdx.x, t = threadIdx.x, w = t / 64, l = lane_id();
-  const uint32_t beg = min(n, b * tile), end = min(n, beg + tile);
-  unsigned int target = bar_base;
-  for (int shift = lo; shift < bits; shift += 8) {
-    h[t] = 0;
+  for (int shift = lo; shift < bits; shift += nb) {
+    const int nbp = min(nb, bits - shift);
+    const uint32_t mask = (1u << nbp) - 1u;
+#pragma unroll
+    for (uint32_t q = 0; q < 4; ++q) (&s_cnt[0][0])[q * RS1_BLOCK + t] = 0;
     __syncthreads();
-    for (uint32_t i = beg + t; i < end; i += RS_BLOCK) atomicAdd(&h[(uint32_t)((ka[i] - kmin) >> shift) & 0xFFu], 1u);
-    __syncthreads();
-    counts[(uint64_t)b * 256 + t] = h[t];
-    target += B;
-    grid_barrier(bar, target);
-    // digit t: its total over all tiles and its count in the tiles before this one
-    uint32_t tot = 0, pre = 0;
-    for (uint32_t x = 0; x < B; ++x) {
-      const uint32_t cx = counts[(uint64_t)x * 256 + t];
-      tot += cx;
-      pre += x < b ? cx : 0u;
+    uint32_t pos[IT];
+#pragma unroll
+    for (uint32_t r = 0; r < IT; ++r) {
+      const uint32_t d = (uint32_t)((key[r] - kmin) >> shift) & mask;
+      pos[r] = wave_digit_rank(first + 64 * r < n, d, nbp, s_cnt[w]);
     }
-    const uint32_t inc = wave_scan_incl(tot);
+    __syncthreads();
+    // exclusive sums in (digit, wave) order: thread t takes four waves of digit t / 4
+    uint32_t c[4], sum = 0;
+#pragma unroll
+    for (uint32_t q = 0; q < 4; ++q) {
+      c[q] = s_cnt[(t & 3) * 4 + q][t >> 2];
+      sum += c[q];
+    }
+    const uint32_t inc = wave_scan_incl(sum);
     if (l == 63) s_w[w] = inc;
     __syncthreads();
-    uint32_t base = 0;
-    for (uint32_t q = 0; q < w; ++q) base += s_w[q];
-    run[t] = base + inc - tot + pre;
-    for (uint32_t r0 = beg; r0 < end; r0 += RS_BLOCK) {  // uniform across the workgroup
+    uint32_t run = inc - sum;
 #pragma unroll
-      for (int q = 0; q < RS_BLOCK / 64; ++q) wcnt[q][t] = 0;
-      __syncthreads();
-      const uint32_t i = r0 + t;
-      const bool valid = i < end;
-      const K key = valid ? ka[i] : (K)0;
-      uint32_t val = 0;
-      if (HAS_VALS && valid) val = va[i];
-      const uint32_t d = (uint32_t)((key - kmin) >> shift) & 0xFFu;
-      uint64_t peers = __ballot(valid);
+    for (uint32_t q = 0; q < W; ++q) run += q < w ? s_w[q] : 0u;
 #pragma unroll
-      for (int bt = 0; bt < 8; ++bt) {
-        const bool bit = (d >> bt) & 1u;
-        const uint64_t bb = __ballot(bit);
-        peers &= bit ? bb : ~bb;
-      }
-      const uint32_t rank = lanes_below(peers);
-      if (valid && rank == 0) wcnt[w][d] = (uint32_t)__popcll(peers);
-      __syncthreads();
-      uint32_t acc = 0;
-#pragma unroll
-      for (int q = 0; q < RS_BLOCK / 64; ++q) {
-        const uint32_t cq = wcnt[q][t];
-        wcnt[q][t] = acc;
-        acc += cq;
-      }
-      __syncthreads();
-      if (valid) {
-        const uint32_t pos = run[d] + wcnt[w][d] + rank;
-        kb[pos] = key;
-        if (HAS_VALS) vb[pos] = val;
-      }
-      __syncthreads();
-      run[t] += acc;
+    for (uint32_t q = 0; q < 4; ++q) {
+      s_cnt[(t & 3) * 4 + q][t >> 2] = run;
+      run += c[q];
     }
-    target += B;
-    grid_barrier(bar, target);  // the output is whole (and the counts free) before the next pass
-    K* tk = ka;
-    ka = kb;
-    kb = tk;
-    uint32_t* tv = va;
-    va = vb;
-    vb = tv;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t r = 0; r < IT; ++r) {
+      const uint32_t d = (uint32_t)((key[r] - kmin) >> shift) & mask;
+      pos[r] += s_cnt[w][d];
+      if (first + 64 * r < n) s_key[pos[r]] = key[r];
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t r = 0; r < IT; ++r)
+      if (first + 64 * r < n) key[r] = s_key[first + 64 * r];
+    if (HAS_VALS) {  // the values take the keys' place in LDS
+      uint32_t* s_val = reinterpret_cast<uint32_t*>(s_key);
+      __syncthreads();
+#pragma unroll
+      for (uint32_t r = 0; r < IT; ++r)
+        if (first + 64 * r < n) s_val[pos[r]] = val[r];
+      __syncthreads();
+#pragma unroll
+      for (uint32_t r = 0; r < IT; ++r)
+        if (first + 64 * r < n) val[r] = s_val[first + 64 * r];
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) {
+    const uint32_t i = first + 64 * r;
+    if (i < n) {
+      keys[i] = key[r];
+      if (HAS_VALS) vals[i] = val[r];
+    }
   }
 }
 
-// LSD passes over bits [lo, bits) of key - kmin (the keys themselves are moved unchanged).  With `kbuf` (and `vbuf`) the result ends up in those
-// buffers by exchanging them with the scratch ones after an odd pass count; otherwise it is
-// copied back into keys / vals.
+// Larger sorts, per pass: every tile of 512 * IT keys counts its digits; the tiles' counts become
+// the number of equal digits in the tiles before (and the digits' totals); every tile ranks its
+// keys again, exchanges them through LDS into digit order and writes runs.  Up to RS_DIRECT_TILES
+// tiles the last step adds up the earlier tiles' counts itself, and a pass is two launches.  Two
+// passes over 64-bit keys with values, against a scan of all counts and a scatter in rounds of 256
+// keys: 65,536 keys 72 -> 21 us, 1,000,000 68 -> 44 us, 15.4 M 630 -> 302 us.  No workgroup waits
+// for another: a single-pass look-back over the tiles, numbered by a ticket so that its waits end,
+// was measured too, and the tickets (one address, about 40 ns each) bounded it above 100 tiles
+// (15.4 M keys: 370 us; 1,000,000: 62 us).
+constexpr uint32_t OS_BLOCK = 512;
+constexpr uint32_t RS_DIRECT_TILES = 64;
+
+// LDS add to a digit counter; when the whole wave has one digit (the high digits of small values)
+// one lane adds for all instead of 64 adds to one address
+__device__ __forceinline__ void count_digit(uint32_t* h, bool valid, uint32_t d) {
+  const uint64_t act = __ballot(valid);
+  if (!act) return;
+  const int lead = __ffsll((unsigned long long)act) - 1;
+  const uint32_t d0 = (uint32_t)__builtin_amdgcn_readlane((int)d, lead);
+  if (__ballot(valid && d == d0) == act) {
+    if ((int)lane_id() == lead) atomicAdd(&h[d0], (uint32_t)__popcll(act));
+  } else if (valid) {
+    atomicAdd(&h[d], 1u);
+  }
+}
+// counts[tile][digit]
+template <typename K, uint32_t IT>
+__global__ void __launch_bounds__(OS_BLOCK) k_rs_count(const K* __restrict__ keys, uint64_t n, int shift, int nb, K kmin,
+                                                       uint32_t* __restrict__ counts) {
+  __shared__ uint32_t h[256];
+  const uint32_t t = threadIdx.x, mask = (1u << nb) - 1u;
+  if (t < 256) h[t] = 0;
+  const uint64_t beg = (uint64_t)blockIdx.x * (OS_BLOCK * IT);
+  K key[IT];
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) {
+    const uint64_t i = beg + r * OS_BLOCK + t;
+    key[r] = i < n ? keys[i] - kmin : (K)0;
+  }
+  __syncthreads();
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) count_digit(h, beg + r * OS_BLOCK + t < n, (uint32_t)(key[r] >> shift) & mask);
+  __syncthreads();
+  if (t < 256) counts[(uint64_t)blockIdx.x * 256 + t] = h[t];
+}
+
+// before[tile][digit] = the counts of the digit in the tiles before; totals[digit].  One workgroup
+// per 16 digits: 64 segments of consecutive tiles, summed, scanned and walked again.
+__global__ void __launch_bounds__(1024) k_rs_columns(const uint32_t* __restrict__ counts, uint32_t tiles,
+                                                     uint64_t* __restrict__ before, uint64_t* __restrict__ totals) {
+  __shared__ uint64_t s_seg[64][16];
+  const uint32_t x = threadIdx.x & 15, seg = threadIdx.x >> 4, d = blockIdx.x * 16 + x;
+  const uint32_t per = (tiles + 63) / 64;
+  const uint32_t b = min(tiles, seg * per), e = min(tiles, b + per);
+  uint64_t sum = 0;
+#pragma unroll 8
+  for (uint32_t i = b; i < e; ++i) sum += counts[(uint64_t)i * 256 + d];
+  s_seg[seg][x] = sum;
+  __syncthreads();
+  // a wave holds 4 segments of 16 digits: each of the first 16 threads scans one digit's segments
+  if (threadIdx.x < 16) {
+    uint64_t run = 0;
+    for (uint32_t q = 0; q < 64; ++q) {
+      const uint64_t v = s_seg[q][threadIdx.x];
+      s_seg[q][threadIdx.x] = run;
+      run += v;
+    }
+    totals[d] = run;
+  }
+  __syncthreads();
+  uint64_t run = s_seg[seg][x];
+#pragma unroll 8
+  for (uint32_t i = b; i < e; ++i) {
+    const uint32_t v = counts[(uint64_t)i * 256 + d];
+    before[(uint64_t)i * 256 + d] = run;
+    run += v;
+  }
+}
+
+// before == nullptr: at most RS_DIRECT_TILES tiles, whose counts are added up here
+template <typename K, bool HAS_VALS, uint32_t IT>
+__global__ void __launch_bounds__(OS_BLOCK) k_rs_pass(const K* __restrict__ keys, const uint32_t* __restrict__ vals,
+                                                      K* __restrict__ okeys, uint32_t* __restrict__ ovals, uint64_t n,
+                                                      int shift, int nb, K kmin, const uint32_t* __restrict__ counts,
+                                                      const uint64_t* __restrict__ before,
+                                                      const uint64_t* __restrict__ totals) {
+  constexpr uint32_t W = OS_BLOCK / 64, TILE = OS_BLOCK * IT, WD = 256 / 64, HALVES = OS_BLOCK / 256;
+  __shared__ K s_key[TILE];
+  __shared__ uint32_t s_val[HAS_VALS ? TILE : 1];
+  __shared__ uint32_t s_cnt[W][256];
+  __shared__ uint32_t s_loc[256];
+  __shared__ uint64_t s_base[256];
+  __shared__ uint32_t s_w[WD];
+  __shared__ uint64_t s_g[WD];
+  __shared__ uint32_t s_sum[HALVES][2][256];
+  const uint32_t t = threadIdx.x, w = t / 64, l = lane_id();
+  const uint32_t mask = (1u << nb) - 1u;
+  const uint32_t tile = blockIdx.x;
+  const uint64_t beg = (uint64_t)tile * TILE;
+  const uint32_t len = (uint32_t)min((uint64_t)TILE, n - beg);
+  const uint32_t first = w * 64 * IT + l;
+  K key[IT];
+  uint32_t val[IT], pos[IT];
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) {
+    const uint32_t i = first + 64 * r;
+    key[r] = i < len ? keys[beg + i] : (K)0;
+    val[r] = HAS_VALS && i < len ? vals[beg + i] : 0u;
+  }
+#pragma unroll
+  for (uint32_t q = 0; q < W * 256 / OS_BLOCK; ++q) (&s_cnt[0][0])[q * OS_BLOCK + t] = 0;
+  // per digit: keys of it in the tiles before, and in all
+  uint64_t g = 0, bef = 0;
+  if (before) {
+    if (t < 256) {
+      g = totals[t];
+      bef = before[(uint64_t)tile * 256 + t];
+    }
+  } else {
+    const uint32_t d = t & 255, half = t >> 8;
+    uint32_t a = 0, b = 0;
+#pragma unroll 8
+    for (uint32_t i = half; i < gridDim.x; i += HALVES) {
+      const uint32_t v = counts[i * 256 + d];
+      a += v;
+      b += i < tile ? v : 0u;
+    }
+    s_sum[half][0][d] = a;
+    s_sum[half][1][d] = b;
+  }
+  __syncthreads();
+  if (!before && t < 256) {
+#pragma unroll
+    for (uint32_t h = 0; h < HALVES; ++h) {
+      g += s_sum[h][0][t];
+      bef += s_sum[h][1][t];
+    }
+  }
+  uint64_t ginc = 0;
+  if (t < 256) {
+    ginc = wave_scan_incl(g);
+    if (l == 63) s_g[w] = ginc;
+  }
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r)
+    pos[r] = wave_digit_rank(first + 64 * r < len, (uint32_t)((key[r] - kmin) >> shift) & mask, nb, s_cnt[w]);
+  __syncthreads();
+  // digit t: its start in the tile, and each wave's start in it
+  uint32_t tot = 0, inc = 0;
+  if (t < 256) {
+#pragma unroll
+    for (uint32_t q = 0; q < W; ++q) {
+      const uint32_t c = s_cnt[q][t];
+      s_cnt[q][t] = tot;
+      tot += c;
+    }
+    inc = wave_scan_incl(tot);
+    if (l == 63) s_w[w] = inc;
+  }
+  __syncthreads();
+  if (t < 256) {
+    uint32_t loc = inc - tot;
+    uint64_t below = ginc - g;
+#pragma unroll
+    for (uint32_t q = 0; q < WD; ++q) {
+      loc += q < w ? s_w[q] : 0u;
+      below += q < w ? s_g[q] : 0ull;
+    }
+    s_loc[t] = loc;
+    s_base[t] = below + bef - loc;  // (wraps below zero and back with the tile position)
+  }
+  __syncthreads();
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) {
+    if (first + 64 * r < len) {
+      const uint32_t d = (uint32_t)((key[r] - kmin) >> shift) & mask;
+      const uint32_t o = s_loc[d] + s_cnt[w][d] + pos[r];
+      s_key[o] = key[r];
+      if (HAS_VALS) s_val[o] = val[r];
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) {
+    const uint32_t i = r * OS_BLOCK + t;
+    if (i < len) {
+      const K k = s_key[i];
+      const uint64_t o = s_base[(uint32_t)((k - kmin) >> shift) & mask] + i;
+      okeys[o] = k;
+      if (HAS_VALS) ovals[o] = s_val[i];
+    }
+  }
+}
+
+// Size of a pass's tiles in units of 256 keys (2, 4, 8 or 16): small tiles rank sooner, few tiles
+// cost less to add up.  Measured (two passes, 32-bit keys with values, at 2 / 4 / 8 / 16): 50,000
+// keys 23 / 20 / 24 / 29 us; 300,000 40 / 31 / 30 / 34; 1,000,000 71 / 47 / 42 / 41; 3.2 M 181 / 117 /
+// 84 / 67.  The autotuner may set it per size class (floor(log2 n)); the result is the same.
+inline uint32_t rs_items(const Ctx& c, uint64_t n) {
+  const int cls = bit_width(n) - 1;
+  uint32_t want = 0;
+  if (cls >= 0 && cls < 40) want = c.tune.sort_rounds[cls];
+  if (!want) want = n <= 65536 ? 4 : n <= 1u << 20 ? 8 : 16;
+  uint32_t it = 2;
+  while (it < want && it < 16) it <<= 1;
+  return it;
+}
+
+// LSD passes over bits [lo, bits) of key - kmin (the keys themselves are moved unchanged).  With
+// `kbuf` (and `vbuf`) the result ends up in those buffers by exchanging them with the scratch ones
+// after an odd pass count; otherwise it is copied back into keys / vals.
 template <typename K>
 void radix_impl(Ctx& c, K* keys, uint32_t* vals, uint64_t n, int bits, int lo = 0, DBuf<K>* kbuf = nullptr,
                 DBuf<uint32_t>* vbuf = nullptr, K kmin = 0) {
   if (n <= 1 || bits <= lo) return;
+  const int passes = (bits - lo + 7) / 8;
+  const int nb = (bits - lo + passes - 1) / passes;
   if (n <= RS1_MAX_N) {
-    DBuf<K> k2(c, n);
-    DBuf<uint32_t> v2(c, vals ? n : 0);
-    const int passes = (bits - lo + 7) / 8;
-    // bytes: keys (and values) read once and written once per pass
-    const uint64_t sb = (uint64_t)passes * n * (2 * sizeof(K) + (vals ? 8 : 0));
-    if (vals)
-      HGP_LAUNCH_B(sb, (k_rs_small<K, true>), 1, RS1_BLOCK, 0, c, keys, vals, k2.get(), v2.get(), (uint32_t)n, lo,
-                   bits, kmin);
-    else
-      HGP_LAUNCH_B(sb, (k_rs_small<K, false>), 1, RS1_BLOCK, 0, c, keys, vals, k2.get(), v2.get(), (uint32_t)n, lo,
-                   bits, kmin);
-    if (passes & 1) {
-      if (kbuf && (!vals || vbuf)) {  // hand the scratch buffers over instead of copying
-        std::swap(*kbuf, k2);
-        if (vals) std::swap(*vbuf, v2);
-        return;
-      }
-      copy_d2d(c, keys, k2.get(), n * sizeof(K));
-      if (vals) copy_d2d(c, vals, v2.get(), n * sizeof(uint32_t));
-    }
+    const uint64_t sb = n * (2 * sizeof(K) + (vals ? 8 : 0));  // keys (and values) read once and written once
+    auto launch = [&](auto items) {
+      constexpr uint32_t IT = decltype(items)::value;
+      if (vals)
+        HGP_LAUNCH_B(sb, (k_rs_block<K, true, IT>), 1, RS1_BLOCK, 0, c, keys, vals, (uint32_t)n, lo, bits, nb, kmin);
+      else
+        HGP_LAUNCH_B(sb, (k_rs_block<K, false, IT>), 1, RS1_BLOCK, 0, c, keys, vals, (uint32_t)n, lo, bits, nb, kmin);
+    };
+    if (n <= 1 * RS1_BLOCK) launch(std::integral_constant<uint32_t, 1>{});
+    else if (n <= 2 * RS1_BLOCK) launch(std::integral_constant<uint32_t, 2>{});
+    else if (n <= 4 * RS1_BLOCK) launch(std::integral_constant<uint32_t, 4>{});
+    else launch(std::integral_constant<uint32_t, RS1_MAX_IT>{});
     return;
   }
-  if (n <= c.tune.coop_max_n) {
-    // one launch for every pass: ceil(n / coop_tile) workgroups (at most COOP_MAX_BLOCKS)
-    const uint32_t tile0 = std::max<uint32_t>(c.tune.coop_tile, (uint32_t)ceil_div(n, COOP_MAX_BLOCKS));
-    const uint32_t tile = (tile0 + RS_BLOCK - 1) / RS_BLOCK * RS_BLOCK;
-    const uint32_t B = ceil_div(n, tile);
-    const int passes = (bits - lo + 7) / 8;
-    const unsigned int base = coop_barrier_base(c, 2u * passes * B);
-    DBuf<K> k2(c, n);
-    DBuf<uint32_t> v2(c, vals ? n : 0);
-    DBuf<uint32_t> counts(c, (uint64_t)256 * B);
-    const uint64_t sb = (uint64_t)passes * n * (2 * sizeof(K) + (vals ? 8 : 0));
-    if (vals)
-      HGP_LAUNCH_B(sb, (k_rs_coop<K, true>), B, RS_BLOCK, 0, c, keys, vals, k2.get(), v2.get(), (uint32_t)n, tile, lo,
-                   bits, kmin, counts.get(), c.coop_bar, base);
-    else
-      HGP_LAUNCH_B(sb, (k_rs_coop<K, false>), B, RS_BLOCK, 0, c, keys, vals, k2.get(), v2.get(), (uint32_t)n, tile,
-                   lo, bits, kmin, counts.get(), c.coop_bar, base);
-    c.coop_issued += 2u * passes * B;
-    if (passes & 1) {
-      if (kbuf && (!vals || vbuf)) {  // hand the scratch buffers over instead of copying
-        std::swap(*kbuf, k2);
-        if (vals) std::swap(*vbuf, v2);
-        return;
-      }
-      copy_d2d(c, keys, k2.get(), n * sizeof(K));
-      if (vals) copy_d2d(c, vals, v2.get(), n * sizeof(uint32_t));
-    }
-    return;
-  }
-  const uint32_t rounds = rs_rounds(c, n);
-  const uint32_t nblocks = ceil_div(n, (uint64_t)RS_BLOCK * rounds);
+  const uint32_t it = rs_items(c, n);
+  const uint64_t tiles64 = (n + (uint64_t)RS_BLOCK * it - 1) / ((uint64_t)RS_BLOCK * it);
+  HGP_REQUIRE(tiles64 < (1ull << 31), HGP_E_CAPACITY, "radix sort: too many tiles");
+  const uint32_t tiles = (uint32_t)tiles64;
+  const bool direct = tiles <= RS_DIRECT_TILES;
   DBuf<K> k2(c, n);
   DBuf<uint32_t> v2(c, vals ? n : 0);
-  DBuf<uint32_t> counts(c, (uint64_t)256 * nblocks);
-  DBuf<uint64_t> offsets(c, (uint64_t)256 * nblocks + 1);
+  DBuf<uint32_t> counts(c, (uint64_t)tiles * 256);
+  DBuf<uint64_t> before(c, direct ? 0 : ((uint64_t)tiles + 1) * 256);  // and the totals
+  uint64_t* totals = direct ? nullptr : before.get() + (uint64_t)tiles * 256;
   K* ka = keys;
   K* kb = k2.get();
   uint32_t* va = vals;
   uint32_t* vb = v2.get();
-  for (int shift = lo; shift < bits; shift += 8) {
-    // bytes: keys read once, one count per (digit, tile) written
-    HGP_LAUNCH_B(n * sizeof(K) + 1024ull * nblocks, (k_rs_hist<K>), nblocks, RS_BLOCK, 0, c, ka, n, shift, nblocks, rounds, kmin,
-                 counts.get());
-    exclusive_scan(c, counts.get(), offsets.get(), (uint64_t)256 * nblocks);
-    // bytes: keys (and values) read once and written once, one offset per (digit, tile) read
-    const uint64_t sb = n * (2 * sizeof(K) + (vals ? 8 : 0)) + 2048ull * nblocks;
-    if (vals)
-      HGP_LAUNCH_B(sb, (k_rs_scatter<K, true>), nblocks, RS_BLOCK, 0, c, ka, va, kb, vb, n, shift, nblocks,
-                   rounds, kmin, offsets.get());
-    else
-      HGP_LAUNCH_B(sb, (k_rs_scatter<K, false>), nblocks, RS_BLOCK, 0, c, ka, va, kb, vb, n, shift, nblocks,
-                   rounds, kmin, offsets.get());
+  // bytes: keys (and values) read once and written once, one offset per (tile, digit) read
+  const uint64_t sb = n * (2 * sizeof(K) + (vals ? 8 : 0)) + 2048ull * tiles;
+  for (int shift = lo; shift < bits; shift += nb) {
+    const int nbp = std::min(nb, bits - shift);
+    auto launch = [&](auto items) {
+      constexpr uint32_t IT = decltype(items)::value;
+      // bytes: keys read once, one count per (tile, digit) written
+      HGP_LAUNCH_B(n * sizeof(K) + 1024ull * tiles, (k_rs_count<K, IT>), tiles, OS_BLOCK, 0, c, ka, n, shift, nbp, kmin,
+                   counts.get());
+      if (!direct) HGP_LAUNCH(k_rs_columns, 16, 1024, 0, c, counts.get(), tiles, before.get(), totals);
+      if (vals)
+        HGP_LAUNCH_B(sb, (k_rs_pass<K, true, IT>), tiles, OS_BLOCK, 0, c, ka, va, kb, vb, n, shift, nbp, kmin,
+                     counts.get(), before.get(), totals);
+      else
+        HGP_LAUNCH_B(sb, (k_rs_pass<K, false, IT>), tiles, OS_BLOCK, 0, c, ka, va, kb, vb, n, shift, nbp, kmin,
+                     counts.get(), before.get(), totals);
+    };
+    if (it == 2) launch(std::integral_constant<uint32_t, 1>{});
+    else if (it == 4) launch(std::integral_constant<uint32_t, 2>{});
+    else if (it == 8) launch(std::integral_constant<uint32_t, 4>{});
+    else launch(std::integral_constant<uint32_t, 8>{});
     std::swap(ka, kb);
     std::swap(va, vb);
   }
@@ -743,9 +756,6 @@ void inclusive_scan(Ctx& c, const int32_t* in, int32_t* out, uint64_t n) { scan_
 
 void radix_sort(Ctx& c, uint32_t* keys, uint32_t* vals, uint64_t n, int bits) { radix_impl<uint32_t>(c, keys, vals, n, bits); }
 void radix_sort(Ctx& c, uint64_t* keys, uint32_t* vals, uint64_t n, int bits) { radix_impl<uint64_t>(c, keys, vals, n, bits); }
-void radix_sort_bits(Ctx& c, uint64_t* keys, uint32_t* vals, uint64_t n, int lo, int hi) {
-  radix_impl<uint64_t>(c, keys, vals, n, hi, lo);
-}
 void radix_sort_buf(Ctx& c, DBuf<uint32_t>& keys, DBuf<uint32_t>& vals, uint64_t n, int lo, int hi) {
   radix_impl<uint32_t>(c, keys.get(), vals.get(), n, hi, lo, &keys, &vals);
 }
@@ -760,8 +770,7 @@ void segment_offsets(Ctx& c, const uint64_t* keys, int shift, uint64_t n, uint32
   HGP_LAUNCH((k_segment_offsets<uint64_t>), ceil_div(n + 1, 256), 256, 0, c, keys, shift, n, nseg, off);
 }
 
-namespace {
-void range_impl(Ctx& c, uint64_t* keys, uint32_t* vals, uint64_t n, DBuf<uint64_t>* kbuf, DBuf<uint32_t>* vbuf) {
+void radix_sort_range(Ctx& c, uint64_t* keys, uint32_t* vals, uint64_t n) {
   if (n <= 1) return;
   DBuf<unsigned long long> mm(c, 2);
   HGP_LAUNCH(k_init_minmax, 1, 1, 0, c, mm.get());  // on the stream: no host-to-device copy
@@ -770,13 +779,7 @@ void range_impl(Ctx& c, uint64_t* keys, uint32_t* vals, uint64_t n, DBuf<uint64_
   copy_d2h(c, h, mm.get(), sizeof h);
   if (h[1] == h[0]) return;  // all keys equal: a stable sort is the identity
   // digits of key - min: the passes cover only the keys' range
-  radix_impl<uint64_t>(c, keys, vals, n, bit_width(h[1] - h[0]), 0, kbuf, vbuf, (uint64_t)h[0]);
-}
-}  // namespace
-
-void radix_sort_range(Ctx& c, uint64_t* keys, uint32_t* vals, uint64_t n) { range_impl(c, keys, vals, n, nullptr, nullptr); }
-void radix_sort_range_buf(Ctx& c, DBuf<uint64_t>& keys, DBuf<uint32_t>& vals, uint64_t n) {
-  range_impl(c, keys.get(), vals.get(), n, &keys, &vals);
+  radix_impl<uint64_t>(c, keys, vals, n, bit_width(h[1] - h[0]), 0, nullptr, nullptr, (uint64_t)h[0]);
 }
 
 Fork::Fork(Ctx& c, bool enabled) : c_(c), enabled_(enabled) {

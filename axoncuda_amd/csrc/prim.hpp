@@ -17,10 +17,8 @@ void inclusive_scan(Ctx& c, const int32_t* in, int32_t* out, uint64_t n);
 // Stable LSD radix sorts over key bits [0, bits); values ride along (nullable).
 void radix_sort(Ctx& c, uint32_t* keys, uint32_t* vals, uint64_t n, int bits);
 void radix_sort(Ctx& c, uint64_t* keys, uint32_t* vals, uint64_t n, int bits);
-// Stable sort by key bits [lo, hi) only: when the input is already ordered by the bits below
-// lo, the result is ordered by bits [0, hi), in (hi - lo) / 8 passes instead of hi / 8.
-void radix_sort_bits(Ctx& c, uint64_t* keys, uint32_t* vals, uint64_t n, int lo, int hi);
-// The same over bits [lo, hi) of buffers the caller owns: after an odd number of passes the
+// The same over bits [lo, hi) only, of buffers the caller owns (when the input is already ordered
+// by the bits below lo, the result is ordered by bits [0, hi)): after an odd number of passes the
 // buffers are exchanged with the sort's scratch ones instead of copied back (the DBufs then
 // hold different allocations; any raw pointer taken before is stale).
 void radix_sort_buf(Ctx& c, DBuf<uint32_t>& keys, DBuf<uint32_t>& vals, uint64_t n, int lo, int hi);
@@ -28,9 +26,6 @@ void radix_sort_buf(Ctx& c, DBuf<uint64_t>& keys, DBuf<uint32_t>& vals, uint64_t
 // Stable sort over the keys' actual range: digits are taken from key - min, so only the bits
 // that the maximum difference needs are sorted; the keys come out unchanged.
 void radix_sort_range(Ctx& c, uint64_t* keys, uint32_t* vals, uint64_t n);
-// The same on buffers the caller owns, exchanged with the scratch ones instead of copied back
-// (see radix_sort_buf).
-void radix_sort_range_buf(Ctx& c, DBuf<uint64_t>& keys, DBuf<uint32_t>& vals, uint64_t n);
 
 // off[s] = first index i with (keys[i] >> shift) >= s, for s in [0, nseg]; keys sorted.
 void segment_offsets(Ctx& c, const uint32_t* keys, int shift, uint64_t n, uint32_t nseg, uint64_t* off);

@@ -105,7 +105,7 @@ enum { HGP_IP_HOST = 0, HGP_IP_DEVICE = 1, HGP_IP_AUTO = 2 };
  * the same result under any valid setting. */
 typedef struct hgp_tuning {
   /* radix sorts of 2^c .. 2^(c+1) - 1 keys: keys per thread in a workgroup's tile (the tile is
-   * 256 x this many keys), 1..16; 0 = the built-in rule (about 512 tiles per sort) */
+   * 256 x this many keys), 1..16, taken as the next of 2, 4, 8 and 16; 0 = the built-in rule */
   uint32_t sort_rounds[40];
   /* candidate scoring of heavy nodes: slots of the first-attempt HBM hash table (a power of
    * two, 2^13..2^24) and its fill limit in sixteenths (4..14), i.e. the table occupancy that
@@ -125,9 +125,8 @@ typedef struct hgp_tuning {
    * stream: bit 0 the candidate tiers, bit 1 the cascade's sorted hedge classes beside the
    * size and inbound events, bit 2 (with bit 1) beside the small-hedge cascade too */
   uint32_t side_streams;
-  /* radix sorts of more than 16,384 and at most coop_max_n keys run all their passes in one
-   * launch of at most 64 workgroups that meet at grid barriers, each taking at least
-   * coop_tile keys (0 disables them; serving workers never use them) */
+  /* accepted, saved and returned, without effect (they bounded a sort with grid barriers that
+   * is no longer there) */
   uint32_t coop_max_n;
   uint32_t coop_tile;
   /* 1 when set by hgp_autotune */

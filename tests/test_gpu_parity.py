@@ -306,6 +306,41 @@ def test_refine_analyze_huge_lists(dev, mode, k, fm_repeat, chainup, n, e, max_s
     assert got["best"] == exp["best"]
 
 
+@pytest.mark.parametrize("p", [1, 2, 63, 64, 65, 1023, 1025, 2048, 4097, 8191, 8192, 8193, 65535, 65536, 65537, 131072,
+                               131073, 300001, 1 << 20, (1 << 20) + 1])
+@pytest.mark.parametrize("n", [2, 100, 70000, 3000000])
+def test_sorts_by_size(dev, p, n, rng):
+    """The radix sorts at the edges of their kernels and tiles, by way of the incidence lists (32-bit
+    keys with values, stable) and the coarse hedges (64-bit keys): one pass to seven, few and many
+    distinct keys."""
+    lens = np.minimum(rng.integers(1, 6, size=p), n).astype(np.int64)
+    lens = lens[:int(np.searchsorted(np.cumsum(lens), p)) + 1]
+    lens[-1] -= lens.sum() - p
+    off = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint64)
+    e = len(lens)
+    # distinct pins within a hedge: a random start and consecutive ids
+    start = rng.integers(0, n, size=e)
+    pos = np.arange(p) - np.repeat(off[:-1].astype(np.int64), lens)
+    pins = ((np.repeat(start, lens) + pos) % n).astype(np.uint32)
+    srcc = np.minimum(rng.integers(0, 2, size=e), lens).astype(np.uint32)
+    hg = O.HG(n, off, pins, srcc, np.ones(e, np.float32))
+    L = G.Level(dev, hg)
+    toff, tch, inb = L.build_touching()
+    hedge = np.repeat(np.arange(e, dtype=np.uint32), lens)
+    key = pins.astype(np.int64) * 2 + (pos < np.repeat(srcc, lens))
+    order = np.argsort(key, kind="stable")
+    assert np.array_equal(tch, hedge[order])
+    assert np.array_equal(toff, np.concatenate([[0], np.cumsum(np.bincount(pins, minlength=n))]).astype(np.uint64))
+    assert np.array_equal(inb, np.bincount(pins[key % 2 == 0], minlength=n).astype(np.uint32))
+    groups = (rng.permutation(n) // 2).astype(np.uint32)
+    d_groups = dev.upload(groups)
+    choff, cp, csrcc, *_ = G.coarsen_hedges(dev, L, d_groups)
+    eo, ep, es = O.coarsen_hedges(hg, groups)
+    assert np.array_equal(choff, eo) and np.array_equal(cp, ep) and np.array_equal(csrcc, es)
+    for x in (d_groups, L.pins, L.off, L.srcc, L.w, L.tch, L.toff, L.inb):
+        dev.free(x)
+
+
 @pytest.mark.parametrize("mode,k,scale,chainup", [
     (1, 2, 1.0, False),            # whole-number gains: few varying bits, cycles of moves
     (0, 300, 1.0, True),
