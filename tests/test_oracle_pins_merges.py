@@ -306,3 +306,21 @@ def test_initial_partitioner_is_independent_of_threads():
         O.set_ip_threads(0)
     many, ps2 = O.initial_partition(g, sizes, 16, 0.03, omega, prune=False)
     assert np.array_equal(one, many) and np.array_equal(ps1, ps2)
+
+
+@pytest.mark.parametrize("n,e,k,weights,digest", [
+    (60, 50, 5, "int", 18324815),          # one block of the gain queue
+    (3000, 3000, 7, "float", 1634108869),    # fractional hedge weights
+    (4200, 9000, 64, "int", 3257163293),     # more than one block of blocks
+    (40000, 60000, 6, "unit", 2456725103),   # node ids of 16 bits
+    (70000, 50000, 2, "int", 2965228201),    # ... and of 32
+])
+def test_initial_partitioner_pinned(n, e, k, weights, digest):
+    """The bisection's partitions, as recorded when its gain queues were plain scans (up to 32,768
+    nodes) and heaps (above): the queue's structure must not show in the result."""
+    rng = seeded(f"ip-pin-{n}-{k}")
+    g = O.dedup(O.HG(*gen.random_hypergraph(n, e, rng, max_size=6, weights=weights)))
+    sizes = rng.integers(1, 9, g.n).astype(np.uint32)
+    omega = O.kway_omega(int(sizes.sum()), k, 0.03)
+    part, _ = O.initial_partition(g, sizes, k, 0.03, omega, prune=False)
+    assert zlib.crc32(part.astype("<u4").tobytes()) == digest
