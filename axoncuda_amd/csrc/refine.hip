@@ -38,9 +38,9 @@ constexpr uint32_t GAIN_LIGHT = 512;
 constexpr uint32_t GAIN_BLOCK_MIN = 4096;  // entries above which a node takes a workgroup even for small k
 constexpr uint32_t GAIN_TINY = 16;  // partition entries handled by one thread in registers
 constexpr uint32_t CAS_SMALL = 16;
+constexpr uint32_t CAS_WAVE = 128;   // pins of a hedge cascaded by one wave in registers
 constexpr uint32_t CAS_LDS = 2048;
 constexpr uint32_t CAS_SORT = 1024;               // pins of a hedge cascaded through sorted events
-constexpr uint32_t CAS_SORT_S = 128;              // ... by the small-LDS instance
 constexpr uint32_t CAS_EV = 2048;                 // event slots: next power of two >= 2 * CAS_SORT
 constexpr uint32_t CAS_SORT_NT = 256;              // threads sorting the events of one such hedge
 constexpr uint64_t HEAVY_BATCH_SLOTS = 32ull << 20;
@@ -1997,6 +1997,7 @@ struct CascadeArgs {
   // leave (low word) and enter (high word) a partition with that move (see k_inbound_deltas)
   const uint32_t* srcc;
   unsigned long long* dio;
+  uint32_t V;  // ranks
 };
 constexpr uint32_t PM2_MAX_K = 0xFFFFu;  // partition ids < 0xFFFF leave 0xFFFF for "no move"
 
@@ -2036,8 +2037,8 @@ __device__ __forceinline__ int64_t cascade_term(int incc, int64_t W, int64_t cp,
 }
 
 // Cascade classes of a level's hedges: min_len..CAS_SMALL pins (the thread-per-hedge kernel; the
-// key orders them by their first pin), the sorted kernels (up to CAS_SORT_S or sort_max
-// pins) and the direct LDS/HBM kernel.  A hedge of one pin adds nothing to the cascade: its pin
+// key orders them by their first pin), up to CAS_WAVE pins (a wave each), up to sort_max pins (the
+// sorted events) and the direct LDS/HBM kernel.  A hedge of one pin adds nothing to the cascade: its pin
 // finds itself alone in p and nobody in q, so the two terms of cascade_term cancel.  It does
 // count for the inbound sets, so min_len is 2 in k-way mode and 1 in inbound-constrained mode.
 __global__ void k_cascade_classes(const uint32_t* __restrict__ hedges, const uint64_t* __restrict__ hoff, uint32_t E,
@@ -2047,12 +2048,13 @@ __global__ void k_cascade_classes(const uint32_t* __restrict__ hedges, const uin
   if (e >= E) return;
   const uint64_t s = hoff[e], hl = hoff[e + 1] - s;
   const bool small = hl >= min_len && hl <= CAS_SMALL;
-  const bool sorted = hl > CAS_SMALL && hl <= sort_max;
+  const bool wave = hl > CAS_SMALL && hl <= CAS_WAVE;
+  const bool sorted = hl > CAS_WAVE && hl <= sort_max;
   f_small[e] = small ? 1u : 0u;
   k_small[e] = small ? ((uint64_t)hedges[s] << 32) | e : 0ull;
-  f_s[e] = (sorted && hl <= CAS_SORT_S) ? 1u : 0u;
-  f_m[e] = (sorted && hl > CAS_SORT_S) ? 1u : 0u;
-  f_big[e] = (hl > CAS_SMALL && !sorted) ? 1u : 0u;
+  f_s[e] = wave ? 1u : 0u;
+  f_m[e] = sorted ? 1u : 0u;
+  f_big[e] = (hl > CAS_WAVE && !sorted) ? 1u : 0u;
 }
 
 // The level's hedges of 2..CAS_SMALL pins as their own CSR, in order of their first pin (built
@@ -2065,6 +2067,39 @@ struct SmallHedges {
   uint32_t m;
 };
 
+// Where the cascade kernels add their terms.  ACC: with few ranks, many hedges meet on the same
+// counters (the coarse levels of an inbound-constrained run have thousands of hedges on tens of
+// nodes), so a workgroup sums in LDS over all its hedges and adds every counter once at its end.
+constexpr uint32_t CAS_ACC_BYTES = 32768;   // LDS counters of a workgroup (8 bytes a rank, 16 with dio)
+constexpr uint32_t CAS_ACC_GRID = 512;      // workgroups of those launches (at most)
+extern __shared__ unsigned long long s_cas_acc[];
+template <bool INCC, bool ACC>
+__device__ __forceinline__ void cas_clear(uint32_t V) {
+  if constexpr (ACC) {
+    for (uint32_t i = threadIdx.x; i < (INCC ? 2 * V : V); i += blockDim.x) s_cas_acc[i] = 0;
+    __syncthreads();
+  }
+}
+template <bool ACC>
+__device__ __forceinline__ void cas_add(const CascadeArgs& a, uint32_t r, int64_t term) {
+  if (term) atomicAdd(ACC ? &s_cas_acc[r] : &a.seq[r], (unsigned long long)term);
+}
+template <bool ACC>
+__device__ __forceinline__ void cas_add_io(const CascadeArgs& a, uint32_t r, bool leaves, bool enters) {
+  const unsigned long long io = (leaves ? 1ull : 0ull) | (enters ? 1ull << 32 : 0ull);
+  if (io) atomicAdd(ACC ? &s_cas_acc[a.V + r] : &a.dio[r], io);
+}
+template <bool INCC, bool ACC>
+__device__ __forceinline__ void cas_flush(const CascadeArgs& a) {
+  if constexpr (ACC) {
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < a.V; i += blockDim.x) {
+      if (s_cas_acc[i]) atomicAdd(&a.seq[i], s_cas_acc[i]);
+      if (INCC && s_cas_acc[a.V + i]) atomicAdd(&a.dio[i], s_cas_acc[a.V + i]);
+    }
+  }
+}
+
 // Hedges of 2..CAS_SMALL pins, one thread each, each XCD given a contiguous range of the
 // first-pin order so that the records its threads gather meet in one L2.
 // P16 (packed records, k < PM2_MAX_K): a pin's partition and target stay packed in one
@@ -2074,9 +2109,8 @@ struct SmallHedges {
 // and its target just before the move.  The hedge leaves the source's inbound set when they are
 // all this node (a hedge that lists a node twice counts it once, at the first of its pins), and
 // enters the target's when there are none: one 64-bit atomic per pin that changes either.
-template <bool P16, bool INCC>
-__global__ void k_cascade_small(CascadeArgs a, SmallHedges h) {
-  const uint32_t i = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+template <bool P16, bool INCC, bool ACC>
+__device__ __forceinline__ void cascade_small_hedge(const CascadeArgs& a, const SmallHedges& h, uint32_t i) {
   if (i >= h.m) return;
   const uint64_t rec = h.rec[i];
   const uint64_t s = rec >> 10;
@@ -2169,16 +2203,101 @@ __global__ void k_cascade_small(CascadeArgs a, SmallHedges h) {
           }
         }
       }
-      const int64_t term = cascade_term(a.incc, W, cp, cq);
-      if (term) atomicAdd(&a.seq[r], (unsigned long long)term);
+      cas_add<ACC>(a, r, cascade_term(a.incc, W, cp, cq));
       if constexpr (INCC) {
-        if (i >= sc && !again) {
-          const unsigned long long io = (dp == own ? 1ull : 0ull) | (dq == 0 ? 1ull << 32 : 0ull);
-          if (io) atomicAdd(&a.dio[r], io);
-        }
+        if (i >= sc && !again) cas_add_io<ACC>(a, r, dp == own, dq == 0);
       }
     }
   }
+}
+template <bool P16, bool INCC, bool ACC>
+__global__ void k_cascade_small(CascadeArgs a, SmallHedges h) {
+  cas_clear<INCC, ACC>(a.V);
+  const uint32_t blocks = (h.m + blockDim.x - 1) / blockDim.x;  // ACC: the grid strides over them
+  for (uint32_t b = blockIdx.x; b < blocks; b += gridDim.x)
+    cascade_small_hedge<P16, INCC, ACC>(a, h, xcd_block(b, blocks) * blockDim.x + threadIdx.x);
+  cas_flush<INCC, ACC>(a);
+}
+
+// Hedges of CAS_SMALL < len <= CAS_WAVE pins, one wave each: lane l holds pins l (and 64 + l), and
+// every pin is read as a scalar in turn and compared with all of them, six vector instructions per
+// pin and register.  The event sort below needs LDS and a chain of barriers for it: 57,337
+// hedges of 65 pins took 180 us that way.
+template <uint32_t R, bool INCC, bool ACC>
+__device__ __forceinline__ void cascade_wave_hedge(const CascadeArgs& a, uint32_t e, uint64_t s, uint32_t len) {
+  const uint32_t l = lane_id();
+  uint32_t x[R], pt[R], mv[R], rk[R];
+#pragma unroll
+  for (uint32_t g = 0; g < R; ++g) x[g] = a.hedges[s + min(64 * g + l, len - 1)];
+  bool any = false;
+#pragma unroll
+  for (uint32_t g = 0; g < R; ++g) {
+    const uint3 rec = pm_at(a, x[g]);
+    const bool in = 64 * g + l < len;
+    pt[g] = in ? rec.x : NONE;  // entries past the end: of no partition, never moving
+    mv[g] = in ? rec.y : NONE;
+    rk[g] = mv[g] != NONE ? rec.z : NONE;
+    any |= mv[g] != NONE;
+  }
+  if (!__ballot(any)) return;
+  // counts over the sources and, apart from them, over the destinations (INCC; else over all pins)
+  const uint32_t sc = INCC ? a.srcc[e] : 0u;
+  uint32_t sp[R], sq[R], dp[R], dq[R], own[R];
+#pragma unroll
+  for (uint32_t g = 0; g < R; ++g) sp[g] = sq[g] = dp[g] = dq[g] = own[g] = 0;
+  auto against = [&](uint32_t pj, uint32_t mj, uint32_t rj, uint32_t (&np)[R], uint32_t (&nq)[R], bool dst) {
+#pragma unroll
+    for (uint32_t g = 0; g < R; ++g) {
+      const uint32_t now = rj < rk[g] ? mj : pj;  // its partition when this lane's pin moves
+      np[g] += now == pt[g];
+      nq[g] += now == mv[g];
+      if (INCC && dst) own[g] += rj == rk[g];
+    }
+  };
+#pragma unroll
+  for (uint32_t g = 0; g < R; ++g) {
+    const uint32_t beg = 64 * g, end = min(64 * g + 64, len);
+    uint32_t j = beg;
+    for (; INCC && j < min(end, sc); ++j)
+      against(lane_value(pt[g], j - beg), lane_value(mv[g], j - beg), lane_value(rk[g], j - beg), sp, sq, false);
+    for (; j < end; j += 4) {
+#pragma unroll
+      for (uint32_t u = 0; u < 4; ++u)
+        if (j + u < end)
+          against(lane_value(pt[g], j + u - beg), lane_value(mv[g], j + u - beg), lane_value(rk[g], j + u - beg), dp, dq,
+                  true);
+    }
+  }
+  const int64_t W = (int64_t)fixed_weight(a.w[e]);
+#pragma unroll
+  for (uint32_t g = 0; g < R; ++g) {
+    const uint32_t i = 64 * g + l;
+    const bool moving = mv[g] != NONE;
+    if (moving) cas_add<ACC>(a, rk[g], cascade_term(a.incc, W, sp[g] + dp[g], sq[g] + dq[g]));
+    if (INCC) {
+      const bool dst = moving && i >= sc;
+      bool again = false;  // an earlier destination pin is the same node
+      if (__ballot(dst && own[g] > 1)) {
+        for (uint32_t j = sc; j < len; ++j) {
+          const uint32_t rj = R > 1 && j >= 64 ? lane_value(rk[R - 1], j - 64) : lane_value(rk[0], j);
+          again |= j < i && rj == rk[g];
+        }
+      }
+      if (dst && !again) cas_add_io<ACC>(a, rk[g], dp[g] == own[g], dq[g] == 0);
+    }
+  }
+}
+template <bool INCC, bool ACC>
+__global__ void __launch_bounds__(256) k_cascade_wave(CascadeArgs a, const uint32_t* __restrict__ list, uint32_t m) {
+  cas_clear<INCC, ACC>(a.V);
+  for (uint32_t b = blockIdx.x * 4 + threadIdx.x / 64; b < m; b += gridDim.x * 4) {
+    const uint32_t e = (uint32_t)__builtin_amdgcn_readfirstlane((int)list[b]);
+    const uint64_t s = a.hoff[e];
+    const uint32_t len = (uint32_t)(a.hoff[e + 1] - s);
+    if (len <= 64) cascade_wave_hedge<1, INCC, ACC>(a, e, s, len);
+    else cascade_wave_hedge<2, INCC, ACC>(a, e, s, len);
+  }
+  cas_flush<INCC, ACC>(a);
 }
 
 // Algorithmic bytes of one k_cascade_small launch, counted when that kernel is profiled (a
@@ -2267,7 +2386,7 @@ __global__ void __launch_bounds__(64) k_cascade_large(CascadeArgs a, const uint3
   }
 }
 
-// Cascade of one hedge through sorted events (hedges of CAS_SMALL < len <= CAS_SORT pins,
+// Cascade of one hedge through sorted events (hedges of CAS_WAVE < len <= CAS_SORT pins,
 // one workgroup per hedge).  The pins' partitions are counted in an LDS hash table; every
 // moving pin contributes an "out" event (source, -1) and an "in" event (target, +1) at its
 // rank.  Sorted by (partition, rank), a move event's exclusive prefix within its partition,
@@ -3044,7 +3163,7 @@ void analyze_round(Ctx& c, const RefineLevel& L, int mode, uint32_t omega, uint3
       pm = DBuf<uint4>(c, n);
       HGP_LAUNCH(k_pack_nodes, g, 256, 0, c, part, st.moves.get(), st.ranks.get(), n, pm.get());
     }
-    CascadeArgs a{L.hedges, L.hoff, L.w, pm.get(), pm2.get(), incc ? 1 : 0, st.seq.get(), L.srcc, dio.get()};
+    CascadeArgs a{L.hedges, L.hoff, L.w, pm.get(), pm2.get(), incc ? 1 : 0, st.seq.get(), L.srcc, dio.get(), V};
     const int crb = std::max(1, bit_width(V));  // rank + 1 <= V
     const int cpb = std::max(1, bit_width(L.k));
     const uint32_t sort_max = cpb + crb + 11 < 64 ? CAS_SORT : 0u;
@@ -3076,15 +3195,27 @@ void analyze_round(Ctx& c, const RefineLevel& L, int mode, uint32_t omega, uint3
         Y.cs = small_csr(c, kc.get(), m, L.hoff, L.hedges, L.w, incc ? L.srcc : nullptr);
       }
     }
+    // few ranks: the counters in LDS (see cas_add)
+    const uint32_t acc_lds = V * (incc ? 16u : 8u);
+    const bool acc = acc_lds <= CAS_ACC_BYTES;
+    // runs f with compile-time (INCC, ACC)
+    auto with_modes = [&](auto&& f) {
+      if (incc && acc) f(std::true_type{}, std::true_type{});
+      else if (incc) f(std::true_type{}, std::false_type{});
+      else if (acc) f(std::false_type{}, std::true_type{});
+      else f(std::false_type{}, std::false_type{});
+    };
     auto small_cascade = [&] {
       const uint32_t m = Y.cs.m;
       if (!m) return;
       const SmallHedges sh{Y.cs.rec.get(), Y.cs.pins.get(), Y.cs.w.get(), m};
       const uint32_t cb = c.tune.cascade_block;  // 256 unless the autotuner chose otherwise
-      if (a.pm2 && incc) HGP_LAUNCH((k_cascade_small<true, true>), ceil_div(m, cb), cb, 0, c, a, sh);
-      else if (incc) HGP_LAUNCH((k_cascade_small<false, true>), ceil_div(m, cb), cb, 0, c, a, sh);
-      else if (a.pm2) HGP_LAUNCH((k_cascade_small<true, false>), ceil_div(m, cb), cb, 0, c, a, sh);
-      else HGP_LAUNCH((k_cascade_small<false, false>), ceil_div(m, cb), cb, 0, c, a, sh);
+      const uint32_t cg = acc ? std::min<uint32_t>(ceil_div(m, cb), CAS_ACC_GRID) : ceil_div(m, cb);
+      with_modes([&](auto mi, auto ma) {
+        constexpr bool INCC = decltype(mi)::value, ACC = decltype(ma)::value;
+        if (a.pm2) HGP_LAUNCH((k_cascade_small<true, INCC, ACC>), cg, cb, ACC ? acc_lds : 0, c, a, sh);
+        else HGP_LAUNCH((k_cascade_small<false, INCC, ACC>), cg, cb, ACC ? acc_lds : 0, c, a, sh);
+      });
       if (prof_match(c, "k_cascade_small") && c.prof_count && c.prof_dev)
         HGP_LAUNCH(k_cascade_small_bytes, ceil_div(m, 256), 256, 0, c, a, sh, c.prof_dev);
     };
@@ -3098,16 +3229,15 @@ void analyze_round(Ctx& c, const RefineLevel& L, int mode, uint32_t omega, uint3
       if (m == 0) continue;
       const uint32_t* lst = Y.cas_list[cls].get();
       cas_fork->on(cls, [&] {
-        auto launch = [&](auto mode_incc) {
-          constexpr bool INCC = decltype(mode_incc)::value;
+        with_modes([&](auto mi, auto ma) {
+          constexpr bool INCC = decltype(mi)::value, ACC = decltype(ma)::value;
           if (cls == 0)
-            HGP_LAUNCH((k_cascade_sorted<CAS_SORT_S, 2 * CAS_SORT_S, 64, INCC>), m, 64, 0, c, a, lst, crb);
+            HGP_LAUNCH((k_cascade_wave<INCC, ACC>), ACC ? std::min<uint32_t>(ceil_div(m, 4), CAS_ACC_GRID) : ceil_div(m, 4),
+                       256, ACC ? acc_lds : 0, c, a, lst, m);
           else if (cls == 1)
             HGP_LAUNCH((k_cascade_sorted<CAS_SORT, CAS_EV, CAS_SORT_NT, INCC>), m, CAS_SORT_NT, 0, c, a, lst, crb);
           else HGP_LAUNCH((k_cascade_large<INCC>), m, 64, 0, c, a, lst);
-        };
-        if (incc) launch(std::true_type{});
-        else launch(std::false_type{});
+        });
       });
     }
     if (early) small_cascade();
@@ -3269,13 +3399,13 @@ SmallCsr small_csr(Ctx& c, const uint64_t* keys, uint32_t m, const uint64_t* hof
 
 float time_cascade_small(Ctx& c, const SmallCsr& cs, const uint2* pm2, uint32_t block, unsigned long long* seq) {
   const uint32_t m = cs.m;
-  CascadeArgs a{nullptr, nullptr, nullptr, nullptr, pm2, 0, seq, nullptr, nullptr};
+  CascadeArgs a{nullptr, nullptr, nullptr, nullptr, pm2, 0, seq, nullptr, nullptr, 0};
   const SmallHedges sh{cs.rec.get(), cs.pins.get(), cs.w.get(), m};
   hipEvent_t t0, t1;
   HGP_HIP(hipEventCreate(&t0));
   HGP_HIP(hipEventCreate(&t1));
   HGP_HIP(hipEventRecord(t0, c.stream));
-  HGP_LAUNCH((k_cascade_small<true, false>), ceil_div(m, block), block, 0, c, a, sh);
+  HGP_LAUNCH((k_cascade_small<true, false, false>), ceil_div(m, block), block, 0, c, a, sh);
   HGP_HIP(hipEventRecord(t1, c.stream));
   HGP_HIP(hipEventSynchronize(t1));
   float ms = 0;
