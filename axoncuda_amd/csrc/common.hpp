@@ -245,11 +245,13 @@ inline void prof_stop(Ctx& c, hipEvent_t a, uint64_t bytes) {
   c.prof.push_back({a, e, bytes});
 }
 
+inline uint64_t grid_threads(dim3 g) { return (uint64_t)g.x * g.y * g.z; }  // 0: nothing to launch
+
 // Kernel launch on the context stream.  HGP_LAUNCH_B also states the launch's algorithmic
 // bytes, which the kernel profiler (hgp_profile_kernel) reports next to the timing.
 #define HGP_LAUNCH_B(bytes, kernel, grid, block, shmem, ctx, ...)                             \
   do {                                                                                      \
-    if ((grid) > 0) {                                                                       \
+    if (::hgp::grid_threads(grid) > 0) {                                                    \
       const bool _prof = ::hgp::prof_match((ctx), #kernel);                                 \
       const uint64_t _bytes = _prof ? (uint64_t)(bytes) : 0; /* before the timed launch */  \
       hipEvent_t _pa = _prof ? ::hgp::prof_start(ctx) : nullptr;                            \

@@ -1745,12 +1745,16 @@ __global__ void k_zero3(unsigned long long* __restrict__ a, uint32_t* __restrict
 struct ChainArrays {
   const uint32_t* orig;  // j -> node
   uint4* pk;             // per entry: gain (lo, hi), size, valid
-  uint2* range;          // per entry: its target partition's entries (empty when invalid)
-  uint32_t* from;        // per entry: where its next proposal scan starts
   uint32_t* next;
   uint32_t* prev;
+  // proposals by table (see k_chain_table); null when they scan
+  uint2* ds;       // per entry: target partition (NONE: invalid), size
+  uint32_t* last;  // per entry: the slot it proposed to in the last iteration
+  // proposals by scan (see k_chain_propose)
+  uint2* range;    // per entry: its target partition's entries (empty when invalid)
+  uint32_t* from;  // per entry: where its next proposal scan starts
   unsigned long long* claim;
-  uint32_t* progress;    // progress[it] != 0: iteration it committed a link
+  uint32_t* progress;  // progress[it] != 0: iteration it committed a link
   // components, by head entry: summed gain, moves, holds an invalid move, exists
   long long* cw;
   uint32_t* csize;
@@ -1767,19 +1771,24 @@ __global__ void k_chain_gather(ChainArrays c, const uint32_t* __restrict__ moves
                                const uint32_t* __restrict__ sizes, const uint64_t* __restrict__ poff, uint32_t n,
                                KeyStats* comp_stats) {
   const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j < 4) c.progress[j] = 0u;
+  if (!c.ds && j < 4) c.progress[j] = 0u;
   if (j == 0) *comp_stats = KeyStats{~0ull, 0ull, 0ull, 0ull, 0ull};
   if (j >= n) return;
   const uint32_t v = c.orig[j];
   const uint32_t q = moves[v];
   const int64_t g = gains[v];
   c.pk[j] = make_uint4((uint32_t)(uint64_t)g, (uint32_t)((uint64_t)g >> 32), sizes[v], q != NONE ? 1u : 0u);
-  const uint2 r = q != NONE ? make_uint2((uint32_t)poff[q], (uint32_t)poff[q + 1]) : make_uint2(0u, 0u);
-  c.range[j] = r;
-  c.from[j] = r.x;
+  if (c.ds) {
+    c.ds[j] = make_uint2(q, sizes[v]);
+    c.last[j] = NONE;
+  } else {
+    const uint2 r = q != NONE ? make_uint2((uint32_t)poff[q], (uint32_t)poff[q + 1]) : make_uint2(0u, 0u);
+    c.range[j] = r;
+    c.from[j] = r.x;
+    c.claim[j] = 0ull;
+  }
   c.next[j] = NONE;
   c.prev[j] = NONE;
-  c.claim[j] = 0ull;
   c.cw[j] = 0;
   c.csize[j] = 0u;
   c.cinv[j] = 0u;
@@ -1787,28 +1796,182 @@ __global__ void k_chain_gather(ChainArrays c, const uint32_t* __restrict__ moves
 }
 __device__ __forceinline__ int size_bucket(uint32_t s) { return s == 0 ? 0 : 31 - __clz(s); }
 
-// Each open move proposes to the best free move out of its destination partition among the
-// first 256 entries of that partition's list.  The list is sorted by gain (descending, valid
-// moves first), so once a choice exists the scan stops at the first lower gain or invalid
-// entry: nothing later can beat it.  An entry that cannot be chosen (invalid, the proposer
-// itself, already linked, or of a size bucket too far) never can again, so the next scan
-// starts at the first entry this one could choose.
-// Claims, in the same launch: the proposer with the smallest size difference, then the lowest
-// index, wins.  Proposals pile onto few targets (the heads of the partition lists) but the
-// lanes of a wave rarely share one, so the workgroup first merges its claims per target in an
-// LDS table and then issues one global atomic per distinct target.  Claims start at zero: the
+// Chaining proposals.  Each open move proposes to the best free move out of its destination
+// partition among the first CHAIN_WINDOW entries of that partition's list: the highest gain among
+// sizes at most a bucket away, then the smallest size difference, then the first entry.  (The list
+// is sorted by gain, valid moves first; a move is never in its destination's list.)  Of a target's
+// proposers the one with the smallest size difference wins, then the lowest index.
+//
+// By table: the choice depends only on the destination and the proposer's size, so per iteration
+// one workgroup per partition (and 256 sizes) finds it for every size up to the level's largest,
+// and a move looks its own up.  Claims are kept per window slot and iteration: an entry is linked
+// once any iteration's claim on its slot is set, and a proposer is once it holds its last slot's
+// claim, so nothing is committed until the end.
+constexpr uint32_t CHAIN_WINDOW = 256;
+constexpr uint32_t CHAIN_TABLE_K = 1024;  // partitions of the table path (at most)
+// table entries (partitions x sizes): up to two a move, or this many
+constexpr uint64_t CHAIN_TABLE_MIN = 131072;
+constexpr uint64_t CHAIN_TABLE_SIZES = 1u << 20;  // sizes (at most: 65,535 workgroups of 256)
+__global__ void __launch_bounds__(CHAIN_WINDOW) k_chain_table(ChainArrays c, const uint64_t* __restrict__ poff,
+                                                              uint32_t nsizes, int it, uint32_t slots,
+                                                              const unsigned long long* __restrict__ claims,
+                                                              uint2* __restrict__ table) {
+  constexpr uint32_t WORDS = CHAIN_WINDOW / 64;
+  __shared__ int64_t s_gain[CHAIN_WINDOW];
+  __shared__ __align__(16) uint32_t s_size[CHAIN_WINDOW];
+  __shared__ uint32_t s_slot[CHAIN_WINDOW], s_cnt[WORDS];
+  static_assert(WORDS == 4, "the scan below picks among four words");
+  // the free entries of each size bucket (bucket b at b + 1; none on either side), and those that
+  // start a run of equal gains
+  __shared__ unsigned long long s_bucket[34][WORDS], s_run[WORDS];
+  const uint32_t q = blockIdx.x, t = threadIdx.x, w = t / 64;
+  for (uint32_t x = t; x < 34 * WORDS; x += CHAIN_WINDOW) (&s_bucket[0][0])[x] = 0;
+  const uint64_t j = poff[q] + t;
+  const uint32_t slot = q * CHAIN_WINDOW + t;
+  uint4 e = make_uint4(0, 0, 0, 0);
+  if (j < poff[q + 1]) e = c.pk[j];
+  bool free = e.w != 0;
+  for (int x = 0; x < it; ++x) free = free && claims[(uint64_t)x * slots + slot] == 0ull;
+  const uint64_t m = __ballot(free);
+  if (lane_id() == 0) s_cnt[w] = (uint32_t)__popcll(m);
+  __syncthreads();
+  uint32_t o = lanes_below(m), cnt = 0;
+#pragma unroll
+  for (uint32_t x = 0; x < WORDS; ++x) {
+    o += x < w ? s_cnt[x] : 0u;
+    cnt += s_cnt[x];
+  }
+  if (free) {
+    s_gain[o] = (int64_t)(((uint64_t)e.y << 32) | e.x);
+    s_size[o] = e.z;
+    s_slot[o] = slot;
+    atomicOr(&s_bucket[size_bucket(e.z) + 1][o / 64], 1ull << (o % 64));
+  }
+  __syncthreads();
+  const uint64_t heads = __ballot(t < cnt && (t == 0 || s_gain[t] != s_gain[t - 1]));
+  if (lane_id() == 0) s_run[w] = heads;
+  __syncthreads();
+  const uint32_t si = blockIdx.y * CHAIN_WINDOW + t;
+  if (si >= nsizes) return;
+  const int bi = size_bucket(si);
+  uint64_t fit[WORDS];  // entries of a fitting bucket
+  uint32_t first = CHAIN_WINDOW;
+#pragma unroll
+  for (uint32_t x = WORDS; x-- > 0;) {
+    fit[x] = s_bucket[bi][x] | s_bucket[bi + 1][x] | s_bucket[bi + 2][x];
+    if (fit[x]) first = 64 * x + (uint32_t)__ffsll((unsigned long long)fit[x]) - 1u;
+  }
+  uint32_t choice = NONE, bd = 0;
+  if (first < CHAIN_WINDOW) {
+    // the first one has the best gain; the nearest size among those of its run
+    uint32_t end = cnt;
+#pragma unroll
+    for (uint32_t x = WORDS; x-- > 0;) {
+      const uint64_t above = x < first / 64 ? 0ull : x > first / 64 ? s_run[x] : s_run[x] & ~lanes_upto(first % 64);
+      if (above) end = 64 * x + (uint32_t)__ffsll((unsigned long long)above) - 1u;
+    }
+    // eight sizes per step: a long run of equal gains costs one LDS round trip per step, not per entry
+    for (uint32_t x0 = first & ~7u; x0 < end && (choice == NONE || bd != 0); x0 += 8) {
+      const uint4 s0 = *reinterpret_cast<const uint4*>(&s_size[x0]), s1 = *reinterpret_cast<const uint4*>(&s_size[x0 + 4]);
+      const uint32_t sz[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
+      const uint64_t word = x0 < 64 ? fit[0] : x0 < 128 ? fit[1] : x0 < 192 ? fit[2] : fit[3];
+      uint32_t bits = (uint32_t)(word >> (x0 & 63u)) & 0xFFu;
+      if (end - x0 < 8) bits &= (1u << (end - x0)) - 1u;
+#pragma unroll
+      for (uint32_t u = 0; u < 8; ++u) {
+        const uint32_t d = si > sz[u] ? si - sz[u] : sz[u] - si;
+        const bool better = ((bits >> u) & 1u) && (choice == NONE || d < bd);
+        choice = better ? x0 + u : choice;
+        bd = better ? d : bd;
+      }
+    }
+    choice = s_slot[choice];
+  }
+  table[(uint64_t)q * nsizes + si] = make_uint2(choice, bd);
+}
+// The links of all iterations: slot's entry follows the claim's winner.
+__global__ void k_chain_links(ChainArrays c, const uint64_t* __restrict__ poff, uint32_t slots,
+                              const unsigned long long* __restrict__ claims) {
+  const uint32_t x = blockIdx.x * blockDim.x + threadIdx.x;
+  if (x >= 4 * slots) return;
+  const unsigned long long k = claims[x];
+  if (k == 0ull) return;
+  const uint32_t slot = x % slots;
+  const uint32_t j = (uint32_t)poff[slot / CHAIN_WINDOW] + slot % CHAIN_WINDOW;
+  const uint32_t p = 0xFFFFFFFFu - (uint32_t)(k & 0xFFFFFFFFull);
+  c.prev[j] = p;
+  c.next[p] = j;
+}
+
+// By scan (many partitions or sizes).  Once a choice exists the scan stops at the first lower
+// gain or invalid entry: nothing later can beat it.  An entry that cannot be chosen (invalid,
+// already linked, or of a size bucket too far) never can again, so the next scan starts at the
+// first entry this one could choose.
+// Claims, in the same launch: proposals pile onto few targets (the heads of the partition lists)
+// but the lanes of a wave rarely share one, so the workgroup first merges its claims per target in
+// an LDS table and then issues one global atomic per distinct target.  Claims start at zero: the
 // buffer is cleared when it is filled, and the commit clears every claim it reads.
 constexpr uint32_t RESOLVE_BLOCK = 1024;
 constexpr uint32_t RESOLVE_SLOTS = 2048;  // > 2 x the workgroup's claims: the table never fills
 constexpr uint32_t PROPOSE_BATCH = 6;     // list entries per load round (60 VGPRs: two workgroups per CU)
+struct ClaimTable {
+  uint32_t tgt[RESOLVE_SLOTS];
+  unsigned long long key[RESOLVE_SLOTS];
+};
+__device__ __forceinline__ void claims_clear(ClaimTable& s) {
+  for (uint32_t t = threadIdx.x; t < RESOLVE_SLOTS; t += RESOLVE_BLOCK) {
+    s.tgt[t] = NONE;
+    s.key[t] = 0ull;
+  }
+}
+// This thread's claim on `choice` (NONE: none) at size difference d, merged over the workgroup and
+// added to claim[]; every thread of the workgroup calls it.
+__device__ __forceinline__ void claims_add(ClaimTable& s, uint32_t choice, uint32_t d, uint32_t i,
+                                           unsigned long long* claim) {
+  __syncthreads();  // the table is cleared
+  if (choice != NONE) {
+    const unsigned long long key = ((unsigned long long)(0xFFFFFFFFu - d) << 32) | (0xFFFFFFFFu - i);
+    uint32_t h = slot_hash(choice) & (RESOLVE_SLOTS - 1);
+    for (;;) {
+      const uint32_t old = atomicCAS(&s.tgt[h], NONE, choice);
+      if (old == NONE || old == choice) break;
+      h = (h + 1) & (RESOLVE_SLOTS - 1);
+    }
+    atomicMax(&s.key[h], key);
+  }
+  __syncthreads();
+  for (uint32_t t = threadIdx.x; t < RESOLVE_SLOTS; t += RESOLVE_BLOCK)
+    if (s.tgt[t] != NONE) atomicMax(&claim[s.tgt[t]], s.key[t]);
+}
+__global__ void __launch_bounds__(RESOLVE_BLOCK) k_chain_lookup(ChainArrays c, uint32_t n, uint32_t nsizes, int it,
+                                                                uint32_t slots, const uint2* __restrict__ table,
+                                                                unsigned long long* claims) {
+  __shared__ ClaimTable s;
+  claims_clear(s);
+  const uint32_t i = blockIdx.x * RESOLVE_BLOCK + threadIdx.x;
+  uint2 choice = make_uint2(NONE, 0u);
+  if (i < n) {
+    const uint2 x = c.ds[i];
+    bool open = x.x != NONE;
+    if (open && it > 0) {
+      const uint32_t l = c.last[i];
+      // (a move keeps its last slot once it has won it)
+      if (l != NONE) {
+        for (int y = 0; y < it; ++y)
+          open = open && (uint32_t)(claims[(uint64_t)y * slots + l] & 0xFFFFFFFFull) != 0xFFFFFFFFu - i;
+      }
+    }
+    if (open) {
+      choice = table[(uint64_t)x.x * nsizes + x.y];
+      c.last[i] = choice.x;
+    }
+  }
+  claims_add(s, choice.x, choice.y, i, claims + (uint64_t)it * slots);
+}
 __global__ void __launch_bounds__(RESOLVE_BLOCK) k_chain_propose(ChainArrays c, uint32_t n, int it) {
   if (chain_stalled(c, it)) return;  // uniform
-  __shared__ uint32_t s_tgt[RESOLVE_SLOTS];
-  __shared__ unsigned long long s_key[RESOLVE_SLOTS];
-  for (uint32_t t = threadIdx.x; t < RESOLVE_SLOTS; t += RESOLVE_BLOCK) {
-    s_tgt[t] = NONE;
-    s_key[t] = 0ull;
-  }
+  __shared__ ClaimTable s;
+  claims_clear(s);
   const uint32_t i = blockIdx.x * RESOLVE_BLOCK + threadIdx.x;
   uint32_t choice = NONE;
   const uint2 range = i < n ? c.range[i] : make_uint2(0u, 0u);
@@ -1816,7 +1979,7 @@ __global__ void __launch_bounds__(RESOLVE_BLOCK) k_chain_propose(ChainArrays c, 
   if (range.x < range.y && c.next[i] == NONE) {
     si = c.pk[i].z;
     const int bi = size_bucket(si);
-    const uint32_t lim = min(range.y, range.x + 256u);
+    const uint32_t lim = min(range.y, range.x + CHAIN_WINDOW);
     const uint32_t j0 = c.from[i];
     uint32_t first = lim;  // first entry that could be chosen (scan end when none)
     int64_t bw = 0;
@@ -1866,21 +2029,8 @@ __global__ void __launch_bounds__(RESOLVE_BLOCK) k_chain_propose(ChainArrays c, 
     }
     c.from[i] = first;
   }
-  __syncthreads();  // the table is cleared
-  if (choice != NONE && c.prev[choice] == NONE) {
-    const uint32_t d = si > choice_size ? si - choice_size : choice_size - si;
-    const unsigned long long key = ((unsigned long long)(0xFFFFFFFFu - d) << 32) | (0xFFFFFFFFu - i);
-    uint32_t h = slot_hash(choice) & (RESOLVE_SLOTS - 1);
-    for (;;) {
-      const uint32_t old = atomicCAS(&s_tgt[h], NONE, choice);
-      if (old == NONE || old == choice) break;
-      h = (h + 1) & (RESOLVE_SLOTS - 1);
-    }
-    atomicMax(&s_key[h], key);
-  }
-  __syncthreads();
-  for (uint32_t t = threadIdx.x; t < RESOLVE_SLOTS; t += RESOLVE_BLOCK)
-    if (s_tgt[t] != NONE) atomicMax(&c.claim[s_tgt[t]], s_key[t]);
+  const bool claims = choice != NONE && c.prev[choice] == NONE;
+  claims_add(s, claims ? choice : NONE, si > choice_size ? si - choice_size : choice_size - si, i, c.claim);
 }
 __global__ void k_chain_commit(ChainArrays c, uint32_t n, int it) {
   uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
@@ -2727,13 +2877,6 @@ __global__ void k_gather_u32(const uint32_t* __restrict__ src, const uint32_t* _
   if (i < m) out[i] = src[idx[i]];
 }
 
-__global__ void k_max_u32(const uint32_t* __restrict__ p, uint32_t n, uint32_t* out) {
-  uint32_t m = 0;
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) m = p[i] > m ? p[i] : m;
-  m = wave_max(m);
-  if (lane_id() == 0) atomicMax(out, m);
-}
-
 }  // namespace
 
 // ==========================================================================================
@@ -2763,6 +2906,8 @@ struct LevelLayout {
   DBuf<uint32_t> large, llist, glist;  // large: all above PP_SMALL pins (masks), or up to PP_WAVE (lists)
   DBuf<uint64_t> goff;
   uint64_t gslots = 0;
+  bool sized = false;
+  uint32_t max_size = 0;  // largest node size of the level
   uint32_t cas_sort_max = 0xFFFFFFFFu;
   DBuf<uint32_t> cas_list[3];
   uint32_t cas_n[3] = {0, 0, 0};
@@ -3044,26 +3189,41 @@ void rank_by_gain(Ctx& c, uint32_t n, const uint32_t* moves, const int64_t* gain
 }
 
 void rank_by_chaining(Ctx& c, uint32_t n, uint32_t k, const uint32_t* part, const uint32_t* moves, const int64_t* gains,
-                      const KeyStats& gst, const uint32_t* sizes, uint32_t* ranks) {
+                      const KeyStats& gst, const uint32_t* sizes, uint32_t max_size, uint32_t* ranks) {
   if (n == 0) return;
   const uint32_t g = ceil_div(n, 256);
   // sorted space: stable by (src partition asc, valid first, gain desc), ties by node id
   DBuf<uint32_t> orig(c, n);
   DBuf<uint64_t> poff(c, (uint64_t)k + 1);
   sort_moves(c, n, k, part, moves, gains, gst, orig, poff.get());
-  DBuf<uint32_t> next(c, n), prev(c, n), from(c, n), progress(c, 4);
-  DBuf<unsigned long long> claim(c, n);
+  // proposals by table: see k_chain_table
+  const uint64_t nsizes = (uint64_t)max_size + 1;
+  const bool table = k <= CHAIN_TABLE_K && nsizes <= CHAIN_TABLE_SIZES && nsizes * k <= std::max<uint64_t>(2ull * n, CHAIN_TABLE_MIN);
+  const uint32_t slots = table ? k * CHAIN_WINDOW : 0u;
+  DBuf<uint32_t> next(c, n), prev(c, n), from(c, table ? 0 : n), last(c, table ? n : 0), progress(c, 4);
+  DBuf<unsigned long long> claim(c, table ? 4ull * slots : n);
   DBuf<uint4> pk(c, n);
-  DBuf<uint2> range(c, n);
+  DBuf<uint2> range(c, table ? 0 : n), ds(c, table ? n : 0), tab(c, table ? nsizes * k : 0);
   DBuf<uint32_t> cflag(c, n), cinv(c, n), csize(c, n);
   DBuf<long long> cw(c, n);
   DBuf<KeyStats> cst(c, 1);
-  ChainArrays ca{orig.get(), pk.get(), range.get(), from.get(), next.get(), prev.get(), claim.get(), progress.get(),
-                 cw.get(), csize.get(), cinv.get(), cflag.get()};
+  ChainArrays ca{orig.get(), pk.get(), next.get(), prev.get(), ds.get(), last.get(), range.get(), from.get(),
+                 claim.get(), progress.get(), cw.get(), csize.get(), cinv.get(), cflag.get()};
   HGP_LAUNCH(k_chain_gather, g, 256, 0, c, ca, moves, gains, sizes, poff.get(), n, cst.get());
-  for (int it = 0; it < 4; ++it) {
-    HGP_LAUNCH(k_chain_propose, ceil_div(n, RESOLVE_BLOCK), RESOLVE_BLOCK, 0, c, ca, n, it);
-    HGP_LAUNCH(k_chain_commit, g, 256, 0, c, ca, n, it);
+  if (table) {
+    fill_u32(c, (uint32_t*)claim.get(), 0u, 8ull * slots);
+    for (int it = 0; it < 4; ++it) {
+      HGP_LAUNCH(k_chain_table, dim3(k, ceil_div(nsizes, CHAIN_WINDOW)), CHAIN_WINDOW, 0, c, ca, poff.get(),
+                 (uint32_t)nsizes, it, slots, claim.get(), tab.get());
+      HGP_LAUNCH(k_chain_lookup, ceil_div(n, RESOLVE_BLOCK), RESOLVE_BLOCK, 0, c, ca, n, (uint32_t)nsizes, it, slots,
+                 tab.get(), claim.get());
+    }
+    HGP_LAUNCH(k_chain_links, ceil_div(4ull * slots, 256), 256, 0, c, ca, poff.get(), slots, claim.get());
+  } else {
+    for (int it = 0; it < 4; ++it) {
+      HGP_LAUNCH(k_chain_propose, ceil_div(n, RESOLVE_BLOCK), RESOLVE_BLOCK, 0, c, ca, n, it);
+      HGP_LAUNCH(k_chain_commit, g, 256, 0, c, ca, n, it);
+    }
   }
   DBuf<uint32_t> comp(c, n), pos(c, n);
   HGP_LAUNCH(k_chain_comp, g, 256, 0, c, ca, n, comp.get(), pos.get(), cst.get());
@@ -3130,10 +3290,16 @@ void analyze_round(Ctx& c, const RefineLevel& L, int mode, uint32_t omega, uint3
   st.gains = DBuf<int64_t>(c, n);
   st.ranks = DBuf<uint32_t>(c, n);
   compute_gains(c, L, pl, mode, omega, rep, discount_of(rep, R), part, psizes, st.moves.get(), st.gains.get());
+  LevelLayout own_layout;
+  LevelLayout& Y = layout ? *layout : own_layout;
+  if (!Y.sized) {
+    Y.sized = true;
+    Y.max_size = n ? reduce_max_u32(c, L.sizes, n) : 0u;
+  }
   const KeyStats gst = gain_stats(c, n, st.moves.get(), st.gains.get());
   st.V = (uint32_t)gst.count;
   if (chainup) rank_by_gain(c, n, st.moves.get(), st.gains.get(), gst, st.ranks.get());
-  else rank_by_chaining(c, n, L.k, part, st.moves.get(), st.gains.get(), gst, L.sizes, st.ranks.get());
+  else rank_by_chaining(c, n, L.k, part, st.moves.get(), st.gains.get(), gst, L.sizes, Y.max_size, st.ranks.get());
   const uint32_t V = st.V;
   st.seq = DBuf<unsigned long long>(c, std::max<uint32_t>(V, 1));
   st.sv = DBuf<int32_t>(c, std::max<uint32_t>(V, 1));
@@ -3167,8 +3333,6 @@ void analyze_round(Ctx& c, const RefineLevel& L, int mode, uint32_t omega, uint3
     const int crb = std::max(1, bit_width(V));  // rank + 1 <= V
     const int cpb = std::max(1, bit_width(L.k));
     const uint32_t sort_max = cpb + crb + 11 < 64 ? CAS_SORT : 0u;
-    LevelLayout local;
-    LevelLayout& Y = layout ? *layout : local;
     if (Y.cas_sort_max != sort_max) {  // the level's cascade classes (its first round)
       Y.cas_sort_max = sort_max;
       DBuf<uint32_t> fl[4];
@@ -3452,13 +3616,10 @@ int64_t connectivity_fixed(Ctx& c, const uint32_t* hedges, const uint64_t* hoff,
   if (e == 0) return 0;
   // partitions in use: max id + 1 (needed to size the per-partition inbound counters)
   const uint64_t P = read_scalar(c, hoff + e);
-  DBuf<uint32_t> mx(c, 1);
-  memset_async(c, mx.get(), 0, 4);
   // max over the partition ids of the pins
   DBuf<uint32_t> pinpart(c, P);
   HGP_LAUNCH(k_gather_u32, ceil_div(P, 256), 256, 0, c, part, hedges, (uint32_t)P, pinpart.get());
-  HGP_LAUNCH(k_max_u32, std::min<uint32_t>(ceil_div(P, 256), 2048), 256, 0, c, pinpart.get(), (uint32_t)P, mx.get());
-  const uint32_t k = read_scalar(c, mx.get()) + 1;
+  const uint32_t k = reduce_max_u32(c, pinpart.get(), P) + 1;
   DBuf<uint32_t> srcc0(c, e);
   memset_async(c, srcc0.get(), 0, (uint64_t)e * 4);
   RefineLevel L{};
