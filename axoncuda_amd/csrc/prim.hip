@@ -6,6 +6,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "block_sort.hpp"
 #include "prim.hpp"
 
 namespace hgp {
@@ -286,115 +287,32 @@ void scan_impl(Ctx& c, const TI* in, TO* out, uint64_t n, bool exclusive) {
 // sort sharing its bits evenly)
 constexpr int RS_BLOCK = 256;
 
-// Ranking.  A wave owns consecutive keys, 64 per round; lanes with equal digits find each other
-// with one ballot per digit bit, the lowest of them adds the group to the wave's own counter of
-// that digit, and a key's rank is the counter before its group plus its place in it.  The
-// counters belong to the wave (LDS operations of a wave are in order), so rounds need no barrier.
-// Returns the rank among the wave's keys of the same digit so far.
-__device__ __forceinline__ uint32_t wave_digit_rank(bool valid, uint32_t d, int nb, uint32_t* cnt) {
-  uint64_t peers = __ballot(valid);
-#pragma unroll
-  for (int b = 0; b < 8; ++b) {
-    if (b < nb) {  // uniform
-      const bool bit = (d >> b) & 1u;
-      const uint64_t bb = __ballot(bit);
-      peers &= bit ? bb : ~bb;
-    }
-  }
-  const uint32_t below = lanes_below(peers);
-  uint32_t before = 0;
-  if (valid) before = cnt[d];
-  __builtin_amdgcn_wave_barrier();
-  if (valid && below == 0) cnt[d] = before + (uint32_t)__popcll(peers);
-  __builtin_amdgcn_wave_barrier();
-  return before + below;
-}
-
 // Whole sort of at most 1024 * IT keys by one workgroup: keys and values stay in registers, every
 // pass ranks them and exchanges them through LDS, and memory is read and written once.  The
 // exchange through global memory this replaces cost 64 cycles per scattered 64-lane store: two
 // passes over 8,191 64-bit keys with values took 37 us and take 20 us this way, 4,096 keys 25 and
 // 13 us, 64 keys 14 and 7.5 us.  Past 8,192 keys one CU's ranking is the bound (16,384 keys: 38 us)
 // and the tiles below are faster (16,385 keys: 18 us).
-constexpr uint32_t RS1_BLOCK = 1024;
+constexpr uint32_t RS1_BLOCK = BLOCK_SORT_THREADS;
 constexpr uint32_t RS1_MAX_IT = 8;
 constexpr uint64_t RS1_MAX_N = (uint64_t)RS1_BLOCK * RS1_MAX_IT;
 
 template <typename K, bool HAS_VALS, uint32_t IT>
 __global__ void __launch_bounds__(RS1_BLOCK) k_rs_block(K* keys, uint32_t* vals, uint32_t n, int lo, int bits, int nb,
                                                         K kmin) {
-  constexpr uint32_t W = RS1_BLOCK / 64;
-  __shared__ K s_key[RS1_BLOCK * IT];
-  __shared__ uint32_t s_cnt[W][256];
-  __shared__ uint32_t s_w[W];
-  const uint32_t t = threadIdx.x, w = t / 64, l = lane_id();
-  const uint32_t first = w * 64 * IT + l;  // this lane's keys: first + 64 * r
+  __shared__ BlockSortMem<K, IT> s;
   K key[IT];
   uint32_t val[IT];
 #pragma unroll
   for (uint32_t r = 0; r < IT; ++r) {
-    const uint32_t i = first + 64 * r;
+    const uint32_t i = block_pos<IT>(r);
     key[r] = i < n ? keys[i] : (K)0;
     val[r] = HAS_VALS && i < n ? vals[i] : 0u;
   }
-  for (int shift = lo; shift < bits; shift += nb) {
-    const int nbp = min(nb, bits - shift);
-    const uint32_t mask = (1u << nbp) - 1u;
-#pragma unroll
-    for (uint32_t q = 0; q < 4; ++q) (&s_cnt[0][0])[q * RS1_BLOCK + t] = 0;
-    __syncthreads();
-    uint32_t pos[IT];
-#pragma unroll
-    for (uint32_t r = 0; r < IT; ++r) {
-      const uint32_t d = (uint32_t)((key[r] - kmin) >> shift) & mask;
-      pos[r] = wave_digit_rank(first + 64 * r < n, d, nbp, s_cnt[w]);
-    }
-    __syncthreads();
-    // exclusive sums in (digit, wave) order: thread t takes four waves of digit t / 4
-    uint32_t c[4], sum = 0;
-#pragma unroll
-    for (uint32_t q = 0; q < 4; ++q) {
-      c[q] = s_cnt[(t & 3) * 4 + q][t >> 2];
-      sum += c[q];
-    }
-    const uint32_t inc = wave_scan_incl(sum);
-    if (l == 63) s_w[w] = inc;
-    __syncthreads();
-    uint32_t run = inc - sum;
-#pragma unroll
-    for (uint32_t q = 0; q < W; ++q) run += q < w ? s_w[q] : 0u;
-#pragma unroll
-    for (uint32_t q = 0; q < 4; ++q) {
-      s_cnt[(t & 3) * 4 + q][t >> 2] = run;
-      run += c[q];
-    }
-    __syncthreads();
-#pragma unroll
-    for (uint32_t r = 0; r < IT; ++r) {
-      const uint32_t d = (uint32_t)((key[r] - kmin) >> shift) & mask;
-      pos[r] += s_cnt[w][d];
-      if (first + 64 * r < n) s_key[pos[r]] = key[r];
-    }
-    __syncthreads();
-#pragma unroll
-    for (uint32_t r = 0; r < IT; ++r)
-      if (first + 64 * r < n) key[r] = s_key[first + 64 * r];
-    if (HAS_VALS) {  // the values take the keys' place in LDS
-      uint32_t* s_val = reinterpret_cast<uint32_t*>(s_key);
-      __syncthreads();
-#pragma unroll
-      for (uint32_t r = 0; r < IT; ++r)
-        if (first + 64 * r < n) s_val[pos[r]] = val[r];
-      __syncthreads();
-#pragma unroll
-      for (uint32_t r = 0; r < IT; ++r)
-        if (first + 64 * r < n) val[r] = s_val[first + 64 * r];
-    }
-    __syncthreads();
-  }
+  block_sort<K, HAS_VALS, IT>(key, val, n, lo, bits, nb, kmin, s);
 #pragma unroll
   for (uint32_t r = 0; r < IT; ++r) {
-    const uint32_t i = first + 64 * r;
+    const uint32_t i = block_pos<IT>(r);
     if (i < n) {
       keys[i] = key[r];
       if (HAS_VALS) vals[i] = val[r];

@@ -19,6 +19,7 @@
 #include <optional>
 #include <type_traits>
 
+#include "block_sort.hpp"
 #include "prim.hpp"
 #include "stages.hpp"
 #include "wave_iter.hpp"
@@ -2131,6 +2132,291 @@ __global__ void k_edge_ranks(const uint32_t* __restrict__ sorted_j, const uint32
   if (r < n) ranks[orig[sorted_j[r]]] = r;
 }
 
+// ---- 3b. ranking of small levels by one workgroup ---------------------------------------------
+// On levels of up to SMALL_N nodes the ranking is some thirty launches of a few microseconds each
+// and two read-backs; one workgroup holds all moves in registers and LDS.  k_rank_front orders the
+// moves (and, ranking by gain, is done), k_rank_back follows the links to the ranks; the proposals
+// between them keep their launches (a table per partition and size needs more than one workgroup).
+// A level of 5,000 nodes: about 150 us in the launches above, 65 us this way.
+// Keys carry the position in their low SMALL_BITS bits, so the sorts move one word per entry.
+constexpr uint32_t SMALL_BITS = 13;
+constexpr uint32_t SMALL_N = 1u << SMALL_BITS;
+struct RankInfo {
+  uint32_t V;     // valid moves
+  uint32_t wide;  // a key did not fit 64 bits: the ranks are not those asked for
+};
+struct RankArgs {
+  const uint32_t* part;
+  const uint32_t* moves;
+  const int64_t* gains;
+  const uint32_t* sizes;
+  uint32_t n, k;
+  int by_gain;
+  uint32_t* ranks;
+  // node records of the cascade (see CascadeArgs)
+  uint4* pm;
+  uint2* pm2;
+  // counters by rank, cleared here
+  unsigned long long* seq;
+  unsigned long long* dio;
+  int32_t* sv;
+  int32_t* iv;
+  RankInfo* info;
+  uint64_t* poff;
+};
+// rank r of node v, and its record for the cascade
+__device__ __forceinline__ void put_rank(const RankArgs& a, uint32_t v, uint32_t r) {
+  a.ranks[v] = r;
+  const uint32_t q = a.moves[v];
+  if (a.pm2) a.pm2[v] = make_uint2(a.part[v] | ((q == NONE ? 0xFFFFu : q) << 16), r);
+  else a.pm[v] = make_uint4(a.part[v], q, r, 0u);
+}
+struct SmallStats {
+  uint64_t mn[BLOCK_SORT_WAVES], mx[BLOCK_SORT_WAVES], bits[BLOCK_SORT_WAVES];
+  uint32_t count[BLOCK_SORT_WAVES];
+};
+// KeyStats over the workgroup's threads (every thread calls it and gets the result)
+__device__ __forceinline__ KeyStats block_stats(uint64_t mn, uint64_t mx, uint64_t bits, uint32_t count, SmallStats& s) {
+  mn = wave_min(mn);
+  mx = wave_max(mx);
+  bits = wave_reduce(bits, [](uint64_t a, uint64_t b) { return a | b; });
+  count = wave_sum(count);
+  if (lane_id() == 0) {
+    const uint32_t w = threadIdx.x / 64;
+    s.mn[w] = mn;
+    s.mx[w] = mx;
+    s.bits[w] = bits;
+    s.count[w] = count;
+  }
+  __syncthreads();
+  KeyStats r{~0ull, 0ull, 0ull, 0ull, 0ull};
+  for (uint32_t w = 0; w < BLOCK_SORT_WAVES; ++w) {
+    r.mn = s.mn[w] < r.mn ? s.mn[w] : r.mn;
+    r.mx = s.mx[w] > r.mx ? s.mx[w] : r.mx;
+    r.bits |= s.bits[w];
+    r.count += s.count[w];
+  }
+  __syncthreads();
+  return r;
+}
+__device__ __forceinline__ int dev_bit_width(uint64_t x) { return x ? 64 - __clzll((long long)x) : 0; }
+
+template <uint32_t IT>
+__global__ void __launch_bounds__(BLOCK_SORT_THREADS) k_rank_front(RankArgs a, ChainArrays c) {
+  __shared__ BlockSortMem<uint64_t, IT> s;
+  __shared__ SmallStats st;
+  const uint32_t n = a.n;
+  uint32_t mv[IT], val[IT];
+  uint64_t key[IT];
+  uint64_t mn = ~0ull, mx = 0, bits = 0;
+  uint32_t count = 0;
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) {
+    const uint32_t v = block_pos<IT>(r);
+    mv[r] = v < n ? a.moves[v] : NONE;
+    key[r] = v < n ? (uint64_t)a.gains[v] : 0ull;
+    if (v < n) {  // counters by rank
+      a.seq[v] = 0ull;
+      if (a.dio) a.dio[v] = 0ull;
+      a.sv[v] = 0;
+      a.iv[v] = 0;
+    }
+    if (mv[r] != NONE) {
+      const uint64_t o = ordered_i64((int64_t)key[r]);
+      mn = o < mn ? o : mn;
+      mx = o > mx ? o : mx;
+      bits |= key[r];
+      ++count;
+    }
+  }
+  const KeyStats ks = block_stats(mn, mx, bits, count, st);
+  const int pb = a.by_gain ? 1 : dev_bit_width(2ull * a.k - 1);
+  int tz = 0, gb = 0;
+  if (ks.count && ks.mx != ks.mn) {
+    tz = ks.bits ? __ffsll((unsigned long long)ks.bits) - 1 : 0;
+    gb = dev_bit_width((ks.mx - ks.mn) >> tz);
+  }
+  const bool wide = gb + pb + (int)SMALL_BITS > 64;  // then every move counts as invalid
+  if (wide) gb = 0;
+  if (threadIdx.x == 0) *a.info = RankInfo{wide ? 0u : (uint32_t)ks.count, wide ? 1u : 0u};
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) {
+    const uint32_t v = block_pos<IT>(r);
+    const bool invalid = wide || mv[r] == NONE;
+    const uint64_t code = invalid || gb == 0 ? 0ull : (ks.mx - ordered_i64((int64_t)key[r])) >> tz;
+    const uint64_t hi = (a.by_gain || v >= n ? 0ull : (uint64_t)a.part[v] << 1) | (invalid ? 1ull : 0ull);
+    key[r] = (((hi << gb) | code) << SMALL_BITS) | v;
+    val[r] = 0;
+  }
+  block_sort<uint64_t, false, IT>(key, val, n, SMALL_BITS, SMALL_BITS + gb + pb, digit_bits(gb + pb), 0ull, s);
+  if (a.by_gain) {
+#pragma unroll
+    for (uint32_t r = 0; r < IT; ++r) {
+      const uint32_t j = block_pos<IT>(r);
+      if (j < n) put_rank(a, (uint32_t)(key[r] & (SMALL_N - 1)), j);
+    }
+    return;
+  }
+  // entries and partition offsets of the sorted order
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) {
+    const uint32_t j = block_pos<IT>(r);
+    if (j >= n) continue;
+    const uint32_t v = (uint32_t)(key[r] & (SMALL_N - 1));
+    const int64_t p = (int64_t)(key[r] >> (SMALL_BITS + gb + 1));
+    const int64_t before = j ? (int64_t)(s.key[j - 1] >> (SMALL_BITS + gb + 1)) : -1;
+    for (int64_t x = before + 1; x <= p; ++x) a.poff[x] = j;
+    if (j == n - 1)
+      for (int64_t x = p + 1; x <= (int64_t)a.k; ++x) a.poff[x] = n;
+    const uint32_t q = wide ? NONE : a.moves[v];
+    const int64_t g = a.gains[v];
+    const uint32_t size = a.sizes[v];
+    const_cast<uint32_t*>(c.orig)[j] = v;
+    c.pk[j] = make_uint4((uint32_t)(uint64_t)g, (uint32_t)((uint64_t)g >> 32), size, q != NONE ? 1u : 0u);
+    c.ds[j] = make_uint2(q, size);
+    c.last[j] = NONE;
+    c.next[j] = NONE;
+    c.prev[j] = NONE;
+  }
+}
+
+// Components of the links, their order and every entry's rank: k_chain_comp .. k_edge_ranks.
+template <uint32_t IT>
+__global__ void __launch_bounds__(BLOCK_SORT_THREADS) k_rank_back(RankArgs a, ChainArrays c) {
+  __shared__ BlockSortMem<uint64_t, IT> s;
+  __shared__ uint32_t s_size[BLOCK_SORT_THREADS * IT];  // per component head: entries (top bit: invalid)
+  __shared__ uint16_t s_prev[BLOCK_SORT_THREADS * IT];
+  __shared__ SmallStats st;
+  __shared__ uint32_t s_odd;
+  constexpr uint32_t INVALID = 0x80000000u, NOPREV = 0xFFFFu;
+  unsigned long long* s_cw = reinterpret_cast<unsigned long long*>(s.key);  // summed gains, until the sort
+  const uint32_t n = a.n;
+  uint32_t comp[IT], dist[IT], val[IT];
+  uint64_t key[IT];
+  if (threadIdx.x == 0) s_odd = 0;
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) {
+    const uint32_t j = block_pos<IT>(r);
+    const uint32_t p = j < n ? c.prev[j] : NONE;
+    s_prev[j] = (uint16_t)(p == NONE ? NOPREV : p);  // p < 2^13
+    s_size[j] = 0;
+    s_cw[j] = 0;
+  }
+  __syncthreads();
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) {
+    const uint32_t j = block_pos<IT>(r);
+    comp[r] = dist[r] = 0;
+    if (j >= n) continue;
+    uint32_t cur = j, mn = j, cc = NONE, ps = 0;
+    for (uint32_t d = 0; d < 256; ++d) {  // as k_chain_comp
+      const uint32_t p = s_prev[cur];
+      if (p == NOPREV) {
+        cc = cur;
+        ps = d;
+        break;
+      }
+      cur = p;
+      mn = cur < mn ? cur : mn;
+    }
+    if (cc == NONE) {
+      cc = mn;
+      ps = 0;
+      s_odd = 1;
+    }
+    comp[r] = cc;
+    dist[r] = ps;
+    const uint4 e = c.pk[j];
+    atomicAdd(&s_size[cc], 1u);
+    if (e.w) atomicAdd(&s_cw[cc], (unsigned long long)(((uint64_t)e.y << 32) | e.x));
+    else atomicOr(&s_size[cc], INVALID);
+  }
+  __syncthreads();
+  // keys of the components (heads): class << cb | code of the summed gain, class 0 valid, 1 invalid,
+  // 2 not a head
+  uint64_t mn = ~0ull, mx = 0, bits = 0;
+  uint32_t count = 0;
+  bool head[IT], inv[IT];
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) {
+    const uint32_t j = block_pos<IT>(r);
+    head[r] = j < n && s_size[j] != 0;
+    inv[r] = head[r] && (s_size[j] & INVALID);
+    key[r] = s_cw[j];
+    if (head[r] && !inv[r]) {
+      const uint64_t o = ordered_i64((int64_t)key[r]);
+      mn = o < mn ? o : mn;
+      mx = o > mx ? o : mx;
+      bits |= key[r];
+      ++count;
+    }
+  }
+  const KeyStats ks = block_stats(mn, mx, bits, count, st);  // (its barriers also end the reads of s_cw)
+  int tz = 0, cb = 0;
+  if (ks.count && ks.mx != ks.mn) {
+    tz = ks.bits ? __ffsll((unsigned long long)ks.bits) - 1 : 0;
+    cb = dev_bit_width((ks.mx - ks.mn) >> tz);
+  }
+  const bool wide = cb + 2 + (int)SMALL_BITS > 64;
+  if (wide) {
+    cb = 0;
+    if (threadIdx.x == 0) a.info->wide = 1u;
+  }
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) {
+    const uint32_t j = block_pos<IT>(r);
+    const uint64_t cls = !head[r] ? 2ull : inv[r] ? 1ull : 0ull;
+    const uint64_t code = cls || cb == 0 ? 0ull : (ks.mx - ordered_i64((int64_t)key[r])) >> tz;
+    key[r] = (((cls << cb) | code) << SMALL_BITS) | j;
+    val[r] = 0;
+  }
+  block_sort<uint64_t, false, IT>(key, val, n, SMALL_BITS, SMALL_BITS + cb + 2, digit_bits(cb + 2), 0ull, s);
+  // starts of the components in their order, and their ranks
+  uint32_t start[IT];
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) {
+    const uint32_t j = block_pos<IT>(r);
+    start[r] = j < n ? s_size[key[r] & (SMALL_N - 1)] & ~INVALID : 0u;
+  }
+  uint32_t own[IT];
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) own[r] = start[r];
+  block_scan(start, s.w);
+  uint32_t* s_start = reinterpret_cast<uint32_t*>(s.key);      // by head
+  uint32_t* s_crank = s_start + BLOCK_SORT_THREADS * IT;       // by head
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) {
+    const uint32_t j = block_pos<IT>(r);
+    if (j < n) {
+      const uint32_t h = (uint32_t)(key[r] & (SMALL_N - 1));
+      s_start[h] = start[r] - own[r];
+      s_crank[h] = j;
+    }
+  }
+  __syncthreads();
+  if (!s_odd) {
+#pragma unroll
+    for (uint32_t r = 0; r < IT; ++r) {
+      const uint32_t j = block_pos<IT>(r);
+      if (j < n) put_rank(a, c.orig[j], s_start[comp[r]] + dist[r]);
+    }
+    return;
+  }
+  // (component rank, distance), ties in entry order
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) {
+    const uint32_t j = block_pos<IT>(r);
+    key[r] = j < n ? (((uint64_t)s_crank[comp[r]] << 8 | dist[r]) << SMALL_BITS) | j : 0ull;
+  }
+  __syncthreads();
+  block_sort<uint64_t, false, IT>(key, val, n, SMALL_BITS, 2 * SMALL_BITS + 8, digit_bits(SMALL_BITS + 8), 0ull, s);
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) {
+    const uint32_t j = block_pos<IT>(r);
+    if (j < n) put_rank(a, c.orig[(uint32_t)(key[r] & (SMALL_N - 1))], j);
+  }
+}
+
 // ---- 4. cascade (hedge-centric) ------------------------------------------------------------
 struct CascadeArgs {
   const uint32_t* hedges;
@@ -2777,8 +3063,7 @@ __device__ __forceinline__ bool better(const Best& a, const Best& b) {  // a str
   if (a.seq != b.seq) return a.seq > b.seq;
   return a.r < b.r;
 }
-__device__ Best block_best(Best x) {
-  __shared__ Best sb[4];
+__device__ __forceinline__ Best wave_best_prefix(Best x) {
   for (int o = 32; o > 0; o >>= 1) {
     Best y;
     y.ok = __shfl_xor(x.ok, o, 64);
@@ -2788,6 +3073,11 @@ __device__ Best block_best(Best x) {
     y.iv = __shfl_xor(x.iv, o, 64);
     if (better(y, x)) x = y;
   }
+  return x;
+}
+__device__ Best block_best(Best x) {
+  __shared__ Best sb[4];
+  x = wave_best_prefix(x);
   if (lane_id() == 0) sb[threadIdx.x / 64] = x;
   __syncthreads();
   Best b = sb[0];
@@ -2827,6 +3117,167 @@ __global__ void __launch_bounds__(256) k_best_final(const Best* __restrict__ par
   Best b = block_best(x);
   if (threadIdx.x == 0) *out = b;
 }
+// A round's events and best prefix on levels of up to SMALL_EVENT_N nodes, by one workgroup after the
+// cascade: the size (and inbound) events sorted by (partition, rank), their running sums per
+// partition, the violations summed per rank, the prefix sums over the ranks and the best of them,
+// in place of fifteen launches and a read-back of V.
+constexpr uint32_t SMALL_EVENT_N = SMALL_N / 2;
+struct RoundOut {
+  Best best;
+  RankInfo info;
+};
+struct EventArgs {
+  const uint32_t* part;
+  const uint32_t* moves;
+  const uint32_t* ranks;
+  const uint32_t* sizes;
+  const uint32_t* psizes;
+  const uint32_t* isz;  // inbound sizes (INCC)
+  const unsigned long long* dio;
+  const RankInfo* info;
+  uint32_t n, omega, delta;
+  int rb, kb;
+  int64_t* seq;  // in: per rank; out: prefix sums
+  int32_t* sv;
+  int32_t* iv;
+  RoundOut* out;
+};
+template <uint32_t IT, bool INCC>
+__global__ void __launch_bounds__(BLOCK_SORT_THREADS) k_round_small(EventArgs a) {
+  constexpr uint32_t CAP = BLOCK_SORT_THREADS * IT;  // events; ranks: half
+  __shared__ BlockSortMem<uint64_t, IT> s;
+  __shared__ int32_t s_sv[CAP / 2], s_iv[CAP / 2];
+  __shared__ uint16_t s_node[CAP / 2];
+  __shared__ int64_t s_w64[BLOCK_SORT_WAVES];
+  __shared__ Best s_best[BLOCK_SORT_WAVES];
+  const RankInfo info = *a.info;
+  const uint32_t V = info.V, m = 2 * V;
+  const int rb = a.rb;
+  Best best;
+  best.ok = 0;
+  best.sv = 0;
+  best.seq = 0;
+  best.r = NONE;
+  best.iv = 0;
+  if (V == 0) {  // uniform
+    if (threadIdx.x == 0) *a.out = RoundOut{best, info};
+    return;
+  }
+  for (uint32_t r = threadIdx.x; r < V; r += BLOCK_SORT_THREADS) s_sv[r] = s_iv[r] = 0;
+  for (uint32_t v = threadIdx.x; v < a.n; v += BLOCK_SORT_THREADS) {
+    const uint32_t q = a.moves[v];
+    if (q == NONE) continue;
+    const uint32_t r = a.ranks[v];
+    s_node[r] = (uint16_t)v;
+    s.key[2 * r] = ((uint64_t)a.part[v] << (rb + 1)) | ((uint64_t)r << 1);
+    s.key[2 * r + 1] = ((uint64_t)q << (rb + 1)) | ((uint64_t)r << 1) | 1u;
+  }
+  __syncthreads();
+  uint64_t key[IT];
+  uint32_t val[IT];
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) {
+    const uint32_t i = block_pos<IT>(r);
+    key[r] = i < m ? s.key[i] : 0ull;
+    val[r] = 0;
+  }
+  __syncthreads();
+  block_sort<uint64_t, false, IT>(key, val, m, rb + 1, rb + 1 + a.kb, digit_bits(a.kb), 0ull, s);
+  bool flag[IT];
+  uint32_t head[IT];
+  int64_t d[IT], cum[IT];
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) {
+    const uint32_t i = block_pos<IT>(r);
+    flag[r] = i < m && (i == 0 || (s.key[i - 1] >> (rb + 1)) != (key[r] >> (rb + 1)));
+    const uint32_t sz = i < m ? a.sizes[s_node[event_rank(key[r], rb)]] : 0u;
+    d[r] = (int64_t)((key[r] & 1u) ? (int32_t)sz : -(int32_t)sz);
+    cum[r] = d[r];
+  }
+  block_last_head<IT>(flag, head, s.w);  // (its barriers also end the reads of s.key)
+  int64_t* s_base = reinterpret_cast<int64_t*>(s.key);  // at a partition's first event: the sum before it
+  block_scan(cum, s_w64);
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r)
+    if (flag[r]) s_base[block_pos<IT>(r)] = cum[r] - d[r];
+  __syncthreads();
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) {
+    if (block_pos<IT>(r) >= m) continue;
+    const uint32_t q = (uint32_t)(key[r] >> (rb + 1)), rk = event_rank(key[r], rb);
+    const int64_t cur = (int64_t)a.psizes[q] + cum[r] - s_base[head[r]], prev = cur - d[r], om = (int64_t)a.omega;
+    const int64_t ex = (cur > om ? cur - om : 0) - (prev > om ? prev - om : 0);
+    if ((int32_t)ex) atomicAdd(&s_sv[rk], (int32_t)ex);
+  }
+  if constexpr (INCC) {
+    // counts of changing events above the summed changes, as k_inbound_deltas
+    constexpr int DB = 48;  // 2^14 events; changes below 2^47 hedges
+    int64_t pk[IT];
+#pragma unroll
+    for (uint32_t r = 0; r < IT; ++r) {
+      const uint32_t i = block_pos<IT>(r);
+      const unsigned long long x = i < m ? a.dio[event_rank(key[r], rb)] : 0ull;
+      d[r] = (key[r] & 1u) ? (int64_t)(x >> 32) : -(int64_t)(x & 0xFFFFFFFFull);
+      pk[r] = i < m ? d[r] + (d[r] != 0 ? (int64_t)1 << DB : 0) : 0;
+      cum[r] = pk[r];
+    }
+    __syncthreads();  // the sums before the partitions have been read
+    block_scan(cum, s_w64);
+#pragma unroll
+    for (uint32_t r = 0; r < IT; ++r)
+      if (flag[r]) s_base[block_pos<IT>(r)] = cum[r] - pk[r];
+    __syncthreads();
+#pragma unroll
+    for (uint32_t r = 0; r < IT; ++r) {
+      if (block_pos<IT>(r) >= m || d[r] == 0) continue;
+      const uint32_t q = (uint32_t)(key[r] >> (rb + 1)), rk = event_rank(key[r], rb);
+      const int64_t x = cum[r] - s_base[head[r]];
+      const int64_t change = (int64_t)((uint64_t)x << (64 - DB)) >> (64 - DB);
+      const bool first = ((x - change) >> DB) == 1;
+      const int64_t cur = (int64_t)a.isz[q] + change, prev = cur - d[r];
+      const bool was_valid = first || prev <= (int64_t)a.delta, is_valid = cur <= (int64_t)a.delta;
+      if (was_valid && !is_valid) atomicAdd(&s_iv[rk], 1);
+      if (!was_valid && is_valid) atomicSub(&s_iv[rk], 1);
+    }
+  }
+  __syncthreads();
+  // prefix sums over the ranks and the best prefix
+  int64_t seq[IT], sv[IT], iv[IT];
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) {
+    const uint32_t i = block_pos<IT>(r);
+    seq[r] = i < V ? a.seq[i] : 0;
+    sv[r] = i < V ? s_sv[i] : 0;
+    iv[r] = i < V ? s_iv[i] : 0;
+  }
+  block_scan(seq, s_w64);
+  block_scan(sv, s_w64);
+  block_scan(iv, s_w64);
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) {
+    const uint32_t i = block_pos<IT>(r);
+    if (i >= V) continue;
+    a.seq[i] = seq[r];
+    a.sv[i] = (int32_t)sv[r];
+    a.iv[i] = (int32_t)iv[r];
+    Best y;
+    y.r = i;
+    y.ok = (int32_t)iv[r] == 0;
+    y.sv = (int32_t)sv[r];
+    y.seq = seq[r];
+    y.iv = (int32_t)iv[r];
+    if (better(y, best)) best = y;
+  }
+  best = wave_best_prefix(best);
+  if (lane_id() == 0) s_best[threadIdx.x / 64] = best;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (uint32_t w = 1; w < BLOCK_SORT_WAVES; ++w)
+      if (better(s_best[w], best)) best = s_best[w];
+    *a.out = RoundOut{best, info};
+  }
+}
+
 // Moves of rank <= best.  With k <= APPLY_LDS_K the size changes are summed per partition in
 // LDS and added once per workgroup (with few partitions, one atomic per moved node would
 // queue every node of the grid on the same few addresses).
@@ -3188,6 +3639,68 @@ void rank_by_gain(Ctx& c, uint32_t n, const uint32_t* moves, const int64_t* gain
   HGP_LAUNCH(k_scatter_ranks, ceil_div(n, 256), 256, 0, c, vals.get(), n, ranks);
 }
 
+// Whether chaining looks its proposals up in a table (see k_chain_table) or scans the lists.
+bool chain_by_table(uint32_t n, uint32_t k, uint32_t max_size) {
+  const uint64_t nsizes = (uint64_t)max_size + 1;
+  return k <= CHAIN_TABLE_K && nsizes <= CHAIN_TABLE_SIZES &&
+         nsizes * k <= std::max<uint64_t>(2ull * n, CHAIN_TABLE_MIN);
+}
+// The four iterations of proposals and claims by table, and their links.  claim: 4 x k x
+// CHAIN_WINDOW words, tab: k x (max_size + 1).
+void propose_by_table(Ctx& c, const ChainArrays& ca, const uint64_t* poff, uint32_t n, uint32_t k, uint32_t max_size,
+                      unsigned long long* claim, uint2* tab) {
+  const uint32_t nsizes = max_size + 1, slots = k * CHAIN_WINDOW;
+  fill_u32(c, (uint32_t*)claim, 0u, 8ull * slots);
+  for (int it = 0; it < 4; ++it) {
+    HGP_LAUNCH(k_chain_table, dim3(k, ceil_div(nsizes, CHAIN_WINDOW)), CHAIN_WINDOW, 0, c, ca, poff, nsizes, it, slots,
+               claim, tab);
+    HGP_LAUNCH(k_chain_lookup, ceil_div(n, RESOLVE_BLOCK), RESOLVE_BLOCK, 0, c, ca, n, nsizes, it, slots, tab, claim);
+  }
+  HGP_LAUNCH(k_chain_links, ceil_div(4ull * slots, 256), 256, 0, c, ca, poff, slots, claim);
+}
+
+// f(items): the smallest items per thread (a compile-time constant) whose workgroup holds m.
+template <typename F>
+void with_items(uint32_t m, F&& f) {
+  if (m <= 1 * BLOCK_SORT_THREADS) f(std::integral_constant<uint32_t, 1>{});
+  else if (m <= 2 * BLOCK_SORT_THREADS) f(std::integral_constant<uint32_t, 2>{});
+  else if (m <= 4 * BLOCK_SORT_THREADS) f(std::integral_constant<uint32_t, 4>{});
+  else f(std::integral_constant<uint32_t, 8>{});
+}
+static_assert(SMALL_N == 8 * BLOCK_SORT_THREADS, "the largest instance holds a small level");
+
+// Ranks of a small level (see k_rank_front): by gain, or by chaining with proposals by table.
+void rank_small(Ctx& c, const RankArgs& a0, uint32_t max_size) {
+  RankArgs a = a0;
+  const uint32_t n = a.n, k = a.k;
+  if (a.by_gain) {
+    with_items(n, [&](auto it) {
+      HGP_LAUNCH((k_rank_front<decltype(it)::value>), 1, BLOCK_SORT_THREADS, 0, c, a, ChainArrays{});
+    });
+    return;
+  }
+  DBuf<uint32_t> orig(c, n), next(c, n), prev(c, n), last(c, n);
+  DBuf<uint4> pk(c, n);
+  DBuf<uint2> ds(c, n), tab(c, ((uint64_t)max_size + 1) * k);
+  DBuf<uint64_t> poff(c, (uint64_t)k + 1);
+  DBuf<unsigned long long> claim(c, 4ull * k * CHAIN_WINDOW);
+  a.poff = poff.get();
+  ChainArrays ca{};
+  ca.orig = orig.get();
+  ca.pk = pk.get();
+  ca.next = next.get();
+  ca.prev = prev.get();
+  ca.ds = ds.get();
+  ca.last = last.get();
+  with_items(n, [&](auto it) {
+    HGP_LAUNCH((k_rank_front<decltype(it)::value>), 1, BLOCK_SORT_THREADS, 0, c, a, ca);
+  });
+  propose_by_table(c, ca, poff.get(), n, k, max_size, claim.get(), tab.get());
+  with_items(n, [&](auto it) {
+    HGP_LAUNCH((k_rank_back<decltype(it)::value>), 1, BLOCK_SORT_THREADS, 0, c, a, ca);
+  });
+}
+
 void rank_by_chaining(Ctx& c, uint32_t n, uint32_t k, const uint32_t* part, const uint32_t* moves, const int64_t* gains,
                       const KeyStats& gst, const uint32_t* sizes, uint32_t max_size, uint32_t* ranks) {
   if (n == 0) return;
@@ -3198,7 +3711,7 @@ void rank_by_chaining(Ctx& c, uint32_t n, uint32_t k, const uint32_t* part, cons
   sort_moves(c, n, k, part, moves, gains, gst, orig, poff.get());
   // proposals by table: see k_chain_table
   const uint64_t nsizes = (uint64_t)max_size + 1;
-  const bool table = k <= CHAIN_TABLE_K && nsizes <= CHAIN_TABLE_SIZES && nsizes * k <= std::max<uint64_t>(2ull * n, CHAIN_TABLE_MIN);
+  const bool table = chain_by_table(n, k, max_size);
   const uint32_t slots = table ? k * CHAIN_WINDOW : 0u;
   DBuf<uint32_t> next(c, n), prev(c, n), from(c, table ? 0 : n), last(c, table ? n : 0), progress(c, 4);
   DBuf<unsigned long long> claim(c, table ? 4ull * slots : n);
@@ -3211,14 +3724,7 @@ void rank_by_chaining(Ctx& c, uint32_t n, uint32_t k, const uint32_t* part, cons
                  claim.get(), progress.get(), cw.get(), csize.get(), cinv.get(), cflag.get()};
   HGP_LAUNCH(k_chain_gather, g, 256, 0, c, ca, moves, gains, sizes, poff.get(), n, cst.get());
   if (table) {
-    fill_u32(c, (uint32_t*)claim.get(), 0u, 8ull * slots);
-    for (int it = 0; it < 4; ++it) {
-      HGP_LAUNCH(k_chain_table, dim3(k, ceil_div(nsizes, CHAIN_WINDOW)), CHAIN_WINDOW, 0, c, ca, poff.get(),
-                 (uint32_t)nsizes, it, slots, claim.get(), tab.get());
-      HGP_LAUNCH(k_chain_lookup, ceil_div(n, RESOLVE_BLOCK), RESOLVE_BLOCK, 0, c, ca, n, (uint32_t)nsizes, it, slots,
-                 tab.get(), claim.get());
-    }
-    HGP_LAUNCH(k_chain_links, ceil_div(4ull * slots, 256), 256, 0, c, ca, poff.get(), slots, claim.get());
+    propose_by_table(c, ca, poff.get(), n, k, max_size, claim.get(), tab.get());
   } else {
     for (int it = 0; it < 4; ++it) {
       HGP_LAUNCH(k_chain_propose, ceil_div(n, RESOLVE_BLOCK), RESOLVE_BLOCK, 0, c, ca, n, it);
@@ -3278,9 +3784,11 @@ struct RoundState {
   Best best;
 };
 
-void analyze_round(Ctx& c, const RefineLevel& L, int mode, uint32_t omega, uint32_t delta, uint32_t R, uint32_t rep,
-                   bool chainup, const uint32_t* part, const uint32_t* psizes, RoundState& st,
-                   LevelLayout* layout = nullptr) {
+// one_group: levels that fit take the one-workgroup stages (see k_rank_front).  Returns false when
+// their keys did not fit; the round is then to be analysed without them.
+bool try_analyze_round(Ctx& c, const RefineLevel& L, int mode, uint32_t omega, uint32_t delta, uint32_t R, uint32_t rep,
+                       bool chainup, const uint32_t* part, const uint32_t* psizes, RoundState& st, LevelLayout* layout,
+                       bool one_group) {
   const uint32_t n = L.n;
   const uint32_t g = ceil_div(n, 256);
   const bool incc = mode == HGP_MODE_INCC;
@@ -3296,39 +3804,55 @@ void analyze_round(Ctx& c, const RefineLevel& L, int mode, uint32_t omega, uint3
     Y.sized = true;
     Y.max_size = n ? reduce_max_u32(c, L.sizes, n) : 0u;
   }
-  const KeyStats gst = gain_stats(c, n, st.moves.get(), st.gains.get());
-  st.V = (uint32_t)gst.count;
-  if (chainup) rank_by_gain(c, n, st.moves.get(), st.gains.get(), gst, st.ranks.get());
-  else rank_by_chaining(c, n, L.k, part, st.moves.get(), st.gains.get(), gst, L.sizes, Y.max_size, st.ranks.get());
-  const uint32_t V = st.V;
-  st.seq = DBuf<unsigned long long>(c, std::max<uint32_t>(V, 1));
-  st.sv = DBuf<int32_t>(c, std::max<uint32_t>(V, 1));
-  st.iv = DBuf<int32_t>(c, std::max<uint32_t>(V, 1));
-  st.best.r = NONE;
-  if (V == 0) return;
-  HGP_LAUNCH(k_zero3, ceil_div(V, 256), 256, 0, c, st.seq.get(), (uint32_t*)st.sv.get(), (uint32_t*)st.iv.get(),
-             (uint64_t)V);
+  const bool small = one_group && n >= 1 && n <= SMALL_N && (chainup || chain_by_table(n, L.k, Y.max_size));
+  // the events and the best prefix too (V stays on the device); inbound events of larger keys are
+  // refused below
+  const int key_bits = bit_width(L.k) + bit_width(L.e) + bit_width(n);
+  const bool fused = small && n <= SMALL_EVENT_N && (!incc || key_bits <= 64);
+  // node records of the cascade, kept until its side streams have joined
+  const bool packed = L.k < PM2_MAX_K;
+  DBuf<uint2> pm2(c, packed ? n : 0);
+  DBuf<uint4> pm(c, packed ? 0 : n);
   DBuf<unsigned long long> dio;
-  if (incc) {
-    dio = DBuf<unsigned long long>(c, V);
-    fill_u32(c, (uint32_t*)dio.get(), 0u, 2ull * V);
+  DBuf<RankInfo> info(c, small ? 1 : 0);
+  st.best.r = NONE;
+  auto counters = [&](uint32_t m) {
+    st.seq = DBuf<unsigned long long>(c, std::max<uint32_t>(m, 1));
+    st.sv = DBuf<int32_t>(c, std::max<uint32_t>(m, 1));
+    st.iv = DBuf<int32_t>(c, std::max<uint32_t>(m, 1));
+    if (incc) dio = DBuf<unsigned long long>(c, std::max<uint32_t>(m, 1));
+  };
+  if (small) {
+    counters(n);
+    rank_small(c, RankArgs{part, st.moves.get(), st.gains.get(), L.sizes, n, L.k, chainup ? 1 : 0, st.ranks.get(), pm.get(),
+                           pm2.get(), st.seq.get(), dio.get(), st.sv.get(), st.iv.get(), info.get(), nullptr},
+               Y.max_size);
+    if (!fused) {
+      const RankInfo ri = read_scalar(c, info.get());
+      if (ri.wide) return false;
+      st.V = ri.V;
+      if (st.V == 0) return true;
+    }
+  } else {
+    const KeyStats gst = gain_stats(c, n, st.moves.get(), st.gains.get());
+    st.V = (uint32_t)gst.count;
+    if (chainup) rank_by_gain(c, n, st.moves.get(), st.gains.get(), gst, st.ranks.get());
+    else rank_by_chaining(c, n, L.k, part, st.moves.get(), st.gains.get(), gst, L.sizes, Y.max_size, st.ranks.get());
+    counters(st.V);
+    if (st.V == 0) return true;
+    HGP_LAUNCH(k_zero3, ceil_div(st.V, 256), 256, 0, c, st.seq.get(), (uint32_t*)st.sv.get(), (uint32_t*)st.iv.get(),
+               (uint64_t)st.V);
+    if (incc) fill_u32(c, (uint32_t*)dio.get(), 0u, 2ull * st.V);
+    if (packed) HGP_LAUNCH(k_pack_nodes2, g, 256, 0, c, part, st.moves.get(), st.ranks.get(), n, pm2.get());
+    else HGP_LAUNCH(k_pack_nodes, g, 256, 0, c, part, st.moves.get(), st.ranks.get(), n, pm.get());
   }
+  const uint32_t V = fused ? n : st.V;  // fused: the bound
   // cascade.  The hedges of 2..CAS_SMALL pins first, alone on the stream; then, with bit 1 of
   // the side_streams tuning, the sorted and direct classes on side streams beside the size
   // events (all classes add their terms to seq and dio with atomics; the node records stay
   // alive until the join before they are read).
-  DBuf<uint4> pm;
-  DBuf<uint2> pm2;
   std::optional<Fork> cas_fork;
   {
-    const bool packed = L.k < PM2_MAX_K;
-    if (packed) {
-      pm2 = DBuf<uint2>(c, n);
-      HGP_LAUNCH(k_pack_nodes2, g, 256, 0, c, part, st.moves.get(), st.ranks.get(), n, pm2.get());
-    } else {
-      pm = DBuf<uint4>(c, n);
-      HGP_LAUNCH(k_pack_nodes, g, 256, 0, c, part, st.moves.get(), st.ranks.get(), n, pm.get());
-    }
     CascadeArgs a{L.hedges, L.hoff, L.w, pm.get(), pm2.get(), incc ? 1 : 0, st.seq.get(), L.srcc, dio.get(), V};
     const int crb = std::max(1, bit_width(V));  // rank + 1 <= V
     const int cpb = std::max(1, bit_width(L.k));
@@ -3408,6 +3932,25 @@ void analyze_round(Ctx& c, const RefineLevel& L, int mode, uint32_t omega, uint3
   }
   const int rb = std::max(1, bit_width(V - 1));
   const int kb = std::max(1, bit_width(L.k));
+  // inbound events: partition, hedge and rank in one 64-bit word; larger levels are refused
+  const int eb = std::max(1, bit_width(L.e));
+  HGP_REQUIRE(!incc || kb + eb + rb <= 64, HGP_E_CAPACITY, "inbound events: key exceeds 64 bits");
+  if (fused) {
+    cas_fork.reset();  // the main stream waits for the cascade's side streams
+    DBuf<RoundOut> out(c, 1);
+    const EventArgs ea{part, st.moves.get(), st.ranks.get(), L.sizes, psizes, pl.inbsz.get(), dio.get(), info.get(), n,
+                       omega, delta, rb, kb, (int64_t*)st.seq.get(), st.sv.get(), st.iv.get(), out.get()};
+    with_items(2 * n, [&](auto it) {
+      constexpr uint32_t IT = decltype(it)::value;
+      if (incc) HGP_LAUNCH((k_round_small<IT, true>), 1, BLOCK_SORT_THREADS, 0, c, ea);
+      else HGP_LAUNCH((k_round_small<IT, false>), 1, BLOCK_SORT_THREADS, 0, c, ea);
+    });
+    const RoundOut o = read_scalar(c, out.get());
+    if (o.info.wide) return false;
+    st.V = o.info.V;
+    st.best = o.best;
+    return true;
+  }
   // size events; in inbound-constrained mode the inbound-set events on the same order (with
   // k-way's Delta = INT32_MAX every prefix is valid)
   {
@@ -3417,12 +3960,7 @@ void analyze_round(Ctx& c, const RefineLevel& L, int mode, uint32_t omega, uint3
     DBuf<int64_t> cum(c, m);
     // inbound events: m of them counted above a change of at most P destination pins either way
     const int db = 63 - bit_width(m);
-    if (incc) {
-      // partition, hedge and rank in one 64-bit word: larger levels are refused
-      const int eb = std::max(1, bit_width(L.e));
-      HGP_REQUIRE(kb + eb + rb <= 64, HGP_E_CAPACITY, "inbound events: key exceeds 64 bits");
-      HGP_REQUIRE(pl.P < (1ull << (db - 1)), HGP_E_CAPACITY, "inbound events: too many moves and pins");
-    }
+    HGP_REQUIRE(!incc || pl.P < (1ull << (db - 1)), HGP_E_CAPACITY, "inbound events: too many moves and pins");
     HGP_LAUNCH(k_size_events, g, 256, 0, c, part, st.moves.get(), st.ranks.get(), L.sizes, n, rb, keys.get(), vals.get());
     // the events sit at 2 * rank (+1), so they are already in rank order: sorting by the
     // partition bits alone orders them by (partition, rank)
@@ -3452,6 +3990,14 @@ void analyze_round(Ctx& c, const RefineLevel& L, int mode, uint32_t omega, uint3
     HGP_LAUNCH(k_best_final, 1, 256, 0, c, partial.get(), blocks, out.get());
     st.best = read_scalar(c, out.get());
   }
+  return true;
+}
+
+void analyze_round(Ctx& c, const RefineLevel& L, int mode, uint32_t omega, uint32_t delta, uint32_t R, uint32_t rep,
+                   bool chainup, const uint32_t* part, const uint32_t* psizes, RoundState& st,
+                   LevelLayout* layout = nullptr) {
+  if (!try_analyze_round(c, L, mode, omega, delta, R, rep, chainup, part, psizes, st, layout, true))
+    (void)try_analyze_round(c, L, mode, omega, delta, R, rep, chainup, part, psizes, st, layout, false);
 }
 
 }  // namespace
