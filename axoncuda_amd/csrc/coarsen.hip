@@ -16,6 +16,7 @@
 // independent) and decided top-down along holder chains; see the oracle for the rule.
 #include <cstdio>
 
+#include "block_sort.hpp"
 #include "prim.hpp"
 #include "stages.hpp"
 #include "wave_iter.hpp"
@@ -781,10 +782,14 @@ __global__ void __launch_bounds__(256) k_cand_heavy(CAND_ARGS, uint32_t nlist, u
 
 // ---------------------------------------------------------------------------------------
 // pairing
+// The device-wide rounds (levels above GROUP_SMALL nodes).  A round is four launches, each a read or
+// two of a few words per node: their number bounds it, not the bytes.  The counts and sums of the
+// next round are cleared where the round before has read them last; `best` alternates between two
+// arrays, since the decisions read it for other nodes than their own.
 __global__ void k_pair_init(const uint32_t* __restrict__ pairs, const uint32_t* __restrict__ scores, uint32_t cnc,
                             uint32_t round, uint32_t n, const uint32_t* __restrict__ raw, uint32_t* __restrict__ parent,
-                            uint32_t* __restrict__ wgt, uint32_t* __restrict__ nchild, uint32_t* __restrict__ pending,
-                            uint64_t* __restrict__ S, uint64_t* __restrict__ best, uint32_t* __restrict__ processed) {
+                            uint32_t* __restrict__ wgt, uint32_t* __restrict__ haschild, uint32_t* __restrict__ pending,
+                            uint32_t* __restrict__ processed, uint32_t* __restrict__ locked0) {
   uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
   if (v >= n) return;
   const bool locked = raw[v] != NONE;
@@ -801,21 +806,11 @@ __global__ void k_pair_init(const uint32_t* __restrict__ pairs, const uint32_t* 
   }
   parent[v] = par;
   wgt[v] = wt;
-  nchild[v] = 0;
-  pending[v] = 0;
-  S[v] = 0;
-  best[v] = 0;
   processed[v] = locked ? 1u : 0u;
-}
-
-__global__ void k_pair_count(const uint32_t* __restrict__ parent, uint32_t n, uint32_t* __restrict__ nchild,
-                             uint32_t* __restrict__ pending) {
-  uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= n) return;
-  const uint32_t p = parent[v];
-  if (p != NONE) {
-    atomicAdd(&nchild[p], 1u);
-    atomicAdd(&pending[p], 1u);
+  locked0[v] = locked ? 1u : 0u;
+  if (par != NONE) {
+    haschild[par] = 1u;
+    atomicAdd(&pending[par], 1u);
   }
 }
 
@@ -825,7 +820,8 @@ __global__ void k_pair_count(const uint32_t* __restrict__ parent, uint32_t n, ui
 // its two updates to complete before it decrements the parent's pending count, and the last
 // child reads the parent's values after that decrement returned, so it sees every child's
 // contribution without device-wide cache write-backs or invalidations.
-__device__ void sweep_up(uint32_t cur, const uint32_t* __restrict__ parent, const uint32_t* __restrict__ wgt,
+// `root`, if a node, is climbed to but not past (its pointer is being cut).
+__device__ void sweep_up(uint32_t cur, uint32_t root, const uint32_t* parent, const uint32_t* __restrict__ wgt,
                          uint32_t* pending, unsigned long long* S, unsigned long long* best, uint32_t* processed) {
   for (;;) {
     const uint64_t Sv = atomicAdd(&S[cur], 0ull);
@@ -833,7 +829,7 @@ __device__ void sweep_up(uint32_t cur, const uint32_t* __restrict__ parent, cons
     const uint64_t bg = bv >> 32;
     const uint64_t wout = Sv + bg;
     __hip_atomic_store(&processed[cur], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const uint32_t p = parent[cur];
+    const uint32_t p = cur == root ? NONE : parent[cur];
     if (p == NONE) return;
     const int64_t gain = (int64_t)wgt[cur] - (int64_t)bg;
     const uint64_t key = ((uint64_t)(gain > 0 ? gain : 0) << 32) | cur;
@@ -849,41 +845,34 @@ __device__ void sweep_up(uint32_t cur, const uint32_t* __restrict__ parent, cons
   }
 }
 
-__global__ void k_pair_sweep(const uint32_t* __restrict__ raw, const uint32_t* __restrict__ parent,
-                             const uint32_t* __restrict__ wgt, const uint32_t* __restrict__ nchild, uint32_t n,
+__global__ void k_pair_sweep(const uint32_t* __restrict__ locked0, const uint32_t* __restrict__ parent,
+                             const uint32_t* __restrict__ wgt, const uint32_t* __restrict__ haschild, uint32_t n,
                              uint32_t* pending, unsigned long long* S, unsigned long long* best, uint32_t* processed) {
   uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
   if (v >= n) return;
-  if (raw[v] != NONE || nchild[v] != 0) return;
-  sweep_up(v, parent, wgt, pending, S, best, processed);
+  if (locked0[v] || haschild[v]) return;
+  sweep_up(v, NONE, parent, wgt, pending, S, best, processed);
 }
 
-// nodes left unprocessed sit on cycles of the pointer graph: flag each cycle's minimum
-__global__ void k_pair_cycles(const uint32_t* __restrict__ raw, const uint32_t* __restrict__ parent,
-                              const uint32_t* __restrict__ processed, uint32_t n, uint32_t* __restrict__ cycmin) {
+// Nodes left unprocessed sit on cycles of the pointer graph: each cycle's minimum cuts its own
+// pointer and sums the rest of the cycle up.  The nodes of a cycle walk it in the same launch: one
+// that meets the cut has met the minimum, so only the minimum itself ever finds itself smallest,
+// and all other children of a cycle's nodes have been summed before this launch.
+__global__ void k_pair_cycles(uint32_t* parent, const uint32_t* __restrict__ wgt, uint32_t n, uint32_t* pending,
+                              unsigned long long* S, unsigned long long* best, uint32_t* processed) {
   uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
   if (v >= n) return;
-  uint32_t flag = 0;
-  if (raw[v] == NONE && !processed[v] && parent[v] != NONE) {
-    uint32_t m = v, x = parent[v];
-    for (uint32_t steps = 0; x != v && x != NONE && steps < n; ++steps) {
-      m = x < m ? x : m;
-      x = parent[x];
-    }
-    flag = (m == v) ? 1u : 0u;
-  }
-  cycmin[v] = flag;
-}
-
-__global__ void k_pair_break(const uint32_t* __restrict__ cycmin, uint32_t* parent, const uint32_t* __restrict__ wgt,
-                             uint32_t n, uint32_t* pending, unsigned long long* S, unsigned long long* best,
-                             uint32_t* processed) {
-  uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= n || !cycmin[v]) return;
   const uint32_t p = parent[v];
-  parent[v] = NONE;  // read by no other thread of this launch
+  if (processed[v] || p == NONE) return;
+  uint32_t m = v, x = p;
+  for (uint32_t steps = 0; x != v && x != NONE && steps < n; ++steps) {
+    m = x < m ? x : m;
+    x = parent[x];
+  }
+  if (m != v) return;
+  parent[v] = NONE;
   const uint32_t old = atomicSub(&pending[p], 1u);
-  if (old == 1u) sweep_up(p, parent, wgt, pending, S, best, processed);
+  if (old == 1u) sweep_up(p, v, parent, wgt, pending, S, best, processed);
 }
 
 __device__ __forceinline__ uint32_t holder_of(const unsigned long long* best, uint32_t v) {
@@ -891,11 +880,8 @@ __device__ __forceinline__ uint32_t holder_of(const unsigned long long* best, ui
   return (b >> 32) > 0 ? (uint32_t)b : NONE;
 }
 
-__global__ void k_pair_decide(const uint32_t* __restrict__ parent, const unsigned long long* __restrict__ best,
-                              const uint32_t* __restrict__ locked0, uint32_t n, uint32_t* __restrict__ raw) {
-  uint32_t y = blockIdx.x * blockDim.x + threadIdx.x;
-  if (y >= n || locked0[y]) return;
-  const uint32_t p = parent[y];
+// Matches the chain below y, if y heads one: y takes its holder, and so on below that one.
+__device__ __forceinline__ void decide_from(uint32_t y, uint32_t p, const unsigned long long* best, uint32_t* raw) {
   if (p != NONE && holder_of(best, p) == y) return;  // y hangs below its parent's chain
   uint32_t cur = y;
   while (cur != NONE) {
@@ -907,9 +893,17 @@ __global__ void k_pair_decide(const uint32_t* __restrict__ parent, const unsigne
   }
 }
 
-__global__ void k_locked_snapshot(const uint32_t* __restrict__ raw, uint32_t n, uint32_t* __restrict__ locked0) {
-  uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v < n) locked0[v] = raw[v] != NONE;
+__global__ void k_pair_decide(const uint32_t* __restrict__ parent, const unsigned long long* __restrict__ best,
+                              const uint32_t* __restrict__ locked0, uint32_t n, uint32_t* __restrict__ raw,
+                              uint32_t* __restrict__ haschild, uint32_t* __restrict__ pending,
+                              unsigned long long* __restrict__ S, unsigned long long* __restrict__ best_next) {
+  uint32_t y = blockIdx.x * blockDim.x + threadIdx.x;
+  if (y >= n) return;
+  haschild[y] = 0;
+  pending[y] = 0;
+  S[y] = 0;
+  best_next[y] = 0;
+  if (!locked0[y]) decide_from(y, parent[y], best, raw);
 }
 
 // orphans
@@ -951,6 +945,202 @@ __global__ void k_apply_ids(const uint32_t* __restrict__ raw, const uint64_t* __
   const uint32_t g = (uint32_t)nid[raw[v]];
   groups[v] = g;
   atomicAdd(&gsizes[g], sizes[v]);
+}
+
+// Everything above for levels of up to GROUP_SMALL nodes, by one workgroup with the pointer forest in
+// LDS: the rounds, the orphans' order and pairs, and the relabelling are some 130 launches of two to
+// four microseconds on such a level, bound by launches and by the latency of atomics in memory.  The
+// pointers of the next round are loaded while a round is worked on.  A round without pointers
+// changes nothing and is passed over.
+// Multi-level run on 9,248 nodes (8 layers of 1,156, 16 rounds a level): 11,946 launches in all before,
+// 8,874 now, 75.1 -> 69.8 ms on the device; 118 us for a level of 2,049 to 4,096 nodes.  A level of more
+// nodes has too little LDS for its forest.  There, 800k nodes, the rounds in four launches instead
+// of seven take a one-level contraction from 5.76 to 5.49 ms.
+constexpr uint32_t GROUP_SMALL = 4096;
+
+template <uint32_t IT>
+struct GroupMem {
+  static constexpr uint32_t N = BLOCK_SORT_THREADS * IT;
+  uint32_t parent[N], wgt[N], pending[N], raw[N];
+  union {
+    struct {
+      unsigned long long S[N], best[N];
+    };
+    BlockSortMem<uint64_t, IT> sort;
+  };
+};
+
+// as sweep_up; a wave's operations on LDS are performed in order
+template <uint32_t IT>
+__device__ void sweep_up_lds(uint32_t cur, uint32_t root, GroupMem<IT>& s) {
+  for (;;) {
+    const uint64_t bg = s.best[cur] >> 32;
+    const uint64_t wout = s.S[cur] + bg;
+    const uint32_t p = cur == root ? NONE : s.parent[cur];
+    if (p == NONE) return;
+    const int64_t gain = (int64_t)s.wgt[cur] - (int64_t)bg;
+    const uint64_t key = ((uint64_t)(gain > 0 ? gain : 0) << 32) | cur;
+    atomicAdd(&s.S[p], (unsigned long long)wout);
+    atomicMax(&s.best[p], (unsigned long long)key);
+    const uint32_t old = __hip_atomic_fetch_sub(&s.pending[p], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
+    if (old != 1u) return;
+    cur = p;
+  }
+}
+
+template <uint32_t IT>
+__global__ void __launch_bounds__(BLOCK_SORT_THREADS)
+    k_group_small(const uint32_t* __restrict__ pairs, const uint32_t* __restrict__ scores, uint32_t cnc, uint32_t n,
+                  const uint32_t* __restrict__ sizes, const uint32_t* __restrict__ inb, uint32_t omega, uint32_t delta,
+                  int size_bits, uint32_t* __restrict__ raw_out, uint32_t* __restrict__ groups,
+                  uint32_t* __restrict__ gsizes, uint32_t* __restrict__ new_n) {
+  __shared__ GroupMem<IT> s;
+  uint32_t v[IT], cand[IT], sc[IT];
+  bool orphan[IT];
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) {
+    v[r] = block_pos<IT>(r);
+    s.raw[v[r]] = NONE;
+    const bool in = v[r] < n;
+    cand[r] = in ? pairs[(uint64_t)v[r] * cnc] : NONE;
+    sc[r] = in ? scores[(uint64_t)v[r] * cnc] : 0;
+    orphan[r] = in && cand[r] == NONE;
+  }
+  for (uint32_t round = 0; round < cnc; ++round) {
+    uint32_t par[IT], wt[IT], locked = 0;
+#pragma unroll
+    for (uint32_t r = 0; r < IT; ++r) {
+      par[r] = cand[r];
+      wt[r] = sc[r];
+      if (round + 1 < cnc && v[r] < n) {
+        cand[r] = pairs[(uint64_t)v[r] * cnc + round + 1];
+        sc[r] = scores[(uint64_t)v[r] * cnc + round + 1];
+      }
+      s.parent[v[r]] = par[r];
+      s.pending[v[r]] = 0;
+      s.S[v[r]] = 0;
+      s.best[v[r]] = 0;
+    }
+    __syncthreads();  // also orders the rows of raw
+    bool any = false;
+#pragma unroll
+    for (uint32_t r = 0; r < IT; ++r) {
+      const bool l = s.raw[v[r]] != NONE;
+      locked |= (uint32_t)l << r;
+      const uint32_t t = par[r];
+      if (l || t == NONE || s.raw[t] != NONE || (s.parent[t] == v[r] && v[r] < t)) par[r] = NONE;
+      any |= par[r] != NONE;
+    }
+    if (!__syncthreads_or(any)) continue;
+#pragma unroll
+    for (uint32_t r = 0; r < IT; ++r) {
+      s.parent[v[r]] = par[r];
+      s.wgt[v[r]] = wt[r];
+      if (par[r] != NONE) atomicAdd(&s.pending[par[r]], 1u);
+    }
+    __syncthreads();
+    uint32_t leaf = 0;
+#pragma unroll
+    for (uint32_t r = 0; r < IT; ++r)
+      leaf |= (uint32_t)(par[r] != NONE && s.pending[v[r]] == 0) << r;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t r = 0; r < IT; ++r)
+      if (leaf >> r & 1u) sweep_up_lds(v[r], NONE, s);
+    __syncthreads();
+    // nodes that still wait for a child are on a cycle
+    uint32_t onc = 0;
+#pragma unroll
+    for (uint32_t r = 0; r < IT; ++r) onc |= (uint32_t)(s.pending[v[r]] != 0) << r;
+    if (__syncthreads_or(onc)) {
+      uint32_t cut = 0;
+#pragma unroll
+      for (uint32_t r = 0; r < IT; ++r) {
+        if (!(onc >> r & 1u)) continue;
+        uint32_t m = v[r], x = par[r];
+        for (uint32_t steps = 0; x != v[r] && x != NONE && steps < n; ++steps) {
+          m = x < m ? x : m;
+          x = s.parent[x];
+        }
+        cut |= (uint32_t)(m == v[r]) << r;
+      }
+      __syncthreads();
+#pragma unroll
+      for (uint32_t r = 0; r < IT; ++r) {
+        if (!(cut >> r & 1u)) continue;
+        const uint32_t p = par[r];
+        par[r] = NONE;
+        const uint32_t old = __hip_atomic_fetch_sub(&s.pending[p], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (old == 1u) sweep_up_lds(p, v[r], s);
+      }
+      __syncthreads();
+    }
+#pragma unroll
+    for (uint32_t r = 0; r < IT; ++r)
+      if (v[r] < n && !(locked >> r & 1u)) decide_from(v[r], par[r], s.best, s.raw);
+    __syncthreads();
+  }
+  // orphans in node order, sorted stably by size: the smallest with the largest, and so on inwards
+  uint32_t x[IT];
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) x[r] = orphan[r];
+  block_scan(x, s.sort.w);
+  if (threadIdx.x == BLOCK_SORT_THREADS - 1) s.wgt[0] = x[IT - 1];
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r)
+    if (orphan[r]) s.sort.key[x[r] - 1] = ((uint64_t)sizes[v[r]] << 32) | v[r];
+  __syncthreads();
+  const uint32_t m = s.wgt[0];
+  if (m >= 2) {
+    uint64_t key[IT];
+    uint32_t none[IT] = {};
+#pragma unroll
+    for (uint32_t r = 0; r < IT; ++r) key[r] = v[r] < m ? s.sort.key[v[r]] : 0;
+    __syncthreads();
+    block_sort<uint64_t, false, IT>(key, none, m, 32, 32 + size_bits, digit_bits(size_bits), 0, s.sort);
+    for (uint32_t k = threadIdx.x; k < m / 2; k += BLOCK_SORT_THREADS) {
+      const uint32_t L = (uint32_t)s.sort.key[k], R = (uint32_t)s.sort.key[m - 1 - k];
+      if (sizes[L] + sizes[R] <= omega && inb[L] + inb[R] <= delta) {
+        const uint32_t g = L < R ? L : R;
+        s.raw[L] = g;
+        s.raw[R] = g;
+      }
+    }
+  }
+  __syncthreads();
+  // zero-based ids in ascending order of the raw ids
+  uint32_t raw[IT];
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) {
+    raw[r] = s.raw[v[r]];
+    if (raw[r] == NONE) raw[r] = v[r];
+    if (raw_out && v[r] < n) raw_out[v[r]] = raw[r];
+    s.wgt[v[r]] = 0;
+    s.pending[v[r]] = 0;
+  }
+  __syncthreads();
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r)
+    if (v[r] < n) s.wgt[raw[r]] = 1u;
+  __syncthreads();
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) x[r] = s.wgt[v[r]];
+  block_scan(x, s.sort.w);
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) s.parent[v[r]] = x[r] - 1;  // of the marked nodes only
+  __syncthreads();
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) {
+    if (v[r] >= n) continue;
+    const uint32_t g = s.parent[raw[r]];
+    groups[v[r]] = g;
+    atomicAdd(&s.pending[g], sizes[v[r]]);
+  }
+  if (threadIdx.x == BLOCK_SORT_THREADS - 1) *new_n = x[IT - 1];
+  __syncthreads();
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r)
+    if (v[r] < n) gsizes[v[r]] = s.pending[v[r]];
 }
 
 }  // namespace
@@ -1109,25 +1299,28 @@ void candidates(Ctx& c, const uint32_t* hedges, const uint64_t* hoff, const uint
   }
 }
 
-void group_nodes(Ctx& c, const uint32_t* inb, const uint32_t* pairs, const uint32_t* scores, const uint32_t* sizes,
-                 uint32_t n, uint32_t cnc, uint32_t omega, uint32_t delta, uint32_t& new_n, uint32_t*& groups_out,
-                 uint32_t*& gsizes_out, uint32_t** ungroups_out, uint64_t** uoff_out, uint32_t* raw_out) {
+// Groups of levels above GROUP_SMALL nodes: pairing rounds, orphans and relabelling device-wide.
+static void group_large(Ctx& c, const uint32_t* inb, const uint32_t* pairs, const uint32_t* scores,
+                        const uint32_t* sizes, uint32_t n, uint32_t cnc, uint32_t omega, uint32_t delta,
+                        uint32_t& new_n, uint32_t* groups, DBuf<uint32_t>& gsizes, uint32_t* raw_out) {
   const uint32_t g = ceil_div(n, 256);
-  DBuf<uint32_t> raw(c, n), parent(c, n), wgt(c, n), nchild(c, n), pending(c, n), processed(c, n), cycmin(c, n),
-      locked0(c, n);
-  DBuf<unsigned long long> S(c, n), best(c, n);
+  DBuf<uint32_t> raw(c, n), parent(c, n), wgt(c, n), processed(c, n), locked0(c, n);
+  DBuf<uint32_t> counts(c, 2ull * n);             // haschild, pending
+  DBuf<unsigned long long> sums(c, 3ull * n);     // S, best of even and of odd rounds
+  uint32_t *haschild = counts.get(), *pending = haschild + n;
+  unsigned long long* S = sums.get();
   fill_u32(c, raw.get(), NONE, n);
+  memset_async(c, counts.get(), 0, 2ull * n * sizeof(uint32_t));
+  memset_async(c, sums.get(), 0, 2ull * n * sizeof(unsigned long long));
   for (uint32_t i = 0; i < cnc; ++i) {
-    HGP_LAUNCH(k_pair_init, g, 256, 0, c, pairs, scores, cnc, i, n, raw.get(), parent.get(), wgt.get(), nchild.get(),
-               pending.get(), (uint64_t*)S.get(), (uint64_t*)best.get(), processed.get());
-    HGP_LAUNCH(k_pair_count, g, 256, 0, c, parent.get(), n, nchild.get(), pending.get());
-    HGP_LAUNCH(k_pair_sweep, g, 256, 0, c, raw.get(), parent.get(), wgt.get(), nchild.get(), n, pending.get(), S.get(),
-               best.get(), processed.get());
-    HGP_LAUNCH(k_pair_cycles, g, 256, 0, c, raw.get(), parent.get(), processed.get(), n, cycmin.get());
-    HGP_LAUNCH(k_pair_break, g, 256, 0, c, cycmin.get(), parent.get(), wgt.get(), n, pending.get(), S.get(), best.get(),
+    unsigned long long *best = S + (i & 1 ? 2ull : 1ull) * n, *best_next = S + (i & 1 ? 1ull : 2ull) * n;
+    HGP_LAUNCH(k_pair_init, g, 256, 0, c, pairs, scores, cnc, i, n, raw.get(), parent.get(), wgt.get(), haschild,
+               pending, processed.get(), locked0.get());
+    HGP_LAUNCH(k_pair_sweep, g, 256, 0, c, locked0.get(), parent.get(), wgt.get(), haschild, n, pending, S, best,
                processed.get());
-    HGP_LAUNCH(k_locked_snapshot, g, 256, 0, c, raw.get(), n, locked0.get());
-    HGP_LAUNCH(k_pair_decide, g, 256, 0, c, parent.get(), best.get(), locked0.get(), n, raw.get());
+    HGP_LAUNCH(k_pair_cycles, g, 256, 0, c, parent.get(), wgt.get(), n, pending, S, best, processed.get());
+    HGP_LAUNCH(k_pair_decide, g, 256, 0, c, parent.get(), best, locked0.get(), n, raw.get(), haschild, pending, S,
+               best_next);
   }
   // orphans
   {
@@ -1152,9 +1345,31 @@ void group_nodes(Ctx& c, const uint32_t* inb, const uint32_t* pairs, const uint3
   DBuf<uint64_t> nid(c, (uint64_t)n + 1);
   exclusive_scan(c, flag.get(), nid.get(), n);
   new_n = (uint32_t)read_scalar(c, nid.get() + n);
-  DBuf<uint32_t> groups(c, n), gsizes(c, std::max<uint32_t>(new_n, 1));
+  gsizes = DBuf<uint32_t>(c, std::max<uint32_t>(new_n, 1));
   memset_async(c, gsizes.get(), 0, (uint64_t)new_n * sizeof(uint32_t));
-  HGP_LAUNCH(k_apply_ids, g, 256, 0, c, raw.get(), nid.get(), sizes, n, groups.get(), gsizes.get());
+  HGP_LAUNCH(k_apply_ids, g, 256, 0, c, raw.get(), nid.get(), sizes, n, groups, gsizes.get());
+}
+
+void group_nodes(Ctx& c, const uint32_t* inb, const uint32_t* pairs, const uint32_t* scores, const uint32_t* sizes,
+                 uint32_t n, uint32_t cnc, uint32_t omega, uint32_t delta, uint32_t& new_n, uint32_t*& groups_out,
+                 uint32_t*& gsizes_out, uint32_t** ungroups_out, uint64_t** uoff_out, uint32_t* raw_out) {
+  DBuf<uint32_t> groups(c, n), gsizes;
+  if (n <= GROUP_SMALL) {
+    gsizes = DBuf<uint32_t>(c, std::max<uint32_t>(n, 1));
+    DBuf<uint32_t> raw(c, raw_out ? n : 0), count(c, 1);
+    const int size_bits = std::max(1, bit_width(omega));
+    auto run = [&](auto it) {
+      HGP_LAUNCH((k_group_small<decltype(it)::value>), 1, BLOCK_SORT_THREADS, 0, c, pairs, scores, cnc, n, sizes, inb,
+                 omega, delta, size_bits, raw_out ? raw.get() : nullptr, groups.get(), gsizes.get(), count.get());
+    };
+    if (n <= BLOCK_SORT_THREADS) run(std::integral_constant<uint32_t, 1>{});
+    else if (n <= 2 * BLOCK_SORT_THREADS) run(std::integral_constant<uint32_t, 2>{});
+    else run(std::integral_constant<uint32_t, 4>{});
+    if (raw_out) copy_d2h(c, raw_out, raw.get(), (uint64_t)n * sizeof(uint32_t));
+    new_n = read_scalar(c, count.get());
+  } else {
+    group_large(c, inb, pairs, scores, sizes, n, cnc, omega, delta, new_n, groups.get(), gsizes, raw_out);
+  }
   if (ungroups_out) {
     DBuf<uint32_t> keys(c, n), vals(c, n);
     copy_d2d(c, keys.get(), groups.get(), (uint64_t)n * sizeof(uint32_t));

@@ -194,6 +194,27 @@ def test_group_nodes_cycles(dev, rng):
     assert k == ek and np.array_equal(groups, eg)
 
 
+@pytest.mark.parametrize("n", [1, 2, 64, 1023, 1024, 1025, 2048, 2049, 4095, 4096, 4097])
+@pytest.mark.parametrize("cnc", [1, 4])
+def test_group_nodes_by_size(dev, n, cnc, rng):
+    """Levels at the edges of the one-workgroup pairing: random pointers (chains, cycles of all
+    lengths, pointers to locked nodes and to the node itself), and orphans of many sizes."""
+    pairs = rng.integers(0, n, size=(n, cnc)).astype(np.uint32)
+    near = rng.random((n, cnc)) < 0.5  # half of them along one long cycle
+    pairs[near] = ((np.arange(n)[:, None] + 1) % n * np.ones((1, cnc))).astype(np.uint32)[near]
+    pairs[rng.random((n, cnc)) < 0.2] = 0xFFFFFFFF
+    pairs[rng.random(n) < 0.3] = 0xFFFFFFFF  # orphans
+    scores = rng.integers(0, 8, size=(n, cnc)).astype(np.uint32)
+    sizes = rng.integers(1, 300, size=n).astype(np.uint32)
+    inb = rng.integers(0, 50, size=n).astype(np.uint32)
+    omega, delta = 310, 70
+    d_inb, d_pairs, d_scores, d_sizes = (dev.upload(x) for x in (inb, pairs.ravel(), scores.ravel(), sizes))
+    k, groups, gs, ung, uoff, *_ = G.group_nodes(dev, n, d_inb, d_pairs, d_scores, d_sizes, cnc, omega, delta)
+    ek, eg, egs, eung, euoff, _ = O.group_nodes(n, inb, pairs.ravel(), scores.ravel(), sizes, cnc, omega, delta)
+    assert k == ek and np.array_equal(groups, eg) and np.array_equal(gs, egs)
+    assert np.array_equal(ung, eung) and np.array_equal(uoff, euoff)
+
+
 @pytest.mark.parametrize("case", CASES, ids=[c[0] for c in CASES])
 def test_coarsening(dev, case, rng):
     """coarse hedges, coarse touching, coarse neighbours, uncoarsen"""
