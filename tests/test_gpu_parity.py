@@ -151,6 +151,25 @@ def test_candidates_heavy_tables(dev, n, hubs, expect, rng):
         assert np.array_equal(scores, es), f"scores differ (delta={delta})"
 
 
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 257, 65535, 65536, 65537])
+def test_candidates_by_size(dev, n, rng):
+    """Levels whose nodes split into runs of 64 (and, above 65,536 nodes, of 128) when they are laid
+    out by class: nodes without hedges, and hubs of every class with an LDS table by wave or workgroup."""
+    if n < 64:
+        hg = O.HG(n, np.array([0, 1], np.uint64), np.zeros(1, np.uint32), np.ones(1, np.uint32), np.ones(1, np.float32))
+    else:
+        hubs = [(h, c, 40, n) for h, c in ((0, 3), (1, 8), (n // 2, 20), (n - 1, 60), (n - 2, 110), (n - 3, 200))]
+        hg = hub_graph(n, hubs, n // 4, rng)
+    L = G.Level(dev, hg)
+    L.build_touching()
+    ro, rt, ri = O.touching(hg)
+    sizes = rng.integers(1, 3, size=hg.n).astype(np.uint32)
+    for delta in (2**31 - 1, 30):
+        pairs, scores, *_ = G.candidates(dev, L, sizes, 4, 6, delta)
+        ep, es = O.candidates(hg, ro, rt, ri, sizes, 4, 6, delta)
+        assert np.array_equal(pairs, ep) and np.array_equal(scores, es), delta
+
+
 @pytest.mark.parametrize("case", CASES, ids=[c[0] for c in CASES])
 @pytest.mark.parametrize("cnc", [1, 3, 16])
 def test_group_nodes(dev, case, cnc, rng):
