@@ -10,6 +10,7 @@
 // Coarse hedges (coarsenHedges, :563-676) and neighbour sets (buildNeighbors :242-340,
 // coarsenNeighbors :342-561) are sort-unique problems: the (segment, value) pairs are
 // radix-sorted on exactly the bits they need and run heads are compacted with scans.
+#include "block_sort.hpp"
 #include "prim.hpp"
 #include "stages.hpp"
 #include "wave_iter.hpp"
@@ -18,17 +19,97 @@ namespace hgp {
 
 namespace {
 
-__global__ void k_touch_keys(const uint32_t* __restrict__ hedges, const uint64_t* __restrict__ hoff,
-                             const uint32_t* __restrict__ srcc, uint32_t E, uint32_t* __restrict__ keys,
-                             uint32_t* __restrict__ vals) {
-  uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= E) return;
-  uint64_t s = hoff[e], t = hoff[e + 1];
-  uint32_t sc = srcc[e];
-  for (uint64_t i = s; i < t; ++i) {
-    keys[i] = hedges[i] * 2u + ((i - s) < sc ? 1u : 0u);
-    vals[i] = e;
+// Hedges of pins.  A workgroup owns a tile of consecutive pins, finds the hedges that meet it by a
+// search of the offsets in 64 steps at once, marks the pins where hedges start, and gives every pin
+// the last mark at or before it: pins are read and keys written in full lines, and a long hedge is
+// shared by as many workgroups as it has tiles.  (A thread per hedge writes with the stride of the
+// hedges' lengths, and the longest hedge is one thread's serial work.)  The kernel is bound by its
+// reads and writes: at 3.2M pins of 800k nodes' hedges 169 -> 18 us (k_touch_keys) and 290 -> 33 us
+// (k_chedge_keys, which reads a group per pin).  Up to 256k pins a thread takes one pin, so that
+// small levels spread over the chip; above, four.
+template <uint32_t IT>
+struct PinTile {
+  uint32_t mark[BLOCK_SORT_THREADS * IT];
+  uint32_t w[BLOCK_SORT_WAVES];
+  uint32_t first, end;
+};
+
+// number of the m ascending entries that are <= key; every lane of the wave calls it
+__device__ __forceinline__ uint32_t wave_upper_bound(const uint64_t* __restrict__ x, uint32_t m, uint64_t key) {
+  uint32_t lo = 0, hi = m;  // entries below lo are <= key, those from hi on are not
+  while (hi - lo > 64) {
+    const uint32_t step = (hi - lo) / 64;
+    const uint32_t c = (uint32_t)__popcll(__ballot(x[lo + lane_id() * step] <= key));
+    if (c == 0) return lo;
+    if (c < 64) hi = lo + c * step;
+    lo += (c - 1) * step + 1;
   }
+  return lo + (uint32_t)__popcll(__ballot(lo + lane_id() < hi && x[lo + lane_id()] <= key));
+}
+
+// hedge[r], in_hedge[r]: the hedge of pin block_pos<IT>(r) of the tile at `base`, and the pin's place
+// in it.  Pins from p on get none.  Every thread calls it.
+template <uint32_t IT>
+__device__ __forceinline__ void pin_hedges(const uint64_t* __restrict__ hoff, uint32_t E, uint64_t p, uint64_t base,
+                                           uint32_t (&hedge)[IT], uint64_t (&in_hedge)[IT], PinTile<IT>& s) {
+  constexpr uint32_t T = BLOCK_SORT_THREADS * IT;
+  const uint32_t len = (uint32_t)min((uint64_t)T, p - base);
+  if (threadIdx.x < 64) {
+    const uint32_t c = wave_upper_bound(hoff, E, base);
+    if (lane_id() == 0) s.first = c ? c - 1 : 0;
+  } else if (threadIdx.x < 128) {
+    const uint32_t c = wave_upper_bound(hoff, E, base + len - 1);
+    if (lane_id() == 0) s.end = c;
+  }
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) s.mark[threadIdx.x + BLOCK_SORT_THREADS * r] = NONE;
+  __syncthreads();
+  const uint32_t h0 = s.first, h1 = s.end;
+  for (uint32_t h = h0 + threadIdx.x; h < h1; h += BLOCK_SORT_THREADS) {
+    const uint64_t a = hoff[h], b = hoff[h + 1];
+    if (b > a && b > base) s.mark[a > base ? a - base : 0] = h;  // hedges without pins start nowhere
+  }
+  __syncthreads();
+  bool flag[IT];
+  uint32_t head[IT];
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) flag[r] = s.mark[block_pos<IT>(r)] != NONE;
+  block_last_head(flag, head, s.w);
+  const uint64_t before = base - hoff[h0];  // pins of the first hedge in earlier tiles
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) {
+    const uint32_t i = block_pos<IT>(r);
+    hedge[r] = i < len && head[r] != NONE ? s.mark[head[r]] : NONE;
+    in_hedge[r] = i - head[r] + (head[r] == 0 ? before : 0);
+  }
+}
+
+template <uint32_t IT>
+__global__ void __launch_bounds__(BLOCK_SORT_THREADS)
+    k_touch_keys(const uint32_t* __restrict__ hedges, const uint64_t* __restrict__ hoff,
+                 const uint32_t* __restrict__ srcc, uint32_t E, uint64_t p, uint32_t* __restrict__ keys,
+                 uint32_t* __restrict__ vals) {
+  __shared__ PinTile<IT> s;
+  const uint64_t base = (uint64_t)blockIdx.x * BLOCK_SORT_THREADS * IT;
+  uint32_t h[IT];
+  uint64_t k[IT];
+  pin_hedges(hoff, E, p, base, h, k, s);
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) {
+    if (h[r] == NONE) continue;
+    const uint64_t i = base + block_pos<IT>(r);
+    keys[i] = hedges[i] * 2u + (k[r] < srcc[h[r]] ? 1u : 0u);
+    vals[i] = h[r];
+  }
+}
+
+// f(items, tiles): pins per thread (a compile-time constant) and the number of tiles of p pins
+template <typename F>
+void with_pin_tiles(uint64_t p, F f) {
+  if (p <= 256ull * BLOCK_SORT_THREADS)
+    f(std::integral_constant<uint32_t, 1>{}, ceil_div(p, BLOCK_SORT_THREADS));
+  else
+    f(std::integral_constant<uint32_t, 4>{}, ceil_div(p, 4ull * BLOCK_SORT_THREADS));
 }
 
 // inbound_count[v]: number of even keys (destination incidences) in v's segment
@@ -109,15 +190,22 @@ __global__ void k_low_bits(const uint64_t* __restrict__ keys, uint64_t n, uint64
 }
 
 // coarse hedge keys: (e << (gb+1)) | (group << 1) | is_source
-__global__ void k_chedge_keys(const uint32_t* __restrict__ hedges, const uint64_t* __restrict__ hoff,
-                              const uint32_t* __restrict__ srcc, const uint32_t* __restrict__ groups, uint32_t E,
-                              int gb, uint64_t* __restrict__ keys) {
-  uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= E) return;
-  uint64_t s = hoff[e], t = hoff[e + 1];
-  uint32_t sc = srcc[e];
-  for (uint64_t i = s; i < t; ++i)
-    keys[i] = ((uint64_t)e << (gb + 1)) | ((uint64_t)groups[hedges[i]] << 1) | ((i - s) < sc ? 1u : 0u);
+template <uint32_t IT>
+__global__ void __launch_bounds__(BLOCK_SORT_THREADS)
+    k_chedge_keys(const uint32_t* __restrict__ hedges, const uint64_t* __restrict__ hoff,
+                  const uint32_t* __restrict__ srcc, const uint32_t* __restrict__ groups, uint32_t E, uint64_t p,
+                  int gb, uint64_t* __restrict__ keys) {
+  __shared__ PinTile<IT> s;
+  const uint64_t base = (uint64_t)blockIdx.x * BLOCK_SORT_THREADS * IT;
+  uint32_t h[IT];
+  uint64_t k[IT];
+  pin_hedges(hoff, E, p, base, h, k, s);
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) {
+    if (h[r] == NONE) continue;
+    const uint64_t i = base + block_pos<IT>(r);
+    keys[i] = ((uint64_t)h[r] << (gb + 1)) | ((uint64_t)groups[hedges[i]] << 1) | (k[r] < srcc[h[r]] ? 1u : 0u);
+  }
 }
 
 // run heads of (e, group): a head whose first entry is a destination is a destination
@@ -164,14 +252,22 @@ __global__ void k_chedge_write(const uint64_t* __restrict__ keys, uint64_t n, in
   }
 }
 
-__global__ void k_max_group_of_pins(const uint32_t* __restrict__ hedges, const uint32_t* __restrict__ groups, uint64_t p,
-                                    uint32_t* out) {
+// One atomic per workgroup: same-address atomics, tens of nanoseconds each, bound one per wave
+// (108 us at 800k nodes).
+__global__ void __launch_bounds__(1024)
+    k_max_group_of_pins(const uint32_t* __restrict__ hedges, const uint32_t* __restrict__ groups, uint64_t p,
+                        uint32_t* out) {
+  __shared__ uint32_t s_m[16];
   uint32_t m = 0;
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < p; i += (uint64_t)gridDim.x * blockDim.x) {
     const uint32_t g = groups[hedges[i]];
     m = g > m ? g : m;
   }
   m = wave_max(m);
+  if (lane_id() == 0) s_m[threadIdx.x / 64] = m;
+  __syncthreads();
+  if (threadIdx.x >= 64) return;
+  m = wave_max(lane_id() < 16 ? s_m[lane_id()] : 0u);
   if (lane_id() == 0) atomicMax(out, m);
 }
 
@@ -212,7 +308,10 @@ void build_touching(Ctx& c, const uint32_t* hedges, const uint64_t* hoff, const 
   const uint64_t p = e ? read_scalar(c, hoff + e) : 0;
   DBuf<uint32_t> keys(c, p);
   DBuf<uint32_t> vals(c, p);
-  HGP_LAUNCH(k_touch_keys, ceil_div(e, 256), 256, 0, c, hedges, hoff, srcc, e, keys.get(), vals.get());
+  with_pin_tiles(p, [&](auto it, uint32_t tiles) {
+    HGP_LAUNCH((k_touch_keys<decltype(it)::value>), tiles, BLOCK_SORT_THREADS, 0, c, hedges, hoff, srcc, e, p,
+               keys.get(), vals.get());
+  });
   radix_sort(c, keys.get(), vals.get(), p, bit_width(2ull * n + 1));
   DBuf<uint64_t> off(c, (uint64_t)n + 1);
   segment_offsets(c, keys.get(), 1, p, n, off.get());
@@ -256,7 +355,7 @@ void coarsen_hedges(Ctx& c, const uint32_t* hedges, const uint64_t* hoff, const 
   if (new_n == 0 && hsize > 0) {  // derive the coarse node count from the groups of the pins
     DBuf<uint32_t> mx(c, 1);
     memset_async(c, mx.get(), 0, 4);
-    HGP_LAUNCH(k_max_group_of_pins, std::min<uint32_t>(ceil_div(hsize, 256), 2048), 256, 0, c, hedges, groups, hsize,
+    HGP_LAUNCH(k_max_group_of_pins, std::min<uint32_t>(ceil_div(hsize, 1024), 512), 1024, 0, c, hedges, groups, hsize,
                mx.get());
     new_n = read_scalar(c, mx.get()) + 1;
   }
@@ -265,7 +364,10 @@ void coarsen_hedges(Ctx& c, const uint32_t* hedges, const uint64_t* hoff, const 
   HGP_REQUIRE(eb + gb + 1 <= 64, HGP_E_CAPACITY, "coarsen_hedges: hedge and group ids exceed 64 key bits");
   const uint64_t p = hsize;
   DBuf<uint64_t> keys(c, p);
-  HGP_LAUNCH(k_chedge_keys, ceil_div(e, 256), 256, 0, c, hedges, hoff, srcc, groups, e, gb, keys.get());
+  with_pin_tiles(p, [&](auto it, uint32_t tiles) {
+    HGP_LAUNCH((k_chedge_keys<decltype(it)::value>), tiles, BLOCK_SORT_THREADS, 0, c, hedges, hoff, srcc, groups, e, p,
+               gb, keys.get());
+  });
   radix_sort(c, keys.get(), nullptr, p, eb + gb + 1);
   DBuf<uint32_t> srcf(c, p), dstf(c, p);
   HGP_LAUNCH(k_chedge_flags, ceil_div(p, 256), 256, 0, c, keys.get(), p, srcf.get(), dstf.get());

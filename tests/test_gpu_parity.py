@@ -101,6 +101,38 @@ def test_candidates_table_tiers(dev, n, big, deltas, rng):
         assert np.array_equal(scores, es), f"scores differ (delta={delta})"
 
 
+@pytest.mark.parametrize("pins", [1, 1023, 1024, 1025, 262143, 262144, 262145, 300001])
+def test_construction_by_pins(dev, pins, rng):
+    """Pin counts at the edges of the tiles of pins: hedges without pins in runs, at tile edges and at
+    both ends, hedges of a few pins, and hedges of several tiles."""
+    n, lens = max(2, pins // 8), [0, 0]
+    left = pins
+    while left:
+        kind = rng.random()
+        ln = 0 if kind < 0.2 else int(rng.integers(1, 9)) if kind < 0.999 else int(rng.integers(500, 20000))
+        if left in (pins, pins - 1024, pins - 4096):
+            lens += [0] * 5
+        ln = min(ln, left, 1024 - (pins - left) if pins - left < 1024 else left)  # a hedge starts at pin 1024
+        lens.append(ln)
+        left -= ln
+    lens = np.array(lens + [0, 0, 0])
+    off = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint64)
+    p = rng.integers(0, n, size=pins).astype(np.uint32)
+    srcc = np.minimum(rng.integers(0, 3, size=len(lens)), lens).astype(np.uint32)
+    hg = O.HG(n, off, p, srcc, np.ones(len(lens), np.float32))
+    L = G.Level(dev, hg)
+    L.build_touching()
+    ro, rt, ri = O.touching(hg)
+    assert np.array_equal(dev.download(L.toff, n + 1, np.uint64), ro)
+    assert np.array_equal(dev.download(L.tch, pins, np.uint32), rt)
+    assert np.array_equal(dev.download(L.inb, n, np.uint32), ri)
+    groups = rng.integers(0, n // 2, size=n).astype(np.uint32)
+    groups[:2] = [0, n // 2 - 1]
+    choff, cp, csrcc, *_ = G.coarsen_hedges(dev, L, dev.upload(groups))
+    eo, ep, es = O.coarsen_hedges(hg, groups)
+    assert np.array_equal(choff, eo) and np.array_equal(cp, ep) and np.array_equal(csrcc, es)
+
+
 def hub_graph(n, hubs, n_small, rng):
     """Hub nodes, each on `count` hedges of `size` pins drawn from a pool of `pool` nodes, so
     their visit bounds (and worst-case tables) are far above their distinct neighbours."""
