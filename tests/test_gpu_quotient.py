@@ -56,6 +56,22 @@ def test_quotient_matches_oracle(dev, src_prob, k, rng):
     check(dev, hg, part)
 
 
+@pytest.mark.parametrize("few", [0, 40])
+def test_quotient_by_members(dev, few, rng):
+    """Merged hedges of 1 .. 1000 members at the edges of a lane's and a wave's share, beside `few`
+    merged hedges of one member; the members of all are mixed in hedge order."""
+    counts = [1, 8, 9, 63, 64, 65, 127, 128, 129, 1000] + [1] * few
+    k = len(counts) + 1
+    which = rng.permutation(np.repeat(np.arange(len(counts)), counts))  # hedge -> its set {which, k - 1}
+    part = np.repeat(np.arange(k), 50).astype(np.uint32)
+    pins = np.empty((len(which), 2), np.uint32)
+    pins[:, 0] = which * 50 + rng.integers(0, 50, len(which))
+    pins[:, 1] = (k - 1) * 50 + rng.integers(0, 50, len(which))
+    hg = O.HG(len(part), 2 * np.arange(len(which) + 1), pins.ravel(), np.zeros(len(which)),
+              (rng.random(len(which)) * 10.0 ** rng.integers(-6, 6, len(which))).astype(np.float32))
+    check(dev, hg, part)
+
+
 def test_quotient_of_a_partition_from_the_pipeline(dev, rng):
     n, off, pins, srcc, w = gen.snn_like(6, 800, 12, rng)
     prod = H.Hypergraph.from_csr(n, off, pins, srcc, w, dedup=True)
