@@ -191,10 +191,10 @@ __global__ void k_q_member_keys(const uint32_t* __restrict__ rep, const uint64_t
 }
 
 // Per merged hedge: its sizes, and its weight, the sum of its members' in hedge order, one after the
-// other.  A few partitions merge thousands of hedges into one: a thread per merged hedge waited for
-// two dependent loads per member (200k nodes cut in 64: 444 us, now 134 us).  A wave takes Q_META_GROUPS merged hedges: those of a
-// few members a lane each, the others together -- the lanes load 64 members' weights, the next 64
-// on their way, and the sum goes through them by lane.
+// other.  A few partitions merge thousands of hedges into one, and a thread per merged hedge waits
+// for two dependent loads per member (200k nodes cut in 64: 444 us).  A wave takes Q_META_GROUPS
+// merged hedges: those of a few members a lane each, the others together -- the lanes load 64
+// members' weights, the next 64 on their way, and the sum goes through them by lane (134 us).
 constexpr uint32_t Q_META_GROUPS = 16, Q_META_FEW = 8;
 
 __global__ void __launch_bounds__(256)

@@ -2434,6 +2434,7 @@ struct CascadeArgs {
   const uint32_t* srcc;
   unsigned long long* dio;
   uint32_t V;  // ranks
+  uint32_t copies;  // 1, or CAS_COPIES arrays of V terms each behind seq (and dio), to be summed
 };
 constexpr uint32_t PM2_MAX_K = 0xFFFFu;  // partition ids < 0xFFFF leave 0xFFFF for "no move"
 
@@ -2515,6 +2516,33 @@ __device__ __forceinline__ void cas_clear(uint32_t V) {
     for (uint32_t i = threadIdx.x; i < (INCC ? 2 * V : V); i += blockDim.x) s_cas_acc[i] = 0;
     __syncthreads();
   }
+}
+// More ranks (inbound-constrained mode, up to CAS_COPY_V): a copy of the counters for each XCD
+// (workgroups go round them), so that an addition finds its line in the XCD's own L2 instead of
+// fetching it from another's; k_cascade_sum adds the copies up.  k_cascade_wave on the 65-pin hedges
+// of 8 layers of 1,156 nodes 73 -> 32 us, of 8,191 nodes 216 -> 148 us.  In k-way mode a rank is met
+// by a few hedges only, and copies changed nothing up to 262,144 ranks (183 and 181 us); above that
+// their clearing and summing is memory traffic of the size of the pins'.
+constexpr uint32_t CAS_COPIES = 8, CAS_COPY_V = 1u << 18;
+template <bool INCC>
+__device__ __forceinline__ void cas_own_copy(CascadeArgs& a) {
+  if (!INCC || a.copies == 1) return;
+  const uint64_t at = (uint64_t)(blockIdx.x % CAS_COPIES) * a.V;
+  a.seq += at;
+  a.dio += at;
+}
+__global__ void k_cascade_sum(const unsigned long long* __restrict__ seqs, const unsigned long long* __restrict__ dios,
+                              uint32_t V, unsigned long long* __restrict__ seq, unsigned long long* __restrict__ dio) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= V) return;
+  unsigned long long s = 0, d = 0;
+#pragma unroll
+  for (uint32_t q = 0; q < CAS_COPIES; ++q) {
+    s += seqs[(uint64_t)q * V + i];
+    d += dios[(uint64_t)q * V + i];
+  }
+  seq[i] = s;
+  dio[i] = d;
 }
 template <bool ACC>
 __device__ __forceinline__ void cas_add(const CascadeArgs& a, uint32_t r, int64_t term) {
@@ -2648,6 +2676,7 @@ __device__ __forceinline__ void cascade_small_hedge(const CascadeArgs& a, const 
 }
 template <bool P16, bool INCC, bool ACC>
 __global__ void k_cascade_small(CascadeArgs a, SmallHedges h) {
+  cas_own_copy<INCC>(a);
   cas_clear<INCC, ACC>(a.V);
   const uint32_t blocks = (h.m + blockDim.x - 1) / blockDim.x;  // ACC: the grid strides over them
   for (uint32_t b = blockIdx.x; b < blocks; b += gridDim.x)
@@ -2725,6 +2754,7 @@ __device__ __forceinline__ void cascade_wave_hedge(const CascadeArgs& a, uint32_
 }
 template <bool INCC, bool ACC>
 __global__ void __launch_bounds__(256) k_cascade_wave(CascadeArgs a, const uint32_t* __restrict__ list, uint32_t m) {
+  cas_own_copy<INCC>(a);
   cas_clear<INCC, ACC>(a.V);
   for (uint32_t b = blockIdx.x * 4 + threadIdx.x / 64; b < m; b += gridDim.x * 4) {
     const uint32_t e = (uint32_t)__builtin_amdgcn_readfirstlane((int)list[b]);
@@ -2761,6 +2791,7 @@ __global__ __launch_bounds__(256) void k_cascade_small_bytes(CascadeArgs a, Smal
 // INCC: as in k_cascade_small.
 template <bool INCC>
 __global__ void __launch_bounds__(64) k_cascade_large(CascadeArgs a, const uint32_t* __restrict__ list) {
+  cas_own_copy<INCC>(a);
   __shared__ uint32_t s_pt[CAS_LDS], s_mv[CAS_LDS], s_rk[CAS_LDS];
   const uint32_t e = list[blockIdx.x];
   const uint32_t l = lane_id();
@@ -2858,6 +2889,7 @@ __global__ void __launch_bounds__(NT) k_cascade_sorted(CascadeArgs a, const uint
   __shared__ int32_t s_cp[PINS], s_cq[PINS];
   __shared__ uint8_t s_out[INCC ? PINS : 1], s_in[INCC ? PINS : 1];  // the hedge leaves / enters an inbound set
   __shared__ uint32_t s_moving;
+  cas_own_copy<INCC>(a);
   const uint32_t e = list[blockIdx.x];
   const uint32_t l = lane_id(), tid = threadIdx.x;
   const uint64_t s = a.hoff[e];
@@ -3851,9 +3883,21 @@ bool try_analyze_round(Ctx& c, const RefineLevel& L, int mode, uint32_t omega, u
   // the side_streams tuning, the sorted and direct classes on side streams beside the size
   // events (all classes add their terms to seq and dio with atomics; the node records stay
   // alive until the join before they are read).
+  // few ranks: the counters in LDS (see cas_add); more, in inbound-constrained mode: a copy for each
+  // XCD (see cas_own_copy)
+  const uint64_t acc_lds = (uint64_t)V * (incc ? 16u : 8u);
+  const bool acc = acc_lds <= CAS_ACC_BYTES, copied = incc && !acc && V <= CAS_COPY_V;
+  const uint64_t copy_n = (uint64_t)CAS_COPIES * V;
+  DBuf<unsigned long long> copies(c, copied ? 2 * copy_n : 0);
+  if (copied) fill_u32(c, (uint32_t*)copies.get(), 0u, 2 * copies.n);
   std::optional<Fork> cas_fork;
   {
-    CascadeArgs a{L.hedges, L.hoff, L.w, pm.get(), pm2.get(), incc ? 1 : 0, st.seq.get(), L.srcc, dio.get(), V};
+    CascadeArgs a{L.hedges, L.hoff, L.w, pm.get(), pm2.get(), incc ? 1 : 0, st.seq.get(), L.srcc, dio.get(), V, 1};
+    if (copied) {
+      a.seq = copies.get();
+      a.dio = copies.get() + copy_n;
+      a.copies = CAS_COPIES;
+    }
     const int crb = std::max(1, bit_width(V));  // rank + 1 <= V
     const int cpb = std::max(1, bit_width(L.k));
     const uint32_t sort_max = cpb + crb + 11 < 64 ? CAS_SORT : 0u;
@@ -3883,9 +3927,6 @@ bool try_analyze_round(Ctx& c, const RefineLevel& L, int mode, uint32_t omega, u
         Y.cs = small_csr(c, kc.get(), m, L.hoff, L.hedges, L.w, incc ? L.srcc : nullptr);
       }
     }
-    // few ranks: the counters in LDS (see cas_add)
-    const uint32_t acc_lds = V * (incc ? 16u : 8u);
-    const bool acc = acc_lds <= CAS_ACC_BYTES;
     // runs f with compile-time (INCC, ACC)
     auto with_modes = [&](auto&& f) {
       if (incc && acc) f(std::true_type{}, std::true_type{});
@@ -3930,13 +3971,19 @@ bool try_analyze_round(Ctx& c, const RefineLevel& L, int mode, uint32_t omega, u
     }
     if (early) small_cascade();
   }
+  auto join_cascade = [&] {  // the main stream waits for the cascade's side streams
+    cas_fork.reset();
+    if (copied)
+      HGP_LAUNCH(k_cascade_sum, ceil_div(V, 256), 256, 0, c, copies.get(), copies.get() + copy_n, V, st.seq.get(),
+                 dio.get());
+  };
   const int rb = std::max(1, bit_width(V - 1));
   const int kb = std::max(1, bit_width(L.k));
   // inbound events: partition, hedge and rank in one 64-bit word; larger levels are refused
   const int eb = std::max(1, bit_width(L.e));
   HGP_REQUIRE(!incc || kb + eb + rb <= 64, HGP_E_CAPACITY, "inbound events: key exceeds 64 bits");
   if (fused) {
-    cas_fork.reset();  // the main stream waits for the cascade's side streams
+    join_cascade();
     DBuf<RoundOut> out(c, 1);
     const EventArgs ea{part, st.moves.get(), st.ranks.get(), L.sizes, psizes, pl.inbsz.get(), dio.get(), info.get(), n,
                        omega, delta, rb, kb, (int64_t*)st.seq.get(), st.sv.get(), st.iv.get(), out.get()};
@@ -3971,7 +4018,7 @@ bool try_analyze_round(Ctx& c, const RefineLevel& L, int mode, uint32_t omega, u
     HGP_LAUNCH(k_size_flags, ceil_div(m, 256), 256, 0, c, keys.get(), vals.get(), cum.get(), poff.get(), m, rb, psizes,
                omega, st.sv.get());
     inclusive_scan(c, st.sv.get(), st.sv.get(), V);
-    cas_fork.reset();  // the main stream waits for the cascade's side streams
+    join_cascade();
     if (incc) {
       HGP_LAUNCH(k_inbound_deltas, ceil_div(m, 256), 256, 0, c, keys.get(), dio.get(), m, rb, db, cum.get());
       inclusive_scan(c, cum.get(), cum.get(), m);

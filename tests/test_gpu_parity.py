@@ -513,6 +513,35 @@ def test_refine_analyze_inbound_by_hedge_size(dev, k, dup, rng):
     assert dup or got["best"] == exp["best"]
 
 
+@pytest.mark.parametrize("n", [1, 2, 65, 1024, 1025, 2048, 2049, 4096, 4097, 8192, 8193])
+@pytest.mark.parametrize("mode,k", [(1, 40), (0, 40), (1, 3000), (0, 3000)])
+def test_refine_analyze_by_level_size(dev, n, mode, k, rng):
+    """Levels at the edges of the one-workgroup ranking (8,192 nodes) and events (4,096), of their
+    items per thread and of the ranks whose counters fit LDS; partitions by table and by scan."""
+    lens = np.minimum(np.concatenate([rng.integers(1, 18, size=2 * n), rng.integers(17, 130, size=min(n, 200))]), n)
+    off = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint64)
+    start, step = rng.integers(0, n, size=len(lens)), 1 + 2 * rng.integers(0, 50, size=len(lens))
+    pos = np.arange(int(off[-1])) - np.repeat(off[:-1].astype(np.int64), lens)
+    pins = ((np.repeat(start, lens) + pos * np.repeat(step, lens)) % n).astype(np.uint32)
+    srcc = np.minimum(rng.integers(0, 3, size=len(lens)), lens - 1).astype(np.uint32)
+    hg = O.dedup(O.HG(n, off, pins, srcc, (rng.random(len(lens)) + 0.5).astype(np.float32)))
+    sizes = rng.integers(1, 4, size=n).astype(np.uint32)
+    part = rng.integers(0, k, size=n).astype(np.uint32)
+    psizes = np.bincount(part, weights=sizes, minlength=k).astype(np.uint32)
+    omega, delta = int(psizes.max()) + 3, 2**31 - 1
+    if mode == 0:
+        delta = max(1, int(O.inbound_sizes(hg, part, k).max()) - 1)
+    L = G.Level(dev, hg)
+    L.build_touching()
+    ro, rt, ri = O.touching(hg)
+    for chainup in (False, True):
+        got = G.refine_analyze(dev, L, sizes, k, mode, omega, delta, 16, 0, chainup, part, psizes)
+        exp = O.refine_analyze(mode, omega, delta, 16, hg, ro, rt, ri, sizes, k, 0, chainup, part, psizes)
+        for key in ("moves", "gains", "ranks", "seq", "sv", "iv"):
+            assert np.array_equal(got[key], exp[key]), f"{key} differs (chainup={chainup})"
+        assert got["best"] == exp["best"]
+
+
 @pytest.mark.parametrize("rc", REFINE_CASES, ids=[r[0] for r in REFINE_CASES])
 def test_refine_loop(dev, rc, rng):
     name, mode, k, case_name = rc
