@@ -98,17 +98,20 @@ __global__ void __launch_bounds__(256) k_visit_bound_heavy(const uint64_t* __res
   }
 }
 
-// candidate key = (final score << 32) | v, or 0 when v is filtered out
-__device__ __forceinline__ uint64_t cand_key(uint32_t u, uint32_t v, uint32_t score, uint32_t inter, uint32_t size_u,
-                                             uint32_t inb_u, const uint32_t* __restrict__ sizes,
-                                             const uint32_t* __restrict__ inb, uint32_t omega, uint32_t delta) {
-  if ((uint32_t)(size_u + sizes[v]) > omega) return 0;
-  if ((uint32_t)((inb[v] - inter) + inb_u) > delta) return 0;
-  const uint32_t s = score + noise64(u, v);
-  if (s == 0) return 0;
-  return ((uint64_t)s << 32) | v;
+// What ranking reads of a node: (size, inbound count) in one word pair.
+__global__ void k_node_records(const uint32_t* __restrict__ sizes, const uint32_t* __restrict__ inb, uint32_t n,
+                               uint2* __restrict__ rec) {
+  const uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
+  if (v < n) rec[v] = make_uint2(sizes[v], inb[v]);
 }
 
+// candidate key = (final score << 32) | v, or 0 when v is filtered out; r: v's record
+__device__ __forceinline__ uint64_t cand_key(uint32_t u, uint32_t v, uint32_t score, uint32_t inter, uint2 ru, uint2 r,
+                                             uint32_t omega, uint32_t delta) {
+  const uint32_t s = score + noise64(u, v);
+  const bool drop = (uint32_t)(ru.x + r.x) > omega || (uint32_t)((r.y - inter) + ru.y) > delta || s == 0;
+  return drop ? 0ull : ((uint64_t)s << 32) | v;
+}
 
 // k >> b, 0 for b >= 64
 __device__ __forceinline__ uint64_t shr64(uint64_t k, uint32_t b) { return b >= 64 ? 0ull : k >> b; }
@@ -123,7 +126,7 @@ template <bool INTER, uint32_t CAP = CAND_CAP, uint32_t NW = 4>
 __global__ void __launch_bounds__(64 * NW) k_cand_light(const uint32_t* __restrict__ hedges, const uint64_t* __restrict__ hoff,
                                                     const uint32_t* __restrict__ srcc, const uint32_t* __restrict__ tch,
                                                     const uint64_t* __restrict__ toff, const uint32_t* __restrict__ inb,
-                                                    const float* __restrict__ w, const uint32_t* __restrict__ sizes,
+                                                    const float* __restrict__ w, const uint2* __restrict__ nrec,
                                                     const uint32_t* __restrict__ list, uint32_t nlist,
                                                     const uint64_t* __restrict__ bound, uint32_t cnc, uint32_t omega,
                                                     uint32_t delta, uint32_t* __restrict__ pairs,
@@ -167,14 +170,25 @@ __global__ void __launch_bounds__(64 * NW) k_cand_light(const uint32_t* __restri
   }, [] { return false; });
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-  const uint32_t size_u = sizes[u];
+  const uint2 ru = nrec[u];
+  // the records of all slots are loaded together, whether the slot is used or not: a size and an
+  // inbound count per used slot, each behind the test of the one before, were the longest chain of
+  // the kernel (800k nodes: the 1024-slot instance 650 -> 451 us, the 512-slot one 600 -> 505 us)
   uint64_t cand[SLOTS];
+  uint32_t id[SLOTS];
+  uint2 rec[SLOTS];
 #pragma unroll
   for (uint32_t s = 0; s < SLOTS; ++s) {
     const uint32_t slot = l + 64 * s;
-    const uint32_t v = slot < cap ? keys[slot] : NONE;
-    cand[s] = v == NONE ? 0ull
-                        : cand_key(u, v, score[slot], INTER ? inter[slot] : 0u, size_u, inb_u, sizes, inb, omega, delta);
+    id[s] = slot < cap ? keys[slot] : NONE;
+  }
+#pragma unroll
+  for (uint32_t s = 0; s < SLOTS; ++s) rec[s] = nrec[id[s] != NONE ? id[s] : u];
+#pragma unroll
+  for (uint32_t s = 0; s < SLOTS; ++s) {
+    const uint32_t slot = l + 64 * s;
+    const uint64_t k = cand_key(u, id[s], score[slot], INTER ? inter[slot] : 0u, ru, rec[s], omega, delta);
+    cand[s] = id[s] != NONE ? k : 0ull;
   }
   // The top cnc keys by a radix select (as block_select_write, for one wave): the keys are in
   // registers now, so the table's score array holds the histogram (CAP >= 128 bins) and its
@@ -571,11 +585,16 @@ __global__ void k_heavy_max_cap(const uint32_t* __restrict__ heavy, const uint32
   if (lane_id() == 0) atomicMax(out, m);
 }
 
+constexpr uint32_t RANK_BATCH = 8;
+
 // Scores one node with a whole workgroup of NW waves: the waves split its touching hedges
 // and insert into the table, then every entry is ranked.  The table is LDS or the block's
 // HBM region (GMEM).  Hashed: keys[] holds node ids.  Direct (cap == level size): slot = node
 // id and keys[] is a presence bitmap.  INTER keeps the shared-inbound counts that the
 // inbound-union filter needs; without it (Delta >= twice the hedge count) they are 0.
+//
+// Ranking loads RANK_BATCH slots' records together (see k_cand_light; k_cand_medium<2048> at 800k
+// nodes 950 -> 826 us).
 //
 // OPT (optimistic): the node's distinct neighbours may exceed the table.  New keys are
 // counted; past `limit` the workgroup stops and the caller hands the node to a larger table.  At most one insert per thread is in flight when
@@ -589,14 +608,14 @@ __device__ __forceinline__ bool cand_block_node(uint32_t u, uint32_t cap, bool d
                                                 const uint64_t* __restrict__ hoff, const uint32_t* __restrict__ srcc,
                                                 const uint32_t* __restrict__ tch, const uint64_t* __restrict__ toff,
                                                 const uint32_t* __restrict__ inb, const float* __restrict__ w,
-                                                const uint32_t* __restrict__ sizes, uint32_t cnc, uint32_t omega,
+                                                const uint2* __restrict__ nrec, uint32_t cnc, uint32_t omega,
                                                 uint32_t delta, uint32_t* __restrict__ pairs,
                                                 uint32_t* __restrict__ scores, uint64_t* s_w,
                                                 uint32_t* s_state = nullptr, uint32_t limit = 0) {
   const uint32_t nkeys = direct ? (cap + 31) / 32 : cap;
   const uint64_t t0 = toff[u], t1 = toff[u + 1];
   const uint32_t inb_u = inb[u];
-  const uint32_t size_u = sizes[u];
+  const uint2 ru = nrec[u];
   const uint32_t wv = threadIdx.x / 64;
   const uint64_t cnt = t1 - t0;
   const uint64_t a = t0 + cnt * wv / NW, b = t0 + cnt * (wv + 1) / NW;
@@ -656,18 +675,25 @@ __device__ __forceinline__ bool cand_block_node(uint32_t u, uint32_t cap, bool d
     if constexpr (SELECT) {
       // each slot's key, its high word written over the score (0: no candidate)
       uint64_t kmax = 0;
-      for (uint32_t s = threadIdx.x; s < cap; s += blockDim.x) {
-        uint32_t v;
-        if (direct) {
-          if (!((keys[s >> 5] >> (s & 31u)) & 1u)) continue;
-          v = s;
-        } else {
-          v = keys[s];
-          if (v == NONE) continue;
+      for (uint32_t s0 = threadIdx.x; s0 < cap; s0 += RANK_BATCH * 64 * NW) {
+        uint32_t id[RANK_BATCH];
+        uint2 rec[RANK_BATCH];
+#pragma unroll
+        for (uint32_t q = 0; q < RANK_BATCH; ++q) {
+          const uint32_t s = s0 + q * 64 * NW;
+          id[q] = NONE;
+          if (s < cap) id[q] = !direct ? keys[s] : (keys[s >> 5] >> (s & 31u)) & 1u ? s : NONE;
         }
-        const uint64_t k = cand_key(u, v, score[s], INTER ? inter[s] : 0u, size_u, inb_u, sizes, inb, omega, delta);
-        score[s] = (uint32_t)(k >> 32);
-        kmax = k > kmax ? k : kmax;
+#pragma unroll
+        for (uint32_t q = 0; q < RANK_BATCH; ++q) rec[q] = nrec[id[q] != NONE ? id[q] : u];
+#pragma unroll
+        for (uint32_t q = 0; q < RANK_BATCH; ++q) {
+          const uint32_t s = s0 + q * 64 * NW;
+          if (id[q] == NONE) continue;
+          const uint64_t k = cand_key(u, id[q], score[s], INTER ? inter[s] : 0u, ru, rec[q], omega, delta);
+          score[s] = (uint32_t)(k >> 32);
+          kmax = k > kmax ? k : kmax;
+        }
       }
       block_select_write<NW>(cap, direct, keys, score, kmax, cnc, u, pairs, scores, (SelectScratch*)s_w);
       return true;
@@ -681,7 +707,7 @@ __device__ __forceinline__ bool cand_block_node(uint32_t u, uint32_t cap, bool d
         v = keys[s];
         if (v == NONE) continue;
       }
-      top_insert(top, cand_key(u, v, score[s], INTER ? inter[s] : 0u, size_u, inb_u, sizes, inb, omega, delta));
+      top_insert(top, cand_key(u, v, score[s], INTER ? inter[s] : 0u, ru, nrec[v], omega, delta));
     }
     // the pin ids visited; per touching hedge its list entry, offsets, weight (and source count)
     if (CH > 1) __syncthreads();  // the next pass clears the table
@@ -693,7 +719,7 @@ __device__ __forceinline__ bool cand_block_node(uint32_t u, uint32_t cap, bool d
 #define CAND_ARGS                                                                                                   \
   const uint32_t *__restrict__ hedges, const uint64_t *__restrict__ hoff, const uint32_t *__restrict__ srcc,        \
       const uint32_t *__restrict__ tch, const uint64_t *__restrict__ toff, const uint32_t *__restrict__ inb,        \
-      const float *__restrict__ w, const uint32_t *__restrict__ sizes, const uint32_t *__restrict__ list,           \
+      const float *__restrict__ w, const uint2 *__restrict__ nrec, const uint32_t *__restrict__ list,               \
       const uint32_t *__restrict__ caps, uint32_t cnc, uint32_t omega, uint32_t delta, uint32_t *__restrict__ pairs, \
       uint32_t *__restrict__ scores
 
@@ -708,7 +734,7 @@ __global__ void __launch_bounds__(64 * NW) k_cand_medium(CAND_ARGS) {
   __shared__ uint64_t s_w[SELECT_WORDS];
   const uint32_t u = list[xcd_block(blockIdx.x, gridDim.x)];
   cand_block_node<false, INTER, NW>(u, caps[u], false, s_keys, s_score, s_inter, hedges, hoff, srcc, tch, toff, inb, w,
-                                    sizes, cnc, omega, delta, pairs, scores, s_w);
+                                    nrec, cnc, omega, delta, pairs, scores, s_w);
 }
 
 // One node per 1024-thread workgroup with a hashed LDS table of up to CAND_BIG_SLOTS.
@@ -721,7 +747,7 @@ __global__ void __launch_bounds__(1024) k_cand_big(CAND_ARGS) {
   __shared__ uint64_t s_w[256];
   const uint32_t u = list[xcd_block(blockIdx.x, gridDim.x)];
   cand_block_node<false, INTER, 16>(u, caps[u], false, s_keys, s_score, s_inter, hedges, hoff, srcc, tch, toff, inb,
-                                    w, sizes, cnc, omega, delta, pairs, scores, s_w);
+                                    w, nrec, cnc, omega, delta, pairs, scores, s_w);
 }
 
 // One node per 1024-thread workgroup with a hashed LDS table of CAND_BIG8_SLOTS (64 KB, no
@@ -733,7 +759,7 @@ __global__ void __launch_bounds__(1024) k_cand_big8(CAND_ARGS) {
   __shared__ uint64_t s_w[256];
   const uint32_t u = list[xcd_block(blockIdx.x, gridDim.x)];
   cand_block_node<false, false, 16>(u, caps[u], false, s_keys, s_score, s_inter, hedges, hoff, srcc, tch, toff, inb, w,
-                                    sizes, cnc, omega, delta, pairs, scores, s_w);
+                                    nrec, cnc, omega, delta, pairs, scores, s_w);
 }
 
 // Nodes whose worst-case table exceeds LDS: try the largest LDS table that fits (their
@@ -759,7 +785,7 @@ __global__ void __launch_bounds__(1024) k_cand_opt(CAND_ARGS, uint32_t* __restri
   __shared__ uint32_t s_state[2];
   const uint32_t u = list[xcd_block(blockIdx.x, gridDim.x)];
   const bool done = cand_block_node<false, INTER, 16, true, false, CH>(u, SLOTS, false, s_keys, s_score, s_inter,
-                                                                       hedges, hoff, srcc, tch, toff, inb, w, sizes,
+                                                                       hedges, hoff, srcc, tch, toff, inb, w, nrec,
                                                                        cnc, omega, delta, pairs, scores, s_w, s_state,
                                                                        LIMIT);
   if (!done && threadIdx.x == 0) ovf[atomicAdd(ovf_count, 1u)] = u;
@@ -778,7 +804,7 @@ __global__ void __launch_bounds__(1024) k_cand_direct(CAND_ARGS) {
   // without the pipelined traversal: with it this kernel measured no faster (its occupancy is
   // set by the LDS score array)
   cand_block_node<false, INTER, 16, false, true, 1, false>(u, caps[u], true, s_bits, s_score, s_inter, hedges, hoff,
-                                                           srcc, tch, toff, inb, w, sizes, cnc, omega, delta, pairs,
+                                                           srcc, tch, toff, inb, w, nrec, cnc, omega, delta, pairs,
                                                            scores, s_w);
 }
 
@@ -803,12 +829,12 @@ __global__ void __launch_bounds__(256) k_cand_heavy(CAND_ARGS, uint32_t nlist, u
     const uint32_t cap = caps[u];
     if (try_cap == 0 || cap <= try_cap) {
       cand_block_node<true, true, 4>(u, cap, cap == n, keys, score, inter, hedges, hoff, srcc, tch, toff, inb, w,
-                                     sizes, cnc, omega, delta, pairs, scores, s_w);
+                                     nrec, cnc, omega, delta, pairs, scores, s_w);
     } else if (cap == n) {
       if (threadIdx.x == 0) ovf[atomicAdd(ovf_count, 1u)] = u;
     } else {
       const bool done = cand_block_node<true, true, 4, true>(u, try_cap, false, keys, score, inter, hedges, hoff, srcc,
-                                                             tch, toff, inb, w, sizes, cnc, omega, delta, pairs,
+                                                             tch, toff, inb, w, nrec, cnc, omega, delta, pairs,
                                                              scores, s_w, s_state, try_fill);
       if (!done && threadIdx.x == 0) ovf[atomicAdd(ovf_count, 1u)] = u;
       __syncthreads();  // s_state is reused by the next node
@@ -1225,6 +1251,9 @@ void candidates(Ctx& c, const uint32_t* hedges, const uint64_t* hoff, const uint
                  nb = cnt.n[6], nd = cnt.n[7], nh = cnt.n[8];
   const uint32_t *small = tl[0], *mid = tl[1], *light = tl[2], *med_s = tl[3], *med = tl[4], *big8 = tl[5],
                  *big = tl[6], *direct = tl[7], *heavy = tl[8];
+  DBuf<uint2> node_rec(c, n);
+  const uint2* nrec = node_rec.get();
+  HGP_LAUNCH(k_node_records, g, 256, 0, c, sizes, inb, n, node_rec.get());
   // the tiers write disjoint rows of pairs and scores: light and medium nodes on side streams
   // beside the big and heavy ones (which allocate, so they stay on the main stream)
   Fork fk(c, c.tune.side_streams & 1u);
@@ -1232,25 +1261,25 @@ void candidates(Ctx& c, const uint32_t* hedges, const uint64_t* hoff, const uint
     // visit bounds up to CAND_LIGHT_S: 128-slot tables, 8 waves per workgroup
     if (inter)
       HGP_LAUNCH((k_cand_light<true, 2 * CAND_LIGHT_S, 8>), ceil_div(ns, 8), 512, 0, c, hedges, hoff, srcc, tch, toff,
-                 inb, w, sizes, small, ns, bound.get(), cnc, omega, delta, pairs, scores);
+                 inb, w, nrec, small, ns, bound.get(), cnc, omega, delta, pairs, scores);
     else
       HGP_LAUNCH((k_cand_light<false, 2 * CAND_LIGHT_S, 8>), ceil_div(ns, 8), 512, 0, c, hedges, hoff, srcc, tch, toff,
-                 inb, w, sizes, small, ns, bound.get(), cnc, omega, delta, pairs, scores);
+                 inb, w, nrec, small, ns, bound.get(), cnc, omega, delta, pairs, scores);
     if (inter)
       HGP_LAUNCH((k_cand_light<true, 2 * CAND_LIGHT_M, 8>), ceil_div(nmid, 8), 512, 0, c, hedges, hoff, srcc, tch,
-                 toff, inb, w, sizes, mid, nmid, bound.get(), cnc, omega, delta, pairs, scores);
+                 toff, inb, w, nrec, mid, nmid, bound.get(), cnc, omega, delta, pairs, scores);
     else
       HGP_LAUNCH((k_cand_light<false, 2 * CAND_LIGHT_M, 8>), ceil_div(nmid, 8), 512, 0, c, hedges, hoff, srcc, tch,
-                 toff, inb, w, sizes, mid, nmid, bound.get(), cnc, omega, delta, pairs, scores);
+                 toff, inb, w, nrec, mid, nmid, bound.get(), cnc, omega, delta, pairs, scores);
     if (inter)
-      HGP_LAUNCH(k_cand_light<true>, ceil_div(nl, 4), 256, 0, c, hedges, hoff, srcc, tch, toff, inb, w, sizes,
+      HGP_LAUNCH(k_cand_light<true>, ceil_div(nl, 4), 256, 0, c, hedges, hoff, srcc, tch, toff, inb, w, nrec,
                  light, nl, bound.get(), cnc, omega, delta, pairs, scores);
     else
-      HGP_LAUNCH(k_cand_light<false>, ceil_div(nl, 4), 256, 0, c, hedges, hoff, srcc, tch, toff, inb, w, sizes,
+      HGP_LAUNCH(k_cand_light<false>, ceil_div(nl, 4), 256, 0, c, hedges, hoff, srcc, tch, toff, inb, w, nrec,
                  light, nl, bound.get(), cnc, omega, delta, pairs, scores);
   });
 #define CAND_LAUNCH(K, list, cnt, threads)                                                                          \
-  HGP_LAUNCH(K, cnt, threads, 0, c, hedges, hoff, srcc, tch, toff, inb, w, sizes, list, caps.get(), cnc, omega, delta, \
+  HGP_LAUNCH(K, cnt, threads, 0, c, hedges, hoff, srcc, tch, toff, inb, w, nrec, list, caps.get(), cnc, omega, delta, \
              pairs, scores)
   fk.on(1, [&] {
     if (inter) CAND_LAUNCH((k_cand_medium<true, CAND_MED_S>), med_s, nms, 256);
@@ -1273,10 +1302,10 @@ void candidates(Ctx& c, const uint32_t* hedges, const uint64_t* hoff, const uint
   DBuf<uint32_t> ovf(c, nh), novf(c, 1);
   memset_async(c, novf.get(), 0, 4);
   if (inter)
-    HGP_LAUNCH((k_cand_opt<true, 1>), nh, 1024, 0, c, hedges, hoff, srcc, tch, toff, inb, w, sizes, heavy,
+    HGP_LAUNCH((k_cand_opt<true, 1>), nh, 1024, 0, c, hedges, hoff, srcc, tch, toff, inb, w, nrec, heavy,
                caps.get(), cnc, omega, delta, pairs, scores, ovf.get(), novf.get());
   else
-    HGP_LAUNCH((k_cand_opt<false, 1>), nh, 1024, 0, c, hedges, hoff, srcc, tch, toff, inb, w, sizes, heavy,
+    HGP_LAUNCH((k_cand_opt<false, 1>), nh, 1024, 0, c, hedges, hoff, srcc, tch, toff, inb, w, nrec, heavy,
                caps.get(), cnc, omega, delta, pairs, scores, ovf.get(), novf.get());
   uint32_t no = read_scalar(c, novf.get());
   const uint32_t no1 = no;
@@ -1285,10 +1314,10 @@ void candidates(Ctx& c, const uint32_t* hedges, const uint64_t* hoff, const uint
     DBuf<uint32_t> ovf_b(c, no);
     memset_async(c, novf.get(), 0, 4);
     if (inter)
-      HGP_LAUNCH((k_cand_opt<true, OPT_CHUNKS>), no, 1024, 0, c, hedges, hoff, srcc, tch, toff, inb, w, sizes, ovf.get(),
+      HGP_LAUNCH((k_cand_opt<true, OPT_CHUNKS>), no, 1024, 0, c, hedges, hoff, srcc, tch, toff, inb, w, nrec, ovf.get(),
                  caps.get(), cnc, omega, delta, pairs, scores, ovf_b.get(), novf.get());
     else
-      HGP_LAUNCH((k_cand_opt<false, OPT_CHUNKS>), no, 1024, 0, c, hedges, hoff, srcc, tch, toff, inb, w, sizes,
+      HGP_LAUNCH((k_cand_opt<false, OPT_CHUNKS>), no, 1024, 0, c, hedges, hoff, srcc, tch, toff, inb, w, nrec,
                  ovf.get(), caps.get(), cnc, omega, delta, pairs, scores, ovf_b.get(), novf.get());
     no = read_scalar(c, novf.get());
     ovf = std::move(ovf_b);
@@ -1312,7 +1341,7 @@ void candidates(Ctx& c, const uint32_t* hedges, const uint64_t* hoff, const uint
     const uint64_t region = read_scalar(c, mc.get());
     const uint64_t grid = std::max<uint64_t>(1, std::min<uint64_t>({(uint64_t)cntl, HEAVY_TABLE_SLOTS / region, 4096}));
     DBuf<uint32_t> gk(c, grid * region), gs(c, grid * region), gi(c, grid * region);
-    HGP_LAUNCH(k_cand_heavy, (uint32_t)grid, 256, 0, c, hedges, hoff, srcc, tch, toff, inb, w, sizes, lst, caps.get(),
+    HGP_LAUNCH(k_cand_heavy, (uint32_t)grid, 256, 0, c, hedges, hoff, srcc, tch, toff, inb, w, nrec, lst, caps.get(),
                cnc, omega, delta, pairs, scores, cntl, n, region, gk.get(), gs.get(), gi.get(), try_cap, try_fill, ovf2.get(),
                novf2.get());
     if (c.verbose >= 2)
