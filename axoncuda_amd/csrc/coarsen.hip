@@ -354,7 +354,7 @@ __device__ __forceinline__ void block_top_write(uint64_t (&top)[TOPN], uint32_t 
 // Exact top-cnc (cnc <= 16) of the candidate keys of a node's LDS table, written to the
 // node's pairs/scores in descending key order (NONE / 0 past the candidates).  Slot s holds
 // its key's high word in hi[s] (0: no candidate) and its low word (the neighbour id) in
-// keys[s], or s itself when the table is indexed by node id.  Keys are distinct (they embed
+// keys[s], or s itself when the table is indexed by node id; slots are STRIDE words apart in hi.  Keys are distinct (they embed
 // the neighbour id).  A radix select: each pass histograms the next 8 bits below those fixed
 // so far, over the keys that share the fixed bits, and fixes the bin that holds the cnc-th
 // largest key; it stops once every key of that bin is taken.  The first pass starts below
@@ -371,7 +371,7 @@ struct SelectScratch {
 };
 constexpr uint32_t SELECT_WORDS = (sizeof(SelectScratch) + 7) / 8;  // 8-byte words of the scratch
 static_assert(SELECT_WORDS <= 256, "the 1024-thread kernels' 256-word scratch holds a SelectScratch");
-template <int NW>
+template <int NW, uint32_t STRIDE = 1>
 __device__ __forceinline__ void block_select_write(uint32_t cap, bool direct, const uint32_t* keys, const uint32_t* hi,
                                                    uint64_t kmax, uint32_t cnc, uint32_t u,
                                                    uint32_t* __restrict__ pairs, uint32_t* __restrict__ scores,
@@ -380,7 +380,7 @@ __device__ __forceinline__ void block_select_write(uint32_t cap, bool direct, co
   constexpr uint32_t B = 64 * NW;
   const uint32_t tid = threadIdx.x, l = lane_id(), wv = tid / 64;
   auto key_at = [&](uint32_t s) -> uint64_t {
-    const uint32_t h = hi[s];
+    const uint32_t h = hi[STRIDE * s];
     return h ? ((uint64_t)h << 32) | (direct ? s : keys[s]) : 0ull;
   };
   kmax = wave_max(kmax);
@@ -513,7 +513,7 @@ __global__ void k_cand_tiers(const uint64_t* __restrict__ bound, uint32_t n, uin
       else if (c <= CAND_MED_CAP) t = 4;
       else if (c <= big8_cap) t = 5;
       else if (c <= big_cap) t = 6;  // hashed, on any level
-      else if (n <= direct_n) t = 7;
+      else if (n <= direct_n && b < 1ull << 31) t = 7;  // PACKED counts in 31 bits
       else t = 8;
       tier[v] = (uint8_t)t;
       // indexed by node id: the direct tier, and heavy nodes whose table would not be smaller than n;
@@ -599,10 +599,14 @@ constexpr uint32_t RANK_BATCH = 8;
 // OPT (optimistic): the node's distinct neighbours may exceed the table.  New keys are
 // counted; past `limit` the workgroup stops and the caller hands the node to a larger table.  At most one insert per thread is in flight when
 // the limit trips, so the table never fills.  Returns false when the node overflowed.
+// PACKED (direct, with shared-inbound counts, fewer than 2^31 visits): `score` holds one 64-bit word
+// per slot: the score in the high half, the shared-inbound count below it and, in bit 31, whether a
+// visit did not count.  A counted visit is one addition; a slot without visits has a zero low half
+// (k_cand_direct on 257-pin hedges, against a bitmap, a score and a count per visit: 2.44 -> 2.14 ms).
 // TOPN: length of the per-thread candidate lists, 16 unless every thread owns at most TOPN
 // table slots (then its list holds all of them).
 template <bool GMEM, bool INTER, int NW, bool OPT = false, bool P2 = true, int CH = 1, bool PIPE = true,
-          int TOPN = 16>
+          int TOPN = 16, bool PACKED = false>
 __device__ __forceinline__ bool cand_block_node(uint32_t u, uint32_t cap, bool direct, uint32_t* keys, uint32_t* score,
                                                 uint32_t* inter, const uint32_t* __restrict__ hedges,
                                                 const uint64_t* __restrict__ hoff, const uint32_t* __restrict__ srcc,
@@ -631,11 +635,17 @@ __device__ __forceinline__ bool cand_block_node(uint32_t u, uint32_t cap, bool d
   // CH > 1: the neighbours are split by id modulo CH and scored one class per pass, so the
   // table holds a CH-th of them; the per-thread top lists carry over between passes.
   for (int chunk = 0; chunk < CH; ++chunk) {
+    unsigned long long* acc = reinterpret_cast<unsigned long long*>(score);  // PACKED
     for (uint32_t s = threadIdx.x; s < cap; s += blockDim.x) {
+      if (PACKED) {
+        acc[s] = 0;
+        continue;
+      }
       score[s] = 0;
       if (INTER) inter[s] = 0;
     }
-    for (uint32_t s = threadIdx.x; s < nkeys; s += blockDim.x) keys[s] = direct ? 0u : NONE;
+    if (!PACKED)
+      for (uint32_t s = threadIdx.x; s < nkeys; s += blockDim.x) keys[s] = direct ? 0u : NONE;
     if (OPT && threadIdx.x == 0) {
       s_state[0] = 0;  // new keys
       s_state[1] = 0;  // overflow flag
@@ -643,12 +653,15 @@ __device__ __forceinline__ bool cand_block_node(uint32_t u, uint32_t cap, bool d
     if (GMEM) __threadfence();
     __syncthreads();
     auto hvf = [&](uint32_t e, uint32_t len) { return make_uint2(fixed_weight(w[e]) / len, INTER ? srcc[e] : 0u); };
-    wave_visit_pins_hv_until<PIPE>(tch, a, b, hoff, hedges, hvf, [&](const PinVisitHV& pv) {
+    wave_visit_pins_hv_until<PIPE, NW == 16>(tch, a, b, hoff, hedges, hvf, [&](const PinVisitHV& pv) {
       if (!pv.act || pv.pin == u) return;
       if (CH > 1 && pv.pin % CH != (uint32_t)chunk) return;
       const uint32_t contrib = pv.hv.x;  // floor(W / |e|), computed once per touching hedge
       const bool shared_in = INTER && (pv.j - t0) < inb_u && pv.pos >= pv.hv.y;
-      if (direct) {
+      if (PACKED) {
+        atomicAdd(&acc[pv.pin], ((unsigned long long)contrib << 32) | (shared_in ? 1u : 0u));
+        if (!shared_in) atomicOr(&score[2 * pv.pin], 1u << 31);
+      } else if (direct) {
         const uint32_t bit = 1u << (pv.pin & 31u);
         if (!(atomic_load_relaxed(&keys[pv.pin >> 5]) & bit)) atomicOr(&keys[pv.pin >> 5], bit);
         atomicAdd(&score[pv.pin], contrib);
@@ -682,7 +695,9 @@ __device__ __forceinline__ bool cand_block_node(uint32_t u, uint32_t cap, bool d
         for (uint32_t q = 0; q < RANK_BATCH; ++q) {
           const uint32_t s = s0 + q * 64 * NW;
           id[q] = NONE;
-          if (s < cap) id[q] = !direct ? keys[s] : (keys[s >> 5] >> (s & 31u)) & 1u ? s : NONE;
+          if (s >= cap) continue;
+          if (PACKED) id[q] = score[2 * s] ? s : NONE;
+          else id[q] = !direct ? keys[s] : (keys[s >> 5] >> (s & 31u)) & 1u ? s : NONE;
         }
 #pragma unroll
         for (uint32_t q = 0; q < RANK_BATCH; ++q) rec[q] = nrec[id[q] != NONE ? id[q] : u];
@@ -690,10 +705,16 @@ __device__ __forceinline__ bool cand_block_node(uint32_t u, uint32_t cap, bool d
         for (uint32_t q = 0; q < RANK_BATCH; ++q) {
           const uint32_t s = s0 + q * 64 * NW;
           if (id[q] == NONE) continue;
-          const uint64_t k = cand_key(u, id[q], score[s], INTER ? inter[s] : 0u, ru, rec[q], omega, delta);
-          score[s] = (uint32_t)(k >> 32);
+          uint32_t& sc = PACKED ? score[2 * s + 1] : score[s];
+          const uint32_t shared = PACKED ? score[2 * s] & 0x7FFFFFFFu : INTER ? inter[s] : 0u;
+          const uint64_t k = cand_key(u, id[q], sc, shared, ru, rec[q], omega, delta);
+          sc = (uint32_t)(k >> 32);
           kmax = k > kmax ? k : kmax;
         }
+      }
+      if constexpr (PACKED) {  // unvisited slots are zero in both words
+        block_select_write<NW, 2>(cap, true, nullptr, score + 1, kmax, cnc, u, pairs, scores, (SelectScratch*)s_w);
+        return true;
       }
       block_select_write<NW>(cap, direct, keys, score, kmax, cnc, u, pairs, scores, (SelectScratch*)s_w);
       return true;
@@ -796,16 +817,15 @@ __global__ void __launch_bounds__(1024) k_cand_opt(CAND_ARGS, uint32_t* __restri
 template <bool INTER>
 __global__ void __launch_bounds__(1024) k_cand_direct(CAND_ARGS) {
   constexpr uint32_t N = INTER ? CAND_DIRECT_N / 2 : CAND_DIRECT_N;
-  __shared__ uint32_t s_bits[N / 32];
-  __shared__ uint32_t s_score[N];
-  __shared__ uint32_t s_inter[INTER ? N : 1];
+  __shared__ uint32_t s_bits[INTER ? 1 : N / 32];
+  __shared__ alignas(8) uint32_t s_score[INTER ? 2 * N : N];
   __shared__ uint64_t s_w[256];
   const uint32_t u = list[xcd_block(blockIdx.x, gridDim.x)];
   // without the pipelined traversal: with it this kernel measured no faster (its occupancy is
   // set by the LDS score array)
-  cand_block_node<false, INTER, 16, false, true, 1, false>(u, caps[u], true, s_bits, s_score, s_inter, hedges, hoff,
-                                                           srcc, tch, toff, inb, w, nrec, cnc, omega, delta, pairs,
-                                                           scores, s_w);
+  cand_block_node<false, INTER, 16, false, true, 1, false, 16, INTER>(u, caps[u], true, s_bits, s_score, nullptr,
+                                                                      hedges, hoff, srcc, tch, toff, inb, w, nrec, cnc,
+                                                                      omega, delta, pairs, scores, s_w);
 }
 
 // Heavy nodes: a persistent grid, each workgroup owning `region` slots of HBM tables and

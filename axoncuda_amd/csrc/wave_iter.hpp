@@ -192,11 +192,16 @@ __device__ __forceinline__ void wave_visit_pins_until(const uint32_t* __restrict
 // The same traversal with two per-hedge values computed once per touching hedge by the lane
 // that loads it, `hvf(e, len)`, and handed to every visit of that hedge's pins in `hv`.  With
 // PIPE the next step's pin is loading while the current step is visited (one more step's
-// registers live across the visit).
+// registers live across the visit).  With LONG, a chunk of hedges of LONG_HEDGE pins on average goes
+// hedge by hedge instead: finding owners and fetching their fields is some 60 of a step's 80 vector
+// instructions, which bound the traversal, against part-filled steps at the hedges' ends.
+// k_cand_direct on 257-pin hedges 2.65 -> 2.44 ms; hedges of 65 pins, two steps for one, lose (253 ->
+// 353 us), so they stay below the line.
+constexpr uint32_t LONG_HEDGE = 128, LONG_STEPS = 4;
 struct PinVisitHV : PinVisit {
   uint2 hv;
 };
-template <bool PIPE = true, typename H, typename F, typename S>
+template <bool PIPE = true, bool LONG = false, typename H, typename F, typename S>
 __device__ __forceinline__ void wave_visit_pins_hv_until(const uint32_t* __restrict__ tch, uint64_t t0, uint64_t t1,
                                                          const uint64_t* __restrict__ hoff,
                                                          const uint32_t* __restrict__ hedges, H&& hvf, F&& visit,
@@ -213,6 +218,51 @@ __device__ __forceinline__ void wave_visit_pins_hv_until(const uint32_t* __restr
       s = hoff[e];
       len = (uint32_t)(hoff[e + 1] - s);
       hv = hvf(e, len);
+    }
+    const uint32_t m = (uint32_t)min((uint64_t)64, t1 - jb);
+    if (LONG && wave_sum((uint64_t)len) >= (uint64_t)LONG_HEDGE * m) {
+      // long hedges, one after the other: the hedge is uniform, so a step is a load and the visit.
+      // LONG_STEPS of the next hedge's loads are on their way during the visits of the current one.
+      struct Part {
+        uint32_t q, at, len, pin[LONG_STEPS];
+      };
+      auto fetch = [&](uint32_t q, uint32_t at) {
+        Part p;
+        p.q = q;
+        p.at = at;
+        p.len = lane_value(len, q);
+        const uint32_t* from = hedges + lane_value(s, q);
+#pragma unroll
+        for (uint32_t i = 0; i < LONG_STEPS; ++i) {
+          const uint32_t pos = at + 64 * i + l;
+          p.pin[i] = pos < p.len ? from[pos] : 0u;
+        }
+        return p;
+      };
+      Part cur = fetch(0, 0);
+      for (;;) {
+        const bool more = cur.at + 64 * LONG_STEPS < cur.len;
+        const uint32_t q = more ? cur.q : cur.q + 1, at = more ? cur.at + 64 * LONG_STEPS : 0u;
+        Part nxt = cur;
+        if (q < m) nxt = fetch(q, at);
+        PinVisitHV pv;
+        pv.e = lane_value(e, cur.q);
+        pv.len = cur.len;
+        pv.hv = make_uint2(lane_value(hv.x, cur.q), lane_value(hv.y, cur.q));
+        pv.j = jb + cur.q;
+#pragma unroll
+        for (uint32_t i = 0; i < LONG_STEPS; ++i) {
+          if (cur.at + 64 * i >= cur.len) break;
+          if ((cur.q | cur.at | i) && stop()) return;
+          pv.pos = cur.at + 64 * i + l;
+          pv.act = pv.pos < cur.len;
+          pv.pin = cur.pin[i];
+          visit(pv);
+        }
+        if (q >= m) break;
+        cur = nxt;
+      }
+      continue;
     }
     const uint32_t incl = wave_scan_incl(len);
     const uint32_t total = __shfl(incl, 63, 64);

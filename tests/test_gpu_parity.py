@@ -133,6 +133,33 @@ def test_construction_by_pins(dev, pins, rng):
     assert np.array_equal(choff, eo) and np.array_equal(cp, ep) and np.array_equal(csrcc, es)
 
 
+@pytest.mark.parametrize("short", [0, 300])
+def test_candidates_long_hedges(dev, short, rng):
+    """Hedges at the edges of the steps of the hedge-by-hedge traversal (64 pins a step, four steps
+    a batch) with hubs in all of them, beside `short` hedges of a few pins that mix into the hubs'
+    lists; contributions of zero, sources and destinations."""
+    n, hubs = 9000, np.array([0, 17, 4321, 8998, 8999])
+    lens = [128, 129, 191, 192, 193, 255, 256, 257, 258, 319, 320, 321, 511, 512, 513, 767, 769, 1024, 1025] * 4
+    off, pins, srcc = [0], [], []
+    for i, ln in enumerate(lens + [3, 5, 8] * (short // 3)):
+        h = hubs[: 2 if ln < 9 else 5]
+        row = np.concatenate([h, rng.choice(np.setdiff1d(np.arange(n), hubs), size=ln - len(h), replace=False)])
+        pins.extend(int(x) for x in rng.permutation(row))
+        off.append(len(pins))
+        srcc.append(i % 3 if ln > 3 else 1)
+    w = rng.random(len(srcc)).astype(np.float32)
+    w[::4] = 0.0
+    hg = O.HG(n, np.array(off, np.uint64), np.array(pins, np.uint32), np.array(srcc, np.uint32), w)
+    L = G.Level(dev, hg)
+    L.build_touching()
+    ro, rt, ri = O.touching(hg)
+    sizes = rng.integers(1, 3, size=n).astype(np.uint32)
+    for delta in (2**31 - 1, 40):
+        pairs, scores, *_ = G.candidates(dev, L, sizes, 16, 6, delta)
+        ep, es = O.candidates(hg, ro, rt, ri, sizes, 16, 6, delta)
+        assert np.array_equal(pairs, ep) and np.array_equal(scores, es), delta
+
+
 def hub_graph(n, hubs, n_small, rng):
     """Hub nodes, each on `count` hedges of `size` pins drawn from a pool of `pool` nodes, so
     their visit bounds (and worst-case tables) are far above their distinct neighbours."""
