@@ -2137,7 +2137,8 @@ __global__ void k_edge_ranks(const uint32_t* __restrict__ sorted_j, const uint32
 // and two read-backs; one workgroup holds all moves in registers and LDS.  k_rank_front orders the
 // moves (and, ranking by gain, is done), k_rank_back follows the links to the ranks; the proposals
 // between them keep their launches (a table per partition and size needs more than one workgroup).
-// A level of 5,000 nodes: about 150 us in the launches above, 65 us this way.
+// With k_round_small, an inbound-constrained run on 9,248 nodes: 16,230 launches before, 11,946 so,
+// 83.8 -> 75.1 ms on the device (k_rank_front 12 us to 1,024 moves, 43 us to 8,192; k_rank_back 68).
 // Keys carry the position in their low SMALL_BITS bits, so the sorts move one word per entry.
 constexpr uint32_t SMALL_BITS = 13;
 constexpr uint32_t SMALL_N = 1u << SMALL_BITS;
@@ -3108,7 +3109,7 @@ __device__ __forceinline__ Best wave_best_prefix(Best x) {
   return x;
 }
 __device__ Best block_best(Best x) {
-  __shared__ Best sb[4];
+  __shared__ Best sb[16];
   x = wave_best_prefix(x);
   if (lane_id() == 0) sb[threadIdx.x / 64] = x;
   __syncthreads();
@@ -3148,6 +3149,91 @@ __global__ void __launch_bounds__(256) k_best_final(const Best* __restrict__ par
     if (better(part[i], x)) x = part[i];
   Best b = block_best(x);
   if (threadIdx.x == 0) *out = b;
+}
+
+// Prefix sums of the ranks' terms and violations, and the best prefix, in three launches: tiles are
+// summed, every tile adds up the sums of the tiles before it, scans its own ranks and finds its best
+// prefix, and k_best_final takes the best of those.  Single scans of the three arrays and a sweep
+// for the best are eight launches at least, and are bound by them (16 rounds on 500k nodes: 11.0 ->
+// 10.7 ms; a run on 20k nodes 19.4 -> 18.2 ms, on 3.2M nodes 324.6 -> 320.4 ms on the device).
+// A tile reads the sums before it, so up to PREFIX_TILES tiles (above, the scans).
+struct PrefixSums {
+  int64_t seq;
+  int32_t sv, iv;
+};
+constexpr uint32_t PREFIX_TILES = 4096;
+template <uint32_t IT, bool INCC>
+__device__ __forceinline__ void prefix_load(const int64_t* seq, const int32_t* sv, const int32_t* iv, uint32_t V,
+                                            int64_t (&a)[IT], int32_t (&b)[IT], int32_t (&d)[IT]) {
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) {
+    const uint64_t i = (uint64_t)blockIdx.x * BLOCK_SORT_THREADS * IT + block_pos<IT>(r);
+    a[r] = i < V ? seq[i] : 0;
+    b[r] = i < V ? sv[i] : 0;
+    d[r] = INCC && i < V ? iv[i] : 0;
+  }
+}
+// sums over the workgroup, to every thread
+__device__ __forceinline__ PrefixSums prefix_block_sum(PrefixSums x) {
+  __shared__ PrefixSums s[BLOCK_SORT_WAVES];
+  x = PrefixSums{wave_sum(x.seq), wave_sum(x.sv), wave_sum(x.iv)};
+  if (lane_id() == 0) s[threadIdx.x / 64] = x;
+  __syncthreads();
+  PrefixSums t{0, 0, 0};
+#pragma unroll
+  for (uint32_t q = 0; q < BLOCK_SORT_WAVES; ++q) t = PrefixSums{t.seq + s[q].seq, t.sv + s[q].sv, t.iv + s[q].iv};
+  return t;
+}
+template <uint32_t IT, bool INCC>
+__global__ void __launch_bounds__(BLOCK_SORT_THREADS)
+    k_prefix_sums(const int64_t* __restrict__ seq, const int32_t* __restrict__ sv, const int32_t* __restrict__ iv,
+                  uint32_t V, PrefixSums* __restrict__ sums) {
+  int64_t a[IT];
+  int32_t b[IT], d[IT];
+  prefix_load<IT, INCC>(seq, sv, iv, V, a, b, d);
+  PrefixSums x{0, 0, 0};
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) x = PrefixSums{x.seq + a[r], x.sv + b[r], x.iv + d[r]};
+  x = prefix_block_sum(x);
+  if (threadIdx.x == 0) sums[blockIdx.x] = x;
+}
+template <uint32_t IT, bool INCC>
+__global__ void __launch_bounds__(BLOCK_SORT_THREADS)
+    k_prefix_best(int64_t* __restrict__ seq, int32_t* __restrict__ sv, int32_t* __restrict__ iv, uint32_t V,
+                  const PrefixSums* __restrict__ sums, Best* __restrict__ out) {
+  __shared__ int64_t s_a[BLOCK_SORT_WAVES];
+  __shared__ int32_t s_b[BLOCK_SORT_WAVES], s_d[BLOCK_SORT_WAVES];
+  PrefixSums before{0, 0, 0};
+  for (uint32_t j = threadIdx.x; j < blockIdx.x; j += BLOCK_SORT_THREADS) {
+    const PrefixSums y = sums[j];
+    before = PrefixSums{before.seq + y.seq, before.sv + y.sv, before.iv + y.iv};
+  }
+  int64_t a[IT];
+  int32_t b[IT], d[IT];
+  prefix_load<IT, INCC>(seq, sv, iv, V, a, b, d);
+  before = prefix_block_sum(before);
+  block_scan(a, s_a);
+  block_scan(b, s_b);
+  if (INCC) block_scan(d, s_d);
+  Best x{};
+  x.r = NONE;
+#pragma unroll
+  for (uint32_t r = 0; r < IT; ++r) {
+    const uint64_t i = (uint64_t)blockIdx.x * BLOCK_SORT_THREADS * IT + block_pos<IT>(r);
+    if (i >= V) continue;
+    Best y{};
+    y.r = (uint32_t)i;
+    y.seq = a[r] + before.seq;
+    y.sv = b[r] + before.sv;
+    y.iv = INCC ? d[r] + before.iv : 0;
+    y.ok = y.iv == 0;
+    seq[i] = y.seq;
+    sv[i] = y.sv;
+    if (INCC) iv[i] = y.iv;
+    if (better(y, x)) x = y;
+  }
+  x = block_best(x);
+  if (threadIdx.x == 0) out[blockIdx.x] = x;
 }
 // A round's events and best prefix on levels of up to SMALL_EVENT_N nodes, by one workgroup after the
 // cascade: the size (and inbound) events sorted by (partition, rank), their running sums per
@@ -4017,26 +4103,48 @@ bool try_analyze_round(Ctx& c, const RefineLevel& L, int mode, uint32_t omega, u
     segment_offsets(c, keys.get(), rb + 1, m, L.k, poff.get());
     HGP_LAUNCH(k_size_flags, ceil_div(m, 256), 256, 0, c, keys.get(), vals.get(), cum.get(), poff.get(), m, rb, psizes,
                omega, st.sv.get());
-    inclusive_scan(c, st.sv.get(), st.sv.get(), V);
     join_cascade();
     if (incc) {
       HGP_LAUNCH(k_inbound_deltas, ceil_div(m, 256), 256, 0, c, keys.get(), dio.get(), m, rb, db, cum.get());
       inclusive_scan(c, cum.get(), cum.get(), m);
       HGP_LAUNCH(k_inbound_flags, ceil_div(m, 256), 256, 0, c, keys.get(), dio.get(), cum.get(), poff.get(), m, rb, db,
                  pl.inbsz.get(), delta, st.iv.get());
-      inclusive_scan(c, st.iv.get(), st.iv.get(), V);
     }
   }
-  inclusive_scan(c, (const int64_t*)st.seq.get(), (int64_t*)st.seq.get(), V);
-  // best prefix
-  {
+  // prefix sums and best prefix; one item a thread up to 65,536 ranks, so that more workgroups share them
+  const bool few = V <= 64 * BLOCK_SORT_THREADS;
+  const uint32_t tiles = ceil_div(V, few ? BLOCK_SORT_THREADS : 4 * BLOCK_SORT_THREADS);
+  DBuf<Best> out(c, 1);
+  if (tiles <= PREFIX_TILES) {
+    DBuf<PrefixSums> sums(c, tiles);
+    DBuf<Best> partial(c, tiles);
+    auto run = [&](auto it, auto mi) {
+      constexpr uint32_t IT = decltype(it)::value;
+      constexpr bool INCC = decltype(mi)::value;
+      if (tiles > 1)
+        HGP_LAUNCH((k_prefix_sums<IT, INCC>), tiles, BLOCK_SORT_THREADS, 0, c, (const int64_t*)st.seq.get(),
+                   st.sv.get(), st.iv.get(), V, sums.get());
+      HGP_LAUNCH((k_prefix_best<IT, INCC>), tiles, BLOCK_SORT_THREADS, 0, c, (int64_t*)st.seq.get(), st.sv.get(),
+                 st.iv.get(), V, sums.get(), partial.get());
+    };
+    using One = std::integral_constant<uint32_t, 1>;
+    using Four = std::integral_constant<uint32_t, 4>;
+    if (incc && few) run(One{}, std::true_type{});
+    else if (incc) run(Four{}, std::true_type{});
+    else if (few) run(One{}, std::false_type{});
+    else run(Four{}, std::false_type{});
+    HGP_LAUNCH(k_best_final, 1, 256, 0, c, partial.get(), tiles, out.get());
+  } else {
     const uint32_t blocks = std::min<uint32_t>(ceil_div(V, 256), 1024);
-    DBuf<Best> partial(c, blocks), out(c, 1);
+    DBuf<Best> partial(c, blocks);
+    inclusive_scan(c, st.sv.get(), st.sv.get(), V);
+    if (incc) inclusive_scan(c, st.iv.get(), st.iv.get(), V);
+    inclusive_scan(c, (const int64_t*)st.seq.get(), (int64_t*)st.seq.get(), V);
     HGP_LAUNCH(k_best_partial, blocks, 256, 0, c, (const int64_t*)st.seq.get(), st.sv.get(), st.iv.get(), V,
                partial.get());
     HGP_LAUNCH(k_best_final, 1, 256, 0, c, partial.get(), blocks, out.get());
-    st.best = read_scalar(c, out.get());
   }
+  st.best = read_scalar(c, out.get());
   return true;
 }
 

@@ -540,11 +540,12 @@ def test_refine_analyze_inbound_by_hedge_size(dev, k, dup, rng):
     assert dup or got["best"] == exp["best"]
 
 
-@pytest.mark.parametrize("n", [1, 2, 65, 1024, 1025, 2048, 2049, 4096, 4097, 8192, 8193])
+@pytest.mark.parametrize("n", [1, 2, 65, 1024, 1025, 2048, 2049, 4096, 4097, 8192, 8193, 65536, 65537])
 @pytest.mark.parametrize("mode,k", [(1, 40), (0, 40), (1, 3000), (0, 3000)])
 def test_refine_analyze_by_level_size(dev, n, mode, k, rng):
     """Levels at the edges of the one-workgroup ranking (8,192 nodes) and events (4,096), of their
-    items per thread and of the ranks whose counters fit LDS; partitions by table and by scan."""
+    items per thread, of the ranks whose counters fit LDS and of the tiles of the prefix sums;
+    partitions by table and by scan."""
     lens = np.minimum(np.concatenate([rng.integers(1, 18, size=2 * n), rng.integers(17, 130, size=min(n, 200))]), n)
     off = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint64)
     start, step = rng.integers(0, n, size=len(lens)), 1 + 2 * rng.integers(0, 50, size=len(lens))
