@@ -1074,8 +1074,8 @@ template <uint32_t IT>
 __global__ void __launch_bounds__(BLOCK_SORT_THREADS)
     k_group_small(const uint32_t* __restrict__ pairs, const uint32_t* __restrict__ scores, uint32_t cnc, uint32_t n,
                   const uint32_t* __restrict__ sizes, const uint32_t* __restrict__ inb, uint32_t omega, uint32_t delta,
-                  int size_bits, uint32_t* __restrict__ raw_out, uint32_t* __restrict__ groups,
-                  uint32_t* __restrict__ gsizes, uint32_t* __restrict__ new_n) {
+                  uint32_t* __restrict__ raw_out, uint32_t* __restrict__ groups, uint32_t* __restrict__ gsizes,
+                  uint32_t* __restrict__ new_n) {
   __shared__ GroupMem<IT> s;
   uint32_t v[IT], cand[IT], sc[IT];
   bool orphan[IT];
@@ -1162,18 +1162,27 @@ __global__ void __launch_bounds__(BLOCK_SORT_THREADS)
       if (v[r] < n && !(locked >> r & 1u)) decide_from(v[r], par[r], s.best, s.raw);
     __syncthreads();
   }
-  // orphans in node order, sorted stably by size: the smallest with the largest, and so on inwards
-  uint32_t x[IT];
+  // orphans in node order, sorted stably by size: the smallest with the largest, and so on inwards (a
+  // size may be above omega, so the sort's bits are those of the largest orphan)
+  uint32_t x[IT], top = 0;
 #pragma unroll
   for (uint32_t r = 0; r < IT; ++r) x[r] = orphan[r];
   block_scan(x, s.sort.w);
   if (threadIdx.x == BLOCK_SORT_THREADS - 1) s.wgt[0] = x[IT - 1];
 #pragma unroll
-  for (uint32_t r = 0; r < IT; ++r)
-    if (orphan[r]) s.sort.key[x[r] - 1] = ((uint64_t)sizes[v[r]] << 32) | v[r];
+  for (uint32_t r = 0; r < IT; ++r) {
+    if (!orphan[r]) continue;
+    const uint32_t size = sizes[v[r]];
+    s.sort.key[x[r] - 1] = ((uint64_t)size << 32) | v[r];
+    top = max(top, size);
+  }
+  top = wave_max(top);
+  if (lane_id() == 0) s.wgt[1 + threadIdx.x / 64] = top;
   __syncthreads();
   const uint32_t m = s.wgt[0];
   if (m >= 2) {
+    for (uint32_t w = 0; w < BLOCK_SORT_WAVES; ++w) top = max(top, s.wgt[1 + w]);
+    const int size_bits = 32 - __clz(top | 1u);
     uint64_t key[IT];
     uint32_t none[IT] = {};
 #pragma unroll
@@ -1407,7 +1416,8 @@ static void group_large(Ctx& c, const uint32_t* inb, const uint32_t* pairs, cons
     if (m >= 2) {
       DBuf<uint64_t> keys(c, m);
       HGP_LAUNCH(k_orphan_keys, g, 256, 0, c, f.get(), pos.get(), sizes, n, keys.get());
-      radix_sort(c, keys.get(), nullptr, m, 32 + std::max(1, bit_width(omega)));
+      DBuf<uint32_t> none;  // the keys are in node order; a size may be above omega
+      radix_sort_buf(c, keys, none, m, 32, 64);
       HGP_LAUNCH(k_orphan_pair, ceil_div(m / 2, 256), 256, 0, c, keys.get(), m, sizes, inb, omega, delta, raw.get());
     }
   }
@@ -1432,10 +1442,9 @@ void group_nodes(Ctx& c, const uint32_t* inb, const uint32_t* pairs, const uint3
   if (n <= GROUP_SMALL) {
     gsizes = DBuf<uint32_t>(c, std::max<uint32_t>(n, 1));
     DBuf<uint32_t> raw(c, raw_out ? n : 0), count(c, 1);
-    const int size_bits = std::max(1, bit_width(omega));
     auto run = [&](auto it) {
       HGP_LAUNCH((k_group_small<decltype(it)::value>), 1, BLOCK_SORT_THREADS, 0, c, pairs, scores, cnc, n, sizes, inb,
-                 omega, delta, size_bits, raw_out ? raw.get() : nullptr, groups.get(), gsizes.get(), count.get());
+                 omega, delta, raw_out ? raw.get() : nullptr, groups.get(), gsizes.get(), count.get());
     };
     if (n <= BLOCK_SORT_THREADS) run(std::integral_constant<uint32_t, 1>{});
     else if (n <= 2 * BLOCK_SORT_THREADS) run(std::integral_constant<uint32_t, 2>{});

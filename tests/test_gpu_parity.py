@@ -293,6 +293,25 @@ def test_group_nodes_by_size(dev, n, cnc, rng):
     assert np.array_equal(ung, eung) and np.array_equal(uoff, euoff)
 
 
+@pytest.mark.parametrize("n", [100, 4096, 4097, 20000])
+@pytest.mark.parametrize("omega", [1, 100, 70000])
+def test_group_nodes_orphans_above_the_limit(dev, n, omega, rng):
+    """Orphans are paired in the order of their sizes, also of sizes above the limit, whatever bits
+    those have: sizes up to 2^31 - 1 (two of them do not wrap) beside sizes that fit in pairs."""
+    pairs = np.full((n, 2), 0xFFFFFFFF, np.uint32)
+    some = rng.random(n) < 0.2
+    pairs[some, 0] = rng.integers(0, n, size=int(some.sum()))
+    sizes = rng.integers(1, omega // 2 + 2, size=n).astype(np.uint32)
+    above = rng.random(n) < 0.3
+    sizes[above] = (2.0 ** rng.uniform(np.log2(omega + 1), 31, size=int(above.sum()))).astype(np.uint32)
+    scores = rng.integers(0, 8, size=(n, 2)).astype(np.uint32)
+    inb = rng.integers(0, 50, size=n).astype(np.uint32)
+    d_inb, d_pairs, d_scores, d_sizes = (dev.upload(x) for x in (inb, pairs.ravel(), scores.ravel(), sizes))
+    k, groups, gs, *_ = G.group_nodes(dev, n, d_inb, d_pairs, d_scores, d_sizes, 2, omega, 70)
+    ek, eg, egs, *_ = O.group_nodes(n, inb, pairs.ravel(), scores.ravel(), sizes, 2, omega, 70)
+    assert k == ek and np.array_equal(groups, eg) and np.array_equal(gs, egs)
+
+
 @pytest.mark.parametrize("case", CASES, ids=[c[0] for c in CASES])
 def test_coarsening(dev, case, rng):
     """coarse hedges, coarse touching, coarse neighbours, uncoarsen"""
