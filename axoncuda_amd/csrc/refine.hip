@@ -1575,7 +1575,8 @@ __global__ void k_small_lens(const uint64_t* __restrict__ keys, uint32_t m, cons
 }
 __global__ void k_small_fill(const uint64_t* __restrict__ keys, uint32_t m, const uint64_t* __restrict__ hoff,
                              const uint32_t* __restrict__ hedges, const float* __restrict__ w,
-                             const uint32_t* __restrict__ srcc, uint64_t* __restrict__ rec, uint32_t* __restrict__ pins, float* __restrict__ sw) {
+                             const uint32_t* __restrict__ srcc, uint64_t* __restrict__ rec, uint32_t* __restrict__ pins,
+                             float* __restrict__ sw) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= m) return;
   const uint32_t e = small_hedge_id(keys, i);
@@ -1583,7 +1584,10 @@ __global__ void k_small_fill(const uint64_t* __restrict__ keys, uint32_t m, cons
   for (uint64_t j = 0; j < len; ++j) pins[o + j] = hedges[s + j];
   for (uint64_t j = len; j < ((len + 3) & ~3ull); ++j) pins[o + j] = hedges[s + len - 1];
   sw[i] = w[e];
-  rec[i] = (o << 10) | ((uint64_t)(srcc ? srcc[e] : 0u) << 5) | len;
+  // device callers' source counts are not checked: one above the length means all pins, and has to
+  // keep to its five bits
+  const uint64_t sources = srcc ? min((uint64_t)srcc[e], len) : 0ull;
+  rec[i] = (o << 10) | (sources << 5) | len;
 }
 __global__ void k_compact(const uint32_t* __restrict__ flag, const uint64_t* __restrict__ pos, uint32_t n,
                           uint32_t* __restrict__ out) {

@@ -559,6 +559,34 @@ def test_refine_analyze_inbound_by_hedge_size(dev, k, dup, rng):
     assert dup or got["best"] == exp["best"]
 
 
+@pytest.mark.parametrize("k", [40, 66000])
+def test_refine_analyze_source_counts_above_the_length(dev, k, rng):
+    """A source count above the hedge's length (the stages take device arrays as they are) makes all
+    its pins sources, in the records of the small hedges too, where counts have five bits."""
+    lens = np.resize([1, 2, 3, 4, 5, 8, 15, 16, 17, 40, 64, 65, 128, 129, 300, 1024, 1025], 1200)
+    n, e = 3000, len(lens)
+    off = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint64)
+    pins = np.concatenate([rng.choice(n, size=ln, replace=False) for ln in lens]).astype(np.uint32)
+    srcc = np.minimum(rng.integers(0, 3, size=e), lens).astype(np.uint32)
+    high = rng.random(e) < 0.3
+    srcc[high] = rng.choice(np.array([17, 31, 32, 33, 63, 1024, 1 << 16, 2**31, 2**32 - 1], np.uint32), size=int(high.sum()))
+    assert (srcc > lens).any()
+    hg = O.HG(n, off, pins, srcc, np.ones(e, np.float32))
+    sizes = rng.integers(1, 3, size=n).astype(np.uint32)
+    part = rng.integers(0, min(k, 300), size=n).astype(np.uint32)
+    psizes = np.bincount(part, weights=sizes, minlength=k).astype(np.uint32)
+    omega, delta = int(psizes.max()) + 3, int(O.inbound_sizes(hg, part, k).max()) - 1
+    L = G.Level(dev, hg)
+    L.build_touching()
+    for chainup in (False, True):
+        got = G.refine_analyze(dev, L, sizes, k, 0, omega, delta, 16, 0, chainup, part, psizes)
+        exp = O.refine_analyze(0, omega, delta, 16, hg, *O.touching(hg), sizes, k, 0, chainup, part, psizes)
+        assert exp["iv"].any()
+        for key in ("moves", "gains", "ranks", "seq", "sv", "iv"):
+            assert np.array_equal(got[key], exp[key]), f"{key} differs (chainup={chainup})"
+        assert got["best"] == exp["best"]
+
+
 @pytest.mark.parametrize("n", [1, 2, 65, 1024, 1025, 2048, 2049, 4096, 4097, 8192, 8193, 65536, 65537])
 @pytest.mark.parametrize("mode,k", [(1, 40), (0, 40), (1, 3000), (0, 3000)])
 def test_refine_analyze_by_level_size(dev, n, mode, k, rng):
