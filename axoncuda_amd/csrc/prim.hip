@@ -678,6 +678,7 @@ __global__ void __launch_bounds__(256) k_max(const T* __restrict__ p, uint64_t n
 void exclusive_scan(Ctx& c, const uint32_t* in, uint64_t* out, uint64_t n) { scan_impl<uint32_t, uint64_t>(c, in, out, n, true); }
 void exclusive_scan(Ctx& c, const uint64_t* in, uint64_t* out, uint64_t n) { scan_impl<uint64_t, uint64_t>(c, in, out, n, true); }
 void inclusive_scan(Ctx& c, const int64_t* in, int64_t* out, uint64_t n) { scan_impl<int64_t, int64_t>(c, in, out, n, false); }
+void inclusive_scan(Ctx& c, const uint64_t* in, uint64_t* out, uint64_t n) { scan_impl<uint64_t, uint64_t>(c, in, out, n, false); }
 void inclusive_scan(Ctx& c, const int32_t* in, int32_t* out, uint64_t n) { scan_impl<int32_t, int32_t>(c, in, out, n, false); }
 
 void radix_sort(Ctx& c, uint32_t* keys, uint32_t* vals, uint64_t n, int bits) { radix_impl<uint32_t>(c, keys, vals, n, bits); }

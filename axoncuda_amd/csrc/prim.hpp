@@ -12,6 +12,7 @@ void exclusive_scan(Ctx& c, const uint32_t* in, uint64_t* out, uint64_t n);
 void exclusive_scan(Ctx& c, const uint64_t* in, uint64_t* out, uint64_t n);
 // out[i] = sum in[0..i]; in-place allowed.
 void inclusive_scan(Ctx& c, const int64_t* in, int64_t* out, uint64_t n);
+void inclusive_scan(Ctx& c, const uint64_t* in, uint64_t* out, uint64_t n);
 void inclusive_scan(Ctx& c, const int32_t* in, int32_t* out, uint64_t n);
 
 // Stable LSD radix sorts over key bits [0, bits); values ride along (nullable).

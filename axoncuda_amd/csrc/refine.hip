@@ -3059,17 +3059,20 @@ __global__ void k_size_flags(const uint64_t* __restrict__ keys, const uint32_t* 
 // per moving inbound incidence (on an 8 x 8191-neuron network of fan-out 64 the events, their
 // 43-bit sort and the searches of their runs took 250 of a 530 ms partitioning).
 // Scanned together: the signed change in the low `db` bits, and above them the number of events
-// that change anything (the first of a partition assumes it started valid).
+// that change anything (the first of a partition assumes it started valid).  A partition's change
+// is that of its inbound-set size, within the number of hedges either way, and it has at most one
+// event per move, so with db = 64 - rb its count of events differs from 1 beyond the first; the sums
+// over all partitions wrap, their differences within one do not.
 __global__ void k_inbound_deltas(const uint64_t* __restrict__ keys, const unsigned long long* __restrict__ dio,
-                                 uint64_t m, int rb, int db, int64_t* __restrict__ out) {
+                                 uint64_t m, int rb, int db, uint64_t* __restrict__ out) {
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= m) return;
   const unsigned long long x = dio[event_rank(keys[i], rb)];
-  const int64_t d = (keys[i] & 1u) ? (int64_t)(x >> 32) : -(int64_t)(x & 0xFFFFFFFFull);
-  out[i] = d + (d != 0 ? (int64_t)1 << db : 0);
+  const uint64_t d = (keys[i] & 1u) ? x >> 32 : 0ull - (x & 0xFFFFFFFFull);
+  out[i] = d + (d != 0 ? 1ull << db : 0ull);
 }
 __global__ void k_inbound_flags(const uint64_t* __restrict__ keys, const unsigned long long* __restrict__ dio,
-                                const int64_t* __restrict__ cum, const uint64_t* __restrict__ poff, uint64_t m, int rb,
+                                const uint64_t* __restrict__ cum, const uint64_t* __restrict__ poff, uint64_t m, int rb,
                                 int db, const uint32_t* __restrict__ isz, uint32_t delta, int32_t* iv) {
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= m) return;
@@ -3080,9 +3083,9 @@ __global__ void k_inbound_flags(const uint64_t* __restrict__ keys, const unsigne
   if (d == 0) return;
   const uint32_t q = (uint32_t)(key >> (rb + 1));
   const uint64_t st = poff[q];
-  const int64_t c = cum[i] - (st == 0 ? 0 : cum[st - 1]);
-  const int64_t change = (int64_t)((uint64_t)c << (64 - db)) >> (64 - db);
-  const bool first = ((c - change) >> db) == 1;
+  const uint64_t c = cum[i] - (st == 0 ? 0 : cum[st - 1]);
+  const int64_t change = (int64_t)(c << (64 - db)) >> (64 - db);
+  const bool first = ((c - (uint64_t)change) >> db) == 1;
   const int64_t cur = (int64_t)isz[q] + change, prev = cur - d;
   // the first event of a partition assumes it started valid (kernels/refinement.cu:643-644)
   const bool was_valid = first || prev <= (int64_t)delta, is_valid = cur <= (int64_t)delta;
@@ -3927,10 +3930,8 @@ bool try_analyze_round(Ctx& c, const RefineLevel& L, int mode, uint32_t omega, u
     Y.max_size = n ? reduce_max_u32(c, L.sizes, n) : 0u;
   }
   const bool small = one_group && n >= 1 && n <= SMALL_N && (chainup || chain_by_table(n, L.k, Y.max_size));
-  // the events and the best prefix too (V stays on the device); inbound events of larger keys are
-  // refused below
-  const int key_bits = bit_width(L.k) + bit_width(L.e) + bit_width(n);
-  const bool fused = small && n <= SMALL_EVENT_N && (!incc || key_bits <= 64);
+  // the events and the best prefix too (V stays on the device)
+  const bool fused = small && n <= SMALL_EVENT_N;
   // node records of the cascade, kept until its side streams have joined
   const bool packed = L.k < PM2_MAX_K;
   DBuf<uint2> pm2(c, packed ? n : 0);
@@ -4069,9 +4070,8 @@ bool try_analyze_round(Ctx& c, const RefineLevel& L, int mode, uint32_t omega, u
   };
   const int rb = std::max(1, bit_width(V - 1));
   const int kb = std::max(1, bit_width(L.k));
-  // inbound events: partition, hedge and rank in one 64-bit word; larger levels are refused
-  const int eb = std::max(1, bit_width(L.e));
-  HGP_REQUIRE(!incc || kb + eb + rb <= 64, HGP_E_CAPACITY, "inbound events: key exceeds 64 bits");
+  // events: partition, rank and direction in one 64-bit word (up to 2^31 moves of any partitions)
+  HGP_REQUIRE(kb + rb + 1 <= 64, HGP_E_CAPACITY, "events: key exceeds 64 bits");
   if (fused) {
     join_cascade();
     DBuf<RoundOut> out(c, 1);
@@ -4095,9 +4095,6 @@ bool try_analyze_round(Ctx& c, const RefineLevel& L, int mode, uint32_t omega, u
     DBuf<uint64_t> keys(c, m), poff(c, (uint64_t)L.k + 1);
     DBuf<uint32_t> vals(c, m);
     DBuf<int64_t> cum(c, m);
-    // inbound events: m of them counted above a change of at most P destination pins either way
-    const int db = 63 - bit_width(m);
-    HGP_REQUIRE(!incc || pl.P < (1ull << (db - 1)), HGP_E_CAPACITY, "inbound events: too many moves and pins");
     HGP_LAUNCH(k_size_events, g, 256, 0, c, part, st.moves.get(), st.ranks.get(), L.sizes, n, rb, keys.get(), vals.get());
     // the events sit at 2 * rank (+1), so they are already in rank order: sorting by the
     // partition bits alone orders them by (partition, rank)
@@ -4109,9 +4106,12 @@ bool try_analyze_round(Ctx& c, const RefineLevel& L, int mode, uint32_t omega, u
                omega, st.sv.get());
     join_cascade();
     if (incc) {
-      HGP_LAUNCH(k_inbound_deltas, ceil_div(m, 256), 256, 0, c, keys.get(), dio.get(), m, rb, db, cum.get());
-      inclusive_scan(c, cum.get(), cum.get(), m);
-      HGP_LAUNCH(k_inbound_flags, ceil_div(m, 256), 256, 0, c, keys.get(), dio.get(), cum.get(), poff.get(), m, rb, db,
+      const int db = 64 - rb;  // above 2^31 moves it holds the changes of fewer than 2^32 hedges
+      HGP_REQUIRE(L.e < 1ull << (db - 1), HGP_E_CAPACITY, "inbound events: too many moves and hedges");
+      uint64_t* sums = reinterpret_cast<uint64_t*>(cum.get());
+      HGP_LAUNCH(k_inbound_deltas, ceil_div(m, 256), 256, 0, c, keys.get(), dio.get(), m, rb, db, sums);
+      inclusive_scan(c, sums, sums, m);
+      HGP_LAUNCH(k_inbound_flags, ceil_div(m, 256), 256, 0, c, keys.get(), dio.get(), sums, poff.get(), m, rb, db,
                  pl.inbsz.get(), delta, st.iv.get());
     }
   }

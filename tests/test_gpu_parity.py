@@ -617,6 +617,102 @@ def test_refine_analyze_by_level_size(dev, n, mode, k, rng):
         assert got["best"] == exp["best"]
 
 
+def inbound_violations(hg, part, moves, ranks, k, delta):
+    """The running inbound violations from their definition: the destinations of every (hedge,
+    partition) counted move by move in rank order, the inbound size of every partition from the
+    counts that reach or leave zero, and its crossings of delta (a partition's first change starts
+    from a valid state)."""
+    lens = np.diff(hg.off.astype(np.int64))
+    hedge = np.repeat(np.arange(hg.e), lens)
+    dst = np.arange(len(hg.pins)) - hg.off[:-1].astype(np.int64)[hedge] >= hg.srcc.astype(np.int64)[hedge]
+    hedge, node = hedge[dst], hg.pins[dst]
+    own = hedge * k + part[node]  # (hedge, partition) of every destination
+    m = moves[node] != 2**32 - 1
+    rank = ranks[node].astype(np.int64)[m]
+    key = np.concatenate([own[m], hedge[m] * k + moves[node].astype(np.int64)[m]])
+    step, rank = np.concatenate([-np.ones(len(rank), np.int64), np.ones(len(rank), np.int64)]), np.tile(rank, 2)
+
+    def running(key, step, start):  # sums up to each event of its key's run, added to the run's start
+        total, first = np.cumsum(step), np.concatenate([[True], key[1:] != key[:-1]])
+        return total - np.repeat((total - step)[first], np.diff(np.append(np.flatnonzero(first), len(key)))) + start
+
+    o = np.lexsort((rank, key))
+    key, step, rank = key[o], step[o], rank[o]
+    ids, cnt = np.unique(own, return_counts=True)
+    at = np.minimum(np.searchsorted(ids, key), len(ids) - 1)
+    now = running(key, step, np.where(ids[at] == key, cnt[at], 0))
+    change = (now > 0).astype(np.int64) - (now - step > 0)
+    c = change != 0
+    q, change, rank = key[c] % k, change[c], rank[c]
+    o = np.lexsort((rank, q))
+    q, change, rank = q[o], change[o], rank[o]
+    size = running(q, change, np.bincount(ids % k, minlength=k)[q])
+    was = (size - change > delta) & np.concatenate([[False], q[1:] == q[:-1]])
+    return np.cumsum(np.bincount(rank, weights=(size > delta).astype(np.int64) - was, minlength=hg.n)).astype(np.int32)
+
+
+@pytest.mark.parametrize("n,e,k,chainup", [
+    (300_000, 300_000, 2000, False),         # above the ranks that have copies of the cascade's counters
+    (300_000, 300_000, 2000, True),
+    (600_000, (1 << 20) + 1, 1 << 24, True),  # partition, hedge and rank in more than 64 bits together
+    (600_000, (1 << 20) + 1, 1 << 24, False),
+])
+def test_refine_analyze_inbound_many_ranks(dev, n, e, k, chainup, rng):
+    """Inbound-constrained rounds of more than 262,144 moves: the cascade's counters in memory, the
+    inbound events of many partitions, hedges of every cascade class.  (The oracle goes through all
+    partitions for every node, so the largest case checks the violations alone, from their definition.)"""
+    lens = rng.integers(1, 5, size=e)
+    lens[rng.permutation(e)[:600]] = np.resize([16, 17, 64, 65, 128, 129, 700, 1024, 1025, 2049], 600)
+    off = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint64)
+    start, step = rng.integers(0, n, size=e), 1 + 2 * rng.integers(0, 50, size=e)
+    pos = np.arange(int(off[-1])) - np.repeat(off[:-1].astype(np.int64), lens)
+    pins = ((np.repeat(start, lens) + pos * np.repeat(step, lens)) % n).astype(np.uint32)
+    srcc = np.minimum(rng.integers(0, 2, size=e), lens - 1).astype(np.uint32)
+    hg = O.HG(n, off, pins, srcc, (rng.random(e) + 0.5).astype(np.float32))
+    sizes = rng.integers(1, 4, size=n).astype(np.uint32)
+    part = (np.arange(n) * 7 // 13 % min(k, 3000) * (k // min(k, 3000))).astype(np.uint32)
+    psizes = np.bincount(part, weights=sizes, minlength=k).astype(np.uint32)
+    omega, delta = int(psizes.max()) + 3, max(1, int(O.inbound_sizes(hg, part, k).max()) - 1)
+    L = G.Level(dev, hg)
+    L.build_touching()
+    got = G.refine_analyze(dev, L, sizes, k, 0, omega, delta, 16, 0, chainup, part, psizes)
+    ranks = int((got["moves"] != 2**32 - 1).sum())
+    assert ranks > 262144 and got["iv"].any()
+    iv = inbound_violations(hg, part, got["moves"], got["ranks"], k, delta)
+    assert np.array_equal(got["iv"][:ranks], iv[:ranks])
+    if k >= 1 << 24:
+        assert k.bit_length() + e.bit_length() + (ranks - 1).bit_length() > 64
+        return
+    exp = O.refine_analyze(0, omega, delta, 16, hg, *O.touching(hg), sizes, k, 0, chainup, part, psizes)
+    for key in ("moves", "gains", "ranks", "seq", "sv", "iv"):
+        assert np.array_equal(got[key], exp[key]), f"{key} differs"
+    assert got["best"] == exp["best"]
+
+
+@pytest.mark.parametrize("movers", [1, 2, 3, 4, 5, 8, 9])
+def test_refine_analyze_inbound_few_ranks(dev, movers, rng):
+    """A device-wide inbound-constrained round of a handful of moves, all into one partition that is
+    over its limit from the start: the first of its events counts as starting valid, no later one."""
+    n, k = 5000, 12
+    n, off, pins, srcc, w = gen.random_hypergraph(n, 8000, rng, max_size=12, src_prob=0.3, max_src=2)
+    hg = O.dedup(O.HG(n, off, pins, srcc, w))
+    sizes = rng.integers(1, 3, size=n).astype(np.uint32)
+    part = np.zeros(n, np.uint32)
+    part[rng.permutation(n)[:movers]] = 1 + np.arange(movers) % (k - 1)
+    psizes = np.full(k, 100, np.uint32)  # only partition 0 takes nodes
+    psizes[0] = 1
+    L = G.Level(dev, hg)
+    L.build_touching()
+    for delta in (10, int(O.inbound_sizes(hg, part, k).max())):
+        for chainup in (False, True):
+            exp = O.refine_analyze(0, 50, delta, 16, hg, *O.touching(hg), sizes, k, 0, chainup, part, psizes)
+            assert int((exp["moves"] != 2**32 - 1).sum()) == movers
+            got = G.refine_analyze(dev, L, sizes, k, 0, 50, delta, 16, 0, chainup, part, psizes)
+            for key in ("moves", "gains", "ranks", "seq", "sv", "iv"):
+                assert np.array_equal(got[key], exp[key]), f"{key} differs"
+            assert got["best"] == exp["best"]
+
+
 @pytest.mark.parametrize("rc", REFINE_CASES, ids=[r[0] for r in REFINE_CASES])
 def test_refine_loop(dev, rc, rng):
     name, mode, k, case_name = rc
