@@ -3484,6 +3484,9 @@ struct LevelLayout {
   uint64_t gslots = 0;
   bool sized = false;
   uint32_t max_size = 0;  // largest node size of the level
+  // a round's keys did not fit the one-workgroup ranking, and no later round tries it (hubs of 20,000 heavy
+  // hedges, 4,000 nodes, k = 1,000: 104 ms with gains and ranks done twice a round, 54 ms so)
+  bool wide = false;
   uint32_t cas_sort_max = 0xFFFFFFFFu;
   DBuf<uint32_t> cas_list[3];
   uint32_t cas_n[3] = {0, 0, 0};
@@ -3909,27 +3912,15 @@ struct RoundState {
   Best best;
 };
 
-// one_group: levels that fit take the one-workgroup stages (see k_rank_front).  Returns false when
-// their keys did not fit; the round is then to be analysed without them.
-bool try_analyze_round(Ctx& c, const RefineLevel& L, int mode, uint32_t omega, uint32_t delta, uint32_t R, uint32_t rep,
-                       bool chainup, const uint32_t* part, const uint32_t* psizes, RoundState& st, LevelLayout* layout,
-                       bool one_group) {
+// Ranks the round's moves (st.moves, st.gains), sums the cascade over them and finds the best prefix.
+// Levels that fit take the one-workgroup stages (see k_rank_front) unless Y.wide.  Returns false when the
+// keys turn out too wide for them after the last kernel, and sets Y.wide: it is then called again.
+bool rank_round(Ctx& c, const RefineLevel& L, int mode, uint32_t omega, uint32_t delta, bool chainup,
+                const uint32_t* part, const uint32_t* psizes, const PartitionLists& pl, RoundState& st, LevelLayout& Y) {
   const uint32_t n = L.n;
   const uint32_t g = ceil_div(n, 256);
   const bool incc = mode == HGP_MODE_INCC;
-  PartitionLists pl;
-  build_partition_lists(c, L, part, pl, incc, layout, !incc && L.k <= MASK_K);
-  st.moves = DBuf<uint32_t>(c, n);
-  st.gains = DBuf<int64_t>(c, n);
-  st.ranks = DBuf<uint32_t>(c, n);
-  compute_gains(c, L, pl, mode, omega, rep, discount_of(rep, R), part, psizes, st.moves.get(), st.gains.get());
-  LevelLayout own_layout;
-  LevelLayout& Y = layout ? *layout : own_layout;
-  if (!Y.sized) {
-    Y.sized = true;
-    Y.max_size = n ? reduce_max_u32(c, L.sizes, n) : 0u;
-  }
-  const bool small = one_group && n >= 1 && n <= SMALL_N && (chainup || chain_by_table(n, L.k, Y.max_size));
+  bool small = !Y.wide && n >= 1 && n <= SMALL_N && (chainup || chain_by_table(n, L.k, Y.max_size));
   // the events and the best prefix too (V stays on the device)
   const bool fused = small && n <= SMALL_EVENT_N;
   // node records of the cascade, kept until its side streams have joined
@@ -3952,11 +3943,16 @@ bool try_analyze_round(Ctx& c, const RefineLevel& L, int mode, uint32_t omega, u
                Y.max_size);
     if (!fused) {
       const RankInfo ri = read_scalar(c, info.get());
-      if (ri.wide) return false;
-      st.V = ri.V;
-      if (st.V == 0) return true;
+      if (ri.wide) {
+        Y.wide = true;
+        small = false;
+      } else {
+        st.V = ri.V;
+        if (st.V == 0) return true;
+      }
     }
-  } else {
+  }
+  if (!small) {
     const KeyStats gst = gain_stats(c, n, st.moves.get(), st.gains.get());
     st.V = (uint32_t)gst.count;
     if (chainup) rank_by_gain(c, n, st.moves.get(), st.gains.get(), gst, st.ranks.get());
@@ -4083,7 +4079,10 @@ bool try_analyze_round(Ctx& c, const RefineLevel& L, int mode, uint32_t omega, u
       else HGP_LAUNCH((k_round_small<IT, false>), 1, BLOCK_SORT_THREADS, 0, c, ea);
     });
     const RoundOut o = read_scalar(c, out.get());
-    if (o.info.wide) return false;
+    if (o.info.wide) {
+      Y.wide = true;
+      return false;
+    }
     st.V = o.info.V;
     st.best = o.best;
     return true;
@@ -4155,8 +4154,22 @@ bool try_analyze_round(Ctx& c, const RefineLevel& L, int mode, uint32_t omega, u
 void analyze_round(Ctx& c, const RefineLevel& L, int mode, uint32_t omega, uint32_t delta, uint32_t R, uint32_t rep,
                    bool chainup, const uint32_t* part, const uint32_t* psizes, RoundState& st,
                    LevelLayout* layout = nullptr) {
-  if (!try_analyze_round(c, L, mode, omega, delta, R, rep, chainup, part, psizes, st, layout, true))
-    (void)try_analyze_round(c, L, mode, omega, delta, R, rep, chainup, part, psizes, st, layout, false);
+  const uint32_t n = L.n;
+  const bool incc = mode == HGP_MODE_INCC;
+  PartitionLists pl;
+  build_partition_lists(c, L, part, pl, incc, layout, !incc && L.k <= MASK_K);
+  st.moves = DBuf<uint32_t>(c, n);
+  st.gains = DBuf<int64_t>(c, n);
+  st.ranks = DBuf<uint32_t>(c, n);
+  compute_gains(c, L, pl, mode, omega, rep, discount_of(rep, R), part, psizes, st.moves.get(), st.gains.get());
+  LevelLayout own_layout;
+  LevelLayout& Y = layout ? *layout : own_layout;
+  if (!Y.sized) {
+    Y.sized = true;
+    Y.max_size = n ? reduce_max_u32(c, L.sizes, n) : 0u;
+  }
+  if (!rank_round(c, L, mode, omega, delta, chainup, part, psizes, pl, st, Y))
+    (void)rank_round(c, L, mode, omega, delta, chainup, part, psizes, pl, st, Y);
 }
 
 }  // namespace

@@ -713,6 +713,76 @@ def test_refine_analyze_inbound_few_ranks(dev, movers, rng):
             assert got["best"] == exp["best"]
 
 
+# (mode, n, k, chainup, hedges of each hub, where the keys are too wide).  By table a key is 13 bits of
+# position, the partition and validity, and the range of the gains; by gain it holds no partition.
+WIDE_CASES = [
+    (1, 4000, 1000, False, 20000, "moves"),   # up to 4,096 nodes: found out after the round's last kernel
+    (0, 4000, 1000, False, 20000, "moves"),
+    (1, 8000, 1000, False, 20000, "moves"),   # above: found out before the cascade
+    (0, 8000, 1000, False, 20000, "moves"),
+    (1, 4000, 4, True, 270000, "moves"),
+    (0, 8000, 4, True, 270000, "moves"),
+    (1, 4000, 2, False, 110000, "chains"),    # every move fits, the sum of a chain's gains does not
+    (1, 8000, 2, False, 110000, "chains"),
+]
+
+
+def wide_level(n, k, e, rng):
+    """Hub 0, in partition 0, shares heavy hedges of two pins with nodes of partition 1, and hub 1 the
+    other way round, so each gains them all; a few hedges of the smallest weight leave the gains
+    without common trailing zeros."""
+    part = rng.integers(0, k, size=n).astype(np.uint32)
+    part[:2] = [0, 1]
+    a, b = 2 + np.flatnonzero(part[2:] == 1), 2 + np.flatnonzero(part[2:] == 0)
+    pairs = np.concatenate([np.stack([np.zeros(e, np.int64), rng.choice(a, e)], 1),
+                            np.stack([np.ones(e, np.int64), rng.choice(b, e)], 1),
+                            rng.permutation(np.arange(2, n))[:200].reshape(100, 2)])
+    w = np.concatenate([16383 - rng.random(2 * e), np.full(100, 2.0 ** -18)]).astype(np.float32)
+    hg = O.HG(n, 2 * np.arange(len(w) + 1).astype(np.uint64), pairs.ravel().astype(np.uint32), np.zeros(len(w), np.uint32), w)
+    sizes = rng.integers(1, 3, size=n).astype(np.uint32)
+    sizes[:2] = 1
+    return hg, sizes, part, np.bincount(part, weights=sizes, minlength=k).astype(np.uint32)
+
+
+def range_bits(gains):
+    """Bits of the range of the gains above the trailing zeros that all share."""
+    low = int(np.bitwise_or.reduce(gains))
+    return ((int(gains.max()) - int(gains.min())) // (low & -low)).bit_length()
+
+
+@pytest.mark.parametrize("mode,n,k,chainup,e,where", WIDE_CASES)
+def test_refine_analyze_wide_keys_on_small_levels(dev, mode, n, k, chainup, e, where, rng):
+    """Levels of up to 8,192 nodes whose keys do not fit the one-workgroup ranking are ranked
+    device-wide instead, within the same round."""
+    hg, sizes, part, psizes = wide_level(n, k, e, rng)
+    omega = int(psizes.max()) + 2
+    L = G.Level(dev, hg)
+    L.build_touching()
+    exp = O.refine_analyze(mode, omega, 2**31 - 1, 16, hg, *O.touching(hg), sizes, k, 0, chainup, part, psizes)
+    gains = exp["gains"][exp["moves"] != 2**32 - 1]
+    bits = range_bits(gains) + 13 + (1 if chainup else (2 * k - 1).bit_length())
+    assert (bits > 64) == (where == "moves")
+    if where == "chains":
+        assert int(exp["ranks"][1]) == int(exp["ranks"][0]) + 1 or int(exp["ranks"][0]) == int(exp["ranks"][1]) + 1
+        assert (int(exp["gains"][0]) + int(exp["gains"][1]) - int(gains.min())).bit_length() + 2 + 13 > 64
+    got = G.refine_analyze(dev, L, sizes, k, mode, omega, 2**31 - 1, 16, 0, chainup, part, psizes)
+    for key in ("moves", "gains", "ranks", "seq", "sv", "iv"):
+        assert np.array_equal(got[key], exp[key]), f"{key} differs"
+    assert got["best"] == exp["best"]
+
+
+@pytest.mark.parametrize("mode,n,k,chainup,e,where", [c for c in WIDE_CASES if not c[3]])
+def test_refine_loop_wide_keys_on_small_levels(dev, mode, n, k, chainup, e, where, rng):
+    """All rounds of such a level, whose layout is kept from round to round."""
+    hg, sizes, part, psizes = wide_level(n, k, e, rng)
+    omega = int(psizes.max()) + 2
+    L = G.Level(dev, hg)
+    L.build_touching()
+    gp, gps, gpin = G.refine(dev, L, sizes, k, mode, omega, 2**31 - 1, 16, True, part, psizes)
+    ep, eps_, epin = O.refine(mode, omega, 2**31 - 1, 16, hg, *O.touching(hg), sizes, k, True, part, psizes)
+    assert np.array_equal(gp, ep) and np.array_equal(gps, eps_) and np.array_equal(gpin, epin)
+
+
 @pytest.mark.parametrize("rc", REFINE_CASES, ids=[r[0] for r in REFINE_CASES])
 def test_refine_loop(dev, rc, rng):
     name, mode, k, case_name = rc
