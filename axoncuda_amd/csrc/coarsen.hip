@@ -653,7 +653,8 @@ __device__ __forceinline__ bool cand_block_node(uint32_t u, uint32_t cap, bool d
     if (GMEM) __threadfence();
     __syncthreads();
     auto hvf = [&](uint32_t e, uint32_t len) { return make_uint2(fixed_weight(w[e]) / len, INTER ? srcc[e] : 0u); };
-    wave_visit_pins_hv_until<PIPE, NW == 16>(tch, a, b, hoff, hedges, hvf, [&](const PinVisitHV& pv) {
+    constexpr uint32_t LONG = NW != 16 ? 0 : OPT ? LONG_HEDGE_OPT : LONG_HEDGE;
+    wave_visit_pins_hv_until<PIPE, LONG>(tch, a, b, hoff, hedges, hvf, [&](const PinVisitHV& pv) {
       if (!pv.act || pv.pin == u) return;
       if (CH > 1 && pv.pin % CH != (uint32_t)chunk) return;
       const uint32_t contrib = pv.hv.x;  // floor(W / |e|), computed once per touching hedge

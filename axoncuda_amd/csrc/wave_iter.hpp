@@ -192,16 +192,19 @@ __device__ __forceinline__ void wave_visit_pins_until(const uint32_t* __restrict
 // The same traversal with two per-hedge values computed once per touching hedge by the lane
 // that loads it, `hvf(e, len)`, and handed to every visit of that hedge's pins in `hv`.  With
 // PIPE the next step's pin is loading while the current step is visited (one more step's
-// registers live across the visit).  With LONG, a chunk of hedges of LONG_HEDGE pins on average goes
-// hedge by hedge instead: finding owners and fetching their fields is some 60 of a step's 80 vector
-// instructions, which bound the traversal, against part-filled steps at the hedges' ends.
-// k_cand_direct on 257-pin hedges 2.65 -> 2.44 ms; hedges of 65 pins, two steps for one, lose (253 ->
-// 353 us), so they stay below the line.
-constexpr uint32_t LONG_HEDGE = 128, LONG_STEPS = 4;
+// registers live across the visit).  With LONG, a chunk of hedges of LONG pins on average goes hedge by
+// hedge instead: finding owners and fetching their fields is some 60 of a step's 80 vector instructions,
+// which bound the traversal, against part-filled steps at the hedges' ends.  k_cand_direct on 257-pin
+// hedges 2.65 -> 2.44 ms; hedges of 65 pins, two steps for one, lose (253 -> 353 us).  Where the line
+// lies between them, on levels of hedges of one length (whole calls, shared steps and hedge by hedge):
+// at 129 pins, three steps for two, the direct tier is still ahead (2,127 us at 120 pins, 1,679 at 129)
+// and the hashed tiers alike, while the optimistic tier loses from 132 to 144 pins (29.6 -> 30.4 ms at
+// 135), is even at 150 and ahead from 160 on (28.9 -> 28.4, at 193 29.7 -> 27.9).
+constexpr uint32_t LONG_HEDGE = 128, LONG_HEDGE_OPT = 160, LONG_STEPS = 4;
 struct PinVisitHV : PinVisit {
   uint2 hv;
 };
-template <bool PIPE = true, bool LONG = false, typename H, typename F, typename S>
+template <bool PIPE = true, uint32_t LONG = 0, typename H, typename F, typename S>
 __device__ __forceinline__ void wave_visit_pins_hv_until(const uint32_t* __restrict__ tch, uint64_t t0, uint64_t t1,
                                                          const uint64_t* __restrict__ hoff,
                                                          const uint32_t* __restrict__ hedges, H&& hvf, F&& visit,
@@ -220,7 +223,7 @@ __device__ __forceinline__ void wave_visit_pins_hv_until(const uint32_t* __restr
       hv = hvf(e, len);
     }
     const uint32_t m = (uint32_t)min((uint64_t)64, t1 - jb);
-    if (LONG && wave_sum((uint64_t)len) >= (uint64_t)LONG_HEDGE * m) {
+    if (LONG && wave_sum((uint64_t)len) >= (uint64_t)LONG * m) {
       // long hedges, one after the other: the hedge is uniform, so a step is a load and the visit.
       // LONG_STEPS of the next hedge's loads are on their way during the visits of the current one.
       struct Part {

@@ -160,6 +160,30 @@ def test_candidates_long_hedges(dev, short, rng):
         assert np.array_equal(pairs, ep) and np.array_equal(scores, es), delta
 
 
+@pytest.mark.parametrize("delta", [2**31 - 1, 40])
+def test_candidates_long_hedges_optimistic(dev, delta, rng):
+    """Nodes whose tables are tried in LDS, with 1,024 touching hedges (64 a wave) of one length on
+    either side of the line to the hedge-by-hedge traversal, and one hub with hedges of all of them."""
+    n, lens = 50000, [128, 144, 159, 160, 161, 193]
+    off, pins = [0], []
+    for h, ln in enumerate(lens):
+        pool = rng.choice(np.arange(10, n), size=4000, replace=False)  # distinct neighbours that fit
+        for i in range(1024):
+            row = np.concatenate([[h], [7] * (i % 16 == 0), rng.choice(pool, size=ln, replace=False)])[:ln]
+            pins.extend(int(x) for x in rng.permutation(row))
+            off.append(len(pins))
+    e = len(off) - 1
+    hg = O.HG(n, np.array(off, np.uint64), np.array(pins, np.uint32), np.arange(e).astype(np.uint32) % 2,
+              rng.random(e).astype(np.float32))
+    L = G.Level(dev, hg)
+    L.build_touching()
+    ro, rt, ri = O.touching(hg)
+    sizes = rng.integers(1, 3, size=n).astype(np.uint32)
+    pairs, scores, *_ = G.candidates(dev, L, sizes, 16, 6, delta)
+    ep, es = O.candidates(hg, ro, rt, ri, sizes, 16, 6, delta)
+    assert np.array_equal(pairs, ep) and np.array_equal(scores, es)
+
+
 def hub_graph(n, hubs, n_small, rng):
     """Hub nodes, each on `count` hedges of `size` pins drawn from a pool of `pool` nodes, so
     their visit bounds (and worst-case tables) are far above their distinct neighbours."""
