@@ -495,7 +495,7 @@ constexpr uint32_t TIERS = 9;
 constexpr uint32_t TIER_WAVES = 1024;  // runs of nodes at most
 
 __global__ void k_cand_tiers(const uint64_t* __restrict__ bound, uint32_t n, uint32_t run, uint32_t direct_n,
-                             uint32_t big8_cap, uint32_t big_cap, uint8_t* __restrict__ tier,
+                             uint64_t direct_visits, uint32_t big8_cap, uint32_t big_cap, uint8_t* __restrict__ tier,
                              uint32_t* __restrict__ cap, uint32_t* __restrict__ counts) {
   const uint32_t w = blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64, waves = gridDim.x * (blockDim.x / 64);
   const uint64_t first = (uint64_t)w * run;
@@ -513,7 +513,7 @@ __global__ void k_cand_tiers(const uint64_t* __restrict__ bound, uint32_t n, uin
       else if (c <= CAND_MED_CAP) t = 4;
       else if (c <= big8_cap) t = 5;
       else if (c <= big_cap) t = 6;  // hashed, on any level
-      else if (n <= direct_n && b < 1ull << 31) t = 7;  // PACKED counts in 31 bits
+      else if (n <= direct_n && b <= direct_visits) t = 7;
       else t = 8;
       tier[v] = (uint8_t)t;
       // indexed by node id: the direct tier, and heavy nodes whose table would not be smaller than n;
@@ -1263,8 +1263,10 @@ void candidates(Ctx& c, const uint32_t* hedges, const uint64_t* hoff, const uint
   const uint32_t tg = ceil_div(ceil_div(n, run), 4);
   DBuf<uint8_t> tier(c, n);
   DBuf<uint32_t> lists(c, n), tcount(c, TIERS * 4 * tg), total(c, TIERS);
-  HGP_LAUNCH(k_cand_tiers, tg, 256, 0, c, bound.get(), n, run, direct_n, big8_cap, big_cap, tier.get(), caps.get(),
-             tcount.get());
+  // the direct tier's packed words hold the shared-inbound counts in 31 bits
+  const uint64_t direct_visits = inter ? (1ull << 31) - 1 : ~0ull;
+  HGP_LAUNCH(k_cand_tiers, tg, 256, 0, c, bound.get(), n, run, direct_n, direct_visits, big8_cap, big_cap, tier.get(),
+             caps.get(), tcount.get());
   HGP_LAUNCH(k_tier_sums, 1, BLOCK_SORT_THREADS, 0, c, tcount.get(), 4 * tg, total.get());
   HGP_LAUNCH(k_split_tiers, tg, 256, 0, c, tier.get(), tcount.get(), n, run, lists.get());
   struct TierCounts {

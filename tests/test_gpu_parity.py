@@ -184,6 +184,27 @@ def test_candidates_long_hedges_optimistic(dev, delta, rng):
     assert np.array_equal(pairs, ep) and np.array_equal(scores, es)
 
 
+@pytest.mark.parametrize("delta", [2**31 - 1, 1])
+def test_candidates_of_two_billion_visits(dev, delta, rng):
+    """A node of more than 2^31 visits on a level indexed by node id: its incidence list names one hedge
+    of all nodes over and over (the stage takes the list as it is), with and without shared-inbound counts."""
+    n, times = 16384, 131100
+    assert times * (n - 1) >= 1 << 31
+    hg = O.HG(n, np.array([0, n], np.uint64), rng.permutation(n).astype(np.uint32), np.ones(1, np.uint32),
+              np.array([0.8], np.float32))
+    L = G.Level(dev, hg)
+    toff = np.full(n + 1, times, np.uint64)
+    toff[0] = 0
+    tch, inb = np.zeros(times, np.uint32), np.zeros(n, np.uint32)
+    L.tch, L.toff, L.inb = (dev.upload(x) for x in (tch, toff, inb))
+    sizes = rng.integers(1, 3, size=n).astype(np.uint32)
+    print(f"case: {times * (n - 1)} visits, delta {delta}", flush=True)
+    pairs, scores, *_ = G.candidates(dev, L, sizes, 4, 3, delta)
+    ep, es = O.candidates(hg, toff, tch, inb, sizes, 4, 3, delta)
+    assert ep[0] != 2**32 - 1
+    assert np.array_equal(pairs, ep) and np.array_equal(scores, es)
+
+
 def hub_graph(n, hubs, n_small, rng):
     """Hub nodes, each on `count` hedges of `size` pins drawn from a pool of `pool` nodes, so
     their visit bounds (and worst-case tables) are far above their distinct neighbours."""
