@@ -5,7 +5,7 @@
 // Each knob of Ctx::tune changes speed only (every stage returns the same result under any
 // valid setting), so the tuner times the candidates of each knob on synthetic inputs built on
 // the device and keeps the fastest:
-//   * radix-sort tile (keys per workgroup = 256 x rounds) for each size class 2^15 .. 2^max;
+//   * radix-sort tile (256 x 2, 4, 8 or 16 keys) for each size class 2^15 .. 2^max;
 //   * the key-count at which scans switch from the single-pass look-back to three passes;
 //   * workgroup size of the thread-per-hedge cascade (64 .. 1024);
 //   * size and fill limit (occupancy) of the heavy candidate nodes' first-attempt HBM hash
@@ -115,7 +115,7 @@ void tune_sorts(Ctx& c, uint32_t max_log2) {
     const uint64_t n = 1ull << cls;
     uint32_t best_r = 0;
     float best = 1e30f;
-    for (uint32_t r = 1; r <= 16; r *= 2) {
+    for (uint32_t r = 2; r <= 16; r *= 2) {  // the settings that differ (see rs_items)
       c.tune.sort_rounds[cls] = r;
       const float ms = t.best_of(
           [&] {
@@ -126,7 +126,7 @@ void tune_sorts(Ctx& c, uint32_t max_log2) {
       if (ms < best) best = ms, best_r = r;
     }
     c.tune.sort_rounds[cls] = best_r;
-    if (c.verbose >= 2) fprintf(stderr, "  tune: sort of 2^%u keys: %u rounds per tile (%.3f ms)\n", cls, best_r, best);
+    if (c.verbose >= 2) fprintf(stderr, "  tune: sort of 2^%u keys: tiles of 256 x %u keys (%.3f ms)\n", cls, best_r, best);
   }
 }
 

@@ -75,7 +75,7 @@ def test_autotune_picks_values_in_range(dev):
         got = tuning(dev)
         assert got.as_dict() == out.as_dict()
         assert out.tuned == 1
-        assert all(out.sort_rounds[c] in (1, 2, 4, 8, 16) for c in range(15, 21))
+        assert all(out.sort_rounds[c] in (2, 4, 8, 16) for c in range(15, 21))
         assert out.cascade_block in (64, 128, 256, 512, 1024)
         assert out.heavy_table_slots in (1 << 15, 1 << 16, 1 << 17, 1 << 18)
         assert out.heavy_table_fill16 in (10, 12, 14)
