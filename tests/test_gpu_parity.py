@@ -509,7 +509,7 @@ def test_sorts_by_size(dev, p, n, rng):
     (0, 300, 1.0, True),
     (0, 4096, 0.37, False),        # the largest partition order ranked by counting
     (0, 4097, 0.37, False),        # ... and the smallest sorted one
-    (0, 1 << 19, 16000.0, False),  # gain and partition bits together above 64: two sorts
+    (0, 1 << 19, 16000.0, False),  # 64-bit keys (two sorts: test_refine_analyze_two_sorts)
     (0, 1 << 19, 16000.0, True),
 ])
 def test_refine_analyze_move_keys(dev, mode, k, scale, chainup, rng):
@@ -533,8 +533,8 @@ def test_refine_analyze_move_keys(dev, mode, k, scale, chainup, rng):
     got = G.refine_analyze(dev, L, sizes, k, mode, omega, delta, 16, 0, chainup, part, psizes)
     exp = O.refine_analyze(mode, omega, delta, 16, hg, ro, rt, ri, sizes, k, 0, chainup, part, psizes)
     if heavy:
-        g = exp["gains"][exp["moves"] != 2**32 - 1]
-        assert (int(g.max()) - int(g.min())).bit_length() + 20 > 64, "the case must need two sorts"
+        bits = range_bits(exp["gains"][exp["moves"] != 2**32 - 1]) + (1 if chainup else (2 * k - 1).bit_length())
+        assert 32 < bits <= 64, "the case must need a 64-bit key"
     for key in ("moves", "gains", "ranks", "seq", "sv", "iv"):
         assert np.array_equal(got[key], exp[key]), f"{key} differs"
     assert got["best"] == exp["best"]
@@ -776,7 +776,7 @@ def wide_level(n, k, e, rng):
     """Hub 0, in partition 0, shares heavy hedges of two pins with nodes of partition 1, and hub 1 the
     other way round, so each gains them all; a few hedges of the smallest weight leave the gains
     without common trailing zeros."""
-    part = rng.integers(0, k, size=n).astype(np.uint32)
+    part = rng.integers(0, min(k, 1000), size=n).astype(np.uint32)
     part[:2] = [0, 1]
     a, b = 2 + np.flatnonzero(part[2:] == 1), 2 + np.flatnonzero(part[2:] == 0)
     pairs = np.concatenate([np.stack([np.zeros(e, np.int64), rng.choice(a, e)], 1),
@@ -811,6 +811,22 @@ def test_refine_analyze_wide_keys_on_small_levels(dev, mode, n, k, chainup, e, w
         assert int(exp["ranks"][1]) == int(exp["ranks"][0]) + 1 or int(exp["ranks"][0]) == int(exp["ranks"][1]) + 1
         assert (int(exp["gains"][0]) + int(exp["gains"][1]) - int(gains.min())).bit_length() + 2 + 13 > 64
     got = G.refine_analyze(dev, L, sizes, k, mode, omega, 2**31 - 1, 16, 0, chainup, part, psizes)
+    for key in ("moves", "gains", "ranks", "seq", "sv", "iv"):
+        assert np.array_equal(got[key], exp[key]), f"{key} differs"
+    assert got["best"] == exp["best"]
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+def test_refine_analyze_two_sorts(dev, mode, rng):
+    """Gain and partition bits together above 64: the device-wide ranking sorts by gain, then by partition."""
+    n, k = 4000, 1 << 19
+    hg, sizes, part, psizes = wide_level(n, k, 20000, rng)
+    omega = int(psizes.max()) + 2
+    L = G.Level(dev, hg)
+    L.build_touching()
+    exp = O.refine_analyze(mode, omega, 2**31 - 1, 16, hg, *O.touching(hg), sizes, k, 0, False, part, psizes)
+    assert range_bits(exp["gains"][exp["moves"] != 2**32 - 1]) + (2 * k - 1).bit_length() > 64
+    got = G.refine_analyze(dev, L, sizes, k, mode, omega, 2**31 - 1, 16, 0, False, part, psizes)
     for key in ("moves", "gains", "ranks", "seq", "sv", "iv"):
         assert np.array_equal(got[key], exp[key]), f"{key} differs"
     assert got["best"] == exp["best"]

@@ -50,19 +50,21 @@ def test_incc_pipeline_matches_oracle(dev, ipm, rng):
 
 
 @pytest.mark.parametrize("budget", [1, 40000])
-def test_incc_inbound_events_in_partition_ranges(dev, budget, rng):
-    """An event budget far below what a round's inbound-set events need splits them into
-    ranges of partitions (one partition per range at a budget of one byte) processed one
-    after the other: the partition is still the oracle's."""
+def test_incc_event_budget_is_without_effect(dev, budget, rng):
+    """refine_event_budget is accepted and bounds nothing (the inbound-set events take a fixed number
+    of bytes per move): the partition is the oracle's and that of the default budget, and so is
+    the peak of device memory."""
     n, off, pins, srcc, w = gen.snn_like(6, 800, 12, rng)
     prod, orc = hg_pair(n, off, pins, srcc, w)
     omega, delta, maxp = 64, 600, 4800
     prm = G.params(H.HGP_MODE_INCC, omega, delta, maxp)
+    base, base_st = G.partition(dev, prod, prm)
     prm.refine_event_budget = budget
     print(f"case: INCC pipeline event budget {budget}", flush=True)
-    part, _ = G.partition(dev, prod, prm)
+    part, st = G.partition(dev, prod, prm)
     exp, _ = O.partition(orc, 0, omega, delta, maxp)
-    assert np.array_equal(part, exp)
+    assert np.array_equal(part, exp) and np.array_equal(part, base)
+    assert st.peak_device_bytes == base_st.peak_device_bytes
 
 
 def test_pipeline_deterministic(dev, rng):

@@ -24,7 +24,7 @@ def extremes():
     """(name, setter) pairs of valid but far-from-default settings."""
     def small(t):
         for i in range(40):
-            t.sort_rounds[i] = 1
+            t.sort_rounds[i] = 2  # the smallest tile (1 is taken as 2)
         t.cascade_block = 64
         t.heavy_table_slots = 1 << 13
         t.heavy_table_fill16 = 4
@@ -32,8 +32,6 @@ def extremes():
         t.mask_wide4_degree = 0  # every level's mask gains 16 waves per node
         t.mask_wide16_degree = 0
         t.side_streams = 0
-        t.coop_max_n = 1 << 22  # every sort above 16 K keys in one launch of 64 workgroups
-        t.coop_tile = 256
 
     def large(t):
         for i in range(40):
@@ -45,7 +43,6 @@ def extremes():
         t.mask_wide4_degree = 1 << 31  # a wave per node on every level
         t.mask_wide16_degree = 1 << 31
         t.side_streams = 3
-        t.coop_max_n = 0  # no sort in one launch
 
     def four_waves(t):
         t.mask_wide4_degree = 0  # 4 waves per node on every level
