@@ -844,6 +844,34 @@ def test_refine_loop_wide_keys_on_small_levels(dev, mode, n, k, chainup, e, wher
     assert np.array_equal(gp, ep) and np.array_equal(gps, eps_) and np.array_equal(gpin, epin)
 
 
+@pytest.mark.parametrize("mode", [0, 1])
+def test_refine_analyze_above_the_prefix_tiles(dev, mode, rng):
+    """More ranks than the tiles of the prefix sums hold (4,096 of 4,096): single scans and a sweep for
+    the best prefix.  A million hedges among a few thousand of the nodes and all of them."""
+    n, e, k = 4096 * 4096 + 5000, 1_000_000, 2
+    pins = rng.integers(0, n, size=3 * e).astype(np.uint32)
+    pins[rng.random(3 * e) < 0.5] %= 4000
+    hg = O.HG(n, 3 * np.arange(e + 1).astype(np.uint64), pins, (np.arange(e) % 2).astype(np.uint32),
+              (rng.random(e) + 0.5).astype(np.float32))
+    hg = O.dedup(hg)
+    sizes = np.ones(n, np.uint32)
+    part = rng.integers(0, k, size=n).astype(np.uint32)
+    psizes = np.bincount(part, minlength=k).astype(np.uint32)
+    omega = int(psizes.max()) + 2
+    delta = int(O.inbound_sizes(hg, part, k).max()) - 1 if mode == 0 else 2**31 - 1
+    print(f"case: {n} ranks, mode {mode}", flush=True)
+    exp = O.refine_analyze(mode, omega, delta, 16, hg, *O.touching(hg), sizes, k, 0, True, part, psizes)
+    assert int((exp["moves"] != 2**32 - 1).sum()) > 4096 * 4096
+    L = G.Level(dev, hg)
+    L.build_touching()
+    got = G.refine_analyze(dev, L, sizes, k, mode, omega, delta, 16, 0, True, part, psizes)
+    for key in ("moves", "gains", "ranks", "seq", "sv", "iv"):
+        assert np.array_equal(got[key], exp[key]), f"{key} differs"
+    assert got["best"] == exp["best"]
+    for x in (L.pins, L.off, L.srcc, L.w, L.tch, L.toff, L.inb):
+        dev.free(x)
+
+
 @pytest.mark.parametrize("rc", REFINE_CASES, ids=[r[0] for r in REFINE_CASES])
 def test_refine_loop(dev, rc, rng):
     name, mode, k, case_name = rc
