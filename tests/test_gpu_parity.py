@@ -604,6 +604,38 @@ def test_refine_analyze_inbound_by_hedge_size(dev, k, dup, rng):
     assert dup or got["best"] == exp["best"]
 
 
+@pytest.mark.parametrize("dup", [False, True])
+@pytest.mark.parametrize("mode,k", [(0, 6), (1, 6), (0, 66000), (1, 66000)])
+def test_refine_analyze_long_hedges(dev, mode, k, dup, rng):
+    """Hedges cascaded by comparing all pins, at the edges of the LDS copy of the pins: sources from none
+    to all, and (not deduplicated) nodes listed twice as destinations and as source and destination."""
+    n, off, pins, srcc = 6000, [0], [], []
+    for i, ln in enumerate([1025, 1026, 1500, 2047, 2048, 2049, 2050, 3001] * 3):
+        nodes = list(rng.choice(n, size=ln, replace=False))
+        ns = [0, 1, 3, ln // 2, ln - 1, ln][i % 6]
+        if dup and 0 < ns < ln - 5:
+            nodes[-1], nodes[-2] = nodes[0], nodes[-3]
+        pins.extend(int(x) for x in nodes)
+        off.append(len(pins))
+        srcc.append(ns)
+    e = len(srcc)
+    hg = O.HG(n, np.array(off, np.uint64), np.array(pins, np.uint32), np.array(srcc, np.uint32),
+              (rng.random(e) + 0.5).astype(np.float32))
+    sizes = rng.integers(1, 3, size=n).astype(np.uint32)
+    part = rng.integers(0, min(k, 300), size=n).astype(np.uint32)
+    psizes = np.bincount(part, weights=sizes, minlength=k).astype(np.uint32)
+    omega = int(psizes.max()) + 3
+    delta = 2**31 - 1 if mode else max(1, int(O.inbound_sizes(hg, part, k).max()) - 1)
+    L = G.Level(dev, hg)
+    L.build_touching()
+    got = G.refine_analyze(dev, L, sizes, k, mode, omega, delta, 16, 0, True, part, psizes)
+    exp = O.refine_analyze(mode, omega, delta, 16, hg, *O.touching(hg), sizes, k, 0, True, part, psizes)
+    # (a node listed twice: see test_refine_analyze_inbound_by_hedge_size)
+    for key in ("moves", "gains", "ranks", "sv", "iv") + (() if dup else ("seq",)):
+        assert np.array_equal(got[key], exp[key]), f"{key} differs"
+    assert dup or got["best"] == exp["best"]
+
+
 @pytest.mark.parametrize("k", [40, 66000])
 def test_refine_analyze_source_counts_above_the_length(dev, k, rng):
     """A source count above the hedge's length (the stages take device arrays as they are) makes all
