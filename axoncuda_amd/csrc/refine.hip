@@ -32,6 +32,10 @@ constexpr uint32_t PP_SMALL = 16;
 constexpr uint32_t PP_WAVE = 256;       // pins of a hedge whose list a wave sorts in registers
 constexpr uint32_t PP_REPLICAS = 64;    // copies of the inbound sizes that the list kernels add to (at most)
 constexpr uint32_t PP_REPLICA_CAP = 16384;  // ... and their counters together
+// levels of up to so many hedges, and of so many above PP_SMALL pins, add to one copy: clearing and
+// summing copies are launches of their own (inbound sizes of 250 to 7,500 hedges 50 to 56 us with
+// copies, 47 to 52 without; from 75,000 hedges on, or with 3,500 hedges of 300 pins, 240 without and 99 with)
+constexpr uint32_t PP_ONE_COPY = 65536, PP_ONE_COPY_LARGE = 256;
 constexpr uint32_t PP_HIST_CAP = 8192;  // partitions whose inbound counts aggregate in LDS
 constexpr uint32_t PP_LDS_CAP = 4096;  // 3 x 16 KiB of dynamic LDS per wave
 constexpr uint32_t GAIN_CAP = 1024;
@@ -65,8 +69,9 @@ __global__ void __launch_bounds__(256) k_pp_small(const uint32_t* __restrict__ h
                                                   const uint32_t* __restrict__ srcc, const uint32_t* __restrict__ part,
                                                   const float* __restrict__ w, uint32_t E, uint2* __restrict__ pp,
                                                   uint32_t* __restrict__ lambda,
-                                                  uint4* __restrict__ hinfo, uint32_t* __restrict__ large_flag,
-                                                  uint32_t* inbsz, uint32_t k_lds, uint32_t k, uint32_t replicas) {
+                                                  uint4* __restrict__ hinfo, uint64_t* __restrict__ large_flag,
+                                                  uint32_t wave_max, uint32_t* inbsz, uint32_t k_lds, uint32_t k,
+                                                  uint32_t replicas) {
   extern __shared__ uint32_t hist[];
   if (INB) inbsz += (uint64_t)(blockIdx.x & (replicas - 1)) * k;
   if (INB && k_lds) {
@@ -76,10 +81,9 @@ __global__ void __launch_bounds__(256) k_pp_small(const uint32_t* __restrict__ h
   const uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
   if (e < E) {
     const uint64_t s = hoff[e], t = hoff[e + 1];
-    if (t - s > PP_SMALL) {
-      if (large_flag) large_flag[e] = 1u;
-    } else {
-      if (large_flag) large_flag[e] = 0u;
+    // the lists of longer hedges: counted in the low word, those above wave_max pins in the high one
+    if (large_flag) large_flag[e] = t - s <= PP_SMALL ? 0ull : t - s <= wave_max ? 1ull : 1ull << 32;
+    if (t - s <= PP_SMALL) {
       const uint32_t len = (uint32_t)(t - s);
       const uint32_t sc = INB ? srcc[e] : 0u;
       // Pins and their partitions are fetched in batches of unconditional loads (indexes
@@ -249,12 +253,12 @@ __global__ void __launch_bounds__(256) k_pp_wave(const uint32_t* __restrict__ he
   }
 }
 
-// out[q] = the sum of the replicas' counters of partition q
-__global__ void k_sum_replicas(const uint32_t* __restrict__ in, uint32_t k, uint32_t replicas,
+// out[q] (+)= the sum of the replicas' counters of partition q
+__global__ void k_sum_replicas(const uint32_t* __restrict__ in, uint32_t k, uint32_t replicas, int add,
                                uint32_t* __restrict__ out) {
   const uint32_t q = blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= k) return;
-  uint32_t t = 0;
+  uint32_t t = add ? out[q] : 0u;
 #pragma unroll 16
   for (uint32_t r = 0; r < replicas; ++r) t += in[(uint64_t)r * k + q];
   out[q] = t;
@@ -371,6 +375,14 @@ __global__ void k_flag_longer(const uint32_t* __restrict__ list, uint32_t m, con
   if (i >= m) return;
   const uint32_t e = list[i];
   flag[i] = hoff[e + 1] - hoff[e] > len ? 1u : 0u;
+}
+// the hedges flagged in the low word to a[], in the high word to b[] (pos: exclusive sums of the flags)
+__global__ void k_pp_lists(const uint64_t* __restrict__ flag, const uint64_t* __restrict__ pos, uint32_t E,
+                           uint32_t* __restrict__ a, uint32_t* __restrict__ b) {
+  const uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= E || !flag[e]) return;
+  if (flag[e] == 1ull) a[(uint32_t)pos[e]] = e;
+  else b[pos[e] >> 32] = e;
 }
 // stable split of list entries: flagged ones to a[], the rest to b[]
 __global__ void k_split_list(const uint32_t* __restrict__ flag, const uint64_t* __restrict__ pos,
@@ -3531,24 +3543,36 @@ void build_partition_lists(Ctx& c, const RefineLevel& L, const uint32_t* part, P
   pl.pp = DBuf<uint2>(c, P);
   pl.hinfo = DBuf<uint4>(c, L.e);
   pl.lambda = DBuf<uint32_t>(c, L.e);
-  DBuf<uint32_t> isz;  // replicas of the inbound sizes
+  // The inbound sizes are added to one copy of the counters or, where many hedges meet on them, to
+  // replicas that are summed afterwards.
+  DBuf<uint32_t> isz;  // the replicas
   uint32_t replicas = 1;
-  if (want_inbound) {
-    const uint32_t k1 = std::max<uint32_t>(L.k, 1);
+  const uint32_t k1 = std::max<uint32_t>(L.k, 1);
+  auto add_replicas = [&] {
     while (replicas < PP_REPLICAS && 2ull * replicas * k1 <= PP_REPLICA_CAP) replicas <<= 1;
-    pl.inbsz = DBuf<uint32_t>(c, k1);
+    if (replicas == 1) return;
     isz = DBuf<uint32_t>(c, (uint64_t)replicas * k1);
     fill_u32(c, isz.get(), 0u, (uint64_t)replicas * k1);
+  };
+  auto counters = [&] { return isz.get() ? isz.get() : pl.inbsz.get(); };
+  if (want_inbound) {
+    pl.inbsz = DBuf<uint32_t>(c, k1);
+    if (L.e > PP_ONE_COPY || Y.nl + Y.nlds + Y.ng > PP_ONE_COPY_LARGE) add_replicas();
+    if (!isz.get()) fill_u32(c, pl.inbsz.get(), 0u, k1);
   }
-  DBuf<uint32_t> lflag;
-  if (!Y.ready) lflag = DBuf<uint32_t>(c, L.e);
+  const bool apart = !isz.get();  // the short hedges' counts are in inbsz itself
+  // (the wave's keys hold a partition id and a bit when the inbound sizes are wanted)
+  const uint32_t wave_max = want_inbound && L.k > 0x7FFFFFFFu ? PP_SMALL : PP_WAVE;
+  DBuf<uint64_t> lflag;
+  if (!Y.ready) lflag = DBuf<uint64_t>(c, L.e);
   if (want_inbound) {
     const uint32_t k_lds = L.k <= PP_HIST_CAP ? L.k : 0u;
     HGP_LAUNCH((k_pp_small<true>), ceil_div(L.e, 256), 256, k_lds * sizeof(uint32_t), c, L.hedges, L.hoff, L.srcc, part,
-               L.w, L.e, pl.pp.get(), pl.lambda.get(), pl.hinfo.get(), lflag.get(), isz.get(), k_lds, L.k, replicas);
+               L.w, L.e, pl.pp.get(), pl.lambda.get(), pl.hinfo.get(), lflag.get(), wave_max, counters(), k_lds, L.k,
+               replicas);
   } else {
     HGP_LAUNCH((k_pp_small<false>), ceil_div(L.e, 256), 256, 0, c, L.hedges, L.hoff, L.srcc, part, L.w, L.e,
-               pl.pp.get(), pl.lambda.get(), pl.hinfo.get(), lflag.get(), (uint32_t*)nullptr, 0u, 0u, 1u);
+               pl.pp.get(), pl.lambda.get(), pl.hinfo.get(), lflag.get(), wave_max, (uint32_t*)nullptr, 0u, 0u, 1u);
   }
   // Distinct partitions per hedge <= min(k, len).  Tables of up to PP_LDS_CAP slots sit in
   // LDS; hedges needing more (len and k both above ~2K) get HBM tables.
@@ -3558,33 +3582,28 @@ void build_partition_lists(Ctx& c, const RefineLevel& L, const uint32_t* part, P
     Y.ready = true;
     DBuf<uint64_t> pos(c, (uint64_t)L.e + 1);
     exclusive_scan(c, lflag.get(), pos.get(), L.e);
-    Y.nl = (uint32_t)read_scalar(c, pos.get() + L.e);
-    if (Y.nl) {
+    const uint64_t lists = read_scalar(c, pos.get() + L.e);
+    Y.nl = (uint32_t)lists;
+    Y.nlds = (uint32_t)(lists >> 32);
+    if (lists) {
       Y.large = DBuf<uint32_t>(c, Y.nl);
-      DBuf<uint32_t> small(c, L.e - Y.nl);
-      // k_split puts flagged (large) entries first list
-      HGP_LAUNCH(k_split, ceil_div(L.e, 256), 256, 0, c, lflag.get(), pos.get(), L.e, Y.large.get(), small.get());
-      // moves the listed hedges of more than max_len pins to a list of their own
-      auto split_longer = [&](DBuf<uint32_t>& list, uint32_t& m, uint64_t max_len, DBuf<uint32_t>& longer, uint32_t& ml) {
-        if (m == 0) return;
-        DBuf<uint32_t> flag(c, m);
-        DBuf<uint64_t> lpos(c, (uint64_t)m + 1);
-        HGP_LAUNCH(k_flag_longer, ceil_div(m, 256), 256, 0, c, list.get(), m, L.hoff, max_len, flag.get());
-        exclusive_scan(c, flag.get(), lpos.get(), m);
-        ml = (uint32_t)read_scalar(c, lpos.get() + m);
-        if (ml == 0) return;
-        DBuf<uint32_t> rest(c, m - ml);
-        longer = DBuf<uint32_t>(c, ml);
-        HGP_LAUNCH(k_split_list, ceil_div(m, 256), 256, 0, c, flag.get(), lpos.get(), list.get(), m, longer.get(),
-                   rest.get());
-        list = std::move(rest);
-        m -= ml;
-      };
-      // (the wave's keys hold a partition id and a bit when the inbound sizes are wanted)
-      const bool wide_ids = want_inbound && L.k > 0x7FFFFFFFu;
-      split_longer(Y.large, Y.nl, wide_ids ? PP_SMALL : PP_WAVE, Y.llist, Y.nlds);
-      if (L.k > lds_max_len) split_longer(Y.llist, Y.nlds, lds_max_len, Y.glist, Y.ng);
+      Y.llist = DBuf<uint32_t>(c, Y.nlds);
+      HGP_LAUNCH(k_pp_lists, ceil_div(L.e, 256), 256, 0, c, lflag.get(), pos.get(), L.e, Y.large.get(), Y.llist.get());
+    }
+    if (Y.nlds && L.k > lds_max_len) {
+      DBuf<uint32_t> gflag(c, Y.nlds);
+      DBuf<uint64_t> gpos(c, (uint64_t)Y.nlds + 1);
+      HGP_LAUNCH(k_flag_longer, ceil_div(Y.nlds, 256), 256, 0, c, Y.llist.get(), Y.nlds, L.hoff, (uint64_t)lds_max_len,
+                 gflag.get());
+      exclusive_scan(c, gflag.get(), gpos.get(), Y.nlds);
+      Y.ng = (uint32_t)read_scalar(c, gpos.get() + Y.nlds);
       if (Y.ng) {
+        DBuf<uint32_t> lds_list(c, Y.nlds - Y.ng);
+        Y.glist = DBuf<uint32_t>(c, Y.ng);
+        HGP_LAUNCH(k_split_list, ceil_div(Y.nlds, 256), 256, 0, c, gflag.get(), gpos.get(), Y.llist.get(), Y.nlds,
+                   Y.glist.get(), lds_list.get());
+        Y.llist = std::move(lds_list);
+        Y.nlds -= Y.ng;
         DBuf<uint64_t> gcap(c, Y.ng);
         Y.goff = DBuf<uint64_t>(c, (uint64_t)Y.ng + 1);
         HGP_LAUNCH(k_pp_gcap, ceil_div(Y.ng, 256), 256, 0, c, Y.glist.get(), Y.ng, L.hoff, L.k, gcap.get());
@@ -3593,23 +3612,25 @@ void build_partition_lists(Ctx& c, const RefineLevel& L, const uint32_t* part, P
       }
     }
   }
+  if (want_inbound && !isz.get() && Y.nl + Y.nlds + Y.ng > PP_ONE_COPY_LARGE) add_replicas();
   DBuf<uint32_t> gtab(c, 3 * Y.gslots);
   auto launch = [&](auto inb) {
     constexpr bool INB = decltype(inb)::value;
     if (Y.nl)
       HGP_LAUNCH((k_pp_wave<INB>), ceil_div(Y.nl, 4), 256, 0, c, L.hedges, L.hoff, L.srcc, part, L.w, Y.large.get(),
-                 Y.nl, pl.pp.get(), pl.lambda.get(), pl.hinfo.get(), isz.get(), L.k, replicas);
+                 Y.nl, pl.pp.get(), pl.lambda.get(), pl.hinfo.get(), counters(), L.k, replicas);
     if (Y.nlds)
       HGP_LAUNCH((k_pp_large<INB, false>), Y.nlds, 64, 3 * cap * sizeof(uint32_t), c, L.hedges, L.hoff, L.srcc, part,
                  L.w, Y.llist.get(), cap, L.k, (const uint64_t*)nullptr, (uint32_t*)nullptr, pl.pp.get(),
-                 pl.lambda.get(), pl.hinfo.get(), isz.get(), replicas);
+                 pl.lambda.get(), pl.hinfo.get(), counters(), replicas);
     if (Y.ng)
       HGP_LAUNCH((k_pp_large<INB, true>), Y.ng, 64, 0, c, L.hedges, L.hoff, L.srcc, part, L.w, Y.glist.get(), cap, L.k,
-                 Y.goff.get(), gtab.get(), pl.pp.get(), pl.lambda.get(), pl.hinfo.get(), isz.get(), replicas);
+                 Y.goff.get(), gtab.get(), pl.pp.get(), pl.lambda.get(), pl.hinfo.get(), counters(), replicas);
   };
   if (want_inbound) {
     launch(std::true_type{});
-    HGP_LAUNCH(k_sum_replicas, ceil_div(L.k, 256), 256, 0, c, isz.get(), L.k, replicas, pl.inbsz.get());
+    if (isz.get())
+      HGP_LAUNCH(k_sum_replicas, ceil_div(L.k, 256), 256, 0, c, isz.get(), L.k, replicas, apart ? 1 : 0, pl.inbsz.get());
   } else {
     launch(std::false_type{});
   }

@@ -568,6 +568,28 @@ def test_partition_lists_by_hedge_length(dev, k, spread, rng):
         assert km1.value == O.connectivity_fixed(hg, part)
 
 
+@pytest.mark.parametrize("short,long", [(1, 0), (200, 256), (200, 257), (65536, 0), (65537, 0), (65000, 1000), (0, 300)])
+@pytest.mark.parametrize("k", [5, 9000])
+def test_inbound_sizes_by_copies(dev, short, long, k, rng):
+    """Inbound sizes added to one copy or to several: by the number of hedges, and by that of the longer
+    ones, in registers, LDS and HBM tables, whose copies come after the short ones' counts."""
+    n = 20000
+    lens = np.concatenate([rng.integers(0, 17, size=short), np.resize([17, 64, 200, 256, 257, 600, 2500], long)])
+    lens = rng.permutation(lens).astype(np.int64)
+    off = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint64)
+    pos = np.arange(int(off[-1])) - np.repeat(off[:-1].astype(np.int64), lens)
+    pins = ((np.repeat(rng.integers(0, n, size=len(lens)), lens) + 7 * pos) % n).astype(np.uint32)
+    srcc = np.minimum(rng.integers(0, 3, size=len(lens)), lens).astype(np.uint32)
+    hg = O.HG(n, off, pins, srcc, np.ones(len(lens), np.float32))
+    part = rng.integers(0, k, size=n).astype(np.uint32)
+    L = G.Level(dev, hg)
+    d_part, d_out = dev.upload(part), dev.alloc(4 * k)
+    for _ in range(2):
+        dev.check(dev.lib.hgp_inbound_sizes(dev.ctx, G.V(L.pins), G.V(L.off), G.V(L.srcc), G.V(d_part), hg.e, k,
+                                            G.V(d_out)), "inbound sizes")
+        assert np.array_equal(dev.download(d_out, k, np.uint32), O.inbound_sizes(hg, part, k))
+
+
 @pytest.mark.parametrize("k", [5, 300, 66000])
 @pytest.mark.parametrize("dup", [False, True])
 def test_refine_analyze_inbound_by_hedge_size(dev, k, dup, rng):
