@@ -649,9 +649,12 @@ __global__ void k_iota_u32(uint32_t* p, uint64_t n) {
   uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = (uint32_t)i;
 }
-// one atomic per workgroup of at most MAX_GRID (8,192 of them, one per wave, on one address took
-// 90 us for 500,000 values)
-constexpr uint32_t MAX_GRID = 256;
+// One atomic per workgroup (8,192 of them, one per wave, on one address took 90 us for 500,000 values):
+// 256 workgroups up to 16 M values, above that one for every 65,536, since 256 keep too few loads in
+// flight for memory (connectivity of 150 M pins 4.4 ms with 2,048 workgroups, 5.1 with 256).
+inline uint32_t max_grid(uint64_t n) {
+  return (uint32_t)std::min<uint64_t>((n + 2047) / 2048, std::min<uint64_t>(std::max<uint64_t>(256, n >> 16), 2048));
+}
 template <typename T, typename A>
 __global__ void __launch_bounds__(256) k_max(const T* __restrict__ p, uint64_t n, A* out) {
   __shared__ T s_m[4];
@@ -752,15 +755,14 @@ void iota_u32(Ctx& c, uint32_t* p, uint64_t n) { HGP_LAUNCH(k_iota_u32, ceil_div
 uint32_t reduce_max_u32(Ctx& c, const uint32_t* p, uint64_t n) {
   DBuf<uint32_t> out(c, 1);
   memset_async(c, out.get(), 0, sizeof(uint32_t));
-  if (n) HGP_LAUNCH((k_max<uint32_t, uint32_t>), std::min<uint32_t>(ceil_div(n, 2048), MAX_GRID), 256, 0, c, p, n, out.get());
+  if (n) HGP_LAUNCH((k_max<uint32_t, uint32_t>), max_grid(n), 256, 0, c, p, n, out.get());
   return read_scalar(c, out.get());
 }
 
 uint64_t reduce_max_u64(Ctx& c, const uint64_t* p, uint64_t n) {
   DBuf<unsigned long long> out(c, 1);
   memset_async(c, out.get(), 0, sizeof(unsigned long long));
-  if (n) HGP_LAUNCH((k_max<uint64_t, unsigned long long>), std::min<uint32_t>(ceil_div(n, 2048), MAX_GRID), 256, 0, c, p, n,
-                    out.get());
+  if (n) HGP_LAUNCH((k_max<uint64_t, unsigned long long>), max_grid(n), 256, 0, c, p, n, out.get());
   return (uint64_t)read_scalar(c, out.get());
 }
 

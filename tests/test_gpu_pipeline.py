@@ -177,6 +177,24 @@ def test_partition_device_rejects_malformed_input(dev):
     assert b"num_nodes" in dev.lib.hgp_ctx_last_error(dev.ctx)
 
 
+@pytest.mark.parametrize("p", [2048, 2049, 600_001, 20_000_000, 150_000_000])
+def test_partition_device_finds_one_bad_pin(dev, p):
+    """The largest pin id is found wherever it is, with few and with many workgroups looking for it."""
+    n, e = 1000, p // 2
+    prm = G.params(H.HGP_MODE_KWAY, n, 2**31 - 1, 2, kway=2, eps=0.03)
+    pins = np.zeros(p, np.uint32)
+    off = np.minimum(2 * np.arange(e + 1, dtype=np.uint64), p)
+    off[-1] = p
+    bufs = [dev.upload(pins), dev.upload(off), dev.upload(np.zeros(e, np.uint32)), dev.upload(np.ones(e, np.float32))]
+    one, zero = np.array([n], np.uint32), np.zeros(1, np.uint32)
+    for at in (0, 63, p // 3, p - 2, p - 1):
+        dev.check(dev.lib.hgp_memcpy_htod(dev.ctx, C.c_void_p(bufs[0] + 4 * at), one.ctypes.data_as(C.c_void_p), 4), "copy")
+        assert partition_device(dev, prm, n, e, bufs)[0] == 1 and b"num_nodes" in dev.lib.hgp_ctx_last_error(dev.ctx)
+        dev.check(dev.lib.hgp_memcpy_htod(dev.ctx, C.c_void_p(bufs[0] + 4 * at), zero.ctypes.data_as(C.c_void_p), 4), "copy")
+    for b in bufs:
+        dev.free(b)
+
+
 def test_kway_max_parts_other_than_k_is_rejected(dev):
     hg = H.Hypergraph.generate("random", n=3000, e=3000, max_size=8, seed=4)
     n, _, _ = hg.sizes()
