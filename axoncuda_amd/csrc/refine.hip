@@ -2537,9 +2537,11 @@ __device__ __forceinline__ void cas_clear(uint32_t V) {
 // More ranks (inbound-constrained mode, up to CAS_COPY_V): a copy of the counters for each XCD
 // (workgroups go round them), so that an addition finds its line in the XCD's own L2 instead of
 // fetching it from another's; k_cascade_sum adds the copies up.  k_cascade_wave on the 65-pin hedges
-// of 8 layers of 1,156 nodes 73 -> 32 us, of 8,191 nodes 216 -> 148 us.  In k-way mode a rank is met
-// by a few hedges only, and copies changed nothing up to 262,144 ranks (183 and 181 us); above that
-// their clearing and summing is memory traffic of the size of the pins'.
+// of 8 layers of 1,156 nodes 73 -> 32 us, of 8,191 nodes 216 -> 148 us.  Above 262,144 ranks a counter
+// is met by too few workgroups at a time for its line to travel much, and clearing and summing the
+// copies eats the rest: refinement of 8 layers of 50,000 nodes, fan-out 64, 49.3 ms without and 48.3 with
+// them, of 131,072 nodes 422 and 421, with fan-out 128 785 and 788, for 128 bytes a rank.  In k-way
+// mode a rank is met by a few hedges only, and copies changed nothing (183 and 181 us).
 constexpr uint32_t CAS_COPIES = 8, CAS_COPY_V = 1u << 18;
 template <bool INCC>
 __device__ __forceinline__ void cas_own_copy(CascadeArgs& a) {

@@ -90,9 +90,11 @@ typedef struct hgp_params {
   uint32_t ip_nodes_per_part;
   uint32_t ip_refine_repeats;
   /* INCC refinement: device bytes for its inbound-set events.  Accepted and without effect: the
-   * stage takes two events per move whatever the number of inbound hedges (under 64 bytes per
-   * node), so nothing is split.  The reference sizes this stage by the moving inbound
-   * incidences, without a bound (sources/refinement.cu:307-491). */
+   * stage takes two events per move whatever the number of inbound hedges, so nothing is split.
+   * Its events (those of the sizes too) and their sort take about 72 bytes per moving node, and
+   * the copies of the cascade's counters 128 more on levels of up to 262,144 moving nodes.  The
+   * reference sizes this stage by the moving inbound incidences, without a bound
+   * (sources/refinement.cu:307-491). */
   uint64_t refine_event_budget;
 } hgp_params;
 
@@ -105,7 +107,8 @@ enum { HGP_IP_HOST = 0, HGP_IP_DEVICE = 1, HGP_IP_AUTO = 2 };
  * the same result under any valid setting. */
 typedef struct hgp_tuning {
   /* radix sorts of 2^c .. 2^(c+1) - 1 keys: keys per thread in a workgroup's tile (the tile is
-   * 256 x this many keys), 1..16, taken as the next of 2, 4, 8 and 16; 0 = the built-in rule */
+   * 256 x this many keys), 1..16, taken as the next of 2, 4, 8 and 16; 0 = the built-in rule.
+   * Sorts of up to 8,192 keys have no tiles; hgp_autotune times the classes from 2^15 on */
   uint32_t sort_rounds[40];
   /* candidate scoring of heavy nodes: slots of the first-attempt HBM hash table (a power of
    * two, 2^13..2^24) and its fill limit in sixteenths (4..14), i.e. the table occupancy that
