@@ -72,7 +72,7 @@ def test_netlist_kway_scaled(dev):
 def test_snn_incc_full_size(dev):
     """The full SNN workload: 8 layers x 131,072 neurons, fan-out 256 from a Gaussian
     receptive field (sigma 16, 363 x 363 grid), 235.8M pins, under -m 1024 4096 with -ipm
-    (about 40 s on one MI355X).  Every constraint holds, the partition count respects the
+    (about 17 s on one MI355X).  Every constraint holds, the partition count respects the
     lower bound, and the device lambda-1 equals the host metric."""
     print("case: snn 8x131072 fanout 256 (full size), ipm", flush=True)
     hg = H.Hypergraph.generate("snn", layers=8, per_layer=131072, grid=363, fanout=256, sigma=16.0, seed=1)
